@@ -9,39 +9,55 @@ namespace {
 // ---------------------------------------------------------------------------
 // Kernels: post-passes over the entry arrays (one entry per lane)
 // ---------------------------------------------------------------------------
-__global__ void __launch_bounds__(kBlock)
+// Bound by what it takes to find a slot's edge (chunk -> record -> entry) once the count
+// of what it changed is cheap: every wavefront adding its own to the one counter took 8 ns
+// a wavefront, 337 us for the 2.66 M slots of the 16-layer mixture-of-experts graph.  Two
+// workgroups of 1 024 lanes per CU stride over the slots instead and add once each: 20 us
+// (eight of 256 lanes 40 us).  Measured and not better: four slots in flight per lane, and
+// wavefronts that read the edge record through the scalar cache (20 and 20-22 us).
+constexpr int kDiscountBlocks = 256 * 2, kDiscountThreads = 1024;
+
+__global__ void __launch_bounds__(kDiscountThreads)
 prefetch_discount_kernel(apc_problem p, const double* __restrict__ per_arg, double scale,
                          double* __restrict__ comm, double* __restrict__ cost,
                          const uint8_t* __restrict__ flags, unsigned long long* n_modified) {
-  const int64_t idx = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+  __shared__ unsigned int s_mine[kDiscountThreads / 64];
   unsigned int mine = 0;
-  if (idx < p.n_slot) {
-    const apc_edge ed = find_edge(p, idx);
-    const int64_t local = idx - ed.off;
-    if (local < (int64_t)ed.ssrc * ed.sdst && (ed.flags & APC_EDGE_PREFETCHABLE) &&
-        ed.src_node >= 0) {
-      double c = comm[idx];
-      if (c > 0.0 && isfinite(c)) {
-        const uint32_t o = (uint32_t)local / (uint32_t)ed.ssrc;
-        c = c * scale;
-        comm[idx] = c;
-        cost[idx] = (c + per_arg[ed.comp_base + o]) + (double)(flags[idx] & APC_ENTRY_TRANSITION);
-        mine = 1;
-      }
+  const int64_t step = (int64_t)gridDim.x * kDiscountThreads;
+  for (int64_t idx = (int64_t)blockIdx.x * kDiscountThreads + threadIdx.x; idx < p.n_slot; idx += step) {
+    const apc_edge* ed = p.edges + p.chunk_edge[idx >> APC_CHUNK_SHIFT];
+    if (!(ed->flags & APC_EDGE_PREFETCHABLE) || ed->src_node < 0) continue;
+    const int64_t local = idx - ed->off;
+    if (local >= (int64_t)ed->ssrc * ed->sdst) continue;  // padding behind the block
+    double c = comm[idx];
+    if (c > 0.0 && isfinite(c)) {
+      const uint32_t o = (uint32_t)local / (uint32_t)ed->ssrc;
+      c = c * scale;
+      comm[idx] = c;
+      cost[idx] = (c + per_arg[ed->comp_base + o]) + (double)(flags[idx] & APC_ENTRY_TRANSITION);
+      ++mine;
     }
   }
-  // wavefront reduction, one atomic per wave
   for (int off = 32; off > 0; off >>= 1) mine += __shfl_down(mine, off, 64);
-  if ((threadIdx.x & 63) == 0 && mine) atomicAdd(n_modified, (unsigned long long)mine);
+  if ((threadIdx.x & 63) == 0) s_mine[threadIdx.x >> 6] = mine;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    unsigned int total = 0;
+#pragma unroll
+    for (int w = 0; w < kDiscountThreads / 64; ++w) total += s_mine[w];
+    if (total) atomicAdd(n_modified, (unsigned long long)total);
+  }
 }
 
+// Every slot of obj is written, the padding between blocks with zero (the caller need not
+// clear it first: 7 us of fill on the graph above).
 __global__ void __launch_bounds__(kBlock)
 objective_kernel(apc_problem p, const double* __restrict__ cost, double* __restrict__ obj) {
   const int64_t idx = (int64_t)blockIdx.x * kBlock + threadIdx.x;
   if (idx >= p.n_slot) return;
   const apc_edge ed = find_edge(p, idx);
-  if (idx - ed.off < (int64_t)ed.ssrc * ed.sdst)
-    obj[idx] = cost[idx] * (double)p.node_multiplier[ed.node];
+  const bool entry = idx - ed.off < (int64_t)ed.ssrc * ed.sdst;
+  obj[idx] = entry ? cost[idx] * (double)p.node_multiplier[ed.node] : 0.0;
 }
 
 // ---------------------------------------------------------------------------
@@ -384,8 +400,9 @@ int apc_apply_prefetch_discount(const apc_problem* p, const double* per_arg, dou
   if (!per_arg || !comm || !cost || !flags || !n_modified)
     return fail(APC_ERR_INVALID, "apc_apply_prefetch_discount: null argument%s");
   unsigned grid;
-  if (int rc = slot_grid(p, kBlock, &grid)) return rc;
-  hipLaunchKernelGGL(prefetch_discount_kernel, dim3(grid), dim3(kBlock), 0, (hipStream_t)stream,
+  if (int rc = slot_grid(p, kDiscountThreads, &grid)) return rc;
+  if (grid > kDiscountBlocks) grid = kDiscountBlocks;
+  hipLaunchKernelGGL(prefetch_discount_kernel, dim3(grid), dim3(kDiscountThreads), 0, (hipStream_t)stream,
                      *p, per_arg, scale, comm, cost, flags, n_modified);
   return check_launch("prefetch_discount_kernel");
 }

@@ -520,7 +520,9 @@ class CostEngine:
 
     def objective_coeffs(self) -> torch.Tensor:
         assert self.built
-        obj = torch.zeros_like(self.cost)
+        obj = torch.empty_like(self.cost)  # the pass writes every slot, zero between the blocks
+        if self.g.num_entries == 0:
+            return obj.zero_()
         _lib.check(
             self.lib.apc_objective_coeffs(C.byref(self.problem), self._ptr(self.cost), self._ptr(obj), self._stream()),
             "apc_objective_coeffs",

@@ -574,7 +574,8 @@ int apc_apply_prefetch_discount(const apc_problem* p, const double* per_arg, dou
                                 unsigned long long* n_modified, void* stream);
 
 /* Replaces the coefficient rule of _set_objective
- * (autoparallel/optimize_sharding.py:879-885): obj = cost * node_multiplier. */
+ * (autoparallel/optimize_sharding.py:879-885): obj = cost * node_multiplier; the
+ * slots between blocks get 0. */
 int apc_objective_coeffs(const apc_problem* p, const double* cost, double* obj, void* stream);
 
 /* Replaces _hash_node (autoparallel/graph_passes/graph_clustering.py:68-82),
