@@ -99,21 +99,6 @@ __device__ __forceinline__ double add_ones(double x, uint32_t n) {
   return x;
 }
 
-// In-order fold of one value per lane into acc: acc = (..((acc + v0) + v1)..) + v63,
-// the association a sequential loop over 64 items has.
-__device__ __forceinline__ double fold_in_order(double acc, double v) {
-  const int lo = __double2loint(v), hi = __double2hiint(v);
-#pragma unroll
-  for (int i = 0; i < 64; ++i)
-    acc += __hiloint2double(__builtin_amdgcn_readlane(hi, i), __builtin_amdgcn_readlane(lo, i));
-  return acc;
-}
-
-// Small batches: one wavefront per assignment.  Lanes take 64 consecutive
-// nodes (then 64 consecutive edges) at a time, gather their terms in parallel,
-// and the terms are folded lane by lane in order, so the sums keep the
-// reference's sequential association (bit-identical to score_kernel) while the
-// gathers of a tile overlap.
 // score_kernel<true> over a window of a larger graph: global node ids for the
 // draw, sums continued from the previous window's.
 template <bool kRandom>
@@ -701,78 +686,215 @@ int launch_table(int per, Args... args) {
   }
 }
 
-template <bool kRandom>
-__global__ void __launch_bounds__(kBlock)
-score_wave_kernel(apc_problem p, const double* __restrict__ per_arg,
+// ---------------------------------------------------------------------------
+// Small batches.  An assignment's sums are chains of dependent additions, but their
+// terms are independent: a workgroup takes 1 << kShift assignments, its first kTermLanes
+// lanes gather the terms of a tile of edges and nodes, one (edge, assignment) pair a lane
+// and kTermUnroll pairs in flight, and leave them in LDS; the wavefronts behind them add the
+// tile before up meanwhile, one lane per (sum, assignment), in node order, then argument
+// order, as score_kernel: same results, bit for bit.  Bound by the latency of three
+// dependent loads per tile (edge record, choices, entry) while the workgroups are few, by
+// the draws' hashes and the misses of the three entry arrays when they fill the chip.
+// Against one wavefront per assignment, which gathered 64 edges side by side and then added
+// them lane by lane through the whole wavefront (three chains of 64 additions a tile):
+// 2 000 assignments of the 12-layer GPT-2 graph (2 892 edges) 234 -> 53 us, 16 384 of a
+// 1 600-node window of the planner DAG 3 920 -> 1 330 us.  512 gathering lanes with four
+// pairs in flight take 10-15% longer, 256 lanes 50%.
+// ---------------------------------------------------------------------------
+constexpr int kTermLanes = 768;
+constexpr int kTermUnroll = 2;
+constexpr int kTermTile = kTermLanes * kTermUnroll;  // (edge, assignment) pairs of a tile
+constexpr int kFoldLds = 2 * kTermTile * 3 * 8;      // two tiles of three terms: 72 KB, two workgroups per CU
+
+// kShift: log2 of the assignments of a workgroup, 6 at most; at 6 a wavefront's lanes share
+// their edge and read its record through the scalar cache.
+template <bool kRandom, int kShift>
+__global__ void __launch_bounds__(kTermLanes + 192, 8)
+score_fold_kernel(apc_problem p, const double* __restrict__ per_arg,
                   const double* __restrict__ comm, const double* __restrict__ cost,
                   const uint8_t* __restrict__ flags, const uint16_t* __restrict__ assign,
                   int64_t stride, uint64_t seed, int64_t first, int64_t n_assign,
                   const int32_t* __restrict__ node_gid, int first_node, const double* __restrict__ init,
                   double* __restrict__ out) {
-  const int64_t a = (int64_t)blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6);
-  if (a >= n_assign) return;  // wave-uniform
-  const int lane = threadIdx.x & 63;
-  auto choice = [&](int v) -> uint32_t {
-    return kRandom ? mix_assignment(seed, first + a, node_gid ? node_gid[v] : v, p.node_nstrat[v])
+  constexpr int kGroup = 1 << kShift;
+  constexpr int kRows = kTermTile >> kShift;  // edges (and nodes) of a tile
+  extern __shared__ __align__(16) double s_terms[];  // [2][3][kTermTile]
+  __shared__ double s_sum[3][kGroup];
+  __shared__ uint32_t s_count[2][kGroup];  // transitions, forbidden entries
+  const int tid = threadIdx.x;
+  const bool gathers = tid < kTermLanes;  // else: adds up
+  const int fold = tid - kTermLanes;
+  const int al = (gathers ? tid : fold) & (kGroup - 1);
+  const int sum = fold >> kShift;  // of a lane that adds up: 0 compute, 1 comm, 2 objective; idle beyond
+  const int64_t a_raw = (int64_t)blockIdx.x * kGroup + al;
+  const int64_t a = a_raw < n_assign ? a_raw : n_assign - 1;  // lanes past the end repeat the last one
+  if (tid < 2 * kGroup) s_count[tid >> kShift][tid & (kGroup - 1)] = 0;
+  const int e_first = first_node < p.n_node ? p.node_edge_off[first_node] : p.n_edge;
+  const int n_edges = p.n_edge - e_first, n_nodes = p.n_node - first_node;
+  const int n_max = n_edges > n_nodes ? n_edges : n_nodes;
+  const int n_tiles = (n_max + kRows - 1) / kRows;
+  uint32_t n_trans = 0, n_forbidden = 0;
+  double acc = 0.0;
+  if (init && !gathers && sum < 3) acc = init[a * 6 + (sum == 0 ? 1 : sum == 1 ? 2 : 4)];
+  auto choice = [&](int v, int nstrat) -> uint32_t {
+    return kRandom ? mix_assignment(seed, first + a, node_gid ? node_gid[v] : v, nstrat)
                    : (uint32_t)assign[(size_t)v * stride + a];
   };
-  // a window of a larger graph: the nodes below first_node (stand-ins) contribute nothing,
-  // and the sums continue from init
-  double t_compute = 0.0, t_comm = 0.0, t_trans = 0.0, obj = 0.0, forbidden = 0.0;
-  if (init) {
-    const double* r = init + a * 6;
-    t_compute = r[1]; t_comm = r[2]; t_trans = r[3]; obj = r[4]; forbidden = r[5];
-  }
-  const int e_first = first_node < p.n_node ? p.node_edge_off[first_node] : p.n_edge;
-  for (int v0 = first_node; v0 < p.n_node; v0 += 64) {
-    const int v = v0 + lane;
-    double term = 0.0;
-    if (v < p.n_node) {
-      const int nargs = p.node_nargs[v];
-      term = per_arg[p.node_comp_off[v] + choice(v)] * (double)(nargs > 1 ? nargs : 1);
-    }
-    t_compute = fold_in_order(t_compute, term);  // + 0.0 for the lanes past the end
-  }
-  for (int e0 = e_first; e0 < p.n_edge; e0 += 64) {
-    const int e = e0 + lane;
-    double c_term = 0.0, o_term = 0.0, tr = 0.0, fb = 0.0;
-    if (e < p.n_edge) {
-      const apc_edge ed = p.edges[e];
-      const uint32_t o = choice(ed.node);
-      const uint32_t j = ed.src_node >= 0 ? choice(ed.src_node) : 0u;
-      const int64_t idx = ed.off + (int64_t)o * ed.ssrc + j;
-      const uint8_t f = flags[idx];
-      o_term = cost[idx] * (double)p.node_multiplier[ed.node];
-      fb = (double)((f & APC_ENTRY_NONFINITE) != 0);
-      if (ed.src_node >= 0) {
-        const double c = comm[idx];
-        if (isfinite(c)) c_term = c;
-        if ((ed.flags & APC_EDGE_SCORE_TRANSITION) && (f & APC_ENTRY_TRANSITION)) tr = 1.0;
+  for (int t = 0; t <= n_tiles; ++t) {
+    if (gathers) {
+      if (t < n_tiles) {
+        double* const s_t = s_terms + (t & 1) * 3 * kTermTile;
+        const int row0 = t * kRows;
+        int e[kTermUnroll], v[kTermUnroll];
+        bool live[kTermUnroll], has_src[kTermUnroll], count_trans[kTermUnroll];
+        int64_t idx[kTermUnroll];
+        int mult[kTermUnroll];
+#pragma unroll
+        for (int u = 0; u < kTermUnroll; ++u) {
+          int row = row0 + ((u * kTermLanes + tid) >> kShift);
+          if (kShift == 6) row = __builtin_amdgcn_readfirstlane(row);
+          live[u] = row < n_edges;
+          e[u] = e_first + (live[u] ? row : 0);
+          v[u] = first_node + (row < n_nodes ? row : 0);
+        }
+        // both chains of loads (edge -> choices -> entry, node -> choice -> per-arg term) are
+        // under way before either is waited for
+        double c_cost[kTermUnroll], c_comm[kTermUnroll], pa[kTermUnroll];
+        uint32_t f[kTermUnroll];
+        int nargs[kTermUnroll];
+        if (row0 < n_nodes) {
+#pragma unroll
+          for (int u = 0; u < kTermUnroll; ++u) {
+            pa[u] = per_arg[p.node_comp_off[v[u]] + choice(v[u], p.node_nstrat[v[u]])];
+            nargs[u] = p.node_nargs[v[u]];
+          }
+        }
+        if (row0 < n_edges) {
+#pragma unroll
+          for (int u = 0; u < kTermUnroll; ++u) {
+            const apc_edge* __restrict__ ed = p.edges + e[u];
+            const int src = ed->src_node, ssrc = ed->ssrc, node = ed->node;
+            has_src[u] = src >= 0;
+            count_trans[u] = has_src[u] && (ed->flags & APC_EDGE_SCORE_TRANSITION);
+            const uint32_t o = choice(node, ed->sdst);
+            const uint32_t j = has_src[u] ? choice(src, ssrc) : 0u;  // ssrc is the producer's strategy count
+            idx[u] = ed->off + (int64_t)o * ssrc + j;
+            mult[u] = p.node_multiplier[node];
+          }
+#pragma unroll
+          for (int u = 0; u < kTermUnroll; ++u) {
+            c_cost[u] = cost[idx[u]];
+            c_comm[u] = comm[idx[u]];
+            f[u] = flags[idx[u]];
+          }
+#pragma unroll
+          for (int u = 0; u < kTermUnroll; ++u) {
+            if (live[u]) {
+              n_forbidden += (f[u] & APC_ENTRY_NONFINITE) != 0;
+              n_trans += count_trans[u] && (f[u] & APC_ENTRY_TRANSITION);
+            }
+            s_t[1 * kTermTile + u * kTermLanes + tid] = has_src[u] && isfinite(c_comm[u]) ? c_comm[u] : 0.0;
+            s_t[2 * kTermTile + u * kTermLanes + tid] = c_cost[u] * (double)mult[u];
+          }
+        }
+        if (row0 < n_nodes) {
+#pragma unroll
+          for (int u = 0; u < kTermUnroll; ++u)
+            s_t[u * kTermLanes + tid] = pa[u] * (double)(nargs[u] > 1 ? nargs[u] : 1);
+        }
       }
+    } else if (t > 0 && sum < 3) {
+      const double* __restrict__ s_t = s_terms + (((t - 1) & 1) * 3 + sum) * kTermTile + al;
+      const int left = (sum == 0 ? n_nodes : n_edges) - (t - 1) * kRows;
+      const int n = left < kRows ? left : kRows;
+      // the next kAhead terms are on their way while these are added: the chain runs at the
+      // latency of an addition, not of an LDS read
+      constexpr int kAhead = 8;
+      const int whole = n / kAhead * kAhead;
+      double x[kAhead], y[kAhead];
+      if (whole > 0) {
+#pragma unroll
+        for (int i = 0; i < kAhead; ++i) x[i] = s_t[i << kShift];
+      }
+      int k = 0;
+      for (; k + 2 * kAhead <= whole; k += 2 * kAhead) {
+#pragma unroll
+        for (int i = 0; i < kAhead; ++i) y[i] = s_t[(k + kAhead + i) << kShift];
+#pragma unroll
+        for (int i = 0; i < kAhead; ++i) acc += x[i];
+        const int at = k + 2 * kAhead < whole ? k + 2 * kAhead : 0;
+#pragma unroll
+        for (int i = 0; i < kAhead; ++i) x[i] = s_t[(at + i) << kShift];
+#pragma unroll
+        for (int i = 0; i < kAhead; ++i) acc += y[i];
+      }
+      if (k < whole) {
+#pragma unroll
+        for (int i = 0; i < kAhead; ++i) acc += x[i];
+        k += kAhead;
+      }
+      for (; k < n; ++k) acc += s_t[k << kShift];
     }
-    t_comm = fold_in_order(t_comm, c_term);
-    obj = fold_in_order(obj, o_term);
-    // small integers: any order is exact; onto the carried sums as so many ones
-    for (int off = 32; off > 0; off >>= 1) {
-      tr += __shfl_xor(tr, off, 64);
-      fb += __shfl_xor(fb, off, 64);
-    }
-    t_trans = add_ones(t_trans, (uint32_t)tr);
-    forbidden = add_ones(forbidden + 0.0, (uint32_t)fb);  // a walk adds 0.0 or 1.0 per edge: a carried -0.0 loses its sign
+    __syncthreads();
   }
-  if (lane == 0) {
+  if (gathers) {
+    if (n_trans) atomicAdd(&s_count[0][al], n_trans);
+    if (n_forbidden) atomicAdd(&s_count[1][al], n_forbidden);
+  } else if (sum < 3) {
+    s_sum[sum][al] = acc;
+  }
+  __syncthreads();
+  if (tid < kGroup && a_raw < n_assign) {
+    // counts: onto the carried sums as so many ones
+    const double t_trans = add_ones(init ? init[a * 6 + 3] : 0.0, s_count[0][tid]);
+    double forbidden = init ? init[a * 6 + 5] : 0.0;
+    if (n_edges > 0) forbidden += 0.0;  // a walk adds 0.0 or 1.0 per edge: a carried -0.0 loses its sign
+    forbidden = add_ones(forbidden, s_count[1][tid]);
+    const double t_compute = s_sum[0][tid], t_comm = s_sum[1][tid];
     double* r = out + a * 6;
     r[0] = (t_compute + t_comm) + t_trans;
     r[1] = t_compute;
     r[2] = t_comm;
     r[3] = t_trans;
-    r[4] = obj;
+    r[4] = s_sum[2][tid];
     r[5] = forbidden;
   }
 }
 
-// below this many assignments one wavefront per assignment is faster than one lane
-constexpr int64_t kScoreWaveBelow = 32768;
+// below this many assignments the terms are gathered side by side, from here on a lane walks
+// the graph for its assignment
+constexpr int64_t kScoreFoldBelow = 32768;
+
+template <bool kRandom, int kShift>
+int launch_fold_k(const apc_problem& p, const double* per_arg, const double* comm, const double* cost,
+                  const uint8_t* flags, const uint16_t* assign, int64_t stride, uint64_t seed, int64_t first,
+                  int64_t n_assign, const int32_t* node_gid, int first_node, const double* init, double* out,
+                  hipStream_t stream) {
+  // dynamic LDS beyond 64 KB needs the limit raised, per kernel and device; cheap enough to do per launch
+  hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(score_fold_kernel<kRandom, kShift>),
+                                     hipFuncAttributeMaxDynamicSharedMemorySize, kFoldLds);
+  if (e != hipSuccess) return fail(APC_ERR_LAUNCH, "hipFuncSetAttribute(score_fold_kernel): %s", hipGetErrorString(e));
+  const int fold_lanes = ((3 << kShift) + 63) / 64 * 64;
+  hipLaunchKernelGGL((score_fold_kernel<kRandom, kShift>), dim3((unsigned)((n_assign + (1 << kShift) - 1) >> kShift)),
+                     dim3(kTermLanes + fold_lanes), kFoldLds, stream, p, per_arg, comm, cost, flags, assign, stride, seed,
+                     first, n_assign, node_gid, first_node, init, out);
+  return check_launch("score_fold_kernel");
+}
+
+template <bool kRandom, typename... Args>
+int launch_fold(int64_t n_assign, Args... args) {
+  // The smallest groups whose workgroups are all resident at once (two per CU), since a
+  // group's time grows with its size: 12 layers of the GPT-2 graph, 2 000 assignments, 45 us in
+  // groups of 8, 67 in 16, 126 in 32; 8 000 assignments 110 us in 16, 130 in 32, 154 in 8.
+  const int sh = n_assign <= 1024 ? 2 : n_assign <= 4096 ? 3 : n_assign <= 8192 ? 4 : n_assign < 16384 ? 5 : 6;
+  switch (sh) {
+    case 2: return launch_fold_k<kRandom, 2>(args...);
+    case 3: return launch_fold_k<kRandom, 3>(args...);
+    case 4: return launch_fold_k<kRandom, 4>(args...);
+    case 5: return launch_fold_k<kRandom, 5>(args...);
+    default: return launch_fold_k<kRandom, 6>(args...);
+  }
+}
 
 template <bool kRandom>
 int launch_compact(int per, dim3 grid, hipStream_t stream, const apc_problem& p, const double* per_arg,
@@ -802,28 +924,23 @@ static int launch_score(const apc_problem* p, const double* per_arg, const doubl
                         const double* cost, const uint8_t* flags, const uint16_t* assign,
                         bool random, uint64_t seed, int64_t first, int64_t n_assign, double* out,
                         hipStream_t stream) {
+  if (n_assign < kScoreFoldBelow)
+    return random ? launch_fold<true>(n_assign, *p, per_arg, comm, cost, flags, assign, n_assign, seed, first, n_assign,
+                                      nullptr, 0, nullptr, out, stream)
+                  : launch_fold<false>(n_assign, *p, per_arg, comm, cost, flags, assign, n_assign, seed, first,
+                                       n_assign, nullptr, 0, nullptr, out, stream);
   const int64_t kChunk = 262144;
   for (int64_t a0 = 0; a0 < n_assign; a0 += kChunk) {
     const int64_t n = (n_assign - a0 < kChunk) ? (n_assign - a0) : kChunk;
     const uint16_t* asg = assign ? assign + a0 : nullptr;
     double* o = out + a0 * 6;
-    if (n_assign < kScoreWaveBelow) {
-      const unsigned grid = (unsigned)((n + (kBlock / 64) - 1) / (kBlock / 64));
-      if (random)
-        hipLaunchKernelGGL(score_wave_kernel<true>, dim3(grid), dim3(kBlock), 0, stream, *p, per_arg,
-                           comm, cost, flags, asg, n_assign, seed, first + a0, n, nullptr, 0, nullptr, o);
-      else
-        hipLaunchKernelGGL(score_wave_kernel<false>, dim3(grid), dim3(kBlock), 0, stream, *p,
-                           per_arg, comm, cost, flags, asg, n_assign, seed, first + a0, n, nullptr, 0, nullptr, o);
-    } else {
-      const unsigned grid = (unsigned)((n + kBlock - 1) / kBlock);
-      if (random)
-        hipLaunchKernelGGL(score_kernel<true>, dim3(grid), dim3(kBlock), 0, stream, *p, per_arg, comm,
-                           cost, flags, asg, n_assign, seed, first + a0, n, o);
-      else
-        hipLaunchKernelGGL(score_kernel<false>, dim3(grid), dim3(kBlock), 0, stream, *p, per_arg,
-                           comm, cost, flags, asg, n_assign, seed, first + a0, n, o);
-    }
+    const unsigned grid = (unsigned)((n + kBlock - 1) / kBlock);
+    if (random)
+      hipLaunchKernelGGL(score_kernel<true>, dim3(grid), dim3(kBlock), 0, stream, *p, per_arg, comm,
+                         cost, flags, asg, n_assign, seed, first + a0, n, o);
+    else
+      hipLaunchKernelGGL(score_kernel<false>, dim3(grid), dim3(kBlock), 0, stream, *p, per_arg,
+                         comm, cost, flags, asg, n_assign, seed, first + a0, n, o);
     if (int rc = check_launch("score kernel")) return rc;
   }
   return 0;
@@ -861,12 +978,9 @@ int apc_score_random_window(const apc_problem* p, const double* per_arg, const d
     return fail(APC_ERR_INVALID, "apc_score_random_window: null argument%s");
   if (first_node < 0 || first_node > p->n_node)
     return fail(APC_ERR_INVALID, "apc_score_random_window: first_node out of range%s");
-  if (n_assign < kScoreWaveBelow) {  // a wavefront per assignment
-    hipLaunchKernelGGL(score_wave_kernel<true>, dim3((unsigned)((n_assign + (kBlock / 64) - 1) / (kBlock / 64))),
-                       dim3(kBlock), 0, (hipStream_t)stream, *p, per_arg, comm, cost, flags, nullptr, n_assign, seed,
-                       first, n_assign, node_gid, (int)first_node, init, out);
-    return check_launch("score_wave_kernel");
-  }
+  if (n_assign < kScoreFoldBelow)
+    return launch_fold<true>(n_assign, *p, per_arg, comm, cost, flags, nullptr, n_assign, seed, first, n_assign, node_gid,
+                             (int)first_node, init, out, (hipStream_t)stream);
   const int64_t kChunk = 262144;  // as launch_score
   for (int64_t a0 = 0; a0 < n_assign; a0 += kChunk) {
     const int64_t n = (n_assign - a0 < kChunk) ? (n_assign - a0) : kChunk;
@@ -888,12 +1002,9 @@ int apc_score_assignments_window(const apc_problem* p, const double* per_arg, co
     return fail(APC_ERR_INVALID, "apc_score_assignments_window: null argument%s");
   if (first_node < 0 || first_node > p->n_node)
     return fail(APC_ERR_INVALID, "apc_score_assignments_window: first_node out of range%s");
-  if (n_assign < kScoreWaveBelow) {  // a wavefront per assignment
-    hipLaunchKernelGGL(score_wave_kernel<false>, dim3((unsigned)((n_assign + (kBlock / 64) - 1) / (kBlock / 64))),
-                       dim3(kBlock), 0, (hipStream_t)stream, *p, per_arg, comm, cost, flags, assign, n_assign, 0, 0,
-                       n_assign, nullptr, (int)first_node, init, out);
-    return check_launch("score_wave_kernel");
-  }
+  if (n_assign < kScoreFoldBelow)
+    return launch_fold<false>(n_assign, *p, per_arg, comm, cost, flags, assign, n_assign, 0, 0, n_assign, nullptr,
+                              (int)first_node, init, out, (hipStream_t)stream);
   const int64_t kChunk = 262144;  // as launch_score
   for (int64_t a0 = 0; a0 < n_assign; a0 += kChunk) {
     const int64_t n = (n_assign - a0 < kChunk) ? (n_assign - a0) : kChunk;
