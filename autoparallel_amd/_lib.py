@@ -12,6 +12,8 @@ LIB_PATH = os.path.join(_HERE, "libapc_hip.so")
 
 MAX_MESH_DIMS = 4
 NUM_DTYPES = 8
+SAMPLE_ARGS = 6  # argument rows an apc_sample_rec names
+SAMPLE_REC_BYTES = 64
 
 
 class ApcModel(C.Structure):
@@ -264,6 +266,14 @@ _SIGNATURES = {
         C.c_int,
         [C.POINTER(ApcProblem), C.c_void_p, C.c_void_p, C.c_uint64, C.c_int64, C.c_int64, C.c_void_p, C.c_int32,
          C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p]),
+    "apc_sample_steps": (
+        C.c_int,
+        [C.c_int32, C.c_int32, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_int32, C.c_int32, C.c_void_p,
+         C.c_int32, C.c_void_p, C.c_void_p]),
+    "apc_sample_feasible_steps": (
+        C.c_int,
+        [C.POINTER(ApcProblem), C.c_void_p, C.c_int32, C.c_int32, C.c_void_p, C.c_void_p, C.c_uint64, C.c_int64,
+         C.c_int64, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p]),
     "apc_sample_rank": (C.c_uint32, [C.c_uint64, C.c_int64, C.c_int32, C.c_uint32]),
     "apc_local_shapes": (
         C.c_int,

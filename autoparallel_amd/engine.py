@@ -30,6 +30,11 @@ _SCORE_STAGE_TILES = 2
 # 2^20, 78 ms from compact records for 2^20)
 _SCORE_TABLE_FROM = 131072
 _SCORE_PER_LANE = 0  # assignments per lane of the compact scorer; 0: the library chooses
+# assignments from which one lane each beats several wavefronts per 64 assignments, by the number
+# of wavefronts.  Measured: Llama-3-8B graph (two), 524 288 assignments 21.2 ms by lanes and 17.5 by
+# wavefronts, 2^20 31.5 and 33.2; planner DAG window (sixteen), 131 072 5.8 and 4.2, 262 144 7.1 and 8.3.
+_SAMPLE_LANES_FROM = {2: 1 << 20, 16: 1 << 18}
+_SAMPLE_WAVES = 0  # 2 or 16: tests
 _READBACK_PINNED = True  # results() copies into pinned host memory (else pageable)
 _LUT_TABLE_FROM = 2048  # table units: larger tables are built tile by tile with per-source terms in LDS
 
@@ -774,6 +779,7 @@ class CostEngine:
             if g.edge_alias is not None:  # an edge without a block of its own reads its root's columns
                 off[~own] = off[g.edge_alias[~own]]
             total = int(size[own].sum())
+            self._keep["column_layout_host"] = np.ascontiguousarray(off, np.int64)
             lay = self._keep["column_layout"] = (
                 torch.from_numpy(off).to(self.device), max(int(words.max()) if g.num_edges else 1, 1),
                 torch.empty(max(total, 1), dtype=torch.int64, device=self.device))
@@ -784,6 +790,38 @@ class CostEngine:
                 self._stream()),
             "apc_pack_allowed_columns")
         return colbits, d_off, max_words
+
+    def _sample_steps(self, first_node: int):
+        """(records on the device, steps, wavefronts) of apc_sample_feasible_steps for the walk
+        from ``first_node`` on, or None for a graph such a walk does not take (columns past its
+        32-bit offsets, a producer behind its consumer).  Made once per first_node; the last one
+        is kept."""
+        g = self.g
+        kept = self._keep.get("sample_steps")
+        if kept is not None and kept[0] == first_node:
+            return kept[1]
+        n = g.num_nodes - first_node
+        plan = None
+        if (n > 0 and g.num_edges > 0 and g.num_nodes < 1 << 24 and (g.edge_src_node < g.edge_node).all()
+                and int(self._keep["column_layout_host"].max()) < 1 << 32):
+            edge_off = np.ascontiguousarray(g.node_edge_off, np.int32)
+            src = np.ascontiguousarray(g.edge_src_node, np.int32)
+            nstrat = np.ascontiguousarray(g.node_nstrat, np.int32)
+            col_off = self._keep["column_layout_host"]
+            long_rows = int((np.diff(edge_off) > _lib.SAMPLE_ARGS).sum())
+            n_step, n_waves = C.c_int32(0), C.c_int32(0)
+            max_step = n + 128 * long_rows
+            recs = np.empty((max_step * 16, _lib.SAMPLE_REC_BYTES), np.uint8)
+            _lib.check(
+                self.lib.apc_sample_steps(
+                    g.num_nodes, g.num_edges, edge_off.ctypes.data, src.ctypes.data, nstrat.ctypes.data,
+                    col_off.ctypes.data, int(first_node), _SAMPLE_WAVES, recs.ctypes.data, max_step,
+                    C.byref(n_step), C.byref(n_waves)),
+                "apc_sample_steps")
+            recs = torch.from_numpy(recs[:n_step.value * n_waves.value]).to(self.device)
+            plan = (recs, n_step.value, n_waves.value)
+        self._keep["sample_steps"] = (first_node, plan)
+        return plan
 
     def sample_feasible(self, seed: int, first: int, count: int, node_gid: Optional[np.ndarray] = None,
                         first_node: int = 0, assign: Optional[torch.Tensor] = None,
@@ -832,6 +870,16 @@ class CostEngine:
                 words.append(w)
             d_keep = torch.from_numpy(np.concatenate(words).view(np.int64)).to(self.device)
             d_keep_off = torch.from_numpy(keep_off).to(self.device)
+        steps = self._sample_steps(first_node) if count < max(_SAMPLE_LANES_FROM.values()) else None
+        if steps is not None and count < _SAMPLE_LANES_FROM[steps[2]]:
+            recs, n_step, n_waves = steps
+            _lib.check(
+                self.lib.apc_sample_feasible_steps(
+                    C.byref(self.problem), self._ptr(recs), n_step, n_waves, self._ptr(colbits), self._ptr(d_off),
+                    int(seed), int(first), int(count), self._ptr(d_gid), self._ptr(d_keep), self._ptr(d_keep_off),
+                    self._ptr(assign), self._ptr(fallback), self._stream()),
+                "apc_sample_feasible_steps")
+            return assign, fallback
         _lib.check(
             self.lib.apc_sample_feasible(
                 C.byref(self.problem), self._ptr(colbits), self._ptr(d_off), int(seed), int(first), int(count),

@@ -688,6 +688,36 @@ int apc_sample_feasible(const apc_problem* p, const uint64_t* colbits, const int
                         int32_t* n_fallback, void* stream);
 uint32_t apc_sample_rank(uint64_t seed, int64_t a, int32_t node, uint32_t count);
 
+/* The same draws by n_waves (2 or 16) wavefronts per 64 assignments, for batches that
+ * do not fill the chip with one lane each.  apc_sample_steps (host, no device needed)
+ * lays the nodes from first_node on out in steps of up to n_waves (asked for, or 0: chosen by how
+ * many nodes are ready at a time; what was taken is stored in n_waves_out) nodes whose producers
+ * all lie in earlier steps: records recs[n_step][n_waves] (room for max_step steps; n_node
+ * steps and 128 more per node with over APC_SAMPLE_ARGS argument rows always suffice), to be copied
+ * to the device.  It needs every producer in front of its consumer (edge_src[e] < node)
+ * and reads nothing that a build writes, so one layout serves every call with the same
+ * graph, first_node and col_off.  apc_sample_feasible_steps then is apc_sample_feasible
+ * over those records, same results bit for bit. */
+#define APC_SAMPLE_ARGS 6
+typedef struct apc_sample_rec {
+  int32_t node; /* -1: nothing for this wavefront in this step */
+  int32_t nstrat;
+  int32_t n_arg; /* argument rows, those past APC_SAMPLE_ARGS included */
+  int32_t reserved;
+  struct {
+    uint32_t from; /* producer in the low 24 bits; above them the place of its choice in the
+                      workgroup's ring, 255: in the matrix only, 128: no producer (choice 0) */
+    uint32_t col; /* col_off / 2 */
+  } arg[APC_SAMPLE_ARGS];
+} apc_sample_rec; /* 64 bytes */
+int apc_sample_steps(int32_t n_node, int32_t n_edge, const int32_t* node_edge_off, const int32_t* edge_src,
+                     const int32_t* node_nstrat, const int64_t* col_off, int32_t first_node, int32_t n_waves,
+                     apc_sample_rec* recs, int32_t max_step, int32_t* n_step, int32_t* n_waves_out);
+int apc_sample_feasible_steps(const apc_problem* p, const apc_sample_rec* recs, int32_t n_step, int32_t n_waves,
+                              const uint64_t* colbits, const int64_t* col_off, uint64_t seed, int64_t first,
+                              int64_t n_assign, const int32_t* node_gid, const uint64_t* row_filter,
+                              const int64_t* filter_off, uint16_t* assign, int32_t* n_fallback, void* stream);
+
 /* apc_score_random_assignments for a graph too large to keep its coefficients
  * resident: the problem holds a window of the graph's nodes (preceded by
  * first_node stand-ins for producers outside the window, which are not scored),
