@@ -14,6 +14,7 @@ MAX_MESH_DIMS = 4
 NUM_DTYPES = 8
 SAMPLE_ARGS = 6  # argument rows an apc_sample_rec names
 SAMPLE_REC_BYTES = 64
+SCORE_STEP_BYTES, SCORE_TILE_BYTES, SCORE_UNIT_BYTES = 64, 128, 16
 
 
 class ApcModel(C.Structure):
@@ -266,6 +267,15 @@ _SIGNATURES = {
         C.c_int,
         [C.POINTER(ApcProblem), C.c_void_p, C.c_void_p, C.c_uint64, C.c_int64, C.c_int64, C.c_void_p, C.c_int32,
          C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p]),
+    "apc_score_tiles": (
+        C.c_int,
+        [C.c_void_p, C.c_int32, C.c_int32, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_int32, C.c_int32,
+         C.c_void_p, C.c_int64, C.c_void_p, C.c_int64, C.c_void_p, C.c_int64, C.c_void_p, C.c_void_p, C.c_void_p]),
+    "apc_score_from_tiles": (
+        C.c_int,
+        [C.POINTER(ApcProblem), C.c_void_p, C.c_void_p, C.c_void_p, C.c_int32, C.c_void_p, C.c_int32, C.c_void_p,
+         C.c_void_p, C.c_void_p, C.c_uint64, C.c_int64, C.c_int64, C.c_void_p, C.c_int32, C.c_void_p, C.c_void_p,
+         C.c_void_p]),
     "apc_sample_steps": (
         C.c_int,
         [C.c_int32, C.c_int32, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_int32, C.c_int32, C.c_void_p,

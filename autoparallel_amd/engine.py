@@ -19,6 +19,10 @@ _UPLOAD_ARENA_MAX_ARRAY = 2 << 20
 _SCORE_LANES_FROM = 32768  # assignments: below, one wavefront per assignment (entry arrays as they are)
 _SCORE_FROM_TABLE = True  # the three ways of scoring a graph with large blocks can be switched off (tests do)
 _SCORE_COMPACT = True
+_SCORE_FROM_TILES = True  # small blocks: matrices through LDS by tiles, while the table stands for the arrays
+# Below, too few wavefronts per CU hide the walk's chain of LDS reads.  Llama-3-8B graph, random and explicit
+# assignments, by tiles and from records: 32 768 8.0 / 8.6 and 7.2 / 10.7 ms, 65 536 5.9 / 6.6 and 7.2 / 10.9.
+_SCORE_TILES_FROM = 65536
 # Matrices of up to this many LDS tiles (64 KB each) go through LDS in the table scorer, larger
 # ones are read in place.  Measured on a 3 000-node window of the stress DAG, 2^20 assignments:
 # 17.9 ms with 1, 17.4 with 2, 18.0 with 4, 18.35 with 8 or 16.  (A lower bound, small matrices
@@ -576,6 +580,20 @@ class CostEngine:
                 "apc_score_table")
             self.last_score_backend = "block_table"
             return out
+        if self._table_clamp is not None and _SCORE_FROM_TILES and count >= _SCORE_TILES_FROM and not self.large_blocks:
+            tiles = self._score_tiles(first_node, assign is not None)
+            if tiles is not None:
+                steps, n_step, d_tiles, n_tile, units = tiles
+                call_steps = torch.empty(n_step * _lib.SCORE_STEP_BYTES, dtype=torch.uint8, device=self.device)
+                _lib.check(
+                    self.lib.apc_score_from_tiles(
+                        C.byref(self.problem), self._ptr(self.per_arg), self._ptr(self.table), self._ptr(steps), n_step,
+                        self._ptr(d_tiles), n_tile, self._ptr(units), self._ptr(call_steps), self._ptr(assign),
+                        int(seed), int(first), int(count), self._ptr(d_gid), self._table_clamp, self._ptr(init),
+                        self._ptr(out), self._stream()),
+                    "apc_score_from_tiles")
+                self.last_score_backend = "block_table_tiles"
+                return out
         if not self._recs_valid:
             self._recs = None  # one kind at a time: either is as large as the entry arrays
             recs = None
@@ -616,6 +634,42 @@ class CostEngine:
             "apc_score_packed")
         self.last_score_backend = "records"
         return out
+
+    def _score_tiles(self, first_node: int, explicit: bool):
+        """The layout apc_score_from_tiles walks from ``first_node`` on, on the device, or None for
+        a graph that form does not take.  Made once per first_node, for random and for explicit
+        assignments; the last of each is kept."""
+        key = "score_tiles_explicit" if explicit else "score_tiles"
+        kept = self._keep.get(key)
+        if kept is not None and kept[0] == first_node:
+            return kept[1]
+        g = self.g
+        plan = None
+        if self.table_mode == "full" and first_node < g.num_nodes:
+            edges = np.ascontiguousarray(g.edge_records(False))
+            a = [np.ascontiguousarray(x, t) for x, t in (
+                (g.node_edge_off, np.int32), (g.node_nstrat, np.int32), (g.node_nargs, np.int32),
+                (g.node_comp_off, np.int64))]
+            max_step = g.num_nodes + g.num_edges
+            chunks = (g.edge_sdst.astype(np.int64) * g.edge_ssrc + 31) // 32
+            max_unit = int(chunks.sum() + ((g.node_nstrat.astype(np.int64) + 31) // 32).sum()) + max_step
+            steps = np.empty((max_step, _lib.SCORE_STEP_BYTES), np.uint8)
+            tiles = np.empty((max_step, _lib.SCORE_TILE_BYTES), np.uint8)
+            units = np.empty((max_unit, _lib.SCORE_UNIT_BYTES), np.uint8)
+            n = [C.c_int32(0) for _ in range(3)]
+            _lib.check(
+                self.lib.apc_score_tiles(
+                    edges.ctypes.data, g.num_edges, g.num_nodes, *[x.ctypes.data for x in a], int(first_node),
+                    int(explicit), steps.ctypes.data, max_step, tiles.ctypes.data, max_step, units.ctypes.data,
+                    max_unit, *[C.byref(x) for x in n]),
+                "apc_score_tiles")
+            n_step, n_tile, n_unit = [x.value for x in n]
+            if n_step > 0:
+                plan = (torch.from_numpy(steps[:n_step]).to(self.device), n_step,
+                        torch.from_numpy(tiles[:n_tile]).to(self.device), n_tile,
+                        torch.from_numpy(units[:n_unit]).to(self.device))
+        self._keep[key] = (first_node, plan)
+        return plan
 
     def _score_msize(self) -> np.ndarray:
         """int32[num_edges]: the padded size of an edge's matrix in the block table

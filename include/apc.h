@@ -718,6 +718,59 @@ int apc_sample_feasible_steps(const apc_problem* p, const apc_sample_rec* recs, 
                               int64_t n_assign, const int32_t* node_gid, const uint64_t* row_filter,
                               const int64_t* filter_off, uint16_t* assign, int32_t* n_fallback, void* stream);
 
+/* Scoring of large batches on graphs with small blocks, from the block table through LDS.
+ * apc_score_tiles (host, no device needed) lays the walk from first_node on out: a step per
+ * argument row (and per node without one) in node order, then argument order; tiles of
+ * consecutive steps whose matrices, each once, fit an LDS buffer; the copies (units) that
+ * bring a tile in.  edges: the records of the problem (apc_edge), as on the device.
+ * explicit_rows: the layout is for explicit assignments (a tile names the nodes whose
+ * choices it reads, 16 at most), else for random ones.  
+ * *n_step = 0: not a graph for this form (a matrix of more than 4 864 doubles or compressed, a
+ * node with more than 256 strategies, a producer behind its consumer): use another scorer.
+ * The layout depends on the graph alone; it is copied to the device and serves every call.
+ * apc_score_from_tiles scores random (assign NULL) or explicit assignments as
+ * apc_score_table does over nodes first_node..n_node, same bits.  call_steps: 16-byte aligned
+ * scratch of 64 * n_step bytes. */
+#define APC_STEP_FIRST 1      /* first step of its node */
+#define APC_STEP_EDGE 2       /* an argument row */
+#define APC_STEP_TRANSITION 4 /* whose transitions count */
+typedef struct apc_score_step {
+  int32_t node;
+  int32_t src_node; /* producer or -1 */
+  int32_t nstrat;
+  int32_t ssrc;
+  int32_t nargs;
+  int32_t flags;
+  int32_t mat;      /* of the matrix in the tile's buffer, in doubles */
+  int32_t pa;       /* of the node's per-argument terms */
+  int32_t row_node; /* row of packed choices that holds the node's */
+  int32_t row_src;  /* the producer's, -1: none or not kept */
+  int32_t reserved[6];
+} apc_score_step; /* 64 bytes */
+typedef struct apc_score_unit {
+  int64_t src;  /* first element, in the array kind names */
+  uint16_t lds; /* where to, in doubles */
+  uint16_t n;   /* doubles */
+  int32_t kind; /* 0: block table, 1: per_arg, 2: default_vals */
+} apc_score_unit; /* 16 bytes */
+typedef struct apc_score_tile {
+  int32_t step0, step1, unit0, unit1;
+  int32_t n_row;
+  int32_t any_edge; /* of the whole walk, in the first tile */
+  int32_t row[16];  /* nodes whose explicit choices the tile reads */
+  int32_t reserved[10];
+} apc_score_tile; /* 128 bytes */
+int apc_score_tiles(const apc_edge* edges, int32_t n_edge, int32_t n_node, const int32_t* node_edge_off,
+                    const int32_t* node_nstrat, const int32_t* node_nargs, const int64_t* node_comp_off,
+                    int32_t first_node, int32_t explicit_rows, apc_score_step* steps, int64_t max_step,
+                    apc_score_tile* tiles, int64_t max_tile, apc_score_unit* units, int64_t max_unit,
+                    int32_t* n_step, int32_t* n_tile, int32_t* n_unit);
+int apc_score_from_tiles(const apc_problem* p, const double* per_arg, const double* table, const apc_score_step* steps,
+                         int32_t n_step, const apc_score_tile* tiles, int32_t n_tile, const apc_score_unit* units,
+                         void* call_steps, const uint16_t* assign, uint64_t seed, int64_t first,
+                         int64_t n_assign, const int32_t* node_gid, int32_t clamp_inf, const double* init, double* out,
+                         void* stream);
+
 /* apc_score_random_assignments for a graph too large to keep its coefficients
  * resident: the problem holds a window of the graph's nodes (preceded by
  * first_node stand-ins for producers outside the window, which are not scored),
