@@ -14,6 +14,7 @@ MAX_MESH_DIMS = 4
 NUM_DTYPES = 8
 SAMPLE_ARGS = 6  # argument rows an apc_sample_rec names
 SAMPLE_REC_BYTES = 64
+CHECK_MAX_NODES = 131072
 SCORE_STEP_BYTES, SCORE_TILE_BYTES, SCORE_UNIT_BYTES = 64, 128, 16
 
 
@@ -327,6 +328,7 @@ _SIGNATURES = {
         [C.POINTER(ApcProblem), C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_uint64, C.c_int64,
          C.c_int64, C.c_void_p, C.c_int32, C.c_int32, C.c_int32, C.c_int32, C.c_void_p, C.c_void_p, C.c_void_p]),
     "apc_score_table_tile": (C.c_int, []),
+    "apc_check_orders": (C.c_int, [C.c_void_p, C.c_int64, C.c_int32, C.c_void_p, C.c_void_p]),
     "apc_schedule_metrics": (
         C.c_int,
         [C.POINTER(ApcSchedule), C.c_void_p, C.c_int64, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p,

@@ -342,13 +342,21 @@ class ScheduleEstimator:
             assert orders.ndim == 2 and orders.shape[1] == N
             B = orders.shape[0]
             d_orders = torch.from_numpy(orders).to(self.device)
-            # each row a permutation: the kernel indexes node arrays with it (checked on the
-            # device, where sorting the rows of a large batch takes a fraction of the host's time)
-            rows_sorted = torch.sort(d_orders, dim=1).values
-            assert bool((rows_sorted == torch.arange(N, dtype=torch.int32, device=self.device)).all().item()), \
-                "not permutations"
-            del rows_sorted
             order_ptr = C.c_void_p(d_orders.data_ptr())
+            # each row a permutation: the kernel indexes node arrays with it
+            if N <= _lib.CHECK_MAX_NODES:
+                bad = torch.zeros(1, dtype=torch.int32, device=self.device)
+                _lib.check(
+                    self.lib.apc_check_orders(
+                        order_ptr, B, N, C.c_void_p(bad.data_ptr()),
+                        C.c_void_p(torch.cuda.current_stream(self.device).cuda_stream)),
+                    "apc_check_orders")
+                assert int(bad.item()) == 0, "not permutations"
+            else:
+                rows_sorted = torch.sort(d_orders, dim=1).values
+                assert bool((rows_sorted == torch.arange(N, dtype=torch.int32, device=self.device)).all().item()), \
+                    "not permutations"
+                del rows_sorted
         end = torch.empty(max(B * N, 1), dtype=torch.float64, device=self.device)
         rem = torch.empty(max(B * S, 1), dtype=torch.int32, device=self.device)
         times = torch.empty((B, 4), dtype=torch.float64, device=self.device)

@@ -963,6 +963,11 @@ typedef struct apc_schedule {
   int32_t n_comm;
 } apc_schedule;
 
+/* Sets *bad (on the device, cleared by the caller) unless each of the n_sched rows of order
+ * holds every node 0..n_node-1 once, as apc_schedule_metrics needs it. */
+#define APC_CHECK_MAX_NODES 131072
+int apc_check_orders(const int32_t* order, int64_t n_sched, int32_t n_node, int32_t* bad, void* stream);
+
 /* Replaces estimate_graph_metrics
  * (autoparallel/graph_passes/estimate_graph_metrics.py:30-89; the same timeline
  * as create_execution_trace, graph_passes/debug_helpers.py:336-420) for n_sched
