@@ -16,13 +16,16 @@ from .packed import CHUNK_SHIFT, ITEM_ENTRIES, MAX_MESH_DIMS, PackedGraph
 _LARGE_BLOCKS_FROM = 8192  # mean entries per edge block
 _UPLOAD_ARENA_BYTES = 8 << 20  # descriptor arrays of one problem that go up in one copy
 _UPLOAD_ARENA_MAX_ARRAY = 2 << 20
-_SCORE_LANES_FROM = 32768  # assignments: below, one wavefront per assignment (entry arrays as they are)
+_SCORE_LANES_FROM = 32768  # assignments: below, always with the terms side by side (from the table or the arrays)
 _SCORE_FROM_TABLE = True  # the three ways of scoring a graph with large blocks can be switched off (tests do)
 _SCORE_COMPACT = True
+_SCORE_SMALL_FROM_TABLE = True
 _SCORE_FROM_TILES = True  # small blocks: matrices through LDS by tiles, while the table stands for the arrays
-# Below, too few wavefronts per CU hide the walk's chain of LDS reads.  Llama-3-8B graph, random and explicit
-# assignments, by tiles and from records: 32 768 8.0 / 8.6 and 7.2 / 10.7 ms, 65 536 5.9 / 6.6 and 7.2 / 10.9.
-_SCORE_TILES_FROM = 65536
+# Below, the terms of a few assignments gathered side by side are faster than any walk with a lane per
+# assignment (side by side, by tiles): Llama-3-8B graph, random 65 536 2.5 and 5.9 ms, 131 072 5.5 and 4.8, explicit
+# ones 3.2 and 6.6, 7.2 and 5.7; window of the planner DAG (side by side, table scorer) 65 536 1.95 and 5.4, 131 072
+# 4.7 and 5.3, 262 144 11.2 and 5.3.
+_SCORE_TERMS_BELOW = 131072
 # Matrices of up to this many LDS tiles (64 KB each) go through LDS in the table scorer, larger
 # ones are read in place.  Measured on a 3 000-node window of the stress DAG, 2^20 assignments:
 # 17.9 ms with 1, 17.4 with 2, 18.0 with 4, 18.35 with 8 or 16.  (A lower bound, small matrices
@@ -360,7 +363,11 @@ class CostEngine:
         # clamp_inf of the build whose table path wrote the entry arrays as they are now,
         # None once anything else has written them: then scoring cannot read the table instead
         self._table_clamp: Optional[int] = None
-        self.last_score_backend = "entry_arrays"  # what the last large batch was scored from
+        # and the arrays' version counters at that build: small batches, which used to read the
+        # arrays, notice a caller's in-place edit by them (tensors made under inference_mode have none)
+        self._versioned = not self.comm.is_inference()
+        self._table_version = 0
+        self.last_score_backend = "entry_arrays"  # what the last large batch was scored from (small ones: this)
 
     def synchronize(self) -> None:
         torch.cuda.synchronize(self.device)
@@ -452,6 +459,8 @@ class CostEngine:
             _lib.check(rc, "apc_build_all")
         self.built = True
         self._table_clamp = (1 if clamp_inf else 0) if self.table is not None else None
+        if self._versioned:
+            self._table_version = self.comm._version + self.cost._version + self.flags._version + self.per_arg._version
         return self
 
     def build_timed(self, timer, slot: int, clamp_inf: bool = True):
@@ -467,6 +476,8 @@ class CostEngine:
         self._recs_valid = False
         self.built = True
         self._table_clamp = clamp if self.table is not None else None
+        if self._versioned:
+            self._table_version = self.comm._version + self.cost._version + self.flags._version + self.per_arg._version
         return self
 
     def set_node_multiplier(self, mult: np.ndarray) -> None:
@@ -547,6 +558,8 @@ class CostEngine:
         out = torch.empty((A, 6), dtype=torch.float64, device=self.device)
         if self.packed_scoring and A >= _SCORE_LANES_FROM:
             return self._score_packed(assign, 0, 0, A, None, 0, None, out)
+        if self._score_small(assign, 0, 0, A, None, 0, None, out):
+            return out
         _lib.check(
             self.lib.apc_score_assignments(
                 C.byref(self.problem), self._ptr(self.per_arg), self._ptr(self.comm), self._ptr(self.cost),
@@ -555,13 +568,31 @@ class CostEngine:
         )
         return out
 
+    def _score_small(self, assign, seed, first, count, d_gid, first_node, init, out) -> bool:
+        """A small batch from the block table while it stands for the entry arrays; False: not done."""
+        if self._table_clamp is None or not _SCORE_SMALL_FROM_TABLE or not self.packed_scoring or count == 0:
+            return False
+        if not self._versioned or self._table_version != (
+                self.comm._version + self.cost._version + self.flags._version + self.per_arg._version):
+            return False  # edited since the build
+        _lib.check(
+            self.lib.apc_score_fold_table(
+                C.byref(self.problem), self._ptr(self.per_arg), self._ptr(self.table), self._ptr(assign), int(seed),
+                int(first), int(count), self._ptr(d_gid), int(first_node), self._table_clamp, self._ptr(init),
+                self._ptr(out), self._stream()),
+            "apc_score_fold_table")
+        return True
+
     def _score_packed(self, assign, seed, first, count, d_gid, first_node, init, out) -> torch.Tensor:
         """Scoring of a large batch.  A graph with large blocks: from the block
         table while the entry arrays are what the last build made of it
         (apc_score_table, 5x the rate of any walk over records there).  Else,
-        and for graphs with small blocks (where the records win: 15.6 ms against
-        18.0 ms from the table and 31.2 ms from the three arrays for 2^20
-        assignments of the Llama-3-8B graph), from records made here if the entry
+        and for graphs with small blocks: below _SCORE_TERMS_BELOW assignments with
+        the terms gathered side by side from the table (apc_score_fold_table), from
+        there on by tiles of edges (apc_score_from_tiles: 10.4 ms for 2^20 assignments
+        of the Llama-3-8B graph, against 15.6 ms from records, 18.0 ms from the table
+        edge by edge and 31.2 ms from the three arrays).  Where the table does not
+        stand for the arrays, or the graph has no such tiles: from records made here if the entry
         arrays changed since: compact 16-byte
         records, several assignments per lane (apc_score_compact), while every
         cost is (comm + per_arg) + transition or its clamp (checked on the device
@@ -580,7 +611,11 @@ class CostEngine:
                 "apc_score_table")
             self.last_score_backend = "block_table"
             return out
-        if self._table_clamp is not None and _SCORE_FROM_TILES and count >= _SCORE_TILES_FROM and not self.large_blocks:
+        if (_SCORE_FROM_TABLE and count < _SCORE_TERMS_BELOW
+                and self._score_small(assign, seed, first, count, d_gid, first_node, init, out)):
+            self.last_score_backend = "block_table_terms"
+            return out
+        if self._table_clamp is not None and _SCORE_FROM_TABLE and _SCORE_FROM_TILES and not self.large_blocks:
             tiles = self._score_tiles(first_node, assign is not None)
             if tiles is not None:
                 steps, n_step, d_tiles, n_tile, units = tiles
@@ -765,6 +800,8 @@ class CostEngine:
         out = torch.empty((count, 6), dtype=torch.float64, device=self.device)
         if self.packed_scoring and count >= _SCORE_LANES_FROM:
             return self._score_packed(None, seed, first, count, None, 0, None, out)
+        if self._score_small(None, seed, first, count, None, 0, None, out):
+            return out
         _lib.check(
             self.lib.apc_score_random_assignments(
                 C.byref(self.problem), self._ptr(self.per_arg), self._ptr(self.comm), self._ptr(self.cost),
@@ -787,6 +824,8 @@ class CostEngine:
         if self.packed_scoring and count >= _SCORE_LANES_FROM:
             return self._score_packed(None, seed, first, count, d_gid, first_node, init, out)
         self.last_score_backend = "entry_arrays"
+        if self._score_small(None, seed, first, count, d_gid, first_node, init, out):
+            return out
         _lib.check(
             self.lib.apc_score_random_window(
                 C.byref(self.problem), self._ptr(self.per_arg), self._ptr(self.comm), self._ptr(self.cost),
@@ -809,13 +848,15 @@ class CostEngine:
         out = torch.empty((count, 6), dtype=torch.float64, device=self.device)
         if self.packed_scoring and count >= _SCORE_LANES_FROM:
             return self._score_packed(assign, 0, 0, count, None, first_node, init, out)
+        self.last_score_backend = "entry_arrays"
+        if self._score_small(assign, 0, 0, count, None, first_node, init, out):
+            return out
         _lib.check(
             self.lib.apc_score_assignments_window(
                 C.byref(self.problem), self._ptr(self.per_arg), self._ptr(self.comm), self._ptr(self.cost),
                 self._ptr(self.flags), self._ptr(assign), count, int(first_node), self._ptr(init), self._ptr(out),
                 self._stream()),
             "apc_score_assignments_window")
-        self.last_score_backend = "entry_arrays"
         return out
 
     def _allowed_columns(self):

@@ -718,6 +718,13 @@ int apc_sample_feasible_steps(const apc_problem* p, const apc_sample_rec* recs, 
                               int64_t n_assign, const int32_t* node_gid, const uint64_t* row_filter,
                               const int64_t* filter_off, uint16_t* assign, int32_t* n_fallback, void* stream);
 
+/* Scoring of small batches (the terms of 4 to 64 assignments a workgroup gathered side by side)
+ * from the block table, arguments and results as apc_score_table's over nodes
+ * first_node..n_node. */
+int apc_score_fold_table(const apc_problem* p, const double* per_arg, const double* table, const uint16_t* assign,
+                         uint64_t seed, int64_t first, int64_t n_assign, const int32_t* node_gid, int32_t first_node,
+                         int32_t clamp_inf, const double* init, double* out, void* stream);
+
 /* Scoring of large batches on graphs with small blocks, from the block table through LDS.
  * apc_score_tiles (host, no device needed) lays the walk from first_node on out: a step per
  * argument row (and per node without one) in node order, then argument order; tiles of

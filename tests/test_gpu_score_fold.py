@@ -40,8 +40,27 @@ def test_groups_have_the_bits_of_the_lane_walk(engines, which, count, monkeypatc
             eng.score_random_window(11, 5, count, ids, g.num_nodes, init=init),  # nothing to add
             eng.score_window(assign, first_node, init=init))]
 
-    got = all_scores()
+    from_table = all_scores()
+    monkeypatch.setattr(engine_mod, "_SCORE_SMALL_FROM_TABLE", False)
+    from_arrays = all_scores()
     monkeypatch.setattr(engine_mod, "_SCORE_LANES_FROM", 1)  # one lane per assignment, from records
+    monkeypatch.setattr(engine_mod, "_SCORE_FROM_TABLE", False)
     want = all_scores()
-    for a, b in zip(got, want):
-        assert (a == b).all()
+    for a, b, c in zip(from_table, from_arrays, want):
+        assert (a == c).all() and (b == c).all()
+
+
+def test_the_table_stands_for_the_arrays_only_while_it_does(engines):
+    """Clamped and unclamped builds; and where the arrays were edited, the arrays decide."""
+    eng = engines[0][0]
+    for clamp in (False, True):
+        eng.build(clamp_inf=clamp)
+        got = _bits(eng.score_random(3, 0, 70))
+        eng.mark_results_edited()  # from here on the arrays are read
+        assert (got == _bits(eng.score_random(3, 0, 70))).all()
+    for array in (eng.cost, eng.comm):  # an edit in place is noticed without being told
+        eng.build()
+        got = _bits(eng.score_random(3, 0, 70))
+        array.mul_(2.0)
+        assert not (got == _bits(eng.score_random(3, 0, 70))).all()
+    eng.build()

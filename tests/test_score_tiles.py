@@ -114,7 +114,7 @@ def test_scores_have_the_bits_of_the_walk_over_records(name, count, monkeypatch)
         return out
 
     monkeypatch.setattr(engine_mod, "_SCORE_LANES_FROM", 1)
-    monkeypatch.setattr(engine_mod, "_SCORE_TILES_FROM", 1)
+    monkeypatch.setattr(engine_mod, "_SCORE_TERMS_BELOW", 0)
     for clamp in (True, False):
         eng.build(clamp_inf=clamp)
         got = scores("block_table_tiles")
