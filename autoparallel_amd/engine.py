@@ -367,7 +367,7 @@ class CostEngine:
         # arrays, notice a caller's in-place edit by them (tensors made under inference_mode have none)
         self._versioned = not self.comm.is_inference()
         self._table_version = 0
-        self.last_score_backend = "entry_arrays"  # what the last large batch was scored from (small ones: this)
+        self.last_score_backend = "entry_arrays"  # what the last batch was scored from
 
     def synchronize(self) -> None:
         torch.cuda.synchronize(self.device)
@@ -566,6 +566,7 @@ class CostEngine:
                 self._ptr(self.flags), self._ptr(assign), A, self._ptr(out), self._stream()),
             "apc_score_assignments",
         )
+        self.last_score_backend = "entry_arrays"
         return out
 
     def _score_small(self, assign, seed, first, count, d_gid, first_node, init, out) -> bool:
@@ -581,6 +582,7 @@ class CostEngine:
                 int(first), int(count), self._ptr(d_gid), int(first_node), self._table_clamp, self._ptr(init),
                 self._ptr(out), self._stream()),
             "apc_score_fold_table")
+        self.last_score_backend = "block_table_terms"
         return True
 
     def _score_packed(self, assign, seed, first, count, d_gid, first_node, init, out) -> torch.Tensor:
@@ -613,7 +615,6 @@ class CostEngine:
             return out
         if (_SCORE_FROM_TABLE and count < _SCORE_TERMS_BELOW
                 and self._score_small(assign, seed, first, count, d_gid, first_node, init, out)):
-            self.last_score_backend = "block_table_terms"
             return out
         if self._table_clamp is not None and _SCORE_FROM_TABLE and _SCORE_FROM_TILES and not self.large_blocks:
             tiles = self._score_tiles(first_node, assign is not None)
@@ -808,6 +809,7 @@ class CostEngine:
                 self._ptr(self.flags), int(seed), int(first), int(count), self._ptr(out), self._stream()),
             "apc_score_random_assignments",
         )
+        self.last_score_backend = "entry_arrays"
         return out
 
     def score_random_window(self, seed: int, first: int, count: int, node_gid: np.ndarray, first_node: int,
@@ -823,7 +825,6 @@ class CostEngine:
         out = torch.empty((count, 6), dtype=torch.float64, device=self.device)
         if self.packed_scoring and count >= _SCORE_LANES_FROM:
             return self._score_packed(None, seed, first, count, d_gid, first_node, init, out)
-        self.last_score_backend = "entry_arrays"
         if self._score_small(None, seed, first, count, d_gid, first_node, init, out):
             return out
         _lib.check(
@@ -833,6 +834,7 @@ class CostEngine:
                 self._ptr(init), self._ptr(out), self._stream()),
             "apc_score_random_window",
         )
+        self.last_score_backend = "entry_arrays"
         return out
 
     def score_window(self, assign: torch.Tensor, first_node: int, init: Optional[torch.Tensor] = None) -> torch.Tensor:
@@ -848,7 +850,6 @@ class CostEngine:
         out = torch.empty((count, 6), dtype=torch.float64, device=self.device)
         if self.packed_scoring and count >= _SCORE_LANES_FROM:
             return self._score_packed(assign, 0, 0, count, None, first_node, init, out)
-        self.last_score_backend = "entry_arrays"
         if self._score_small(assign, 0, 0, count, None, first_node, init, out):
             return out
         _lib.check(
@@ -857,6 +858,7 @@ class CostEngine:
                 self._ptr(self.flags), self._ptr(assign), count, int(first_node), self._ptr(init), self._ptr(out),
                 self._stream()),
             "apc_score_assignments_window")
+        self.last_score_backend = "entry_arrays"
         return out
 
     def _allowed_columns(self):

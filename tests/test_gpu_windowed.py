@@ -177,10 +177,9 @@ def test_the_node_of_config5_that_no_assignment_can_serve():
         assert any(dead), (o, dead)
 
 
-def test_small_batches_of_explicit_assignments_in_a_window():
-    """apc_score_assignments_window (entry arrays, a lane per assignment) gives the
-    sums of the batch scorers for the same window, stand-ins and carried sums
-    included."""
+def test_small_batches_of_explicit_assignments_in_a_window(monkeypatch):
+    """apc_score_assignments_window (the entry arrays) gives the sums of the other batch
+    scorers for the same window, stand-ins and carried sums included."""
     from autoparallel_amd import engine as E
     from autoparallel_amd.engine import CostEngine
 
@@ -191,13 +190,15 @@ def test_small_batches_of_explicit_assignments_in_a_window():
     rng = np.random.default_rng(0)
     assign = torch.from_numpy(np.stack([rng.integers(0, s, n) for s in g.node_nstrat]).astype(np.int16)).cuda()
     init = torch.rand(n, 6, dtype=torch.float64, device="cuda")
+    monkeypatch.setattr(E, "_SCORE_SMALL_FROM_TABLE", False)
     got = eng.score_window(assign, n_standin, init=init)
     assert eng.last_score_backend == "entry_arrays"
-    saved = E._SCORE_LANES_FROM
-    try:
-        E._SCORE_LANES_FROM = 0
-        want = eng.score_window(assign, n_standin, init=init)
-        assert eng.last_score_backend != "entry_arrays"
-    finally:
-        E._SCORE_LANES_FROM = saved
+    monkeypatch.setattr(E, "_SCORE_LANES_FROM", 0)  # a lane per assignment, from records
+    monkeypatch.setattr(E, "_SCORE_FROM_TABLE", False)
+    want = eng.score_window(assign, n_standin, init=init)
+    assert eng.last_score_backend == "compact_records"
     assert torch.equal(got.view(torch.int64), want.view(torch.int64))
+    monkeypatch.undo()  # and the route a batch of this size takes by itself
+    default = eng.score_window(assign, n_standin, init=init)
+    assert eng.last_score_backend == "block_table_terms"
+    assert torch.equal(default.view(torch.int64), want.view(torch.int64))
