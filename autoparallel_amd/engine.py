@@ -363,10 +363,11 @@ class CostEngine:
         # clamp_inf of the build whose table path wrote the entry arrays as they are now,
         # None once anything else has written them: then scoring cannot read the table instead
         self._table_clamp: Optional[int] = None
-        # and the arrays' version counters at that build: small batches, which used to read the
-        # arrays, notice a caller's in-place edit by them (tensors made under inference_mode have none)
+        # and the arrays' version counters at that build, by which a caller's edit in place shows, as
+        # it does in those of the records' arrays (tensors made under inference_mode have none)
         self._versioned = not self.comm.is_inference()
-        self._table_version = 0
+        self._table_versions: tuple = ()
+        self._recs_versions: tuple = ()
         self.last_score_backend = "entry_arrays"  # what the last batch was scored from
 
     def synchronize(self) -> None:
@@ -460,7 +461,7 @@ class CostEngine:
         self.built = True
         self._table_clamp = (1 if clamp_inf else 0) if self.table is not None else None
         if self._versioned:
-            self._table_version = self.comm._version + self.cost._version + self.flags._version + self.per_arg._version
+            self._table_versions = self._array_versions()
         return self
 
     def build_timed(self, timer, slot: int, clamp_inf: bool = True):
@@ -477,7 +478,7 @@ class CostEngine:
         self.built = True
         self._table_clamp = clamp if self.table is not None else None
         if self._versioned:
-            self._table_version = self.comm._version + self.cost._version + self.flags._version + self.per_arg._version
+            self._table_versions = self._array_versions()
         return self
 
     def set_node_multiplier(self, mult: np.ndarray) -> None:
@@ -569,13 +570,22 @@ class CostEngine:
         self.last_score_backend = "entry_arrays"
         return out
 
+    def _array_versions(self) -> tuple:
+        if not self._versioned:
+            return ()
+        return self.comm._version, self.cost._version, self.flags._version, self.per_arg._version
+
+    def _table_stands(self) -> bool:
+        """Whether the entry arrays are what the last build made of the block table, so that a
+        scorer may read the table in their place.  Every scorer that does so asks here."""
+        return self._table_clamp is not None and self._table_versions == self._array_versions()
+
     def _score_small(self, assign, seed, first, count, d_gid, first_node, init, out) -> bool:
         """A small batch from the block table while it stands for the entry arrays; False: not done."""
-        if self._table_clamp is None or not _SCORE_SMALL_FROM_TABLE or not self.packed_scoring or count == 0:
+        if not _SCORE_SMALL_FROM_TABLE or not self.packed_scoring or count == 0:
             return False
-        if not self._versioned or self._table_version != (
-                self.comm._version + self.cost._version + self.flags._version + self.per_arg._version):
-            return False  # edited since the build
+        if not self._versioned or not self._table_stands():  # without counters an edit would go unnoticed
+            return False
         _lib.check(
             self.lib.apc_score_fold_table(
                 C.byref(self.problem), self._ptr(self.per_arg), self._ptr(self.table), self._ptr(assign), int(seed),
@@ -600,8 +610,8 @@ class CostEngine:
         cost is (comm + per_arg) + transition or its clamp (checked on the device
         when the records are made); else the 32-byte records that carry the cost
         (apc_score_packed)."""
-        if (self._table_clamp is not None and _SCORE_FROM_TABLE and (self.large_blocks or not _SCORE_COMPACT)
-                and count >= _SCORE_TABLE_FROM):
+        from_table = _SCORE_FROM_TABLE and self._table_stands()
+        if from_table and (self.large_blocks or not _SCORE_COMPACT) and count >= _SCORE_TABLE_FROM:
             aux = self._score_edge_aux(d_gid)
             _lib.check(
                 self.lib.apc_score_table(
@@ -613,10 +623,10 @@ class CostEngine:
                 "apc_score_table")
             self.last_score_backend = "block_table"
             return out
-        if (_SCORE_FROM_TABLE and count < _SCORE_TERMS_BELOW
+        if (from_table and count < _SCORE_TERMS_BELOW
                 and self._score_small(assign, seed, first, count, d_gid, first_node, init, out)):
             return out
-        if self._table_clamp is not None and _SCORE_FROM_TABLE and _SCORE_FROM_TILES and not self.large_blocks:
+        if from_table and self._versioned and _SCORE_FROM_TILES and not self.large_blocks:
             tiles = self._score_tiles(first_node, assign is not None)
             if tiles is not None:
                 steps, n_step, d_tiles, n_tile, units = tiles
@@ -630,7 +640,7 @@ class CostEngine:
                     "apc_score_from_tiles")
                 self.last_score_backend = "block_table_tiles"
                 return out
-        if not self._recs_valid:
+        if not self._recs_valid or self._recs_versions != self._array_versions():
             self._recs = None  # one kind at a time: either is as large as the entry arrays
             recs = None
             self._recs_compact = False
@@ -653,6 +663,7 @@ class CostEngine:
                     "apc_pack_score_records")
             self._recs = recs
             self._recs_valid = True
+            self._recs_versions = self._array_versions()
         if self._recs_compact:
             _lib.check(
                 self.lib.apc_score_compact(

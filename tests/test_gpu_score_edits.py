@@ -1,0 +1,65 @@
+"""Scores follow the entry arrays, whatever a batch is scored from: edits in place, arrays put in
+another's place, builds and edits replayed from a graph.  Wanted sums: those of a second engine that
+adopted the arrays as they are (load_results), which has no block table to go by."""
+import numpy as np
+import pytest
+import torch
+
+from autoparallel_amd import graphgen
+from autoparallel_amd.engine import CostEngine
+
+pytestmark = pytest.mark.gpu
+
+COUNTS = [70, 40000, 140000]  # terms side by side, the same from the table, by tiles (or the table edge by edge)
+
+
+@pytest.fixture(scope="module", params=["small_blocks", "large_blocks"])
+def engines(request):
+    g = graphgen.gpt2_graph((2, 3), 1, vocab=4096, seq=512, batch=64)
+    eng, other = CostEngine(g, table_mode="full"), CostEngine(g, table_mode="full")
+    eng.large_blocks = request.param == "large_blocks"
+    return eng, other
+
+
+def _bits(t):
+    return t.cpu().numpy().view(np.uint64)
+
+
+def _as_the_arrays_are(eng, other, count):
+    other.load_results(**{k: getattr(eng, k).cpu().numpy() for k in ("comm", "cost", "flags", "compute", "per_arg")})
+    return _bits(other.score_random(5, 9, count))
+
+
+def _table_backend(eng, count):
+    if count < 131072:
+        return "block_table_terms"
+    return "block_table" if eng.large_blocks else "block_table_tiles"
+
+
+@pytest.mark.parametrize("count", COUNTS)
+@pytest.mark.parametrize("array", ["cost", "comm"])
+def test_edits_in_place_are_followed(engines, array, count):
+    eng, other = engines
+    eng.build()
+    built = _bits(eng.score_random(5, 9, count))
+    assert eng.last_score_backend == _table_backend(eng, count)
+    assert (built == _as_the_arrays_are(eng, other, count)).all()
+    for _ in range(2):  # again after records were made of the first edit
+        getattr(eng, array).mul_(2.0)
+        got = _bits(eng.score_random(5, 9, count))
+        assert (got == _as_the_arrays_are(eng, other, count)).all() and not (got == built).all()
+    eng.build()  # rewrites the arrays: the table stands for them again
+    assert (_bits(eng.score_random(5, 9, count)) == built).all()
+    assert eng.last_score_backend == _table_backend(eng, count)
+
+
+@pytest.mark.parametrize("count", COUNTS[:2])
+def test_arrays_without_edit_counters_are_read(engines, count):
+    """Tensors made under inference mode count no edits: what is scored after a build is the arrays."""
+    other = engines[1]
+    with torch.inference_mode():
+        eng = CostEngine(engines[0].g, table_mode="full").build()
+        eng.cost.mul_(2.0)
+        got = _bits(eng.score_random(5, 9, count))
+        assert eng.last_score_backend == ("entry_arrays" if count < 32768 else "records")
+    assert (got == _as_the_arrays_are(eng, other, count)).all()
