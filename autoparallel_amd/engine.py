@@ -5,6 +5,7 @@ from __future__ import annotations
 
 import ctypes as C
 import threading
+import weakref
 from typing import Dict, Optional
 
 import numpy as np
@@ -158,6 +159,11 @@ def detect_device_name(device=None) -> str:
         if arch.startswith("gfx942"):
             return "AMD Instinct MI300X"
     return name
+
+
+def _edit_count(t: Optional[torch.Tensor]) -> int:
+    """How often torch has edited ``t`` in place; -1 where that is not counted."""
+    return -1 if t is None or t.is_inference() else t._version
 
 
 class CostEngine:
@@ -363,11 +369,12 @@ class CostEngine:
         # clamp_inf of the build whose table path wrote the entry arrays as they are now,
         # None once anything else has written them: then scoring cannot read the table instead
         self._table_clamp: Optional[int] = None
-        # and the arrays' version counters at that build, by which a caller's edit in place shows, as
-        # it does in those of the records' arrays (tensors made under inference_mode have none)
+        # and the arrays builds write, with their version counters at that build: another tensor put in the
+        # place of one, or a caller's edit in place, shows by them (tensors made under inference_mode
+        # have no counters); the same of the arrays that the records were made from
         self._versioned = not self.comm.is_inference()
-        self._table_versions: tuple = ()
-        self._recs_versions: tuple = ()
+        self._built_marks: tuple = ()
+        self._recs_marks: tuple = ()
         self.last_score_backend = "entry_arrays"  # what the last batch was scored from
 
     def synchronize(self) -> None:
@@ -445,6 +452,7 @@ class CostEngine:
             self._build_args = (
                 C.byref(self.problem), self._ptr(self.table), self._ptr(self.compute), self._ptr(self.per_arg),
                 self._ptr(self.status), self._ptr(self.comm), self._ptr(self.cost), self._ptr(self.flags))
+            self._built_marks = self._array_marks()
         return self._build_args
 
     def build(self, clamp_inf: bool = True):
@@ -460,8 +468,7 @@ class CostEngine:
             _lib.check(rc, "apc_build_all")
         self.built = True
         self._table_clamp = (1 if clamp_inf else 0) if self.table is not None else None
-        if self._versioned:
-            self._table_versions = self._array_versions()
+        self._mark_built()
         return self
 
     def build_timed(self, timer, slot: int, clamp_inf: bool = True):
@@ -477,8 +484,7 @@ class CostEngine:
         self._recs_valid = False
         self.built = True
         self._table_clamp = clamp if self.table is not None else None
-        if self._versioned:
-            self._table_versions = self._array_versions()
+        self._mark_built()
         return self
 
     def set_node_multiplier(self, mult: np.ndarray) -> None:
@@ -570,15 +576,24 @@ class CostEngine:
         self.last_score_backend = "entry_arrays"
         return out
 
-    def _array_versions(self) -> tuple:
-        if not self._versioned:
-            return ()
-        return self.comm._version, self.cost._version, self.flags._version, self.per_arg._version
+    def _array_marks(self) -> tuple:
+        return tuple((weakref.ref(t), t.data_ptr(), _edit_count(t))
+                     for t in (self.comm, self.cost, self.flags, self.per_arg))
+
+    def _mark_built(self) -> None:
+        """A build has rewritten the arrays: edits before it are gone."""
+        self._built_marks = tuple((ref, at, _edit_count(ref())) for ref, at, _ in self._built_marks)
+
+    def _unchanged(self, marks: tuple) -> bool:
+        """Whether the arrays are the marked ones, with no edit since."""
+        arrays = (self.comm, self.cost, self.flags, self.per_arg)
+        return len(marks) > 0 and all(ref() is t and at == t.data_ptr() and n == _edit_count(t)
+                                      for (ref, at, n), t in zip(marks, arrays))
 
     def _table_stands(self) -> bool:
         """Whether the entry arrays are what the last build made of the block table, so that a
         scorer may read the table in their place.  Every scorer that does so asks here."""
-        return self._table_clamp is not None and self._table_versions == self._array_versions()
+        return self._table_clamp is not None and self._unchanged(self._built_marks)
 
     def _score_small(self, assign, seed, first, count, d_gid, first_node, init, out) -> bool:
         """A small batch from the block table while it stands for the entry arrays; False: not done."""
@@ -640,7 +655,7 @@ class CostEngine:
                     "apc_score_from_tiles")
                 self.last_score_backend = "block_table_tiles"
                 return out
-        if not self._recs_valid or self._recs_versions != self._array_versions():
+        if not self._recs_valid or not self._unchanged(self._recs_marks):
             self._recs = None  # one kind at a time: either is as large as the entry arrays
             recs = None
             self._recs_compact = False
@@ -663,7 +678,7 @@ class CostEngine:
                     "apc_pack_score_records")
             self._recs = recs
             self._recs_valid = True
-            self._recs_versions = self._array_versions()
+            self._recs_marks = self._array_marks()
         if self._recs_compact:
             _lib.check(
                 self.lib.apc_score_compact(

@@ -63,3 +63,26 @@ def test_arrays_without_edit_counters_are_read(engines, count):
         got = _bits(eng.score_random(5, 9, count))
         assert eng.last_score_backend == ("entry_arrays" if count < 32768 else "records")
     assert (got == _as_the_arrays_are(eng, other, count)).all()
+
+
+@pytest.mark.parametrize("count", COUNTS)
+def test_an_array_in_anothers_place_is_scored(engines, count):
+    """The builds write the arrays the engine was made with; a tensor put in the place of one of them
+    is what the scorers read, also where its edit counter is that of the array it replaced."""
+    eng, other = engines
+    eng.build()
+    built, cost = _bits(eng.score_random(5, 9, count)), eng.cost
+    keep = cost.data
+    try:
+        for put in (lambda: setattr(eng, "cost", cost * 2.0), lambda: setattr(cost, "data", keep * 2.0)):
+            put()
+            for _ in range(2):
+                got = _bits(eng.score_random(5, 9, count))
+                assert (got == _as_the_arrays_are(eng, other, count)).all() and not (got == built).all()
+                eng.build()  # into ``keep``
+            eng.cost, cost.data = cost, keep
+    finally:
+        eng.cost, cost.data = cost, keep
+    eng.build()
+    assert (_bits(eng.score_random(5, 9, count)) == built).all()
+    assert eng.last_score_backend == _table_backend(eng, count)
