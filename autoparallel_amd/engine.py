@@ -369,10 +369,14 @@ class CostEngine:
         # clamp_inf of the build whose table path wrote the entry arrays as they are now,
         # None once anything else has written them: then scoring cannot read the table instead
         self._table_clamp: Optional[int] = None
-        # and the arrays builds write, with their version counters at that build: another tensor put in the
-        # place of one, or a caller's edit in place, shows by them (tensors made under inference_mode
-        # have no counters); the same of the arrays that the records were made from
+        # and the arrays builds write, with their version counters: another tensor put in the place of
+        # one, or a caller's edit in place, shows by them (tensors made under inference_mode have no
+        # counters); the same of the arrays that the records were made from.  A build takes the counters
+        # again only for a caller who has been seen to edit (a build of a small graph is bound by its
+        # host time, of which the four counters are 2%): after a first edit that only a build, and no
+        # scoring, has followed, scoring reads the arrays until the next build.
         self._versioned = not self.comm.is_inference()
+        self._edits_seen = False
         self._built_marks: tuple = ()
         self._recs_marks: tuple = ()
         self.last_score_backend = "entry_arrays"  # what the last batch was scored from
@@ -408,6 +412,7 @@ class CostEngine:
         """To be called by a caller that has written into comm / cost / flags / per_arg
         itself: scoring then reads the arrays as they are (records are made again on the
         next large batch, and the block table no longer stands for the arrays)."""
+        self._edits_seen = True
         self._recs_valid = False
         self._table_clamp = None
 
@@ -468,7 +473,8 @@ class CostEngine:
             _lib.check(rc, "apc_build_all")
         self.built = True
         self._table_clamp = (1 if clamp_inf else 0) if self.table is not None else None
-        self._mark_built()
+        if self._edits_seen:
+            self._mark_built()
         return self
 
     def build_timed(self, timer, slot: int, clamp_inf: bool = True):
@@ -484,7 +490,8 @@ class CostEngine:
         self._recs_valid = False
         self.built = True
         self._table_clamp = clamp if self.table is not None else None
-        self._mark_built()
+        if self._edits_seen:
+            self._mark_built()
         return self
 
     def set_node_multiplier(self, mult: np.ndarray) -> None:
@@ -504,7 +511,7 @@ class CostEngine:
         self.flags.copy_(torch.from_numpy(np.ascontiguousarray(flags, np.uint8)))
         self.compute.copy_(torch.from_numpy(np.ascontiguousarray(compute, np.float64)))
         self.per_arg.copy_(torch.from_numpy(np.ascontiguousarray(per_arg, np.float64)))
-        self.built = True
+        self.built = self._edits_seen = True
         self._recs_valid = False
         self._table_clamp = None
         return self
@@ -593,7 +600,11 @@ class CostEngine:
     def _table_stands(self) -> bool:
         """Whether the entry arrays are what the last build made of the block table, so that a
         scorer may read the table in their place.  Every scorer that does so asks here."""
-        return self._table_clamp is not None and self._unchanged(self._built_marks)
+        if self._table_clamp is None:
+            return False
+        stands = self._unchanged(self._built_marks)
+        self._edits_seen |= not stands
+        return stands
 
     def _score_small(self, assign, seed, first, count, d_gid, first_node, init, out) -> bool:
         """A small batch from the block table while it stands for the entry arrays; False: not done."""

@@ -5,6 +5,7 @@ import numpy as np
 import pytest
 import torch
 
+from autoparallel_amd import engine as engine_mod
 from autoparallel_amd import graphgen
 from autoparallel_amd.engine import CostEngine
 
@@ -86,3 +87,21 @@ def test_an_array_in_anothers_place_is_scored(engines, count):
     eng.build()
     assert (_bits(eng.score_random(5, 9, count)) == built).all()
     assert eng.last_score_backend == _table_backend(eng, count)
+
+
+def test_builds_ask_for_edits_only_where_a_caller_edits(engines, monkeypatch):
+    eng = CostEngine(engines[0].g, table_mode="full").build()
+    asked = []
+    count = engine_mod._edit_count
+    monkeypatch.setattr(engine_mod, "_edit_count", lambda t: asked.append(t) or count(t))
+    eng.build()
+    assert not asked
+    built = _bits(eng.score_random(5, 9, 70))
+    assert asked and eng.last_score_backend == "block_table_terms"
+    eng.cost.mul_(2.0)
+    eng.build()  # the edit is overwritten before it was seen: until the next build the arrays are read
+    assert (_bits(eng.score_random(5, 9, 70)) == built).all() and eng.last_score_backend == "entry_arrays"
+    for rewrite in (lambda: None, lambda: eng.cost.mul_(2.0), lambda: _as_the_arrays_are(eng, eng, 70)):
+        rewrite()
+        eng.build()
+        assert (_bits(eng.score_random(5, 9, 70)) == built).all() and eng.last_score_backend == "block_table_terms"
