@@ -377,6 +377,9 @@ class CostEngine:
         # scoring, has followed, scoring reads the arrays until the next build.
         self._versioned = not self.comm.is_inference()
         self._edits_seen = False
+        # what launches that write the arrays and were recorded in a graph leave in them whenever it is
+        # replayed: the clamp_inf of a build, None for anything else
+        self._recorded_writes: set = set()
         self._built_marks: tuple = ()
         self._recs_marks: tuple = ()
         self.last_score_backend = "entry_arrays"  # what the last batch was scored from
@@ -408,35 +411,49 @@ class CostEngine:
             "apc_node_compute_costs",
         )
 
+    def _capturing(self, stream) -> bool:
+        """Whether ``stream``, the current one (_stream()), records its launches in a graph."""
+        if not stream.value:  # the default stream never does
+            return False
+        with torch.cuda.device(self.device):
+            return torch.cuda.is_current_stream_capturing()
+
+    def _arrays_rewritten(self, stream) -> None:
+        """Something else than a build writes the arrays: now, or whenever a graph is replayed."""
+        self._recs_valid = False
+        self._table_clamp = None
+        if self._capturing(stream):
+            self._recorded_writes.add(None)
+
     def mark_results_edited(self) -> None:
         """To be called by a caller that has written into comm / cost / flags / per_arg
         itself: scoring then reads the arrays as they are (records are made again on the
-        next large batch, and the block table no longer stands for the arrays)."""
+        next large batch, and the block table no longer stands for the arrays).  Edits that
+        a graph makes when it is replayed are marked after the replay, or once for all
+        while they are recorded."""
         self._edits_seen = True
-        self._recs_valid = False
-        self._table_clamp = None
+        self._arrays_rewritten(self._stream())
 
     def edge_costs(self, clamp_inf: bool = True, want_comm: bool = True, want_flags: bool = True):
-        self._recs_valid = False
-        self._table_clamp = None
+        stream = self._stream()
+        self._arrays_rewritten(stream)
         _lib.check(
             self.lib.apc_edge_costs(
                 C.byref(self.problem), self._ptr(self.table), self._ptr(self.per_arg),
                 self._ptr(self.comm) if want_comm else None, self._ptr(self.cost),
-                self._ptr(self.flags) if want_flags else None, int(bool(clamp_inf)), self._stream()),
+                self._ptr(self.flags) if want_flags else None, int(bool(clamp_inf)), stream),
             "apc_edge_costs",
         )
 
     def edge_costs_timed(self, timer, slot: int, clamp_inf: bool = True):
         """edge_costs with HIP events at the kernel's begin and end (a timer from
         apc_timer_create); the launch is otherwise identical."""
-        self._recs_valid = False
-        self._table_clamp = None
+        stream = self._stream()
+        self._arrays_rewritten(stream)
         _lib.check(
             self.lib.apc_edge_costs_timed(
                 C.byref(self.problem), self._ptr(self.table), self._ptr(self.per_arg), self._ptr(self.comm),
-                self._ptr(self.cost), self._ptr(self.flags), int(bool(clamp_inf)), timer, int(slot),
-                self._stream()),
+                self._ptr(self.cost), self._ptr(self.flags), int(bool(clamp_inf)), timer, int(slot), stream),
             "apc_edge_costs_timed",
         )
 
@@ -475,6 +492,8 @@ class CostEngine:
         self._table_clamp = (1 if clamp_inf else 0) if self.table is not None else None
         if self._edits_seen:
             self._mark_built()
+        if stream and self._capturing(C.c_void_p(stream)):
+            self._recorded_writes.add(self._table_clamp)
         return self
 
     def build_timed(self, timer, slot: int, clamp_inf: bool = True):
@@ -492,6 +511,8 @@ class CostEngine:
         self._table_clamp = clamp if self.table is not None else None
         if self._edits_seen:
             self._mark_built()
+        if stream and self._capturing(C.c_void_p(stream)):
+            self._recorded_writes.add(self._table_clamp)
         return self
 
     def set_node_multiplier(self, mult: np.ndarray) -> None:
@@ -512,8 +533,7 @@ class CostEngine:
         self.compute.copy_(torch.from_numpy(np.ascontiguousarray(compute, np.float64)))
         self.per_arg.copy_(torch.from_numpy(np.ascontiguousarray(per_arg, np.float64)))
         self.built = self._edits_seen = True
-        self._recs_valid = False
-        self._table_clamp = None
+        self._arrays_rewritten(self._stream())
         return self
 
     def capture_build(self, clamp_inf: bool = True) -> "torch.cuda.CUDAGraph":
@@ -524,7 +544,8 @@ class CostEngine:
         argument lists).  The graph holds kernel nodes only (no memset nodes);
         it is valid while this engine's buffers live.  build() is run once
         eagerly first so that one-time function attributes are set outside the
-        capture."""
+        capture.  Scoring takes into account that a replay may have followed the
+        last eager build."""
         self.build(clamp_inf)
         torch.cuda.synchronize(self.device)
         graph = torch.cuda.CUDAGraph()
@@ -541,13 +562,13 @@ class CostEngine:
 
     def apply_prefetch_discount(self, scale: float = 0.0) -> int:
         assert self.built
-        self._recs_valid = False
-        self._table_clamp = None
+        stream = self._stream()
+        self._arrays_rewritten(stream)
         n = torch.zeros(1, dtype=torch.int64, device=self.device)
         _lib.check(
             self.lib.apc_apply_prefetch_discount(
                 C.byref(self.problem), self._ptr(self.per_arg), float(scale), self._ptr(self.comm),
-                self._ptr(self.cost), self._ptr(self.flags), self._ptr(n), self._stream()),
+                self._ptr(self.cost), self._ptr(self.flags), self._ptr(n), stream),
             "apc_apply_prefetch_discount",
         )
         return int(n.item())
@@ -599,8 +620,9 @@ class CostEngine:
 
     def _table_stands(self) -> bool:
         """Whether the entry arrays are what the last build made of the block table, so that a
-        scorer may read the table in their place.  Every scorer that does so asks here."""
-        if self._table_clamp is None:
+        scorer may read the table in their place.  Every scorer that does so asks here.
+        Recorded builds may have been replayed since: they change nothing where they clamp alike."""
+        if self._table_clamp is None or self._recorded_writes - {self._table_clamp}:
             return False
         stands = self._unchanged(self._built_marks)
         self._edits_seen |= not stands
@@ -610,13 +632,16 @@ class CostEngine:
         """A small batch from the block table while it stands for the entry arrays; False: not done."""
         if not _SCORE_SMALL_FROM_TABLE or not self.packed_scoring or count == 0:
             return False
+        stream = self._stream()
+        if count < _SCORE_LANES_FROM and self._capturing(stream):  # whatever the arrays hold on a replay
+            return False
         if not self._versioned or not self._table_stands():  # without counters an edit would go unnoticed
             return False
         _lib.check(
             self.lib.apc_score_fold_table(
                 C.byref(self.problem), self._ptr(self.per_arg), self._ptr(self.table), self._ptr(assign), int(seed),
                 int(first), int(count), self._ptr(d_gid), int(first_node), self._table_clamp, self._ptr(init),
-                self._ptr(out), self._stream()),
+                self._ptr(out), stream),
             "apc_score_fold_table")
         self.last_score_backend = "block_table_terms"
         return True
@@ -666,7 +691,8 @@ class CostEngine:
                     "apc_score_from_tiles")
                 self.last_score_backend = "block_table_tiles"
                 return out
-        if not self._recs_valid or not self._unchanged(self._recs_marks):
+        if not self._recs_valid or not self._unchanged(self._recs_marks) or (
+                self._recorded_writes and not self._capturing(self._stream())):  # replayed since, or not
             self._recs = None  # one kind at a time: either is as large as the entry arrays
             recs = None
             self._recs_compact = False

@@ -105,3 +105,63 @@ def test_builds_ask_for_edits_only_where_a_caller_edits(engines, monkeypatch):
         rewrite()
         eng.build()
         assert (_bits(eng.score_random(5, 9, 70)) == built).all() and eng.last_score_backend == "block_table_terms"
+
+
+@pytest.mark.parametrize("count", COUNTS)
+def test_replayed_builds_count(engines, count):
+    """A recorded build leaves its own clamp in the arrays whenever it is replayed; scores follow,
+    and where every recorded build has the last build's clamp the table goes on standing for them."""
+    eng = CostEngine(engines[0].g, table_mode="full")
+    eng.large_blocks = engines[0].large_blocks
+    other = engines[1]
+    graph = eng.capture_build(True)
+    for _ in range(3):
+        eng.build(True)
+        assert (_bits(eng.score_random(5, 9, count)) == _as_the_arrays_are(eng, other, count)).all()
+        assert eng.last_score_backend == _table_backend(eng, count)
+        graph.replay()
+        assert (_bits(eng.score_random(5, 9, count)) == _as_the_arrays_are(eng, other, count)).all()
+        for change in (lambda: eng.build(False), lambda: eng.apply_prefetch_discount(0.5)):
+            change()
+            assert (_bits(eng.score_random(5, 9, count)) == _as_the_arrays_are(eng, other, count)).all()
+            graph.replay()
+            assert (_bits(eng.score_random(5, 9, count)) == _as_the_arrays_are(eng, other, count)).all()
+
+
+def test_recorded_edits_and_entries_count(engines):
+    eng = CostEngine(engines[0].g, table_mode="full")
+    other = engines[1]
+    for record in (lambda: eng.edge_costs(clamp_inf=False), lambda: (eng.cost.mul_(2.0), eng.mark_results_edited())):
+        eng.build(True)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            record()
+        for _ in range(2):
+            eng.build(True)
+            graph.replay()
+            assert (_bits(eng.score_random(5, 9, 70)) == _as_the_arrays_are(eng, other, 70)).all()
+
+
+@pytest.mark.parametrize("explicit", [False, True])
+def test_a_recorded_small_score_reads_the_arrays(engines, explicit):
+    """Replays of a recorded score follow builds, edits and discounts between them."""
+    eng, other = engines
+    g = eng.g
+    rng = np.random.default_rng(1)
+    rows = (rng.integers(0, 1 << 20, (g.num_nodes, 70)) % g.node_nstrat[:, None]).astype(np.int16)
+    assign = torch.from_numpy(rows).cuda()
+    score = (lambda e: e.score(assign)) if explicit else (lambda e: e.score_random(5, 9, 70))
+    eng.build()
+    score(eng)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = score(eng)
+    for change in (lambda: eng.build(True), lambda: eng.apply_prefetch_discount(0.5), lambda: eng.cost.mul_(2.0),
+                   lambda: eng.build(False), lambda: eng.build(True)):
+        change()
+        graph.replay()
+        _as_the_arrays_are(eng, other, 70)
+        assert (_bits(out) == _bits(score(other))).all()
+    assert torch.equal(out.view(torch.int64), score(eng).view(torch.int64))
