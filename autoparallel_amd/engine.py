@@ -43,6 +43,9 @@ _SCORE_PER_LANE = 0  # assignments per lane of the compact scorer; 0: the librar
 # wavefronts, 2^20 31.5 and 33.2; planner DAG window (sixteen), 131 072 5.8 and 4.2, 262 144 7.1 and 8.3.
 _SAMPLE_LANES_FROM = {2: 1 << 20, 16: 1 << 18}
 _SAMPLE_WAVES = 0  # 2 or 16: tests
+# Layouts of a kind (by first_node) an engine makes.  They stay until the engine goes, since a launch on
+# another stream or in a graph may still read one; calls beyond take the route that needs none.
+_LAYOUTS_KEPT = 16
 _READBACK_PINNED = True  # results() copies into pinned host memory (else pageable)
 _LUT_TABLE_FROM = 2048  # table units: larger tables are built tile by tile with per-source terms in LDS
 
@@ -207,6 +210,7 @@ class CostEngine:
         assert g.num_edges == 0 or int(sizes.max()) < 2**31, "edge block too large for 32-bit local index"
 
         self._keep: Dict[str, torch.Tensor] = {}
+        self._layouts: Dict[str, dict] = {"score_tiles": {}, "score_tiles_explicit": {}, "sample_steps": {}}
 
         # The problem is some thirty arrays, most of them a few kilobytes: they go up in
         # one copy.  An array is laid into a pinned staging buffer and gets its address
@@ -637,6 +641,9 @@ class CostEngine:
             return False
         if not self._versioned or not self._table_stands():  # without counters an edit would go unnoticed
             return False
+        return self._score_terms(assign, seed, first, count, d_gid, first_node, init, out, stream)
+
+    def _score_terms(self, assign, seed, first, count, d_gid, first_node, init, out, stream) -> bool:
         _lib.check(
             self.lib.apc_score_fold_table(
                 C.byref(self.problem), self._ptr(self.per_arg), self._ptr(self.table), self._ptr(assign), int(seed),
@@ -691,8 +698,15 @@ class CostEngine:
                     "apc_score_from_tiles")
                 self.last_score_backend = "block_table_tiles"
                 return out
-        if not self._recs_valid or not self._unchanged(self._recs_marks) or (
-                self._recorded_writes and not self._capturing(self._stream())):  # replayed since, or not
+        stream = self._stream()
+        capturing = self._capturing(stream)
+        recs_stand = (self._recs_valid and self._unchanged(self._recs_marks)
+                      and (capturing or not self._recorded_writes))  # else replayed since, or not
+        if capturing and not recs_stand and from_table and self._versioned:
+            # records are not made while a graph is recorded (their check is read by the host)
+            self._score_terms(assign, seed, first, count, d_gid, first_node, init, out, stream)
+            return out
+        if not recs_stand:
             self._recs = None  # one kind at a time: either is as large as the entry arrays
             recs = None
             self._recs_compact = False
@@ -735,13 +749,23 @@ class CostEngine:
         return out
 
     def _score_tiles(self, first_node: int, explicit: bool):
-        """The layout apc_score_from_tiles walks from ``first_node`` on, on the device, or None for
-        a graph that form does not take.  Made once per first_node, for random and for explicit
-        assignments; the last of each is kept."""
-        key = "score_tiles_explicit" if explicit else "score_tiles"
-        kept = self._keep.get(key)
-        if kept is not None and kept[0] == first_node:
-            return kept[1]
+        """The layout apc_score_from_tiles walks from ``first_node`` on, on the device, or None:
+        a graph that form does not take, or no layout at hand (_layout)."""
+        return self._layout("score_tiles_explicit" if explicit else "score_tiles", first_node,
+                            lambda: self._make_score_tiles(first_node, explicit))
+
+    def _layout(self, kind: str, first_node: int, make):
+        """``make()`` for the walk from ``first_node`` on, made once.  None too once
+        _LAYOUTS_KEPT have been made, and while a graph is recorded, where nothing can be copied to
+        the device."""
+        kept = self._layouts[kind]
+        if first_node in kept:
+            return kept[first_node]
+        if len(kept) >= _LAYOUTS_KEPT or self._capturing(self._stream()):
+            return None
+        return kept.setdefault(first_node, make())
+
+    def _make_score_tiles(self, first_node: int, explicit: bool):
         g = self.g
         plan = None
         if self.table_mode == "full" and first_node < g.num_nodes:
@@ -767,7 +791,6 @@ class CostEngine:
                 plan = (torch.from_numpy(steps[:n_step]).to(self.device), n_step,
                         torch.from_numpy(tiles[:n_tile]).to(self.device), n_tile,
                         torch.from_numpy(units[:n_unit]).to(self.device))
-        self._keep[key] = (first_node, plan)
         return plan
 
     def _score_msize(self) -> np.ndarray:
@@ -953,13 +976,12 @@ class CostEngine:
 
     def _sample_steps(self, first_node: int):
         """(records on the device, steps, wavefronts) of apc_sample_feasible_steps for the walk
-        from ``first_node`` on, or None for a graph such a walk does not take (columns past its
-        32-bit offsets, a producer behind its consumer).  Made once per first_node; the last one
-        is kept."""
+        from ``first_node`` on, or None: a graph such a walk does not take (columns past its
+        32-bit offsets, a producer behind its consumer), or no layout at hand (_layout)."""
+        return self._layout("sample_steps", first_node, lambda: self._make_sample_steps(first_node))
+
+    def _make_sample_steps(self, first_node: int):
         g = self.g
-        kept = self._keep.get("sample_steps")
-        if kept is not None and kept[0] == first_node:
-            return kept[1]
         n = g.num_nodes - first_node
         plan = None
         if (n > 0 and g.num_edges > 0 and g.num_nodes < 1 << 24 and (g.edge_src_node < g.edge_node).all()
@@ -980,7 +1002,6 @@ class CostEngine:
                 "apc_sample_steps")
             recs = torch.from_numpy(recs[:n_step.value * n_waves.value]).to(self.device)
             plan = (recs, n_step.value, n_waves.value)
-        self._keep["sample_steps"] = (first_node, plan)
         return plan
 
     def sample_feasible(self, seed: int, first: int, count: int, node_gid: Optional[np.ndarray] = None,

@@ -165,3 +165,51 @@ def test_a_recorded_small_score_reads_the_arrays(engines, explicit):
         _as_the_arrays_are(eng, other, 70)
         assert (_bits(out) == _bits(score(other))).all()
     assert torch.equal(out.view(torch.int64), score(eng).view(torch.int64))
+
+
+def test_scores_and_draws_are_recorded_without_a_layout_at_hand(engines):
+    """A layout cannot be copied to the device while a graph is recorded: a call whose layout is not
+    there yet is recorded over another route, with the same results on every replay."""
+    eng = CostEngine(engines[0].g, table_mode="full")
+    g = eng.g
+    n = 140000
+    gen = torch.Generator(device="cuda").manual_seed(2)
+    nstrat = torch.from_numpy(g.node_nstrat.astype(np.int32)).cuda()[:, None]
+    assign = (torch.randint(0, 1 << 30, (g.num_nodes, n), device="cuda", generator=gen, dtype=torch.int32)
+              % nstrat).to(torch.int16)
+    drawn = torch.zeros((g.num_nodes, 300), dtype=torch.int16, device="cuda").view(torch.uint16)
+    eng.build()
+    eng.sample_feasible(3, 0, 300)
+    eng.score_random(5, 9, 40000)
+    torch.cuda.synchronize()
+    calls = [lambda: eng.score_random(5, 9, n), lambda: eng.score(assign), lambda: eng.score_window(assign, 5),
+             lambda: eng.sample_feasible(3, 0, 300, first_node=7, assign=drawn)[0].view(torch.int16).clone()]
+    recorded = []
+    for call in calls:
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            out = call()
+        recorded.append((graph, out))
+    for _ in range(3):
+        for call, (graph, out) in zip(calls, recorded):
+            out.zero_()
+            graph.replay()
+            got = out.cpu().numpy().tobytes()
+            want = call()
+            torch.cuda.synchronize()
+            assert got == want.cpu().numpy().tobytes()
+
+
+def test_layouts_stay_where_they_are(engines):
+    """A launch on another stream or in a graph may still read a layout when another first_node is
+    asked for: none is let go or moved while the engine lives, and only so many are made."""
+    eng = engines[0]
+    eng.build()
+    eng.sample_feasible(3, 0, 64)
+    kinds = [lambda v: eng._score_tiles(v, False), lambda v: eng._score_tiles(v, True), eng._sample_steps]
+    for kind in kinds:
+        first = kind(0)
+        for v in range(1, 40):
+            kind(v)
+        assert kind(0) is first
+        assert sum(kind(v) is not None for v in range(40)) == engine_mod._LAYOUTS_KEPT

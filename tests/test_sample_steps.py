@@ -110,7 +110,7 @@ def test_draws_equal_the_lane_walks(name, n_waves, count, monkeypatch):
 
     monkeypatch.setattr(engine_mod, "_SAMPLE_WAVES", n_waves)
     got = draws()
-    assert eng._keep["sample_steps"][1][2] == n_waves
+    assert eng._sample_steps(first_node)[2] == n_waves
     monkeypatch.setattr(engine_mod, "_SAMPLE_LANES_FROM", {2: 0, 16: 0})
     for a, b in zip(got, draws()):
         assert (a == b).all()
