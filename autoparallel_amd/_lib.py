@@ -12,6 +12,7 @@ LIB_PATH = os.path.join(_HERE, "libapc_hip.so")
 
 MAX_MESH_DIMS = 4
 NUM_DTYPES = 8
+ERR_UNSUPPORTED = -3
 SAMPLE_ARGS = 6  # argument rows an apc_sample_rec names
 SAMPLE_REC_BYTES = 64
 CHECK_MAX_NODES = 131072

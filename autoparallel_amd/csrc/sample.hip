@@ -533,7 +533,7 @@ int apc_sample_steps(int32_t n_node, int32_t n_edge, const int32_t* node_edge_of
     int left = n, t = 0;
     std::vector<int32_t> taken;
     for (; left > 0; ++t) {
-      if (t >= max_step) return fail(APC_ERR_INVALID, "apc_sample_steps: more steps than max_step%s");
+      if (t >= max_step) return fail(APC_ERR_UNSUPPORTED, "apc_sample_steps: more steps than max_step%s");
       if (t < (int)held.size())
         for (int v : held[t]) ready.push(v);
       taken.clear();

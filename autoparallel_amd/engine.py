@@ -977,7 +977,7 @@ class CostEngine:
     def _sample_steps(self, first_node: int):
         """(records on the device, steps, wavefronts) of apc_sample_feasible_steps for the walk
         from ``first_node`` on, or None: a graph such a walk does not take (columns past its
-        32-bit offsets, a producer behind its consumer), or no layout at hand (_layout)."""
+        32-bit offsets, a producer behind its consumer, more steps than nodes), or no layout at hand (_layout)."""
         return self._layout("sample_steps", first_node, lambda: self._make_sample_steps(first_node))
 
     def _make_sample_steps(self, first_node: int):
@@ -990,16 +990,18 @@ class CostEngine:
             src = np.ascontiguousarray(g.edge_src_node, np.int32)
             nstrat = np.ascontiguousarray(g.node_nstrat, np.int32)
             col_off = self._keep["column_layout_host"]
-            long_rows = int((np.diff(edge_off) > _lib.SAMPLE_ARGS).sum())
             n_step, n_waves = C.c_int32(0), C.c_int32(0)
-            max_step = n + 128 * long_rows
-            recs = np.empty((max_step * 16, _lib.SAMPLE_REC_BYTES), np.uint8)
-            _lib.check(
-                self.lib.apc_sample_steps(
-                    g.num_nodes, g.num_edges, edge_off.ctypes.data, src.ctypes.data, nstrat.ctypes.data,
-                    col_off.ctypes.data, int(first_node), _SAMPLE_WAVES, recs.ctypes.data, max_step,
-                    C.byref(n_step), C.byref(n_waves)),
-                "apc_sample_steps")
+            # A node with more argument rows than a record names waits until its producers have left the
+            # ring, 8 or 64 steps.  A step takes about as long as a node of the lane walk (1.2 and 1.5 us), so a
+            # walk of more steps than nodes is no gain.
+            recs = np.empty((n * 16, _lib.SAMPLE_REC_BYTES), np.uint8)
+            rc = self.lib.apc_sample_steps(
+                g.num_nodes, g.num_edges, edge_off.ctypes.data, src.ctypes.data, nstrat.ctypes.data,
+                col_off.ctypes.data, int(first_node), _SAMPLE_WAVES, recs.ctypes.data, n,
+                C.byref(n_step), C.byref(n_waves))
+            if rc == _lib.ERR_UNSUPPORTED:
+                return None
+            _lib.check(rc, "apc_sample_steps")
             recs = torch.from_numpy(recs[:n_step.value * n_waves.value]).to(self.device)
             plan = (recs, n_step.value, n_waves.value)
         return plan

@@ -693,8 +693,8 @@ uint32_t apc_sample_rank(uint64_t seed, int64_t a, int32_t node, uint32_t count)
  * lays the nodes from first_node on out in steps of up to n_waves (asked for, or 0: chosen by how
  * many nodes are ready at a time; what was taken is stored in n_waves_out) nodes whose producers
  * all lie in earlier steps: records recs[n_step][n_waves] (room for max_step steps; n_node
- * steps and 128 more per node with over APC_SAMPLE_ARGS argument rows always suffice), to be copied
- * to the device.  It needs every producer in front of its consumer (edge_src[e] < node)
+ * steps and 128 more per node with over APC_SAMPLE_ARGS argument rows always suffice, and
+ * APC_ERR_UNSUPPORTED says that max_step do not), to be copied to the device.  It needs every producer in front of its consumer (edge_src[e] < node)
  * and reads nothing that a build writes, so one layout serves every call with the same
  * graph, first_node and col_off.  apc_sample_feasible_steps then is apc_sample_feasible
  * over those records, same results bit for bit. */

@@ -79,7 +79,54 @@ def test_layout_refuses():
         _layout(off, [0], one, [0], 0, 3)
 
 
+def test_layout_says_when_there_are_more_steps_than_room():
+    """A chain of nodes with seven argument rows: each waits until its producer has left the ring."""
+    n = 40
+    src = np.repeat(np.arange(-1, n - 1), 7).astype(np.int32)
+    recs, n_step, waves = np.zeros(129 * n * 16, REC), C.c_int32(), C.c_int32()
+    a = [np.ascontiguousarray(x, t) for x, t in ((7 * np.arange(n + 1), np.int32), (src, np.int32),
+                                                 (np.full(n, 5), np.int32), (np.zeros(7 * n), np.int64))]
+
+    def steps(room):
+        rc = _lib.load().apc_sample_steps(n, 7 * n, *[x.ctypes.data for x in a], 0, 2, recs.ctypes.data, room,
+                                          C.byref(n_step), C.byref(waves))
+        return rc, n_step.value
+
+    rc, most = steps(129 * n)
+    assert rc == 0 and most > 60 * (n - 1)
+    assert steps(most) == (0, most)
+    for room in (most - 1, n):
+        assert steps(room) == (_lib.ERR_UNSUPPORTED, 0)
+
+
+def _long_rows(chain):
+    """Nodes with eight argument rows, one after the other or among many of one row."""
+    import itertools
+
+    from autoparallel_amd import packed
+    from autoparallel_amd.packed import GraphBuilder, NodeDesc
+
+    b = GraphBuilder((2, 2), 4)
+    m = b.meta((8, 16, 32), (512, 32, 1), 4, packed.DT_F32)
+    tuples = list(itertools.product([0x00, 0x40, 0x41, 0x42, 0x80], repeat=2))
+    rng = np.random.default_rng(1)
+
+    def specs(n):
+        return [b.spec(m, tuples[i]) for i in rng.choice(len(tuples), n, replace=False)]
+
+    first = specs(6)
+    at = [b.add_node(NodeDesc("first", in_specs=[[x] for x in first], out_specs=[[x] for x in first], inputs=[],
+                              default_rows=[[[0.0]] for _ in first]))]
+    for v in range(1, 20 if chain else 400):
+        s, rows = specs(int(rng.integers(2, 12))), 8 if chain or v % 100 == 0 else 1
+        inputs = [at[-1]] * 8 if chain else [int(x) for x in rng.integers(max(0, v - 300), v, rows)]
+        at.append(b.add_node(NodeDesc(f"n{v}", in_specs=[[x] * rows for x in s], out_specs=[[x] for x in s],
+                                      inputs=inputs)))
+    return b.pack(), None, 0
+
+
 GRAPHS = {
+    "long_rows": lambda: _long_rows(False),
     "gpt2": lambda: (graphgen.gpt2_graph((2, 3), 2, vocab=4096, seq=512, batch=64), None, 0),
     "llama_8x8": lambda: (graphgen.llama_graph((8, 8), 1, 1024, 8, 4, 2048, 8192, 512, 16), None, 0),
     "stress_512": lambda: (graphgen.stress_graph(60, (2, 2, 4), seed=4, s_min=2, s_max=700), None, 0),
@@ -114,3 +161,10 @@ def test_draws_equal_the_lane_walks(name, n_waves, count, monkeypatch):
     monkeypatch.setattr(engine_mod, "_SAMPLE_LANES_FROM", {2: 0, 16: 0})
     for a, b in zip(got, draws()):
         assert (a == b).all()
+
+
+@pytest.mark.gpu
+def test_a_chain_of_long_argument_rows_is_drawn_by_lanes():
+    eng = engine_mod.CostEngine(_long_rows(True)[0]).build()
+    eng.sample_feasible(3, 17, 64)
+    assert eng._sample_steps(0) is None
