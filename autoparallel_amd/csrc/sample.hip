@@ -643,7 +643,9 @@ int apc_sample_feasible(const apc_problem* p, const uint64_t* colbits, const int
   if ((row_filter == nullptr) != (filter_off == nullptr))
     return fail(APC_ERR_INVALID, "apc_sample_feasible: row_filter and filter_off come together%s");
   const dim3 grid((unsigned)((n_assign + kBlock - 1) / kBlock));
-  if (n_assign < 65536)  // fewer wavefronts than SIMDs
+  // Fewer wavefronts than SIMDs: batches that apc_sample_feasible_steps does not take (a layout that
+  // cannot be had or would be longer than the walk).
+  if (n_assign < 65536)
     hipLaunchKernelGGL(sample_feasible_kernel<true>, grid, dim3(kBlock), 0, (hipStream_t)stream, *p, colbits, col_off,
                        seed, first, n_assign, node_gid, (int)first_node, row_filter, filter_off, assign, n_fallback);
   else

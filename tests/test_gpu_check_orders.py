@@ -32,6 +32,21 @@ def test_check_orders(n_node, n_sched):
         wrong = orders.copy()
         wrong[n_sched - 1, 0] = wrong[n_sched - 1, n_node - 1]
         assert _bad(wrong)
+
+
+def test_check_orders_at_the_limit():
+    """131 072 nodes: four bitmaps fill the 64 KB of LDS a launch may ask for."""
     limit = _lib.CHECK_MAX_NODES
+    rng = np.random.default_rng(0)
+    orders = np.stack([rng.permutation(limit) for _ in range(6)])
+    assert not _bad(orders)
+    for row, col, value in ((5, limit - 1, limit), (0, 0, -1)):
+        wrong = orders.copy()
+        wrong[row, col] = value
+        assert _bad(wrong)
+    for row in (0, 3, 5):  # one node twice, in the bitmap of the first and the last wavefront too
+        wrong = orders.copy()
+        wrong[row, 17] = wrong[row, limit - 1]
+        assert _bad(wrong)
     d = torch.zeros(1, dtype=torch.int32, device="cuda")
     assert _lib.load().apc_check_orders(d.data_ptr(), 1, limit + 1, d.data_ptr(), None) != 0  # refused by the host

@@ -5,6 +5,7 @@ import numpy as np
 import pytest
 import torch
 
+from autoparallel_amd import engine as engine_mod
 from autoparallel_amd import graphgen
 from oracle import cost_oracle as O
 
@@ -28,7 +29,7 @@ def CostEngine():
 
 
 @pytest.mark.parametrize("name", list(GRAPHS))
-def test_sampled_assignments_equal_the_oracles(CostEngine, name):
+def test_sampled_assignments_equal_the_oracles(CostEngine, name, monkeypatch):
     g = GRAPHS[name]()
     print(f"  sampler: {name} nodes={g.num_nodes} E={g.num_entries}", flush=True)
     eng = CostEngine(g).build(clamp_inf=True)
@@ -58,12 +59,17 @@ def test_sampled_assignments_equal_the_oracles(CostEngine, name):
     # and the plain draws of the same counters do select forbidden variables on these graphs
     plain = eng.score_random(9, 1000, n).cpu().numpy()
     assert (plain[:, 5] > 0).mean() > (scores[:, 5] > 0).mean()
-    # a large batch: the same choices for the same counters
-    big, big_fb = eng.sample_feasible(seed=9, first=1000, count=65536)
-    assert np.array_equal(big[:, :n].cpu().numpy(), assign) and np.array_equal(big_fb[:n].cpu().numpy(), fallback)
+    # a large batch: the same choices for the same counters, in steps and by lanes
     a = 65535
     want, want_fb = O.sample_feasible(g, forbidden, 9, 1000 + a)
-    assert big[:, a].cpu().numpy().tolist() == want and int(big_fb[a]) == want_fb
+    for lanes in (False, True):
+        if lanes:
+            monkeypatch.setattr(engine_mod, "_SAMPLE_LANES_FROM", {2: 0, 16: 0})
+        for count in (n, 65536):  # a lane walk of few wavefronts is another instance of the kernel
+            big, big_fb = eng.sample_feasible(seed=9, first=1000, count=count)
+            assert np.array_equal(big[:, :n].cpu().numpy(), assign)
+            assert np.array_equal(big_fb[:n].cpu().numpy(), fallback)
+        assert big[:, a].cpu().numpy().tolist() == want and int(big_fb[a]) == want_fb
 
 
 def test_sampler_continues_from_given_rows(CostEngine):
@@ -150,7 +156,7 @@ def test_bit_columns_are_the_flags_and_wide_nodes_sample_like_the_oracle(CostEng
     assert picked_high
 
 
-def test_filtered_draws_equal_the_oracle_and_never_fall_back(CostEngine):
+def test_filtered_draws_equal_the_oracle_and_never_fall_back(CostEngine, monkeypatch):
     """Row filters from the plan (feasible_plan): the device's draws equal the oracle's
     with the same filters, no node falls back and no forbidden entry is selected, where
     the walk without filters falls back several times per assignment."""
@@ -174,6 +180,11 @@ def test_filtered_draws_equal_the_oracle_and_never_fall_back(CostEngine):
     for a in range(0, n, 7):
         want, want_fb = O.sample_feasible(g, forbidden, 4, a, row_filter=filters)
         assert assign[:, a].tolist() == want and want_fb == 0, a
-    # the launch that fills the chip (another instance of the kernel): the same draws
-    big, big_fb = eng.sample_feasible(seed=4, first=0, count=65536, row_filter=filters)
-    assert int(big_fb.sum().item()) == 0 and (big[:, :n].cpu().numpy() == assign).all()
+    # the launches that fill the chip, in steps and by lanes (another instance of the kernel for
+    # few wavefronts): the same draws
+    for lanes in (False, True):
+        if lanes:
+            monkeypatch.setattr(engine_mod, "_SAMPLE_LANES_FROM", {2: 0, 16: 0})
+        for count in (n, 65536):
+            big, big_fb = eng.sample_feasible(seed=4, first=0, count=count, row_filter=filters)
+            assert int(big_fb.sum().item()) == 0 and (big[:, :n].cpu().numpy() == assign).all()

@@ -88,10 +88,11 @@ def test_layout_leaves_other_graphs_alone():
     assert len(_layout(g, 0, 0)[1]) == 0
 
 
-# one assignment a lane up to 2^18, then two, then four (two, and a second launch, if explicit)
+# one assignment a lane up to 2^18, then two, then four (two, and a second launch, if explicit); past 2^20
+# random ones take a second launch too
 @pytest.mark.gpu
-@pytest.mark.parametrize("count", [1, 129, 33000, 262145, 524289])
-@pytest.mark.parametrize("name", list(GRAPHS))
+@pytest.mark.parametrize("name,count", [(name, count) for name in GRAPHS for count in (1, 129, 33000, 262145, 524289)]
+                         + [("gpt2_2x3", 2**20 + 65)])
 def test_scores_have_the_bits_of_the_walk_over_records(name, count, monkeypatch):
     g = GRAPHS[name]()
     eng = engine_mod.CostEngine(g, table_mode="full").build()
