@@ -23,10 +23,12 @@ _SCORE_COMPACT = True
 _SCORE_SMALL_FROM_TABLE = True
 _SCORE_FROM_TILES = True  # small blocks: matrices through LDS by tiles, while the table stands for the arrays
 # Below, the terms of a few assignments gathered side by side are faster than any walk with a lane per
-# assignment (side by side, by tiles): Llama-3-8B graph, random 65 536 2.5 and 5.9 ms, 131 072 5.5 and 4.8, explicit
-# ones 3.2 and 6.6, 7.2 and 5.7; window of the planner DAG (side by side, table scorer) 65 536 1.95 and 5.4, 131 072
-# 4.7 and 5.3, 262 144 11.2 and 5.3.
-_SCORE_TERMS_BELOW = 131072
+# assignment: up to here a CU takes seven workgroups of 64, an eighth costs more than a walk's lanes do.  In
+# ms, at 65 536, 110 000 and 120 000 random assignments: Llama-3-8B graph side by side 2.35, 4.58, 5.00, by tiles
+# 5.90, 4.97, 4.82 (explicit ones 3.13, 5.88, 6.76 and 6.57, 5.90, 5.74); window of the planner DAG side by
+# side 1.89, 3.61, 4.12, from records 3.84, 3.87, 3.90 (explicit 2.17, 4.11, 4.85 and 4.41, 4.47, 4.50), table
+# scorer 5.3.  The 12-layer GPT-2 graph crosses earlier, at 90 000 (1.22 and 1.24).
+_SCORE_TERMS_BELOW = 114688
 # Matrices of up to this many LDS tiles (64 KB each) go through LDS in the table scorer, larger
 # ones are read in place.  Measured on a 3 000-node window of the stress DAG, 2^20 assignments:
 # 17.9 ms with 1, 17.4 with 2, 18.0 with 4, 18.35 with 8 or 16.  (A lower bound, small matrices
@@ -619,8 +621,10 @@ class CostEngine:
     def _unchanged(self, marks: tuple) -> bool:
         """Whether the arrays are the marked ones, with no edit since."""
         arrays = (self.comm, self.cost, self.flags, self.per_arg)
-        return len(marks) > 0 and all(ref() is t and at == t.data_ptr() and n == _edit_count(t)
-                                      for (ref, at, n), t in zip(marks, arrays))
+        for (ref, at, n), t in zip(marks, arrays):
+            if ref() is not t or t.data_ptr() != at or (n >= 0 and t._version != n):
+                return False
+        return len(marks) > 0
 
     def _table_stands(self) -> bool:
         """Whether the entry arrays are what the last build made of the block table, so that a

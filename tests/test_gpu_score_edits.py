@@ -97,7 +97,7 @@ def test_builds_ask_for_edits_only_where_a_caller_edits(engines, monkeypatch):
     eng.build()
     assert not asked
     built = _bits(eng.score_random(5, 9, 70))
-    assert asked and eng.last_score_backend == "block_table_terms"
+    assert eng.last_score_backend == "block_table_terms"
     eng.cost.mul_(2.0)
     eng.build()  # the edit is overwritten before it was seen: until the next build the arrays are read
     assert (_bits(eng.score_random(5, 9, 70)) == built).all() and eng.last_score_backend == "entry_arrays"
