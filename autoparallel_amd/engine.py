@@ -40,10 +40,14 @@ _SCORE_STAGE_TILES = 2
 # 2^20, 78 ms from compact records for 2^20)
 _SCORE_TABLE_FROM = 131072
 _SCORE_PER_LANE = 0  # assignments per lane of the compact scorer; 0: the library chooses
-# assignments from which one lane each beats several wavefronts per 64 assignments, by the number
-# of wavefronts.  Measured: Llama-3-8B graph (two), 524 288 assignments 21.2 ms by lanes and 17.5 by
-# wavefronts, 2^20 31.5 and 33.2; planner DAG window (sixteen), 131 072 5.8 and 4.2, 262 144 7.1 and 8.3.
-_SAMPLE_LANES_FROM = {2: 1 << 20, 16: 1 << 18}
+# Assignments from which one lane each beats several wavefronts per 64 assignments, by the number
+# of wavefronts.  Lanes go in rounds of 2^18 that cost the same however full, wavefronts by the
+# assignment, so that near the end of a round the lanes win: from seven eighths of the second round (of the
+# first, with sixteen) on.  In ms, wavefronts and lanes: two, at 400 000 and 524 288 assignments, 12-layer GPT-2
+# graph 4.74, 5.93 and 6.02, 6.02, 4-layer 70B decoder on 4x8x8 2.65, 3.22 and 3.36, 3.22, Llama-3-8B graph 13.7,
+# 20.2 and 17.5, 21.2; at 1 048 575 12.2, 11.1 and 6.49, 5.99 and 35.5, 35.4.  Sixteen, at 220 000 and 262 143,
+# window of the planner DAG of 1 600 nodes 5.49, 6.33 and 6.34, 6.30, of 60 nodes 0.242, 0.260 and 0.270, 0.262.
+_SAMPLE_LANES_FROM = {2: 458752, 16: 229376}
 _SAMPLE_WAVES = 0  # 2 or 16: tests
 # Layouts of a kind (by first_node) an engine makes.  They stay until the engine goes, since a launch on
 # another stream or in a graph may still read one; calls beyond take the route that needs none.
