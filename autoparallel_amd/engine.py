@@ -390,7 +390,7 @@ class CostEngine:
         # what launches that write the arrays and were recorded in a graph leave in them whenever it is
         # replayed: the clamp_inf of a build, None for anything else
         self._recorded_writes: set = set()
-        self._built_marks: tuple = ()
+        self._built_marks = self._array_marks()
         self._recs_marks: tuple = ()
         self.last_score_backend = "entry_arrays"  # what the last batch was scored from
 
@@ -398,8 +398,14 @@ class CostEngine:
         torch.cuda.synchronize(self.device)
 
     # -- raw stream -----------------------------------------------------------
+    # The handle alone: a torch.cuda.Stream made for every call costs 3 us of host time, a third
+    # of what issuing a build takes.
+    def _raw_stream(self) -> int:
+        index = self.device.index
+        return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
+
     def _stream(self):
-        return C.c_void_p(torch.cuda.current_stream(self.device).cuda_stream)
+        return C.c_void_p(self._raw_stream())
 
     @staticmethod
     def _ptr(t: Optional[torch.Tensor]):
@@ -484,7 +490,6 @@ class CostEngine:
             self._build_args = (
                 C.byref(self.problem), self._ptr(self.table), self._ptr(self.compute), self._ptr(self.per_arg),
                 self._ptr(self.status), self._ptr(self.comm), self._ptr(self.cost), self._ptr(self.flags))
-            self._built_marks = self._array_marks()
         return self._build_args
 
     def build(self, clamp_inf: bool = True):
@@ -494,7 +499,7 @@ class CostEngine:
         # the argument list is the same from call to call apart from the stream:
         # made once, so that issuing a step costs less host time than the step takes
         args = self._build_args or self.build_args()
-        stream = torch.cuda.current_stream(self.device).cuda_stream
+        stream = self._raw_stream()
         rc = self.lib.apc_build_all(*args, 1 if clamp_inf else 0, stream)
         if rc:
             _lib.check(rc, "apc_build_all")
@@ -511,7 +516,7 @@ class CostEngine:
         the entries (a timer from apc_timer_create); the launches are otherwise
         identical."""
         self.build_args()
-        stream = torch.cuda.current_stream(self.device).cuda_stream
+        stream = self._raw_stream()
         clamp = 1 if clamp_inf else 0
         rc = self.lib.apc_build_all_timed(*self._build_args, clamp, timer, int(slot), stream)
         if rc:
