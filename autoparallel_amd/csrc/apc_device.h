@@ -51,6 +51,47 @@ typedef double double2_t __attribute__((ext_vector_type(2)));
 typedef long long ll2_t __attribute__((ext_vector_type(2)));
 
 // ---------------------------------------------------------------------------
+// Draws.  A counter-based 32-bit mix of (seed, assignment, node), scaled to a count by a
+// multiply-high: callers repeat it on the host (apc_random_assignment, apc_sample_rank), so every
+// scorer and sampler takes it from here.  The walks are bound by instructions, and a 64-bit mix
+// with a modulo that was here before took a quarter of them.
+// ---------------------------------------------------------------------------
+__host__ __device__ __forceinline__ uint32_t finalise32(uint32_t h) {  // murmur3's finaliser
+  h ^= h >> 16;
+  h *= 0x85EBCA6Bu;
+  h ^= h >> 13;
+  h *= 0xC2B2AE35u;
+  h ^= h >> 16;
+  return h;
+}
+
+// the part of every draw of assignment a that does not depend on the node
+__host__ __device__ __forceinline__ uint32_t assignment_hash(uint64_t seed, int64_t a) {
+  uint32_t h = (uint32_t)seed ^ ((uint32_t)(seed >> 32) * 0x27D4EB2Fu);
+  h ^= (uint32_t)(uint64_t)a * 0x9E3779B1u;
+  h ^= (uint32_t)((uint64_t)a >> 32) * 0x85EBCA77u;
+  return h;
+}
+
+// the part that does not depend on the assignment
+__host__ __device__ __forceinline__ uint32_t node_key(int32_t gid) { return (uint32_t)(gid + 1) * 0xC2B2AE3Du; }
+
+// the scorers' draw (apc_random_assignment): uniform in [0, nstrat)
+__host__ __device__ __forceinline__ uint32_t plain_draw(uint32_t h0, int32_t gid, int32_t nstrat) {
+  const uint32_t h = finalise32(h0 ^ node_key(gid));
+  return (uint32_t)(((uint64_t)h * (uint64_t)(uint32_t)nstrat) >> 32);
+}
+
+// x + 1.0 n times over.  While x is a whole number below 2^52 every step is exact, and so
+// is x + n in one step (what the carried sums are in practice: counts); anything else is
+// added one by one, as a sequential walk does.
+__device__ __forceinline__ double add_ones(double x, uint32_t n) {
+  if (x == floor(x) && fabs(x) < 4503599627370496.0 - 4294967296.0) return x + (double)n;
+  for (uint32_t i = 0; i < n; ++i) x += 1.0;
+  return x;
+}
+
+// ---------------------------------------------------------------------------
 // Cost model, scalar device functions (order of operations is the contract)
 // ---------------------------------------------------------------------------
 

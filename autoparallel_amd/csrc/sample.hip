@@ -34,33 +34,10 @@ constexpr int kSampleArgs = 6;   // argument rows of a node whose columns a lane
 constexpr int kSampleWords = 8;  // words of a node's strategies a lane keeps in registers (512 strategies)
 typedef uint64_t u64x2_t __attribute__((ext_vector_type(2)));
 
-__host__ __device__ __forceinline__ uint32_t finalise32(uint32_t h) {
-  h ^= h >> 16;
-  h *= 0x85EBCA6Bu;
-  h ^= h >> 13;
-  h *= 0xC2B2AE35u;
-  h ^= h >> 16;
-  return h;
-}
-
-// the part of every draw of assignment a that does not depend on the node
-__host__ __device__ __forceinline__ uint32_t assignment_hash(uint64_t seed, int64_t a) {
-  uint32_t h = (uint32_t)seed ^ ((uint32_t)(seed >> 32) * 0x27D4EB2Fu);
-  h ^= (uint32_t)(uint64_t)a * 0x9E3779B1u;
-  h ^= (uint32_t)((uint64_t)a >> 32) * 0x85EBCA77u;
-  return h;
-}
-
-// The plain draw of the scorers (apc_random_assignment): uniform in [0, nstrat).
-__host__ __device__ __forceinline__ uint32_t plain_draw(uint32_t h0, int32_t gid, int32_t nstrat) {
-  const uint32_t h = finalise32(h0 ^ ((uint32_t)(gid + 1) * 0xC2B2AE3Du));
-  return (uint32_t)(((uint64_t)h * (uint64_t)(uint32_t)nstrat) >> 32);
-}
-
 // Which of the count allowed strategies of a node is taken, counted in out_idx order:
 // uniform in [0, count), from a hash of its own (not the plain draw's).
 __host__ __device__ __forceinline__ uint32_t rank_draw(uint32_t h0, int32_t gid, uint32_t count) {
-  const uint32_t h = finalise32(h0 ^ ((uint32_t)(gid + 1) * 0xC2B2AE3Du) ^ 0x68E31DA4u);
+  const uint32_t h = finalise32(h0 ^ node_key(gid) ^ 0x68E31DA4u);
   return (uint32_t)(((uint64_t)h * (uint64_t)count) >> 32);
 }
 

@@ -10,21 +10,7 @@ namespace {
 // ---------------------------------------------------------------------------
 __host__ __device__ __forceinline__ uint32_t mix_assignment(uint64_t seed, int64_t a, int32_t node,
                                                             int32_t nstrat) {
-  // counter-based draw: a 32-bit mix of (seed, assignment, node) through
-  // murmur3's finaliser, scaled to [0, nstrat) by a multiply-high.  The part
-  // that does not depend on the node is loop-invariant in the scorers; the
-  // walk is instruction-bound, and the 64-bit mix with a modulo that was
-  // here before took a quarter of it.
-  uint32_t h = (uint32_t)seed ^ ((uint32_t)(seed >> 32) * 0x27D4EB2Fu);
-  h ^= (uint32_t)(uint64_t)a * 0x9E3779B1u;
-  h ^= (uint32_t)((uint64_t)a >> 32) * 0x85EBCA77u;
-  h ^= (uint32_t)(node + 1) * 0xC2B2AE3Du;
-  h ^= h >> 16;
-  h *= 0x85EBCA6Bu;
-  h ^= h >> 13;
-  h *= 0xC2B2AE35u;
-  h ^= h >> 16;
-  return (uint32_t)(((uint64_t)h * (uint64_t)(uint32_t)nstrat) >> 32);
+  return plain_draw(assignment_hash(seed, a), node, nstrat);
 }
 
 // An edge record through one 64-byte load.  In the scorers the index is
@@ -88,15 +74,6 @@ score_kernel(apc_problem p, const double* __restrict__ per_arg, const double* __
   r[3] = t_trans;
   r[4] = obj;
   r[5] = forbidden;
-}
-
-// x + 1.0 n times over.  While x is a whole number below 2^52 every step is exact, and so
-// is x + n in one step (what the carried sums are in practice: counts); anything else is
-// added one by one, as a sequential walk does.
-__device__ __forceinline__ double add_ones(double x, uint32_t n) {
-  if (x == floor(x) && fabs(x) < 4503599627370496.0 - 4294967296.0) return x + (double)n;
-  for (uint32_t i = 0; i < n; ++i) x += 1.0;
-  return x;
 }
 
 // score_kernel<true> over a window of a larger graph: global node ids for the
@@ -301,22 +278,11 @@ score_compact_kernel(apc_problem p, const double* __restrict__ per_arg,
       const double* r = init + asg(k) * 6;
       t_compute[k] = r[1]; t_comm[k] = r[2]; t_trans[k] = r[3]; obj[k] = r[4]; forbidden[k] = r[5];
     }
-    // the part of mix_assignment that does not depend on the node
-    const uint64_t ua = (uint64_t)(first + asg(k));
-    uint32_t h = (uint32_t)seed ^ ((uint32_t)(seed >> 32) * 0x27D4EB2Fu);
-    h ^= (uint32_t)ua * 0x9E3779B1u;
-    h ^= (uint32_t)(ua >> 32) * 0x85EBCA77u;
-    h0[k] = h;
+    h0[k] = assignment_hash(seed, first + asg(k));
   }
   auto choice = [&](int k, int v, int nstrat) -> uint32_t {
     if (!kRandom) return (uint32_t)assign[(size_t)v * stride + asg(k)];
-    uint32_t h = h0[k] ^ ((uint32_t)((node_gid ? node_gid[v] : v) + 1) * 0xC2B2AE3Du);
-    h ^= h >> 16;
-    h *= 0x85EBCA6Bu;
-    h ^= h >> 13;
-    h *= 0xC2B2AE35u;
-    h ^= h >> 16;
-    return (uint32_t)(((uint64_t)h * (uint64_t)(uint32_t)nstrat) >> 32);
+    return plain_draw(h0[k], node_gid ? node_gid[v] : v, nstrat);
   };
   apc_edge nxt;
   if (first_node < p.n_node && p.node_edge_off[first_node] < p.n_edge)
@@ -476,23 +442,12 @@ score_table_kernel(apc_problem p, const double* __restrict__ per_arg, const doub
       const double* r = init + asg(k) * 6;
       t_compute[k] = r[1]; t_comm[k] = r[2]; obj[k] = r[4];
     }
-    // the part of mix_assignment that does not depend on the node
-    const uint64_t ua = (uint64_t)(first + asg(k));
-    uint32_t h = (uint32_t)seed ^ ((uint32_t)(seed >> 32) * 0x27D4EB2Fu);
-    h ^= (uint32_t)ua * 0x9E3779B1u;
-    h ^= (uint32_t)(ua >> 32) * 0x85EBCA77u;
-    h0[k] = h;
+    h0[k] = assignment_hash(seed, first + asg(k));
   }
   // the choice of assignment k at node v, whose id for the draw is gid
   auto choice = [&](int k, int v, int gid, int nstrat) -> uint32_t {
     if (!kRandom) return (uint32_t)assign[(size_t)v * stride + asg(k)];
-    uint32_t h = h0[k] ^ ((uint32_t)(gid + 1) * 0xC2B2AE3Du);
-    h ^= h >> 16;
-    h *= 0x85EBCA6Bu;
-    h ^= h >> 13;
-    h *= 0xC2B2AE35u;
-    h ^= h >> 16;
-    return (uint32_t)(((uint64_t)h * (uint64_t)(uint32_t)nstrat) >> 32);
+    return plain_draw(h0[k], gid, nstrat);
   };
   // Whether the two index lists of a compressed matrix go through LDS too.
   auto lists_staged = [](const apc_edge& x) {

@@ -86,8 +86,8 @@ score_steps_kernel(apc_problem p, const apc_score_step* __restrict__ steps, int 
     f.mat = r.mat; f.pa = r.pa; f.flags = r.flags; f.ssrc = r.ssrc; f.nstrat = r.nstrat;
     f.row_node = r.row_node; f.row_src = r.row_src; f.has_src = r.src_node >= 0; f.nargs = r.nargs;
     f.mult = (int32_t)mult;
-    f.key_node = (uint32_t)((node_gid ? node_gid[r.node] : r.node) + 1) * 0xC2B2AE3Du;
-    if (r.src_node >= 0) f.key_src = (uint32_t)((node_gid ? node_gid[r.src_node] : r.src_node) + 1) * 0xC2B2AE3Du;
+    f.key_node = node_key(node_gid ? node_gid[r.node] : r.node);
+    if (r.src_node >= 0) f.key_src = node_key(node_gid ? node_gid[r.src_node] : r.src_node);
     static_cast<StepFields*>(out)[s] = f;
   } else {
     StepWords w = {};
@@ -99,12 +99,6 @@ score_steps_kernel(apc_problem p, const apc_score_step* __restrict__ steps, int 
     w.hi[1] = r.src_node >= 0;
     static_cast<StepWords*>(out)[s] = w;
   }
-}
-
-__device__ __forceinline__ double ones_added(double x, uint32_t n) {  // x + 1.0, n times over
-  if (x == floor(x) && fabs(x) < 4503599627370496.0 - 4294967296.0) return x + (double)n;
-  for (uint32_t i = 0; i < n; ++i) x += 1.0;
-  return x;
 }
 
 template <bool kRandom, int kPer>
@@ -138,18 +132,10 @@ score_tiles_kernel(apc_problem p, const double* __restrict__ per_arg, const doub
       const double* r = init + asg(k) * 6;
       t_compute[k] = r[1]; t_comm[k] = r[2]; obj[k] = r[4];
     }
-    const uint64_t ua = (uint64_t)(first + asg(k));
-    h0[k] = (uint32_t)seed ^ ((uint32_t)(seed >> 32) * 0x27D4EB2Fu) ^ ((uint32_t)ua * 0x9E3779B1u) ^
-            ((uint32_t)(ua >> 32) * 0x85EBCA77u);
+    h0[k] = assignment_hash(seed, first + asg(k));
   }
-  auto draw = [&](int k, uint32_t key, uint32_t nstrat) -> uint32_t {  // mix_assignment
-    uint32_t h = h0[k] ^ key;
-    h ^= h >> 16;
-    h *= 0x85EBCA6Bu;
-    h ^= h >> 13;
-    h *= 0xC2B2AE35u;
-    h ^= h >> 16;
-    return __umulhi(h, nstrat);
+  auto draw = [&](int k, uint32_t key, uint32_t nstrat) -> uint32_t {  // plain_draw by the node's key
+    return __umulhi(finalise32(h0[k] ^ key), nstrat);
   };
   // The copies of a tile are shared out by wavefronts; a lane holds the record of one of its
   // wavefront's copies, read a tile before the copies are issued.
@@ -328,10 +314,10 @@ score_tiles_kernel(apc_problem p, const double* __restrict__ per_arg, const doub
 #pragma unroll
   for (int k = 0; k < kPer; ++k) {
     if (t_raw + k * lanes >= n_assign) continue;
-    const double t_trans = ones_added(init ? init[asg(k) * 6 + 3] : 0.0, n_trans[k]);
+    const double t_trans = add_ones(init ? init[asg(k) * 6 + 3] : 0.0, n_trans[k]);
     double forbidden = init ? init[asg(k) * 6 + 5] : 0.0;
     if (tiles[0].any_edge) forbidden += 0.0;  // a walk adds 0.0 or 1.0 per edge: a carried -0.0 loses its sign
-    forbidden = ones_added(forbidden, n_forbidden[k]);
+    forbidden = add_ones(forbidden, n_forbidden[k]);
     double* r = out + asg(k) * 6;
     r[0] = (t_compute[k] + t_comm[k]) + t_trans;
     r[1] = t_compute[k];
