@@ -504,11 +504,7 @@ class CostEngine:
         if rc:
             _lib.check(rc, "apc_build_all")
         self.built = True
-        self._table_clamp = (1 if clamp_inf else 0) if self.table is not None else None
-        if self._edits_seen:
-            self._mark_built()
-        if stream and self._capturing(C.c_void_p(stream)):
-            self._recorded_writes.add(self._table_clamp)
+        self._note_build((1 if clamp_inf else 0) if self.table is not None else None, stream)
         return self
 
     def build_timed(self, timer, slot: int, clamp_inf: bool = True):
@@ -523,12 +519,16 @@ class CostEngine:
             _lib.check(rc, "apc_build_all_timed")
         self._recs_valid = False
         self.built = True
-        self._table_clamp = clamp if self.table is not None else None
-        if self._edits_seen:
-            self._mark_built()
-        if stream and self._capturing(C.c_void_p(stream)):
-            self._recorded_writes.add(self._table_clamp)
+        self._note_build(clamp if self.table is not None else None, stream)
         return self
+
+    def _note_build(self, clamp: Optional[int], stream: int) -> None:
+        if stream and self._capturing(C.c_void_p(stream)):  # nothing is written yet
+            self._recorded_writes.add(clamp)
+            return
+        self._table_clamp = clamp
+        if self._edits_seen:  # edits before this build are gone
+            self._built_marks = tuple((ref, at, _edit_count(ref())) for ref, at, _ in self._built_marks)
 
     def set_node_multiplier(self, mult: np.ndarray) -> None:
         """Replace the objective multiplier per node (cluster multiplicity)."""
@@ -608,24 +608,11 @@ class CostEngine:
         out = torch.empty((A, 6), dtype=torch.float64, device=self.device)
         if self.packed_scoring and A >= _SCORE_LANES_FROM:
             return self._score_packed(assign, 0, 0, A, None, 0, None, out)
-        if self._score_small(assign, 0, 0, A, None, 0, None, out):
-            return out
-        _lib.check(
-            self.lib.apc_score_assignments(
-                C.byref(self.problem), self._ptr(self.per_arg), self._ptr(self.comm), self._ptr(self.cost),
-                self._ptr(self.flags), self._ptr(assign), A, self._ptr(out), self._stream()),
-            "apc_score_assignments",
-        )
-        self.last_score_backend = "entry_arrays"
-        return out
+        return self._score_small(assign, 0, 0, A, None, 0, None, out)
 
     def _array_marks(self) -> tuple:
         return tuple((weakref.ref(t), t.data_ptr(), _edit_count(t))
                      for t in (self.comm, self.cost, self.flags, self.per_arg))
-
-    def _mark_built(self) -> None:
-        """A build has rewritten the arrays: edits before it are gone."""
-        self._built_marks = tuple((ref, at, _edit_count(ref())) for ref, at, _ in self._built_marks)
 
     def _unchanged(self, marks: tuple) -> bool:
         """Whether the arrays are the marked ones, with no edit since."""
@@ -635,36 +622,61 @@ class CostEngine:
                 return False
         return len(marks) > 0
 
-    def _table_stands(self) -> bool:
-        """Whether the entry arrays are what the last build made of the block table, so that a
-        scorer may read the table in their place.  Every scorer that does so asks here.
-        Recorded builds may have been replayed since: they change nothing where they clamp alike."""
+    def _standing_clamp(self) -> Optional[int]:
+        """clamp_inf of the build that made the entry arrays what they are, while they still are what
+        it made of the block table, so that a scorer may read the table in their place; else
+        None.  Every scorer that does so asks here.  Recorded builds may have been replayed since the
+        last one: they change nothing where they clamp alike."""
         if self._table_clamp is None or self._recorded_writes - {self._table_clamp}:
-            return False
-        stands = self._unchanged(self._built_marks)
-        self._edits_seen |= not stands
-        return stands
+            return None
+        if self._unchanged(self._built_marks):
+            return self._table_clamp
+        self._edits_seen = True
+        return None
 
-    def _score_small(self, assign, seed, first, count, d_gid, first_node, init, out) -> bool:
-        """A small batch from the block table while it stands for the entry arrays; False: not done."""
-        if not _SCORE_SMALL_FROM_TABLE or not self.packed_scoring or count == 0:
-            return False
+    def _score_small(self, assign, seed, first, count, d_gid, first_node, init, out) -> torch.Tensor:
+        """A batch below _SCORE_LANES_FROM: the terms side by side, from the block table while it stands for
+        the entry arrays, else from the arrays."""
         stream = self._stream()
-        if count < _SCORE_LANES_FROM and self._capturing(stream):  # whatever the arrays hold on a replay
-            return False
-        if not self._versioned or not self._table_stands():  # without counters an edit would go unnoticed
-            return False
-        return self._score_terms(assign, seed, first, count, d_gid, first_node, init, out, stream)
+        if _SCORE_SMALL_FROM_TABLE and self.packed_scoring and count > 0:
+            # recorded, it reads whatever the arrays hold on a replay; without edit counters, an edit
+            # would go unnoticed
+            clamp = self._standing_clamp() if self._versioned and not self._capturing(stream) else None
+            if clamp is not None:
+                return self._score_terms(clamp, assign, seed, first, count, d_gid, first_node, init, out, stream)
+        return self._score_arrays(assign, seed, first, count, d_gid, first_node, init, out, stream)
 
-    def _score_terms(self, assign, seed, first, count, d_gid, first_node, init, out, stream) -> bool:
+    def _score_arrays(self, assign, seed, first, count, d_gid, first_node, init, out, stream) -> torch.Tensor:
+        args = (C.byref(self.problem), self._ptr(self.per_arg), self._ptr(self.comm), self._ptr(self.cost),
+                self._ptr(self.flags))
+        if assign is not None:
+            _lib.check(
+                self.lib.apc_score_assignments_window(
+                    *args, self._ptr(assign), int(count), int(first_node), self._ptr(init), self._ptr(out), stream),
+                "apc_score_assignments_window")
+        elif d_gid is None:
+            _lib.check(
+                self.lib.apc_score_random_assignments(
+                    *args, int(seed), int(first), int(count), self._ptr(out), stream),
+                "apc_score_random_assignments")
+        else:
+            _lib.check(
+                self.lib.apc_score_random_window(
+                    *args, int(seed), int(first), int(count), self._ptr(d_gid), int(first_node), self._ptr(init),
+                    self._ptr(out), stream),
+                "apc_score_random_window")
+        self.last_score_backend = "entry_arrays"
+        return out
+
+    def _score_terms(self, clamp, assign, seed, first, count, d_gid, first_node, init, out, stream) -> torch.Tensor:
         _lib.check(
             self.lib.apc_score_fold_table(
                 C.byref(self.problem), self._ptr(self.per_arg), self._ptr(self.table), self._ptr(assign), int(seed),
-                int(first), int(count), self._ptr(d_gid), int(first_node), self._table_clamp, self._ptr(init),
+                int(first), int(count), self._ptr(d_gid), int(first_node), clamp, self._ptr(init),
                 self._ptr(out), stream),
             "apc_score_fold_table")
         self.last_score_backend = "block_table_terms"
-        return True
+        return out
 
     def _score_packed(self, assign, seed, first, count, d_gid, first_node, init, out) -> torch.Tensor:
         """Scoring of a large batch.  A graph with large blocks: from the block
@@ -681,7 +693,10 @@ class CostEngine:
         cost is (comm + per_arg) + transition or its clamp (checked on the device
         when the records are made); else the 32-byte records that carry the cost
         (apc_score_packed)."""
-        from_table = _SCORE_FROM_TABLE and self._table_stands()
+        stream = self._stream()
+        capturing = self._capturing(stream)
+        clamp = self._standing_clamp() if _SCORE_FROM_TABLE else None
+        from_table = clamp is not None
         if from_table and (self.large_blocks or not _SCORE_COMPACT) and count >= _SCORE_TABLE_FROM:
             aux = self._score_edge_aux(d_gid)
             _lib.check(
@@ -689,15 +704,15 @@ class CostEngine:
                     C.byref(self.problem), self._ptr(self.per_arg), self._ptr(self.table),
                     C.c_void_p(aux.data_ptr()), self._ptr(assign),
                     int(seed), int(first), int(count), self._ptr(d_gid), int(first_node), self.g.num_nodes,
-                    self._table_clamp, min(_SCORE_PER_LANE, 4),
-                    self._ptr(init), self._ptr(out), self._stream()),
+                    clamp, min(_SCORE_PER_LANE, 4),
+                    self._ptr(init), self._ptr(out), stream),
                 "apc_score_table")
             self.last_score_backend = "block_table"
             return out
-        if (from_table and count < _SCORE_TERMS_BELOW
-                and self._score_small(assign, seed, first, count, d_gid, first_node, init, out)):
-            return out
-        if from_table and self._versioned and _SCORE_FROM_TILES and not self.large_blocks:
+        from_table &= self._versioned  # else an edit would go unnoticed
+        if from_table and count < _SCORE_TERMS_BELOW and _SCORE_SMALL_FROM_TABLE:
+            return self._score_terms(clamp, assign, seed, first, count, d_gid, first_node, init, out, stream)
+        if from_table and _SCORE_FROM_TILES and not self.large_blocks:
             tiles = self._score_tiles(first_node, assign is not None)
             if tiles is not None:
                 steps, n_step, d_tiles, n_tile, units = tiles
@@ -706,19 +721,15 @@ class CostEngine:
                     self.lib.apc_score_from_tiles(
                         C.byref(self.problem), self._ptr(self.per_arg), self._ptr(self.table), self._ptr(steps), n_step,
                         self._ptr(d_tiles), n_tile, self._ptr(units), self._ptr(call_steps), self._ptr(assign),
-                        int(seed), int(first), int(count), self._ptr(d_gid), self._table_clamp, self._ptr(init),
-                        self._ptr(out), self._stream()),
+                        int(seed), int(first), int(count), self._ptr(d_gid), clamp, self._ptr(init),
+                        self._ptr(out), stream),
                     "apc_score_from_tiles")
                 self.last_score_backend = "block_table_tiles"
                 return out
-        stream = self._stream()
-        capturing = self._capturing(stream)
         recs_stand = (self._recs_valid and self._unchanged(self._recs_marks)
                       and (capturing or not self._recorded_writes))  # else replayed since, or not
-        if capturing and not recs_stand and from_table and self._versioned:
-            # records are not made while a graph is recorded (their check is read by the host)
-            self._score_terms(assign, seed, first, count, d_gid, first_node, init, out, stream)
-            return out
+        if capturing and not recs_stand:  # records are not made meanwhile: the host reads their check
+            return self._score_arrays(assign, seed, first, count, d_gid, first_node, init, out, stream)
         if not recs_stand:
             self._recs = None  # one kind at a time: either is as large as the entry arrays
             recs = None
@@ -900,16 +911,7 @@ class CostEngine:
         out = torch.empty((count, 6), dtype=torch.float64, device=self.device)
         if self.packed_scoring and count >= _SCORE_LANES_FROM:
             return self._score_packed(None, seed, first, count, None, 0, None, out)
-        if self._score_small(None, seed, first, count, None, 0, None, out):
-            return out
-        _lib.check(
-            self.lib.apc_score_random_assignments(
-                C.byref(self.problem), self._ptr(self.per_arg), self._ptr(self.comm), self._ptr(self.cost),
-                self._ptr(self.flags), int(seed), int(first), int(count), self._ptr(out), self._stream()),
-            "apc_score_random_assignments",
-        )
-        self.last_score_backend = "entry_arrays"
-        return out
+        return self._score_small(None, seed, first, count, None, 0, None, out)
 
     def score_random_window(self, seed: int, first: int, count: int, node_gid: np.ndarray, first_node: int,
                             init: Optional[torch.Tensor] = None) -> torch.Tensor:
@@ -924,17 +926,7 @@ class CostEngine:
         out = torch.empty((count, 6), dtype=torch.float64, device=self.device)
         if self.packed_scoring and count >= _SCORE_LANES_FROM:
             return self._score_packed(None, seed, first, count, d_gid, first_node, init, out)
-        if self._score_small(None, seed, first, count, d_gid, first_node, init, out):
-            return out
-        _lib.check(
-            self.lib.apc_score_random_window(
-                C.byref(self.problem), self._ptr(self.per_arg), self._ptr(self.comm), self._ptr(self.cost),
-                self._ptr(self.flags), int(seed), int(first), int(count), self._ptr(d_gid), int(first_node),
-                self._ptr(init), self._ptr(out), self._stream()),
-            "apc_score_random_window",
-        )
-        self.last_score_backend = "entry_arrays"
-        return out
+        return self._score_small(None, seed, first, count, d_gid, first_node, init, out)
 
     def score_window(self, assign: torch.Tensor, first_node: int, init: Optional[torch.Tensor] = None) -> torch.Tensor:
         """score() for a window of a larger graph: explicit assignments (uint16
@@ -949,16 +941,7 @@ class CostEngine:
         out = torch.empty((count, 6), dtype=torch.float64, device=self.device)
         if self.packed_scoring and count >= _SCORE_LANES_FROM:
             return self._score_packed(assign, 0, 0, count, None, first_node, init, out)
-        if self._score_small(assign, 0, 0, count, None, first_node, init, out):
-            return out
-        _lib.check(
-            self.lib.apc_score_assignments_window(
-                C.byref(self.problem), self._ptr(self.per_arg), self._ptr(self.comm), self._ptr(self.cost),
-                self._ptr(self.flags), self._ptr(assign), count, int(first_node), self._ptr(init), self._ptr(out),
-                self._stream()),
-            "apc_score_assignments_window")
-        self.last_score_backend = "entry_arrays"
-        return out
+        return self._score_small(assign, 0, 0, count, None, first_node, init, out)
 
     def _allowed_columns(self):
         """(colbits, col_off, max_words) of apc_pack_allowed_columns for the flags as they

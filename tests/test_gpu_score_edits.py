@@ -143,6 +143,45 @@ def test_recorded_edits_and_entries_count(engines):
             assert (_bits(eng.score_random(5, 9, 70)) == _as_the_arrays_are(eng, other, 70)).all()
 
 
+@pytest.mark.parametrize("count", COUNTS)
+def test_a_build_that_is_only_recorded_rewrites_nothing(engines, count):
+    eng = CostEngine(engines[0].g, table_mode="full")
+    eng.large_blocks = engines[0].large_blocks
+    other = engines[1]
+    for change in (lambda: eng.apply_prefetch_discount(0.5), lambda: eng.cost.mul_(2.0), lambda: eng.build(False)):
+        eng.build(True)
+        eng.score_random(5, 9, count)
+        change()
+        graph = torch.cuda.CUDAGraph()
+        torch.cuda.synchronize()
+        with torch.cuda.graph(graph):
+            eng.build(True)
+        assert (_bits(eng.score_random(5, 9, count)) == _as_the_arrays_are(eng, other, count)).all()
+        graph.replay()
+        assert (_bits(eng.score_random(5, 9, count)) == _as_the_arrays_are(eng, other, count)).all()
+
+
+@pytest.mark.parametrize("count", COUNTS)
+def test_builds_and_scores_recorded_together(engines, count):
+    """Replays give what the recorded build and edits leave, whatever was built eagerly before."""
+    eng = CostEngine(engines[0].g, table_mode="full")
+    eng.large_blocks = engines[0].large_blocks
+    other = engines[1]
+    eng.build(False)
+    eng.score_random(5, 9, count)
+    for record in (lambda: eng.build(True), lambda: eng.build(False), lambda: eng.build(True).cost.mul_(2.0),
+                   lambda: (eng.build(True), eng.edge_costs(clamp_inf=False))):
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            record()
+            out = eng.score_random(5, 9, count)
+        for _ in range(3):
+            graph.replay()
+            assert (_bits(out) == _as_the_arrays_are(eng, other, count)).all()
+            eng.build(False)
+
+
 @pytest.mark.parametrize("explicit", [False, True])
 def test_a_recorded_small_score_reads_the_arrays(engines, explicit):
     """Replays of a recorded score follow builds, edits and discounts between them."""
