@@ -868,9 +868,12 @@ int launch_fold_k(const apc_problem& p, const double* per_arg, const double* com
 
 template <bool kRandom, bool kTable, typename... Args>
 int launch_fold_t(int64_t n_assign, Args... args) {
-  // The smallest groups whose workgroups are all resident at once (two per CU), since a
-  // group's time grows with its size: 12 layers of the GPT-2 graph, 2 000 assignments, 45 us in
-  // groups of 8, 67 in 16, 126 in 32; 8 000 assignments 110 us in 16, 130 in 32, 154 in 8.
+  // A group's time grows with its size, so the smallest groups whose workgroups are all resident
+  // at once (two per CU, from groups of 8 on): 12 layers of the GPT-2 graph, 2 000 assignments, 45 us in
+  // groups of 8, 67 in 16, 126 in 32; 8 000 assignments 110 us in 16, 130 in 32, 154 in 8.  Groups of
+  // 4 while there is a CU for each: two of them on a CU take as long as one of 8 (2 048
+  // assignments, random and explicit, 49 and 66 us against 50 and 64; Llama-3-8B graph 154 and 181 against
+  // 144 and 180, planner DAG window 254 and 149 against 244 and 155).
   const int sh = n_assign <= 1024 ? 2 : n_assign <= 4096 ? 3 : n_assign <= 8192 ? 4 : n_assign < 16384 ? 5 : 6;
   switch (sh) {
     case 2: return launch_fold_k<kRandom, 2, kTable>(args...);

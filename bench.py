@@ -355,7 +355,8 @@ def main():
                                "construction: each edge's inp_idx is its producer's draw), not ILP-feasible plans",
             "fraction_without_forbidden_entry": float((scores[:, 5] == 0).double().mean().item()),
         }
-        # The bound that applies to a launch from records.  Its inputs are the 16-byte records of the
+        # The bound that applies to a launch from records (the table does not stand for the
+        # entry arrays here: the entry kernel was timed on its own above).  Its inputs are the 16-byte records of the
         # entries (one per slot) and 48 B of sums per assignment: that is all HBM has to
         # deliver, once.  An assignment then reads one record per edge at a position its
         # draws decide: random 16-byte reads served by L2 and the memory-side cache, at
@@ -365,9 +366,8 @@ def main():
         hbm_bytes = 16 * g.num_slots + 48 * n
         out["scoring"]["roofline"] = {
             "kernel": "score_compact_kernel" if eng.last_score_backend == "compact_records" else eng.last_score_backend,
-            "bound": ("cache-miss service rate (random 16-byte reads of records resident in L2 and the "
-                      "memory-side cache); not HBM, not MFMA") if eng.last_score_backend == "compact_records" else
-                     "instructions (draw hashes, binary64 sums; the entries are drawn from LDS); not HBM, not MFMA",
+            "bound": "cache-miss service rate (random 16-byte reads of records resident in L2 and the "
+                     "memory-side cache); not HBM, not MFMA",
             "achieved": reads / t_score,
             "unit": "random reads/s",
             "per_cu_per_ns": reads / t_score / 256 / 1e9,

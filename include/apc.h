@@ -731,7 +731,7 @@ int apc_score_fold_table(const apc_problem* p, const double* per_arg, const doub
  * consecutive steps whose matrices, each once, fit an LDS buffer; the copies (units) that
  * bring a tile in.  edges: the records of the problem (apc_edge), as on the device.
  * explicit_rows: the layout is for explicit assignments (a tile names the nodes whose
- * choices it reads, 16 at most), else for random ones.  
+ * choices it reads, 16 at most), else for random ones.
  * *n_step = 0: not a graph for this form (a matrix of more than 4 864 doubles or compressed, a
  * node with more than 256 strategies, a producer behind its consumer): use another scorer.
  * The layout depends on the graph alone; it is copied to the device and serves every call.

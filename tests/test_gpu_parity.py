@@ -360,7 +360,7 @@ def test_device_scorers_on_a_hand_made_plan(CostEngine):
     # one selected variable is forbidden (C <- Q)
     obj = 2.0 + 4.0 + (0.5 + 16.0) + 10000.0 + (0.25 + 64.0 + 1.0) + (0.125 + 256.0 + 1.0)
     col = np.asarray(assign, np.int16)[:, None]
-    for count in (1, 70, 33000, 140000):  # wave per assignment, lanes, records
+    for count in (1, 70, 33000, 140000):  # terms side by side, lanes over records
         out = eng.score(torch.from_numpy(np.ascontiguousarray(np.tile(col, (1, count)))).cuda()).cpu().numpy()
         assert tuple(out[0, :4]) == want and tuple(out[-1, :4]) == want, (count, eng.last_score_backend, out[0])
         assert out[0, 4] == obj and out[0, 5] == 1.0 and bits_equal(out[0], out[-1])
