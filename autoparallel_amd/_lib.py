@@ -17,6 +17,7 @@ SAMPLE_ARGS = 6  # argument rows an apc_sample_rec names
 SAMPLE_REC_BYTES = 64
 CHECK_MAX_NODES = 131072
 SCORE_STEP_BYTES, SCORE_TILE_BYTES, SCORE_UNIT_BYTES = 64, 128, 16
+SCORE_IMAGE_BYTES = 43008
 
 
 class ApcModel(C.Structure):
@@ -278,6 +279,11 @@ _SIGNATURES = {
         [C.c_void_p, C.c_int32, C.c_int32, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_int32, C.c_int32,
          C.c_void_p, C.c_int64, C.c_void_p, C.c_int64, C.c_void_p, C.c_int64, C.c_void_p, C.c_void_p, C.c_void_p]),
     "apc_score_from_tiles": (
+        C.c_int,
+        [C.POINTER(ApcProblem), C.c_void_p, C.c_void_p, C.c_void_p, C.c_int32, C.c_void_p, C.c_int32, C.c_void_p,
+         C.c_void_p, C.c_void_p, C.c_uint64, C.c_int64, C.c_int64, C.c_void_p, C.c_int32, C.c_void_p, C.c_void_p,
+         C.c_void_p]),
+    "apc_score_images": (
         C.c_int,
         [C.POINTER(ApcProblem), C.c_void_p, C.c_void_p, C.c_void_p, C.c_int32, C.c_void_p, C.c_int32, C.c_void_p,
          C.c_void_p, C.c_void_p, C.c_uint64, C.c_int64, C.c_int64, C.c_void_p, C.c_int32, C.c_void_p, C.c_void_p,

@@ -14,9 +14,9 @@
 // and kept for the next kRows - 1 nodes, packed to a byte per assignment, where three quarters of
 // the edges find their producer's; explicit choices are read a tile ahead into the same place.
 // Below, it is the chain of LDS reads of a step and the few wavefronts a CU has to hide it.
-// Measured, from records and by tiles: 2^20 random assignments of that graph 15.4 -> 10.4 ms,
-// 131 072 7.2 -> 4.8, 131 072 explicit ones 10.9 -> 5.7, 2^20 random ones of the 16-layer
-// mixture-of-experts graph 8.4 -> 5.7.  Not better: step records in LDS instead of scalar loads
+// Measured, from records and by tiles: 2^20 random assignments of that graph 15.4 -> 10.4 ms, of the 16-layer
+// mixture-of-experts graph 8.4 -> 5.7 (explicit ones, and few random ones, are faster from tile images,
+// score_images.hip; explicit ones are walked here where there is no room for the images).  Not better: step records in LDS instead of scalar loads
 // (11.8 for the first figure; eight readfirstlane a step).
 // Sums run in node order, then argument order, as in score_kernel: the same bits.
 #include <algorithm>
@@ -25,18 +25,18 @@
 #include <vector>
 
 #include "apc_device.h"
+#include "score_tiles.h"
 
 namespace {
 
-constexpr int kTileDoubles = 5120;  // 40 KB: one of the two buffers
-constexpr int kRows = 16;           // rows of packed choices: the ring of random ones, a tile's explicit ones
+using namespace apc_tiles;
+
 constexpr int kNoRow = 255;
 constexpr int kMaxLanes = 1024;
 constexpr int kUnitDoubles = 128;   // what one wavefront copies with one 16-byte load per lane
 constexpr int kUnitSingles = 32;    // and with one 4-byte load per lane, where 16 bytes may not be aligned
 
 typedef int32_t i32x4_t __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(3))) void* lds_ptr_t;
 
 // A step as the walk reads it, one scalar load:
 //   [0] matrix (bits 0-12) and per-argument terms (13-25) in the tile's buffer, APC_STEP_* (26-28)
@@ -56,20 +56,6 @@ typedef uint32_t u32x16_t __attribute__((ext_vector_type(16)));
 static_assert(sizeof(StepWords) == 32 && sizeof(StepFields) == 64 && sizeof(apc_score_step) == 64 && sizeof(apc_score_unit) == 16 &&
               sizeof(apc_score_tile) == 128, "layout");
 static_assert(kTileDoubles <= 8192 && kRows < kNoRow, "a step's fields");
-
-// Global memory to LDS without registers in between: lane i's 16 (4) bytes to lds + i * 16 (4).
-// Written by hand, and waited for by hand, so that the loads stay in flight while the lanes draw
-// from the other buffer; m0 is put back because the compiler keeps it for its own uses.
-__device__ __forceinline__ void load16_lds(const double2_t* g, uint32_t lds) {
-  uint32_t saved;
-  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 3\n\tglobal_load_lds_dwordx4 %2, off\n\ts_mov_b32 m0, %0"
-               : "=&s"(saved) : "s"(lds), "v"(g) : "memory");
-}
-__device__ __forceinline__ void load4_lds(const uint32_t* g, uint32_t lds) {
-  uint32_t saved;
-  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 3\n\tglobal_load_lds_dword %2, off\n\ts_mov_b32 m0, %0"
-               : "=&s"(saved) : "s"(lds), "v"(g) : "memory");
-}
 
 // The steps of a call, with the multipliers (they can be replaced between calls) and the ids
 // the draws hash.
@@ -134,11 +120,17 @@ score_tiles_kernel(apc_problem p, const double* __restrict__ per_arg, const doub
     }
     h0[k] = assignment_hash(seed, first + asg(k));
   }
+  // the loads of init end here: the compiler would wait for them where the sums are first added to, in the
+  // loop, and with that for every copy under way
+#pragma unroll
+  for (int k = 0; k < kPer; ++k) asm volatile("" : "+v"(t_compute[k]), "+v"(t_comm[k]), "+v"(obj[k]));
   auto draw = [&](int k, uint32_t key, uint32_t nstrat) -> uint32_t {  // plain_draw by the node's key
     return __umulhi(finalise32(h0[k] ^ key), nstrat);
   };
   // The copies of a tile are shared out by wavefronts; a lane holds the record of one of its
   // wavefront's copies, read a tile before the copies are issued.
+  const uint64_t at_table = (uint64_t)(uintptr_t)table, to_per_arg = (uint64_t)(uintptr_t)per_arg - at_table,
+                 to_default = (uint64_t)(uintptr_t)p.default_vals - at_table;
   struct Head { int step0, step1, unit0, unit1; };
   auto load_head = [&](int t) -> Head {
     union { i32x4_t raw; Head h; } u;
@@ -161,11 +153,14 @@ score_tiles_kernel(apc_problem p, const double* __restrict__ per_arg, const doub
       const int64_t src = (int64_t)((uint64_t)s_hi << 32 | s_lo);
       const uint32_t lds = base + (to & 0xFFFFu) * 8u;
       const int n_double = (int)(to >> 16);
+      // the array by its distance from the table: a choice between what this lambda captured goes
+      // through scratch memory, and the wait for that is one for the copies before
+      const uint64_t from = at_table + (to_per_arg & (kind == 1 ? ~0ull : 0ull)) + (to_default & (kind == 2 ? ~0ull : 0ull)) +
+                            (uint64_t)src * 8u;
       if (kind == 0) {
-        if (2 * lane < n_double) load16_lds(reinterpret_cast<const double2_t*>(table + src) + lane, lds);
+        if (2 * lane < n_double) load16_lds(reinterpret_cast<const double2_t*>(from) + lane, lds);
       } else {
-        const double* const from = kind == 1 ? per_arg : p.default_vals;
-        if (lane < 2 * n_double) load4_lds(reinterpret_cast<const uint32_t*>(from + src) + lane, lds);
+        if (lane < 2 * n_double) load4_lds(reinterpret_cast<const uint32_t*>(from) + lane, lds);
       }
     }
   };
@@ -436,13 +431,13 @@ int apc_score_tiles(const apc_edge* edges, int32_t n_edge, int32_t n_node, const
           any_edge = true;
         }
         // a tile's room: doubles, and with explicit choices rows
-        int need = (ed ? needs(src, kind, matrix) : 0) + (starts ? needs(node_comp_off[v], 1, node_nstrat[v]) : 0);
+        int need = (ed ? needs(src, kind, matrix) : 0) + needs(node_comp_off[v], 1, node_nstrat[v]);
         int rows = 0;
         if (explicit_rows) {
-          if (starts && !row_of.count(v)) ++rows;
+          if (!row_of.count(v)) ++rows;
           if (ed && ed->src_node >= 0 && !row_of.count(ed->src_node)) ++rows;
         }
-        if (used + need > kTileDoubles || n_row + rows > kRows)
+        if (used + need > kTileDoubles || n_row + rows > kRows || (explicit_rows && s - tiles[t].step0 >= kTileSteps))
           if (!new_tile()) return fail(APC_ERR_INVALID, "apc_score_tiles: max_tile or max_unit is too small%s");
         if (s >= max_step) return fail(APC_ERR_INVALID, "apc_score_tiles: max_step is too small%s");
         apc_score_step& r = steps[s];
@@ -452,13 +447,9 @@ int apc_score_tiles(const apc_edge* edges, int32_t n_edge, int32_t n_node, const
         r.nargs = node_nargs[v] > 1 ? node_nargs[v] : 1;
         r.src_node = -1;
         r.row_src = -1;
-        int placed = 0;
-        r.row_node = v & (kRows - 1);
-        if (starts) {
-          r.flags |= APC_STEP_FIRST;
-          placed = r.pa = place(node_comp_off[v], 1, node_nstrat[v]);
-          if (explicit_rows) r.row_node = row(v);
-        }
+        r.row_node = explicit_rows ? row(v) : v & (kRows - 1);
+        if (starts) r.flags |= APC_STEP_FIRST;
+        int placed = r.pa = place(node_comp_off[v], 1, node_nstrat[v]);  // again, where a node goes on in another tile
         if (ed) {
           r.flags |= APC_STEP_EDGE;
           r.ssrc = ed->ssrc;

@@ -24,11 +24,19 @@ _SCORE_SMALL_FROM_TABLE = True
 _SCORE_FROM_TILES = True  # small blocks: matrices through LDS by tiles, while the table stands for the arrays
 # Below, the terms of a few assignments gathered side by side are faster than any walk with a lane per
 # assignment: up to here a CU takes seven workgroups of 64, an eighth costs more than a walk's lanes do.  In
-# ms, at 65 536, 110 000 and 120 000 random assignments: Llama-3-8B graph side by side 2.35, 4.58, 5.00, by tiles
-# 5.90, 4.97, 4.82 (explicit ones 3.13, 5.88, 6.76 and 6.57, 5.90, 5.74); window of the planner DAG side by
-# side 1.89, 3.61, 4.12, from records 3.84, 3.87, 3.90 (explicit 2.17, 4.11, 4.85 and 4.41, 4.47, 4.50), table
-# scorer 5.3.  The 12-layer GPT-2 graph crosses earlier, at 90 000 (1.22 and 1.24).
+# ms, at 110 000 and 120 000 random assignments, window of the planner DAG: side by side 3.61, 4.12, from records
+# 3.87, 3.90 (explicit 4.11, 4.85 and 4.47, 4.50), table scorer 5.3.
 _SCORE_TERMS_BELOW = 114688
+# The same where the walk is one over tile images, which takes as long for 65 536 assignments as for one (a
+# wavefront a SIMD).  In ms, at 49 152, 57 344 and 81 920 random assignments: Llama-3-8B graph side by side 1.85,
+# 2.33, 2.95, by images 2.36, 2.35, 2.88 (explicit ones 2.54, 3.12, 4.08 and 2.45, 2.46, 2.70), 12-layer GPT-2 graph
+# 0.60, 0.75, 0.95 and 0.63, 0.63, 0.80.
+_SCORE_TERMS_BELOW_IMAGES = 57344
+# Random assignments up to which tile images are walked with a lane each; beyond, lanes take two or four, which
+# share a tile's draws of far producers and unpacking.  In ms, images and lanes of several, at 196 608 and 262 144:
+# Llama-3-8B graph 3.65, 4.59 and 4.48, 4.68; 12-layer GPT-2 graph 1.06, 1.31 and 1.31, 1.21.  Explicit ones always: at
+# 131 072, 262 144, 524 288 and 2^20 of the Llama-3-8B graph 2.6, 3.8, 7.5, 14.9 against 5.7, 6.7, 8.5, 17.0.
+_SCORE_IMAGES_UP_TO = 196608
 # Matrices of up to this many LDS tiles (64 KB each) go through LDS in the table scorer, larger
 # ones are read in place.  Measured on a 3 000-node window of the stress DAG, 2^20 assignments:
 # 17.9 ms with 1, 17.4 with 2, 18.0 with 4, 18.35 with 8 or 16.  (A lower bound, small matrices
@@ -682,9 +690,10 @@ class CostEngine:
         """Scoring of a large batch.  A graph with large blocks: from the block
         table while the entry arrays are what the last build made of it
         (apc_score_table, 5x the rate of any walk over records there).  Else,
-        and for graphs with small blocks: below _SCORE_TERMS_BELOW assignments with
+        and for graphs with small blocks: below _SCORE_TERMS_BELOW_IMAGES assignments with
         the terms gathered side by side from the table (apc_score_fold_table), from
-        there on by tiles of edges (apc_score_from_tiles: 10.4 ms for 2^20 assignments
+        there on by tiles of edges (apc_score_images, or with more random ones
+        apc_score_from_tiles: 10.4 ms for 2^20 assignments
         of the Llama-3-8B graph, against 15.6 ms from records, 18.0 ms from the table
         edge by edge and 31.2 ms from the three arrays).  Where the table does not
         stand for the arrays, or the graph has no such tiles: from records made here if the entry
@@ -710,22 +719,30 @@ class CostEngine:
             self.last_score_backend = "block_table"
             return out
         from_table &= self._versioned  # else an edit would go unnoticed
-        if from_table and count < _SCORE_TERMS_BELOW and _SCORE_SMALL_FROM_TABLE:
-            return self._score_terms(clamp, assign, seed, first, count, d_gid, first_node, init, out, stream)
-        if from_table and _SCORE_FROM_TILES and not self.large_blocks:
-            tiles = self._score_tiles(first_node, assign is not None)
-            if tiles is not None:
+        if from_table and _SCORE_FROM_TILES and not self.large_blocks and (
+                count >= _SCORE_TERMS_BELOW_IMAGES or not _SCORE_SMALL_FROM_TABLE or _SCORE_TERMS_BELOW <= count):
+            name, scratch = "apc_score_images", None
+            if assign is not None or count <= _SCORE_IMAGES_UP_TO:
+                tiles = self._score_tiles(first_node, True)
+                if tiles is not None:
+                    scratch = self._scratch((tiles[3] + 1) * _lib.SCORE_IMAGE_BYTES)
+            if scratch is None:
+                name, tiles = "apc_score_from_tiles", self._score_tiles(first_node, assign is not None)
+                if tiles is not None:
+                    scratch = self._scratch(tiles[1] * _lib.SCORE_STEP_BYTES)
+            if scratch is not None:
                 steps, n_step, d_tiles, n_tile, units = tiles
-                call_steps = torch.empty(n_step * _lib.SCORE_STEP_BYTES, dtype=torch.uint8, device=self.device)
                 _lib.check(
-                    self.lib.apc_score_from_tiles(
+                    getattr(self.lib, name)(
                         C.byref(self.problem), self._ptr(self.per_arg), self._ptr(self.table), self._ptr(steps), n_step,
-                        self._ptr(d_tiles), n_tile, self._ptr(units), self._ptr(call_steps), self._ptr(assign),
+                        self._ptr(d_tiles), n_tile, self._ptr(units), self._ptr(scratch), self._ptr(assign),
                         int(seed), int(first), int(count), self._ptr(d_gid), clamp, self._ptr(init),
                         self._ptr(out), stream),
-                    "apc_score_from_tiles")
+                    name)
                 self.last_score_backend = "block_table_tiles"
                 return out
+        if from_table and count < _SCORE_TERMS_BELOW and _SCORE_SMALL_FROM_TABLE:
+            return self._score_terms(clamp, assign, seed, first, count, d_gid, first_node, init, out, stream)
         recs_stand = (self._recs_valid and self._unchanged(self._recs_marks)
                       and (capturing or not self._recorded_writes))  # else replayed since, or not
         if capturing and not recs_stand:  # records are not made meanwhile: the host reads their check
@@ -772,8 +789,17 @@ class CostEngine:
         self.last_score_backend = "records"
         return out
 
+    def _scratch(self, nbytes: int) -> Optional[torch.Tensor]:
+        """Scratch of a call, or None where the device has no room for it: the caller then takes a way that needs
+        less."""
+        try:
+            return torch.empty(nbytes, dtype=torch.uint8, device=self.device)
+        except torch.cuda.OutOfMemoryError:
+            return None
+
     def _score_tiles(self, first_node: int, explicit: bool):
-        """The layout apc_score_from_tiles walks from ``first_node`` on, on the device, or None:
+        """The layout apc_score_from_tiles walks from ``first_node`` on (apc_score_images: one made with
+        ``explicit``), on the device, or None:
         a graph that form does not take, or no layout at hand (_layout)."""
         return self._layout("score_tiles_explicit" if explicit else "score_tiles", first_node,
                             lambda: self._make_score_tiles(first_node, explicit))

@@ -778,6 +778,16 @@ int apc_score_from_tiles(const apc_problem* p, const double* per_arg, const doub
                          int64_t n_assign, const int32_t* node_gid, int32_t clamp_inf, const double* init, double* out,
                          void* stream);
 
+/* As apc_score_from_tiles, over a layout made with explicit_rows (for random assignments too):
+ * every tile is first laid out in one piece, matrices, terms and what its steps do, which a
+ * workgroup then copies without looking anything up.  For up to 2^18 assignments, and any number
+ * of explicit ones.  scratch: 16-byte aligned, (n_tile + 1) * APC_SCORE_IMAGE_BYTES. */
+#define APC_SCORE_IMAGE_BYTES 43008
+int apc_score_images(const apc_problem* p, const double* per_arg, const double* table, const apc_score_step* steps,
+                     int32_t n_step, const apc_score_tile* tiles, int32_t n_tile, const apc_score_unit* units,
+                     void* scratch, const uint16_t* assign, uint64_t seed, int64_t first, int64_t n_assign,
+                     const int32_t* node_gid, int32_t clamp_inf, const double* init, double* out, void* stream);
+
 /* apc_score_random_assignments for a graph too large to keep its coefficients
  * resident: the problem holds a window of the graph's nodes (preceded by
  * first_node stand-ins for producers outside the window, which are not scored),

@@ -124,3 +124,42 @@ def test_scores_have_the_bits_of_the_walk_over_records(name, count, monkeypatch)
         monkeypatch.setattr(engine_mod, "_SCORE_FROM_TILES", True)
         assert all(torch.equal(a, b) for a, b in zip(got, want))
         eng.set_node_multiplier(mult)  # the layout is kept, the multipliers are the call's
+
+
+# a lane per assignment from tile images: rows of explicit choices brought in 16, 4 and 2 bytes a lane (by
+# their number and where they start), two tiles ahead and one (from 768 lanes a workgroup), one launch and two;
+# workgroups without a whole wavefront, and rows that end inside one
+@pytest.mark.gpu
+@pytest.mark.parametrize("name,count,skip", [
+    ("moe_8x8", 8, 0), ("moe_8x8", 1002, 0), ("moe_8x8", 131080, 0), ("gpt2_2x3", 131080, 2), ("gpt2_2x3", 131082, 0),
+    ("gpt2_2x3", 131080, 1), ("stress_60", 163848, 0), ("stress_60", 196616, 0), ("moe_8x8", 196618, 0),
+    ("gpt2_2x3", 262160, 0), ("stress_60", 262154, 0)])
+def test_images_have_the_bits_of_the_walk_over_records(name, count, skip, monkeypatch):
+    g = GRAPHS[name]()
+    eng = engine_mod.CostEngine(g, table_mode="full")
+    eng.large_blocks = False
+    eng.set_node_multiplier(np.arange(g.num_nodes) % 3 - 1)  # -1, 0, 1
+    eng.build()
+    gid = np.arange(g.num_nodes, dtype=np.int32) * 7 + 1
+    gen = torch.Generator(device="cuda").manual_seed(count)
+    nstrat = torch.from_numpy(g.node_nstrat.astype(np.int32)).cuda()[:, None]
+    given = torch.empty(g.num_nodes * count + skip, dtype=torch.int16, device="cuda")[skip:].view(g.num_nodes, count)
+    given.copy_(torch.randint(0, 1 << 30, (g.num_nodes, count), device="cuda", generator=gen, dtype=torch.int32) % nstrat)
+    init = torch.rand((count, 6), dtype=torch.float64, device="cuda", generator=gen) * 1e6
+    init[::3] = -0.0
+
+    def scores(backend):
+        out = []
+        for score in (lambda: eng.score_random(11, 5, count), lambda: eng.score(given),
+                      lambda: eng.score_random_window(11, 5, count, gid, 5, init=init),
+                      lambda: eng.score_window(given, 5, init=init)):
+            out.append(score().view(torch.int64))
+            assert eng.last_score_backend == backend
+        return out
+
+    monkeypatch.setattr(engine_mod, "_SCORE_LANES_FROM", 1)
+    monkeypatch.setattr(engine_mod, "_SCORE_TERMS_BELOW", 0)
+    monkeypatch.setattr(engine_mod, "_SCORE_IMAGES_UP_TO", 1 << 20)
+    got = scores("block_table_tiles")
+    monkeypatch.setattr(engine_mod, "_SCORE_FROM_TILES", False)
+    assert all(torch.equal(a, b) for a, b in zip(got, scores("compact_records")))
