@@ -37,15 +37,16 @@ _SCORE_TERMS_BELOW_IMAGES = 57344
 # Llama-3-8B graph 3.65, 4.59 and 4.48, 4.68; 12-layer GPT-2 graph 1.06, 1.31 and 1.31, 1.21.  Explicit ones always: at
 # 131 072, 262 144, 524 288 and 2^20 of the Llama-3-8B graph 2.6, 3.8, 7.5, 14.9 against 5.7, 6.7, 8.5, 17.0.
 _SCORE_IMAGES_UP_TO = 196608
+_SCORE_STREAM = True  # random assignments on graphs with large blocks: matrices as a stream of pieces through LDS
 # Matrices of up to this many LDS tiles (64 KB each) go through LDS in the table scorer, larger
 # ones are read in place.  Measured on a 3 000-node window of the stress DAG, 2^20 assignments:
 # 17.9 ms with 1, 17.4 with 2, 18.0 with 4, 18.35 with 8 or 16.  (A lower bound, small matrices
 # read in place to save their barrier, only cost time: 17.4 -> 18.9 ms at 1 024 doubles.)
 _SCORE_STAGE_TILES = 2
-# The table scorer pays about 2 us per edge whatever the batch (a matrix copied into LDS on every CU), the
-# walks over records about 14 ns per edge and assignment: from this many assignments on the table wins
-# (measured on a 3 000-node window of the stress DAG: 18 ms per window from the table for any batch up to
-# 2^20, 78 ms from compact records for 2^20)
+# The table scorers pay about 1.4 us per edge (random assignments) or 2 us whatever the batch (a matrix copied into LDS
+# on every CU), the walks over records about 14 ns per edge and assignment: from this many assignments on the table wins
+# (random ones, window of the planner DAG of 1 600 nodes, table and compact records in ms: 131 072 4.1 and 4.0, 200 001
+# 4.3 and 6.5, 2^20 7.1 and 44)
 _SCORE_TABLE_FROM = 131072
 _SCORE_PER_LANE = 0  # assignments per lane of the compact scorer; 0: the library chooses
 # Assignments from which one lane each beats several wavefronts per 64 assignments, by the number
@@ -224,7 +225,8 @@ class CostEngine:
         assert g.num_edges == 0 or int(sizes.max()) < 2**31, "edge block too large for 32-bit local index"
 
         self._keep: Dict[str, torch.Tensor] = {}
-        self._layouts: Dict[str, dict] = {"score_tiles": {}, "score_tiles_explicit": {}, "sample_steps": {}}
+        self._layouts: Dict[str, dict] = {"score_tiles": {}, "score_tiles_explicit": {}, "sample_steps": {},
+                                          "score_pieces": {}}
 
         # The problem is some thirty arrays, most of them a few kilobytes: they go up in
         # one copy.  An array is laid into a pinned staging buffer and gets its address
@@ -689,7 +691,8 @@ class CostEngine:
     def _score_packed(self, assign, seed, first, count, d_gid, first_node, init, out) -> torch.Tensor:
         """Scoring of a large batch.  A graph with large blocks: from the block
         table while the entry arrays are what the last build made of it
-        (apc_score_table, 5x the rate of any walk over records there).  Else,
+        (apc_score_stream, or apc_score_table for explicit assignments and more strategies than that takes; 5x the
+        rate of any walk over records there).  Else,
         and for graphs with small blocks: below _SCORE_TERMS_BELOW_IMAGES assignments with
         the terms gathered side by side from the table (apc_score_fold_table), from
         there on by tiles of edges (apc_score_images, or with more random ones
@@ -707,6 +710,19 @@ class CostEngine:
         clamp = self._standing_clamp() if _SCORE_FROM_TABLE else None
         from_table = clamp is not None
         if from_table and (self.large_blocks or not _SCORE_COMPACT) and count >= _SCORE_TABLE_FROM:
+            pieces = self._score_pieces(first_node) if assign is None and _SCORE_STREAM else None
+            if pieces is not None:
+                d_pieces, n_piece, n_item = pieces
+                scratch = self._scratch(n_item * _lib.SCORE_SIDE_BYTES + n_piece * _lib.SCORE_PIECE_SCRATCH)
+                if scratch is not None:
+                    _lib.check(
+                        self.lib.apc_score_stream(
+                            C.byref(self.problem), self._ptr(self.per_arg), self._ptr(self.table), self._ptr(d_pieces),
+                            n_piece, n_item, self._ptr(scratch), int(seed), int(first), int(count), self._ptr(d_gid),
+                            clamp, self._ptr(init), self._ptr(out), stream),
+                        "apc_score_stream")
+                    self.last_score_backend = "block_table"
+                    return out
             aux = self._score_edge_aux(d_gid)
             _lib.check(
                 self.lib.apc_score_table(
@@ -842,6 +858,38 @@ class CostEngine:
                         torch.from_numpy(tiles[:n_tile]).to(self.device), n_tile,
                         torch.from_numpy(units[:n_unit]).to(self.device))
         return plan
+
+    def _score_pieces(self, first_node: int):
+        """(apc_score_piece records on the device, pieces, items) of apc_score_stream for the walk from
+        ``first_node`` on, or None: a node with too many strategies, nothing to score, or no layout at hand."""
+        return self._layout("score_pieces", first_node, lambda: self._make_score_pieces(first_node))
+
+    def _make_score_pieces(self, first_node: int):
+        g = self.g
+        compressed = self.table_mode == "compressed"
+        _, block_off, _, table_off, usrc, udst = g.block_table(compressed)
+        # rows and columns of a matrix: of distinct words where it is compressed
+        size = g.edge_ssrc.astype(np.int64) * g.edge_sdst
+        squeezed = (table_off >= 0) & (usrc > 0)
+        if squeezed.any():
+            block = np.searchsorted(block_off, table_off[squeezed], side="right") - 1
+            size[squeezed] = usrc[squeezed].astype(np.int64) * udst[block]
+        if g.num_edges and size.max() > 0x7FFFFFFF - _lib.SCORE_PIECE:
+            return None
+        size = size.astype(np.int32)
+        edges = np.ascontiguousarray(g.edge_records(compressed))
+        off, nstrat = [np.ascontiguousarray(x, np.int32) for x in (g.node_edge_off, g.node_nstrat)]
+        most = int((size // _lib.SCORE_PIECE + 1).sum()) + g.num_nodes
+        pieces = np.empty((most, _lib.SCORE_PIECE_BYTES), np.uint8)
+        n_piece, n_item = C.c_int32(0), C.c_int32(0)
+        _lib.check(
+            self.lib.apc_score_pieces(
+                edges.ctypes.data, g.num_edges, g.num_nodes, off.ctypes.data, nstrat.ctypes.data, size.ctypes.data,
+                int(first_node), pieces.ctypes.data, most, C.byref(n_piece), C.byref(n_item)),
+            "apc_score_pieces")
+        if n_piece.value == 0:
+            return None
+        return torch.from_numpy(pieces[:n_piece.value]).to(self.device), n_piece.value, n_item.value
 
     def _score_msize(self) -> np.ndarray:
         """int32[num_edges]: the padded size of an edge's matrix in the block table

@@ -891,6 +891,36 @@ int apc_score_table(const apc_problem* p, const double* per_arg, const double* t
                     const double* init, double* out, void* stream);
 int apc_score_table_tile(void);
 
+/* apc_score_table for random assignments, as a stream of pieces of matrices: no edge is too large, and copies go on
+ * during the draws from earlier pieces, whatever their sizes.  apc_score_pieces (host, no device needed) makes the list:
+ * the argument rows of nodes first_node.. in node order, then argument order, the matrix of an edge with table_off >= 0
+ * (msize[e] elements, even table_off) in pieces of APC_SCORE_PIECE elements at most, a piece for every other edge and for
+ * a node without one, and where and when each goes into the ring.  An item is an edge or such a node.  *n_piece = 0: nothing
+ * to score, or an item for which 10 * S_dst + 2 * S_src is over APC_SCORE_SIDE_BYTES: use apc_score_table.  The list depends
+ * on the graph alone; it is copied to the device and serves every call.
+ * scratch: 16-byte aligned, n_item * APC_SCORE_SIDE_BYTES + n_piece * 96 bytes. */
+#define APC_SCORE_PIECE 8192
+#define APC_SCORE_SIDE_BYTES 8192
+#define APC_PIECE_FIRST_OF_NODE 1
+#define APC_PIECE_FIRST 2 /* of its item */
+#define APC_PIECE_LAST 4
+typedef struct apc_score_piece {
+  int32_t node;
+  int32_t edge; /* or -1 */
+  int32_t item;
+  int32_t flags;
+  int32_t base; /* elements of the matrix in front of this piece */
+  int32_t n;    /* and in it; 0 without a matrix */
+  int32_t lds;  /* place in the ring, bytes */
+  int32_t ask;  /* once pieces in front of this one are done with, all in front of piece ask are asked for */
+} apc_score_piece; /* 32 bytes */
+int apc_score_pieces(const apc_edge* edges, int32_t n_edge, int32_t n_node, const int32_t* node_edge_off,
+                     const int32_t* node_nstrat, const int32_t* msize, int32_t first_node, apc_score_piece* pieces,
+                     int64_t max_piece, int32_t* n_piece, int32_t* n_item);
+int apc_score_stream(const apc_problem* p, const double* per_arg, const double* table, const apc_score_piece* pieces,
+                     int32_t n_piece, int32_t n_item, void* scratch, uint64_t seed, int64_t first, int64_t n_assign,
+                     const int32_t* node_gid, int32_t clamp_inf, const double* init, double* out, void* stream);
+
 /* Replaces remove_invalid_configs (autoparallel/shardings/propagation_rules.py:127-158)
  * and keep_unique_configs (autoparallel/shardings/placement_options.py:151-170) for the
  * candidate strategies of n_set nodes in packed form.  Set s has rows
