@@ -82,6 +82,9 @@ __host__ __device__ __forceinline__ uint32_t plain_draw(uint32_t h0, int32_t gid
   return (uint32_t)(((uint64_t)h * (uint64_t)(uint32_t)nstrat) >> 32);
 }
 
+// the sampler's rank draw hashes the node's key with this, so that it is not the plain draw's
+constexpr uint32_t kRankSalt = 0x68E31DA4u;
+
 // x + 1.0 n times over.  While x is a whole number below 2^52 every step is exact, and so
 // is x + n in one step (what the carried sums are in practice: counts); anything else is
 // added one by one, as a sequential walk does.

@@ -37,7 +37,7 @@ typedef uint64_t u64x2_t __attribute__((ext_vector_type(2)));
 // Which of the count allowed strategies of a node is taken, counted in out_idx order:
 // uniform in [0, count), from a hash of its own (not the plain draw's).
 __host__ __device__ __forceinline__ uint32_t rank_draw(uint32_t h0, int32_t gid, uint32_t count) {
-  const uint32_t h = finalise32(h0 ^ node_key(gid) ^ 0x68E31DA4u);
+  const uint32_t h = finalise32(h0 ^ node_key(gid) ^ kRankSalt);
   return (uint32_t)(((uint64_t)h * (uint64_t)count) >> 32);
 }
 

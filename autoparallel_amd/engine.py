@@ -58,6 +58,10 @@ _SCORE_PER_LANE = 0  # assignments per lane of the compact scorer; 0: the librar
 # window of the planner DAG of 1 600 nodes 5.49, 6.33 and 6.34, 6.30, of 60 nodes 0.242, 0.260 and 0.270, 0.262.
 _SAMPLE_LANES_FROM = {2: 458752, 16: 229376}
 _SAMPLE_WAVES = 0  # 2 or 16: tests
+# Graphs of at most 64 strategies a node: by tiles of nodes through LDS, whatever the batch.  In ms, tiles, and wavefronts
+# or lanes: Llama-3-8B graph, 100, 131 072 and 524 288 assignments 2.0, 2.4, 7.2 and 3.0, 5.1, 21.2; 12-layer GPT-2 graph,
+# 100 and 131 072 0.66, 0.86 and 0.91, 1.56.
+_SAMPLE_TILES = True
 # Layouts of a kind (by first_node) an engine makes.  They stay until the engine goes, since a launch on
 # another stream or in a graph may still read one; calls beyond take the route that needs none.
 _LAYOUTS_KEPT = 16
@@ -226,7 +230,7 @@ class CostEngine:
 
         self._keep: Dict[str, torch.Tensor] = {}
         self._layouts: Dict[str, dict] = {"score_tiles": {}, "score_tiles_explicit": {}, "sample_steps": {},
-                                          "score_pieces": {}}
+                                          "score_pieces": {}, "sample_tiles": {}}
 
         # The problem is some thirty arrays, most of them a few kilobytes: they go up in
         # one copy.  An array is laid into a pinned staging buffer and gets its address
@@ -1044,6 +1048,30 @@ class CostEngine:
             "apc_pack_allowed_columns")
         return colbits, d_off, max_words
 
+    def _sample_tiles(self, first_node: int):
+        """(apc_sample_tile records, argument rows' places, both on the device, tiles, wide) of
+        apc_sample_feasible_tiles for the walk from ``first_node`` on, or None: a graph such a walk does not take, or no
+        layout at hand (_layout)."""
+        return self._layout("sample_tiles", first_node, lambda: self._make_sample_tiles(first_node))
+
+    def _make_sample_tiles(self, first_node: int):
+        g = self.g
+        n = g.num_nodes - first_node
+        if n <= 0 or g.num_edges == 0 or int(g.node_nstrat[first_node:].max()) > 64:
+            return None
+        off, src, ssrc, nstrat = [np.ascontiguousarray(x, np.int32) for x in (
+            g.node_edge_off, g.edge_src_node, g.edge_ssrc, g.node_nstrat)]
+        tiles, rows, n_tile = np.empty((n, _lib.SAMPLE_TILE_BYTES), np.uint8), np.zeros(g.num_edges, np.uint8), C.c_int32(0)
+        _lib.check(
+            self.lib.apc_sample_tiles(
+                g.num_nodes, g.num_edges, off.ctypes.data, src.ctypes.data, ssrc.ctypes.data, nstrat.ctypes.data,
+                int(first_node), tiles.ctypes.data, n, rows.ctypes.data, C.byref(n_tile)),
+            "apc_sample_tiles")
+        if n_tile.value == 0:
+            return None
+        return (torch.from_numpy(tiles[:n_tile.value]).to(self.device), torch.from_numpy(rows).to(self.device),
+                n_tile.value, int(nstrat[first_node:].max() > 32))
+
     def _sample_steps(self, first_node: int):
         """(records on the device, steps, wavefronts) of apc_sample_feasible_steps for the walk
         from ``first_node`` on, or None: a graph such a walk does not take (columns past its
@@ -1123,6 +1151,17 @@ class CostEngine:
                 words.append(w)
             d_keep = torch.from_numpy(np.concatenate(words).view(np.int64)).to(self.device)
             d_keep_off = torch.from_numpy(keep_off).to(self.device)
+        tiles = self._sample_tiles(first_node) if _SAMPLE_TILES and not _SAMPLE_WAVES and count > 0 else None
+        scratch = None if tiles is None else self._scratch((tiles[2] + 1) * _lib.SAMPLE_IMAGE_BYTES)
+        if scratch is not None:
+            d_tiles, d_rows, n_tile, wide = tiles
+            _lib.check(
+                self.lib.apc_sample_feasible_tiles(
+                    C.byref(self.problem), self._ptr(d_tiles), n_tile, self._ptr(d_rows), self._ptr(colbits),
+                    self._ptr(d_off), self._ptr(scratch), int(seed), int(first), int(count), self._ptr(d_gid),
+                    self._ptr(d_keep), self._ptr(d_keep_off), wide, self._ptr(assign), self._ptr(fallback), self._stream()),
+                "apc_sample_feasible_tiles")
+            return assign, fallback
         steps = self._sample_steps(first_node) if count < max(_SAMPLE_LANES_FROM.values()) else None
         if steps is not None and count < _SAMPLE_LANES_FROM[steps[2]]:
             recs, n_step, n_waves = steps

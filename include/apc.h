@@ -718,6 +718,34 @@ int apc_sample_feasible_steps(const apc_problem* p, const apc_sample_rec* recs, 
                               int64_t n_assign, const int32_t* node_gid, const uint64_t* row_filter,
                               const int64_t* filter_off, uint16_t* assign, int32_t* n_fallback, void* stream);
 
+/* The same draws by tiles of nodes through LDS, a lane per assignment, for graphs of at most 64 strategies a node.
+ * apc_sample_tiles (host, no device needed) lays the nodes from first_node on out: tiles of at most
+ * APC_SAMPLE_TILE_NODES nodes and as many argument rows, in node order, with the producers whose choices have left
+ * the ring of the last 64 (at most APC_SAMPLE_TILE_FAR a tile), and arg_row[n_edge], where an argument row's producer's
+ * choices are: the ring (0-63), 64 + place among those producers, APC_SAMPLE_ROW_NONE.  *n_tile = 0: no nodes, or not a
+ * graph for this form (more than 64 strategies, more than 32 argument rows, a producer behind its consumer).  The layout
+ * depends on the graph and first_node alone.  apc_sample_feasible_tiles is apc_sample_feasible over it, same results bit
+ * for bit.  wide: whether a node from first_node on has more than 32 strategies.  scratch: 16-byte aligned,
+ * (n_tile + 1) * APC_SAMPLE_IMAGE_BYTES. */
+#define APC_SAMPLE_TILE_NODES 32
+#define APC_SAMPLE_TILE_FAR 24
+#define APC_SAMPLE_ROW_NONE 255
+#define APC_SAMPLE_IMAGE_BYTES 19456
+typedef struct apc_sample_tile {
+  int32_t node0, n_node, edge0, n_edge;
+  int32_t seq0; /* node0 - first_node */
+  int32_t n_far;
+  int32_t far[APC_SAMPLE_TILE_FAR];
+  int32_t reserved[10];
+} apc_sample_tile; /* 160 bytes */
+int apc_sample_tiles(int32_t n_node, int32_t n_edge, const int32_t* node_edge_off, const int32_t* edge_src,
+                     const int32_t* edge_ssrc, const int32_t* node_nstrat, int32_t first_node, apc_sample_tile* tiles,
+                     int32_t max_tile, uint8_t* arg_row, int32_t* n_tile);
+int apc_sample_feasible_tiles(const apc_problem* p, const apc_sample_tile* tiles, int32_t n_tile, const uint8_t* arg_row,
+                              const uint64_t* colbits, const int64_t* col_off, void* scratch, uint64_t seed, int64_t first,
+                              int64_t n_assign, const int32_t* node_gid, const uint64_t* row_filter,
+                              const int64_t* filter_off, int32_t wide, uint16_t* assign, int32_t* n_fallback, void* stream);
+
 /* Scoring of small batches (the terms of 4 to 64 assignments a workgroup gathered side by side)
  * from the block table, arguments and results as apc_score_table's over nodes
  * first_node..n_node. */
