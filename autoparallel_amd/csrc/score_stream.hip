@@ -33,6 +33,7 @@ constexpr int kAheadMost = 16;  // pieces under way
 constexpr int kFinite = 0x1F8;  // v_cmp_class: normal, denormal, zero
 static_assert(2 * (kPieceDoubles * 8 + kSideBytes) <= kRingBytes, "a piece and the next one");
 
+typedef const __attribute__((address_space(1))) double* global_f64_ptr_t;
 typedef const __attribute__((address_space(3))) uint16_t* lds_u16_ptr_t;
 typedef const __attribute__((address_space(3))) double* lds_f64_ptr_t;
 
@@ -243,7 +244,7 @@ score_stream_kernel(const WalkRec* __restrict__ walk, const AskRec* __restrict__
     }
     if (!(flags & kEdge)) continue;
     if (flags & kInPlace) {
-      const double* const matrix = reinterpret_cast<const double*>((uint64_t)word(14, s) << 32 | word(13, s));
+      const global_f64_ptr_t matrix = (global_f64_ptr_t)((uint64_t)word(14, s) << 32 | word(13, s));
 #pragma unroll
       for (int k = 0; k < kPer; ++k) raw[k] = matrix[at[k]];
       // waited for here, not on every pass through the loop

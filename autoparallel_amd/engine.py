@@ -38,6 +38,7 @@ _SCORE_TERMS_BELOW_IMAGES = 57344
 # 131 072, 262 144, 524 288 and 2^20 of the Llama-3-8B graph 2.6, 3.8, 7.5, 14.9 against 5.7, 6.7, 8.5, 17.0.
 _SCORE_IMAGES_UP_TO = 196608
 _SCORE_STREAM = True  # random assignments on graphs with large blocks: matrices as a stream of pieces through LDS
+_SCORE_TERM_RECORDS = True  # terms side by side from records of the edges and nodes, made in front of them
 # Matrices of up to this many LDS tiles (64 KB each) go through LDS in the table scorer, larger
 # ones are read in place.  Measured on a 3 000-node window of the stress DAG, 2^20 assignments:
 # 17.9 ms with 1, 17.4 with 2, 18.0 with 4, 18.35 with 8 or 16.  (A lower bound, small matrices
@@ -683,12 +684,26 @@ class CostEngine:
         return out
 
     def _score_terms(self, clamp, assign, seed, first, count, d_gid, first_node, init, out, stream) -> torch.Tensor:
-        _lib.check(
-            self.lib.apc_score_fold_table(
-                C.byref(self.problem), self._ptr(self.per_arg), self._ptr(self.table), self._ptr(assign), int(seed),
-                int(first), int(count), self._ptr(d_gid), int(first_node), clamp, self._ptr(init),
-                self._ptr(out), stream),
-            "apc_score_fold_table")
+        g = self.g
+        first_edge = int(g.node_edge_off[first_node])
+        scratch = None
+        if _SCORE_TERM_RECORDS and first_node < g.num_nodes and first_edge < g.num_edges:
+            scratch = self._scratch((g.num_edges - first_edge) * _lib.FOLD_EDGE_BYTES
+                                    + (g.num_nodes - first_node) * _lib.FOLD_NODE_BYTES)
+        if scratch is not None:
+            _lib.check(
+                self.lib.apc_score_terms(
+                    C.byref(self.problem), self._ptr(self.per_arg), self._ptr(self.table), self._ptr(scratch),
+                    self._ptr(assign), int(seed), int(first), int(count), self._ptr(d_gid), int(first_node), first_edge,
+                    clamp, self._ptr(init), self._ptr(out), stream),
+                "apc_score_terms")
+        else:
+            _lib.check(
+                self.lib.apc_score_fold_table(
+                    C.byref(self.problem), self._ptr(self.per_arg), self._ptr(self.table), self._ptr(assign), int(seed),
+                    int(first), int(count), self._ptr(d_gid), int(first_node), clamp, self._ptr(init),
+                    self._ptr(out), stream),
+                "apc_score_fold_table")
         self.last_score_backend = "block_table_terms"
         return out
 

@@ -753,6 +753,14 @@ int apc_score_fold_table(const apc_problem* p, const double* per_arg, const doub
                          uint64_t seed, int64_t first, int64_t n_assign, const int32_t* node_gid, int32_t first_node,
                          int32_t clamp_inf, const double* init, double* out, void* stream);
 
+/* The same from records of edges and nodes, which a launch in front makes: first_edge is node_edge_off[first_node],
+ * below n_edge, and first_node below n_node.  scratch: 16-byte aligned, 48 bytes per edge from first_edge on and 16 per node
+ * from first_node on. */
+int apc_score_terms(const apc_problem* p, const double* per_arg, const double* table, void* scratch,
+                    const uint16_t* assign, uint64_t seed, int64_t first, int64_t n_assign, const int32_t* node_gid,
+                    int32_t first_node, int32_t first_edge, int32_t clamp_inf, const double* init, double* out,
+                    void* stream);
+
 /* Scoring of large batches on graphs with small blocks, from the block table through LDS.
  * apc_score_tiles (host, no device needed) lays the walk from first_node on out: a step per
  * argument row (and per node without one) in node order, then argument order; tiles of
