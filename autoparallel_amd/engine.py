@@ -22,16 +22,15 @@ _SCORE_FROM_TABLE = True  # the three ways of scoring a graph with large blocks 
 _SCORE_COMPACT = True
 _SCORE_SMALL_FROM_TABLE = True
 _SCORE_FROM_TILES = True  # small blocks: matrices through LDS by tiles, while the table stands for the arrays
-# Below, the terms of a few assignments gathered side by side are faster than any walk with a lane per
-# assignment: up to here a CU takes seven workgroups of 64, an eighth costs more than a walk's lanes do.  In
-# ms, at 110 000 and 120 000 random assignments, window of the planner DAG: side by side 3.61, 4.12, from records
-# 3.87, 3.90 (explicit 4.11, 4.85 and 4.47, 4.50), table scorer 5.3.
+# Below, the terms of a few assignments gathered side by side are faster than a walk over records with a lane per
+# assignment: random ones of a window of the planner DAG, 98 304 and 114 688 assignments, 2.49 and 2.98 ms against 3.83 and
+# 3.87, explicit ones 3.10 and 3.79 against 4.40 and 4.45.
 _SCORE_TERMS_BELOW = 114688
-# The same where the walk is one over tile images, which takes as long for 65 536 assignments as for one (a
-# wavefront a SIMD).  In ms, at 49 152, 57 344 and 81 920 random assignments: Llama-3-8B graph side by side 1.85,
-# 2.33, 2.95, by images 2.36, 2.35, 2.88 (explicit ones 2.54, 3.12, 4.08 and 2.45, 2.46, 2.70), 12-layer GPT-2 graph
-# 0.60, 0.75, 0.95 and 0.63, 0.63, 0.80.
-_SCORE_TERMS_BELOW_IMAGES = 57344
+# The same where the walk is one over tile images, which is as long for one assignment as for the 65 536 that are a
+# wavefront a SIMD; terms go in rounds of 16 384.  In ms, terms and images: Llama-3-8B graph, random, at 114 688 and 131 072
+# 2.49, 2.90 and 2.80, 2.91, explicit, at 81 920 and 90 112 2.48, 2.70 and 3.16, 2.70; 12-layer GPT-2 graph 0.77, 0.81 and
+# 0.86, 0.81, and 0.64, 0.72 and 0.81, 0.72.
+_SCORE_TERMS_UP_TO_IMAGES = {"random": 114688, "explicit": 81920}
 # Random assignments up to which tile images are walked with a lane each; beyond, lanes take two or four, which
 # share a tile's draws of far producers and unpacking.  In ms, images and lanes of several, at 196 608 and 262 144:
 # Llama-3-8B graph 3.65, 4.59 and 4.48, 4.68; 12-layer GPT-2 graph 1.06, 1.31 and 1.31, 1.21.  Explicit ones always: at
@@ -44,11 +43,13 @@ _SCORE_TERM_RECORDS = True  # terms side by side from records of the edges and n
 # 17.9 ms with 1, 17.4 with 2, 18.0 with 4, 18.35 with 8 or 16.  (A lower bound, small matrices
 # read in place to save their barrier, only cost time: 17.4 -> 18.9 ms at 1 024 doubles.)
 _SCORE_STAGE_TILES = 2
-# The table scorers pay about 1.4 us per edge (random assignments) or 2 us whatever the batch (a matrix copied into LDS
-# on every CU), the walks over records about 14 ns per edge and assignment: from this many assignments on the table wins
-# (random ones, window of the planner DAG of 1 600 nodes, table and compact records in ms: 131 072 4.1 and 4.0, 200 001
-# 4.3 and 6.5, 2^20 7.1 and 44)
+# The table scorers take as long whatever the batch, 0.85 us a piece of a matrix (random assignments) or 2.5 us an
+# edge (explicit ones), terms side by side about 9 ns (random) and 12 per edge and 1 000 assignments.  In ms, random ones,
+# terms and table: window of the planner DAG (1.6 pieces an edge), 131 072 and 147 456 assignments 3.64, 4.08 and 4.43, 4.15;
+# 8-layer 70B decoder on 2x2x4 (2.6 pieces), 131 072 2.09, 4.52.  Explicit ones, that window, 163 840 and 196 608 6.03,
+# 7.89 and 7.76, 7.89.  The table it is from this many assignments on, times pieces per edge over 1.5 (random) or 1.5.
 _SCORE_TABLE_FROM = 131072
+_SCORE_TABLE_PIECES, _SCORE_TABLE_EXPLICIT = 1.5, 1.5
 _SCORE_PER_LANE = 0  # assignments per lane of the compact scorer; 0: the library chooses
 # Assignments from which one lane each beats several wavefronts per 64 assignments, by the number
 # of wavefronts.  Lanes go in rounds of 2^18 that cost the same however full, wavefronts by the
@@ -712,8 +713,8 @@ class CostEngine:
         table while the entry arrays are what the last build made of it
         (apc_score_stream, or apc_score_table for explicit assignments and more strategies than that takes; 5x the
         rate of any walk over records there).  Else,
-        and for graphs with small blocks: below _SCORE_TERMS_BELOW_IMAGES assignments with
-        the terms gathered side by side from the table (apc_score_fold_table), from
+        and for graphs with small blocks: up to _SCORE_TERMS_UP_TO_IMAGES assignments with
+        the terms gathered side by side from the table (apc_score_terms), from
         there on by tiles of edges (apc_score_images, or with more random ones
         apc_score_from_tiles: 10.4 ms for 2^20 assignments
         of the Llama-3-8B graph, against 15.6 ms from records, 18.0 ms from the table
@@ -728,8 +729,17 @@ class CostEngine:
         capturing = self._capturing(stream)
         clamp = self._standing_clamp() if _SCORE_FROM_TABLE else None
         from_table = clamp is not None
-        if from_table and (self.large_blocks or not _SCORE_COMPACT) and count >= _SCORE_TABLE_FROM:
-            pieces = self._score_pieces(first_node) if assign is None and _SCORE_STREAM else None
+        large = self.large_blocks or not _SCORE_COMPACT
+        pieces = None
+        table_from = _SCORE_TABLE_FROM
+        if from_table and large and count >= table_from and self._versioned:
+            if assign is not None:
+                table_from *= _SCORE_TABLE_EXPLICIT
+            elif _SCORE_STREAM:
+                pieces = self._score_pieces(first_node)
+                if pieces is not None:
+                    table_from *= max(1.0, pieces[1] / pieces[2] / _SCORE_TABLE_PIECES)
+        if from_table and large and count >= table_from:
             if pieces is not None:
                 d_pieces, n_piece, n_item = pieces
                 scratch = self._scratch(n_item * _lib.SCORE_SIDE_BYTES + n_piece * _lib.SCORE_PIECE_SCRATCH)
@@ -755,7 +765,8 @@ class CostEngine:
             return out
         from_table &= self._versioned  # else an edit would go unnoticed
         if from_table and _SCORE_FROM_TILES and not self.large_blocks and (
-                count >= _SCORE_TERMS_BELOW_IMAGES or not _SCORE_SMALL_FROM_TABLE or _SCORE_TERMS_BELOW <= count):
+                count > _SCORE_TERMS_UP_TO_IMAGES["random" if assign is None else "explicit"]
+                or not _SCORE_SMALL_FROM_TABLE or _SCORE_TERMS_BELOW <= count):
             name, scratch = "apc_score_images", None
             if assign is not None or count <= _SCORE_IMAGES_UP_TO:
                 tiles = self._score_tiles(first_node, True)
@@ -776,7 +787,8 @@ class CostEngine:
                     name)
                 self.last_score_backend = "block_table_tiles"
                 return out
-        if from_table and count < _SCORE_TERMS_BELOW and _SCORE_SMALL_FROM_TABLE:
+        terms_below = table_from if large and _SCORE_TERMS_BELOW else _SCORE_TERMS_BELOW
+        if from_table and count < max(terms_below, _SCORE_TERMS_BELOW) and _SCORE_SMALL_FROM_TABLE:
             return self._score_terms(clamp, assign, seed, first, count, d_gid, first_node, init, out, stream)
         recs_stand = (self._recs_valid and self._unchanged(self._recs_marks)
                       and (capturing or not self._recorded_writes))  # else replayed since, or not
