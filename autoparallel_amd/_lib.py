@@ -18,6 +18,7 @@ SAMPLE_REC_BYTES = 64
 CHECK_MAX_NODES = 131072
 SCORE_STEP_BYTES, SCORE_TILE_BYTES, SCORE_UNIT_BYTES = 64, 128, 16
 SCORE_IMAGE_BYTES = 43008
+PAIR_STEP_BYTES, PAIR_TILE_BYTES, PAIR_IMAGE_BYTES = 24, 80, 55296
 FOLD_EDGE_BYTES, FOLD_NODE_BYTES = 48, 16
 SAMPLE_TILE_BYTES, SAMPLE_IMAGE_BYTES = 160, 19456
 SCORE_PIECE, SCORE_SIDE_BYTES = 8192, 8192
@@ -296,6 +297,14 @@ _SIGNATURES = {
         [C.POINTER(ApcProblem), C.c_void_p, C.c_void_p, C.c_void_p, C.c_int32, C.c_void_p, C.c_int32, C.c_void_p,
          C.c_void_p, C.c_void_p, C.c_uint64, C.c_int64, C.c_int64, C.c_void_p, C.c_int32, C.c_void_p, C.c_void_p,
          C.c_void_p]),
+    "apc_pair_tiles": (
+        C.c_int,
+        [C.c_void_p, C.c_int32, C.c_int32, C.c_void_p, C.c_void_p, C.c_int32, C.c_void_p, C.c_int64, C.c_void_p,
+         C.c_int64, C.c_void_p, C.c_void_p]),
+    "apc_score_pairs": (
+        C.c_int,
+        [C.POINTER(ApcProblem), C.c_void_p, C.c_void_p, C.c_void_p, C.c_int32, C.c_void_p, C.c_int32, C.c_void_p,
+         C.c_uint64, C.c_int64, C.c_int64, C.c_void_p, C.c_int32, C.c_void_p, C.c_void_p]),
     "apc_sample_tiles": (
         C.c_int,
         [C.c_int32, C.c_int32, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_int32, C.c_void_p, C.c_int32,

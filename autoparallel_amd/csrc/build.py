@@ -23,7 +23,7 @@ HIPCC_FLAGS = [
 
 
 def build(verbose: bool = True) -> str:
-    srcs = [os.path.join(HERE, f) for f in ("apc.hip", "lut.hip", "score.hip", "score_tiles.hip", "score_fold.hip", "score_images.hip", "score_stream.hip", "sample.hip", "sample_tiles.hip", "passes.hip", "schedule.hip", "nccl_plan.cpp")]
+    srcs = [os.path.join(HERE, f) for f in ("apc.hip", "lut.hip", "score.hip", "score_tiles.hip", "score_fold.hip", "score_images.hip", "score_stream.hip", "score_pairs.hip", "sample.hip", "sample_tiles.hip", "passes.hip", "schedule.hip", "nccl_plan.cpp")]
     cmd = ["hipcc"] + HIPCC_FLAGS + srcs + ["-o", LIB]
     if verbose:
         print(" ".join(cmd), flush=True)

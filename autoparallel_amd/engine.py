@@ -31,9 +31,16 @@ _SCORE_TERMS_BELOW = 114688
 # 2.49, 2.90 and 2.80, 2.91, explicit, at 81 920 and 90 112 2.48, 2.70 and 3.16, 2.70; 12-layer GPT-2 graph 0.77, 0.81 and
 # 0.86, 0.81, and 0.64, 0.72 and 0.81, 0.72.
 _SCORE_TERMS_UP_TO_IMAGES = {"random": 114688, "explicit": 81920}
-# Random assignments up to which tile images are walked with a lane each; beyond, lanes take two or four, which
+# Random assignments that carry no sums: from images of finished entries beyond these many, the second where a tile of
+# theirs has few argument rows, for which its beginning counts.  In ms, finished entries, tile images (from 262 144 on lanes of
+# several), terms: 12-layer GPT-2 graph (10 rows a tile), 90 112 0.62, 0.81, 0.66, 131 072 0.64, 0.81, 0.87, 262 144 0.98,
+# 1.22, 2^20 2.24, 3.42; Llama-3-8B graph (4.2), 131 072 2.98, 2.91, 2.80, 163 840 3.31, 3.65, 3.45, 262 144 3.68, 4.68,
+# 2^20 7.24, 10.41; MoE graph (4.9), 131 072 1.59, 1.57, 1.53.
+_SCORE_PAIRS = True
+_SCORE_PAIRS_FROM, _SCORE_PAIRS_ROWS = (81920, 131072), 8
+# Else, random assignments up to which tile images are walked with a lane each; beyond, lanes take two or four, which
 # share a tile's draws of far producers and unpacking.  In ms, images and lanes of several, at 196 608 and 262 144:
-# Llama-3-8B graph 3.65, 4.59 and 4.48, 4.68; 12-layer GPT-2 graph 1.06, 1.31 and 1.31, 1.21.  Explicit ones always: at
+# Llama-3-8B graph 3.65, 4.59 and 4.48, 4.68; 12-layer GPT-2 graph 1.06, 1.31 and 1.31, 1.21.  Explicit ones at any number: at
 # 131 072, 262 144, 524 288 and 2^20 of the Llama-3-8B graph 2.6, 3.8, 7.5, 14.9 against 5.7, 6.7, 8.5, 17.0.
 _SCORE_IMAGES_UP_TO = 196608
 _SCORE_STREAM = True  # random assignments on graphs with large blocks: matrices as a stream of pieces through LDS
@@ -232,7 +239,7 @@ class CostEngine:
 
         self._keep: Dict[str, torch.Tensor] = {}
         self._layouts: Dict[str, dict] = {"score_tiles": {}, "score_tiles_explicit": {}, "sample_steps": {},
-                                          "score_pieces": {}, "sample_tiles": {}}
+                                          "score_pieces": {}, "sample_tiles": {}, "pair_tiles": {}}
 
         # The problem is some thirty arrays, most of them a few kilobytes: they go up in
         # one copy.  An array is laid into a pinned staging buffer and gets its address
@@ -715,10 +722,10 @@ class CostEngine:
         rate of any walk over records there).  Else,
         and for graphs with small blocks: up to _SCORE_TERMS_UP_TO_IMAGES assignments with
         the terms gathered side by side from the table (apc_score_terms), from
-        there on by tiles of edges (apc_score_images, or with more random ones
-        apc_score_from_tiles: 10.4 ms for 2^20 assignments
-        of the Llama-3-8B graph, against 15.6 ms from records, 18.0 ms from the table
-        edge by edge and 31.2 ms from the three arrays).  Where the table does not
+        there on by tiles of edges (random ones apc_score_pairs: 7.2 ms for 2^20 assignments of the Llama-3-8B graph,
+        against 10.4 by apc_score_from_tiles, which takes random ones that carry sums, 15.6 ms from records, 18.0 ms from
+        the table edge by edge and 31.2 ms from the three arrays; explicit ones, and up to _SCORE_IMAGES_UP_TO that carry
+        sums, apc_score_images).  Where the table does not
         stand for the arrays, or the graph has no such tiles: from records made here if the entry
         arrays changed since: compact 16-byte
         records, several assignments per lane (apc_score_compact), while every
@@ -764,6 +771,21 @@ class CostEngine:
             self.last_score_backend = "block_table"
             return out
         from_table &= self._versioned  # else an edit would go unnoticed
+        if from_table and _SCORE_FROM_TILES and not self.large_blocks and _SCORE_PAIRS and (
+                assign is None and init is None and count > _SCORE_PAIRS_FROM[0]):
+            pairs = self._pair_tiles(first_node)
+            if pairs is not None and (count > _SCORE_PAIRS_FROM[1] or pairs[1] >= _SCORE_PAIRS_ROWS * pairs[3]):
+                steps, n_step, d_tiles, n_tile = pairs
+                scratch = self._scratch((n_tile + 1) * _lib.PAIR_IMAGE_BYTES)
+                if scratch is not None:
+                    _lib.check(
+                        self.lib.apc_score_pairs(
+                            C.byref(self.problem), self._ptr(self.per_arg), self._ptr(self.table), self._ptr(steps),
+                            n_step, self._ptr(d_tiles), n_tile, self._ptr(scratch), int(seed), int(first), int(count),
+                            self._ptr(d_gid), clamp, self._ptr(out), stream),
+                        "apc_score_pairs")
+                    self.last_score_backend = "block_table_tiles"
+                    return out
         if from_table and _SCORE_FROM_TILES and not self.large_blocks and (
                 count > _SCORE_TERMS_UP_TO_IMAGES["random" if assign is None else "explicit"]
                 or not _SCORE_SMALL_FROM_TABLE or _SCORE_TERMS_BELOW <= count):
@@ -889,6 +911,31 @@ class CostEngine:
                         torch.from_numpy(tiles[:n_tile]).to(self.device), n_tile,
                         torch.from_numpy(units[:n_unit]).to(self.device))
         return plan
+
+    def _pair_tiles(self, first_node: int):
+        """The layout apc_score_pairs walks from ``first_node`` on, on the device, or None: a graph that form does not
+        take, or no layout at hand (_layout)."""
+        return self._layout("pair_tiles", first_node, lambda: self._make_pair_tiles(first_node))
+
+    def _make_pair_tiles(self, first_node: int):
+        g = self.g
+        if self.table_mode != "full" or first_node >= g.num_nodes:
+            return None
+        edges = np.ascontiguousarray(g.edge_records(False))
+        off, nstrat = [np.ascontiguousarray(x, np.int32) for x in (g.node_edge_off, g.node_nstrat)]
+        most = g.num_nodes + g.num_edges
+        steps = np.empty((most, _lib.PAIR_STEP_BYTES), np.uint8)
+        tiles = np.empty((most, _lib.PAIR_TILE_BYTES), np.uint8)
+        n_step, n_tile = C.c_int32(0), C.c_int32(0)
+        _lib.check(
+            self.lib.apc_pair_tiles(
+                edges.ctypes.data, g.num_edges, g.num_nodes, off.ctypes.data, nstrat.ctypes.data, int(first_node),
+                steps.ctypes.data, most, tiles.ctypes.data, most, C.byref(n_step), C.byref(n_tile)),
+            "apc_pair_tiles")
+        if n_tile.value == 0:
+            return None
+        return (torch.from_numpy(steps[:n_step.value]).to(self.device), n_step.value,
+                torch.from_numpy(tiles[:n_tile.value]).to(self.device), n_tile.value)
 
     def _score_pieces(self, first_node: int):
         """(apc_score_piece records on the device, pieces, items) of apc_score_stream for the walk from

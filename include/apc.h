@@ -824,6 +824,36 @@ int apc_score_images(const apc_problem* p, const double* per_arg, const double* 
                      void* scratch, const uint16_t* assign, uint64_t seed, int64_t first, int64_t n_assign,
                      const int32_t* node_gid, int32_t clamp_inf, const double* init, double* out, void* stream);
 
+/* apc_score_random_assignments for the largest batches on a graph with small blocks, from images of finished entries:
+ * a launch in front of the walk forms every cost and communication.  apc_pair_tiles (host, no device needed) makes the
+ * layout, which depends on the graph alone and is copied to the device: a step per argument row, and for a node without
+ * one, from node first_node on, in tiles whose entries, 16 bytes each, and whose rows of choices fit a buffer.  *n_tile = 0:
+ * nothing to score, or not a graph of this form (more than 256 strategies, a compressed table, a matrix larger than a
+ * buffer): use apc_score_from_tiles.  scratch: 16-byte aligned, (n_tile + 1) * APC_PAIR_IMAGE_BYTES. */
+#define APC_PAIR_IMAGE_BYTES 55296
+#define APC_PAIR_TILE_UNITS 3328 /* of 16 bytes: an entry, or two terms of a node */
+#define APC_PAIR_TILE_ROWS 12
+typedef struct apc_pair_step {
+  int32_t node;
+  int32_t edge;  /* or -1 */
+  int32_t pairs; /* first unit of its entries in the tile */
+  int32_t terms; /* of the node's terms, at its first step; else -1 */
+  int32_t row_node, row_src; /* slots of the rows of choices; -1: no producer */
+} apc_pair_step; /* 24 bytes */
+typedef struct apc_pair_tile {
+  int32_t step0, step1;
+  int32_t n_row, n_unit;
+  int32_t row[APC_PAIR_TILE_ROWS];  /* nodes whose choices are drawn: the others' lie in their slots */
+  uint8_t slot[APC_PAIR_TILE_ROWS]; /* where to */
+  int32_t reserved;
+} apc_pair_tile; /* 80 bytes */
+int apc_pair_tiles(const apc_edge* edges, int32_t n_edge, int32_t n_node, const int32_t* node_edge_off,
+                   const int32_t* node_nstrat, int32_t first_node, apc_pair_step* steps, int64_t max_step,
+                   apc_pair_tile* tiles, int64_t max_tile, int32_t* n_step, int32_t* n_tile);
+int apc_score_pairs(const apc_problem* p, const double* per_arg, const double* table, const apc_pair_step* steps,
+                    int32_t n_step, const apc_pair_tile* tiles, int32_t n_tile, void* scratch, uint64_t seed, int64_t first,
+                    int64_t n_assign, const int32_t* node_gid, int32_t clamp_inf, double* out, void* stream);
+
 /* apc_score_random_assignments for a graph too large to keep its coefficients
  * resident: the problem holds a window of the graph's nodes (preceded by
  * first_node stand-ins for producers outside the window, which are not scored),

@@ -160,6 +160,7 @@ def test_images_have_the_bits_of_the_walk_over_records(name, count, skip, monkey
     monkeypatch.setattr(engine_mod, "_SCORE_LANES_FROM", 1)
     monkeypatch.setattr(engine_mod, "_SCORE_TERMS_BELOW", 0)
     monkeypatch.setattr(engine_mod, "_SCORE_IMAGES_UP_TO", 1 << 20)
+    monkeypatch.setattr(engine_mod, "_SCORE_PAIRS", False)
     got = scores("block_table_tiles")
     monkeypatch.setattr(engine_mod, "_SCORE_FROM_TILES", False)
     assert all(torch.equal(a, b) for a, b in zip(got, scores("compact_records")))
