@@ -162,7 +162,11 @@ schedule_metrics_kernel(apc_schedule s, const int32_t* __restrict__ order, int64
 // these workgroups, so the time of a launch is the time of one walk: instructions per step
 // times steps.  The step is therefore written without branches: a record names four storages
 // (unused places name a spare row that absorbs their updates), the counts are lowered by LDS
-// atomics that return nothing, and the timeline's cases are selects.
+// atomics that return nothing, and the timeline's cases are selects.  And as memory and timeline
+// share nothing but the order, each has wavefronts of its own.
+// Measured, MI355X, 288 nodes, 64 to 16 384 orders: 187 us in one chain, 115 with two, 97 with a step's record
+// read a step ahead, a storage's counts and bytes in one row, and streams as bits (about 85 instructions a
+// step of the timeline, 2.8 ns each at least).
 constexpr int kRecDwords = 12;  // 48 bytes a node
 constexpr int kRecUses = 4;     // storages a record names itself; further ones are read from use_st
 constexpr int kAhead = 8;       // steps between the request of an order's entry and its use
@@ -185,34 +189,35 @@ struct alignas(16) NodeRec {
   int32_t wr_row;  // row of the end times the node writes: a wait its collective's, a node on a stream of its own
                    // its own, the others a row nobody reads
   int32_t u0;      // its readers' list in use_st
-  int32_t use[kRecUses];  // the first storages of that list; the spare row n_storage in unused places
+  int32_t use[kRecUses];  // rows of the first storages of that list, bytes; the spare row n_storage in unused places
 };
+// A storage's row: the reader counts [order], then the bytes it gives back, so that one address serves both.
+constexpr int kRowBytes = kBlock * 4 + 8;
 static_assert(sizeof(NodeRec) == kRecDwords * 4, "record layout");
 
-// records, bytes a storage gives back and reader counts [storage][order], each with a spare
-// row; the end times [slot][order], if they are kept in LDS too, have two (one always empty,
+// records and a row per storage, with a spare row; the end times [slot][order], if they are kept in LDS too, have two (one always empty,
 // one nobody reads)
 __host__ __device__ inline int64_t schedule_lds_bytes(int n_node, int n_storage) {
-  return (int64_t)n_node * sizeof(NodeRec) + (int64_t)(n_storage + 1) * (8 + kBlock * 4);
+  return (int64_t)n_node * sizeof(NodeRec) + (int64_t)(n_storage + 1) * kRowBytes;
 }
 __host__ __device__ inline int64_t schedule_end_lds_bytes(int n_comm) { return (int64_t)(n_comm + 2) * kBlock * 8; }
 
 // A workgroup walks 64 orders whatever its shape: kWaves wavefronts with 64 / kWaves working
-// lanes each, so that the 64 walks are spread over the CU's SIMDs when the LDS a workgroup
-// needs leaves room for only one or two of them per CU.
+// lanes each for the memory and as many for the timeline, so that the 64 walks are spread over the
+// CU's SIMDs when the LDS a workgroup needs leaves room for only one or two of them per CU.
+// kStreams: streams the timeline tells apart, at least n_stream (one or two selects each a step).
 // kEndLds: the end times are rows [slot][order] of LDS, slot = comm_slot of the node; otherwise
 // rows [node][order] of end_scratch (row -1: none).
-template <bool kIdentity, int kWaves, bool kEndLds>
-__global__ void __launch_bounds__(kBlock * kWaves)
+template <bool kIdentity, int kWaves, bool kEndLds, int kStreams>
+__global__ void __launch_bounds__(kBlock * kWaves * 2)
 schedule_metrics_lds_kernel(apc_schedule s, const int32_t* __restrict__ order, int64_t n_sched,
                             double* __restrict__ end_scratch, double* __restrict__ times,
                             int64_t* __restrict__ peak_out) {
-  constexpr int kThreads = kBlock * kWaves, kWork = kBlock / kWaves;
+  constexpr int kThreads = kBlock * kWaves * 2, kWork = kBlock / kWaves;
   extern __shared__ __align__(16) unsigned char s_raw[];
   const int N = s.n_node, S = s.n_storage;
   NodeRec* const recs = reinterpret_cast<NodeRec*>(s_raw);
-  int64_t* const freed = reinterpret_cast<int64_t*>(s_raw + (size_t)N * sizeof(NodeRec));  // bytes a storage gives back
-  int32_t* const remaining = reinterpret_cast<int32_t*>(freed + (S + 1));
+  unsigned char* const rows = s_raw + (size_t)N * sizeof(NodeRec);
   double* const end_lds = reinterpret_cast<double*>(s_raw + schedule_lds_bytes(N, S));
   const int row_empty = s.n_comm, row_unread = s.n_comm + 1;  // kEndLds
   const int thread = threadIdx.x;
@@ -241,83 +246,119 @@ schedule_metrics_lds_kernel(apc_schedule s, const int32_t* __restrict__ order, i
     if (mem)
       for (int q = s.alloc_off[v]; q < s.alloc_off[v + 1]; ++q) r.alloc += s.st_bytes[s.alloc_st[q]];
 #pragma unroll
-    for (int i = 0; i < kRecUses; ++i) r.use[i] = i < n_use ? s.use_st[r.u0 + i] : S;
+    for (int i = 0; i < kRecUses; ++i) r.use[i] = (i < n_use ? s.use_st[r.u0 + i] : S) * kRowBytes;
     recs[v] = r;
   }
-  for (int k = thread; k <= S; k += kThreads) freed[k] = (k < S && s.st_freeable[k]) ? s.st_bytes[k] : 0;
-  for (int i = thread; i < (S + 1) * kBlock; i += kThreads) remaining[i] = i < S * kBlock ? s.st_users[i / kBlock] : 0;
+  for (int k = thread; k <= S; k += kThreads)
+    *reinterpret_cast<int64_t*>(rows + k * kRowBytes + kBlock * 4) = (k < S && s.st_freeable[k]) ? s.st_bytes[k] : 0;
+  for (int i = thread; i < (S + 1) * kBlock; i += kThreads)
+    reinterpret_cast<int32_t*>(rows + i / kBlock * kRowBytes)[i % kBlock] = i < S * kBlock ? s.st_users[i / kBlock] : 0;
   if (kEndLds)  // absent from global_time: a negative end time (times are never negative)
     for (int i = thread; i < (s.n_comm + 2) * kBlock; i += kThreads) end_lds[i] = -1.0;
   __syncthreads();
 
   // order `lane` of the workgroup's 64: the first kWork lanes of every wavefront work
-  const int lane = (thread >> 6) * kWork + (thread & 63);
+  const int wave = __builtin_amdgcn_readfirstlane(thread >> 6);
+  const bool for_memory = wave < kWaves;
+  const int lane = (wave & (kWaves - 1)) * kWork + (thread & 63);
   const int64_t b = (int64_t)blockIdx.x * kBlock + lane;
   if ((thread & 63) >= kWork || b >= n_sched) return;  // no barrier follows
   double* const end_time = kEndLds ? end_lds + lane : end_scratch + b;  // this order's column
   const int64_t end_stride = kEndLds ? kBlock : n_sched;
-  if (!kEndLds)
-    for (int i = 0; i < N; ++i) end_time[i * end_stride] = -1.0;
-  int32_t* const my_remaining = remaining + lane;
-
-  double cur[APC_SCHED_MAX_STREAMS];
-  bool seen[APC_SCHED_MAX_STREAMS];
-#pragma unroll
-  for (int t = 0; t < APC_SCHED_MAX_STREAMS; ++t) { cur[t] = 0.0; seen[t] = (t == 0); }
-  double compute_time = 0.0, comm_time = 0.0, exposed = 0.0;
-  int64_t live = s.initial_bytes, peak = s.initial_bytes;
   const int32_t* ord = kIdentity ? nullptr : order + b * N;
 
-  auto step = [&](int v) {
-    const NodeRec r = recs[v];
-    const int tid = r.bits & 0xFF;
-    const int n_use = (int)((uint32_t)r.bits >> 16);
-    const bool is_wait = r.bits & kRecWait, is_comm = r.bits & kRecComm, is_compute = r.bits & kRecCompute;
-    const bool is_sync = r.bits & kRecSync, mem = r.bits & kRecMem;
-    const double dur = r.dur;
-    // ---- memory (MemoryTracker.schedule_node): this reader is now scheduled
+  // The order's entries are requested kAhead steps before their use, every time the same
+  // number of loads (past the end the last entry again), so that the wait before a block of
+  // steps is for the loads of the block before and not for the ones just issued.
+  auto entry = [&](int t) -> int {
+    const int tc = t < N ? t : N - 1;
+    return (kIdentity || N == 0) ? tc : ord[tc];  // (an empty graph has no entries to read)
+  };
+  // A step's record is read a step ahead, in front of the accesses that the step has to wait for.
+  auto walk = [&](auto step) {
+    if (N == 0) return;
+    int nxt[kAhead];
 #pragma unroll
-    for (int i = 0; i < kRecUses; ++i)
-      __hip_atomic_fetch_sub(my_remaining + r.use[i] * kBlock, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    if (n_use > kRecUses)
-      for (int q = r.u0 + kRecUses; q < r.u0 + n_use; ++q) my_remaining[s.use_st[q] * kBlock] -= 1;
-    live += r.alloc;
-    peak = live > peak ? live : peak;
+    for (int i = 0; i < kAhead; ++i) nxt[i] = entry(i);
+    NodeRec rec = recs[nxt[0]];
+    for (int t0 = 0; t0 < N; t0 += kAhead) {
+      int now[kAhead];
 #pragma unroll
-    for (int i = 0; i < kRecUses; ++i) {
-      const int left = my_remaining[r.use[i] * kBlock];
-      const int64_t bytes = freed[r.use[i]];
-      live -= (mem && left == 0) ? bytes : 0;
-    }
-    if (n_use > kRecUses && mem)
-      for (int q = r.u0 + kRecUses; q < r.u0 + n_use; ++q) {
-        const int k = s.use_st[q];
-        if (my_remaining[k * kBlock] == 0) live -= freed[k];
+      for (int i = 0; i < kAhead; ++i) {
+        now[i] = nxt[i];
+        nxt[i] = entry(t0 + kAhead + i);
       }
+#pragma unroll
+      for (int i = 0; i < kAhead; ++i) {
+        const NodeRec after = recs[i + 1 < kAhead ? now[i + 1] : nxt[0]];
+        if (t0 + i < N) step(rec);
+        rec = after;
+      }
+    }
+  };
+
+  if (for_memory) {  // MemoryTracker.schedule_node: this reader is now scheduled
+    int64_t live = s.initial_bytes, peak = s.initial_bytes;
+    auto left = [&](int row) -> int32_t* { return reinterpret_cast<int32_t*>(rows + row) + lane; };
+    auto freed = [&](int row) -> int64_t { return *reinterpret_cast<const int64_t*>(rows + row + kBlock * 4); };
+    walk([&](const NodeRec& r) {
+      const int n_use = (int)((uint32_t)r.bits >> 16);
+      const bool mem = r.bits & kRecMem;
+#pragma unroll
+      for (int i = 0; i < kRecUses; ++i)
+        __hip_atomic_fetch_sub(left(r.use[i]), 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      if (n_use > kRecUses)
+        for (int q = r.u0 + kRecUses; q < r.u0 + n_use; ++q) *left(s.use_st[q] * kRowBytes) -= 1;
+      live += r.alloc;
+      peak = live > peak ? live : peak;
+#pragma unroll
+      for (int i = 0; i < kRecUses; ++i) {
+        const int n_left = *left(r.use[i]);  // read in any case: a condition would be a branch
+        const int64_t bytes = freed(r.use[i]);
+        live -= mem & (n_left == 0) ? bytes : 0;
+      }
+      if (n_use > kRecUses && mem)
+        for (int q = r.u0 + kRecUses; q < r.u0 + n_use; ++q)
+          if (*left(s.use_st[q] * kRowBytes) == 0) live -= freed(s.use_st[q] * kRowBytes);
+    });
+    peak_out[b] = peak;
+    return;
+  }
+
+  if (!kEndLds)
+    for (int i = 0; i < N; ++i) end_time[i * end_stride] = -1.0;
+  double cur[kStreams];
+  uint32_t seen = 1;  // a bit per stream
+#pragma unroll
+  for (int t = 0; t < kStreams; ++t) cur[t] = 0.0;
+  double compute_time = 0.0, comm_time = 0.0, exposed = 0.0;
+  walk([&](const NodeRec& r) {
+    const int tid = r.bits & 0xFF;
+    const bool is_wait = r.bits & kRecWait, is_comm = r.bits & kRecComm, is_compute = r.bits & kRecCompute;
+    const bool is_sync = r.bits & kRecSync;
+    const double dur = r.dur;
     // ---- timeline; cur[tid] with tid a lane-varying index: select, not index
     double c0 = cur[0], ct = c0;
-    bool known = false;
 #pragma unroll
-    for (int k = 0; k < APC_SCHED_MAX_STREAMS; ++k)
-      if (k == tid) { ct = cur[k]; known = seen[k]; }
-    if (!known) ct = c0;  // a stream starts at the compute stream's present time
+    for (int k = 1; k < kStreams; ++k) ct = k == tid ? cur[k] : ct;
+    ct = seen >> tid & 1 ? ct : c0;  // a stream starts at the compute stream's present time
     if (kEndLds) {
       // every node reads a row and writes a row: a wait its collective's (the pop of
-      // global_time), a node on a stream of its own its own, the others the spare ones
+      // global_time), a node on a stream of its own its own, the others the spare ones; only a
+      // wait reads a row that can hold a time, and for it ct is c0
       const double e = end_time[r.rd_row * kBlock];
-      const bool got = e >= 0.0;  // only a wait reads a row that can hold a time
-      const double end = got ? e : c0;
-      const double stall_w = end - c0;
-      exposed += (got && stall_w > 0.0) ? stall_w : 0.0;
-      ct = is_wait ? pymax(ct, end) : (is_comm ? pymax(c0, ct) : ct);
+      const bool stalls = (e >= 0.0) & (e > c0);
+      exposed += stalls ? e - c0 : 0.0;
+      ct = is_comm & !(ct > c0) ? c0 : ct;
+      ct = stalls ? e : ct;
       comm_time += is_comm ? dur : 0.0;
       compute_time += is_compute ? dur : 0.0;
       ct += dur + 1.0;
       end_time[r.wr_row * kBlock] = is_wait ? -1.0 : ct;
       const double c0n = c0 + 1.0;
-      const double stall_s = ct - c0n;
-      exposed += (is_sync && stall_s > 0.0) ? stall_s : 0.0;
-      c0 = tid == 0 ? ct : (is_sync ? pymax(c0n, ct) : c0n);
+      const bool waits = is_sync & (ct > c0n);
+      exposed += waits ? ct - c0n : 0.0;
+      c0 = (tid == 0) | waits ? ct : c0n;
     } else {
       if (is_wait) {
         double end = c0;
@@ -352,40 +393,17 @@ schedule_metrics_lds_kernel(apc_schedule s, const int32_t* __restrict__ order, i
     }
     cur[0] = c0;
 #pragma unroll
-    for (int k = 1; k < APC_SCHED_MAX_STREAMS; ++k)
-      if (k == tid) { cur[k] = ct; seen[k] = true; }
-  };
-
-  // The order's entries are requested kAhead steps before their use, every time the same
-  // number of loads (past the end the last entry again), so that the wait before a block of
-  // steps is for the loads of the block before and not for the ones just issued.
-  auto entry = [&](int t) -> int {
-    const int tc = t < N ? t : N - 1;
-    return (kIdentity || N == 0) ? tc : ord[tc];  // (an empty graph has no entries to read)
-  };
-  int nxt[kAhead];
-#pragma unroll
-  for (int i = 0; i < kAhead; ++i) nxt[i] = entry(i);
-  for (int t0 = 0; t0 < N; t0 += kAhead) {
-    int now[kAhead];
-#pragma unroll
-    for (int i = 0; i < kAhead; ++i) {
-      now[i] = nxt[i];
-      nxt[i] = entry(t0 + kAhead + i);
-    }
-#pragma unroll
-    for (int i = 0; i < kAhead; ++i)
-      if (t0 + i < N) step(now[i]);
-  }
+    for (int k = 1; k < kStreams; ++k) cur[k] = k == tid ? ct : cur[k];
+    seen |= 1u << tid;
+  });
   double total = cur[0];
 #pragma unroll
-  for (int k = 1; k < APC_SCHED_MAX_STREAMS; ++k)
-    if (seen[k]) total = pymax(total, cur[k]);
+  for (int k = 1; k < kStreams; ++k)
+    if (seen >> k & 1) total = pymax(total, cur[k]);
   times[b * 4 + 0] = total;
   times[b * 4 + 1] = compute_time;
   times[b * 4 + 2] = comm_time;
   times[b * 4 + 3] = exposed;
-  peak_out[b] = peak;
 }
 
 // Whether every order names each of the n_node nodes once: a wavefront per order marks what it
@@ -477,20 +495,21 @@ extern "C" int apc_schedule_metrics(const apc_schedule* s, const int32_t* order,
     const int64_t share = (grid + 255) / 256;
     if (share < resident) resident = share;
     const int waves = resident >= 4 ? 1 : (resident >= 2 ? 2 : 4);
-#define APC_SCHED_LAUNCH_(IDENT, WAVES, END)                                                                        \
+#define APC_SCHED_LAUNCH_(IDENT, WAVES, END, STREAMS)                                                                \
   do {                                                                                                          \
     if (lds > 64 * 1024) { /* above the default limit of a launch: ask for it (cheap, so asked every time) */   \
-      hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(schedule_metrics_lds_kernel<IDENT, WAVES, END>), \
+      hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(schedule_metrics_lds_kernel<IDENT, WAVES, END, STREAMS>), \
                                          hipFuncAttributeMaxDynamicSharedMemorySize, kLdsLimit);                \
       if (e != hipSuccess) return fail("apc_schedule_metrics: hipFuncSetAttribute failed");                     \
     }                                                                                                           \
-    hipLaunchKernelGGL((schedule_metrics_lds_kernel<IDENT, WAVES, END>), dim3((unsigned)grid), dim3(kBlock * WAVES), \
+    hipLaunchKernelGGL((schedule_metrics_lds_kernel<IDENT, WAVES, END, STREAMS>), dim3((unsigned)grid), dim3(kBlock * WAVES * 2), \
                        (size_t)lds, (hipStream_t)stream, *s, order, n_sched, end_scratch, times, peak);         \
   } while (0)
 #define APC_SCHED_LAUNCH(IDENT, WAVES)                         \
   do {                                                         \
-    if (end_lds) APC_SCHED_LAUNCH_(IDENT, WAVES, true);        \
-    else APC_SCHED_LAUNCH_(IDENT, WAVES, false);               \
+    if (end_lds && s->n_stream <= 4) APC_SCHED_LAUNCH_(IDENT, WAVES, true, 4); \
+    else if (end_lds) APC_SCHED_LAUNCH_(IDENT, WAVES, true, APC_SCHED_MAX_STREAMS); \
+    else APC_SCHED_LAUNCH_(IDENT, WAVES, false, APC_SCHED_MAX_STREAMS);        \
   } while (0)
     if (!order) APC_SCHED_LAUNCH(true, 4);
     else if (waves == 1) APC_SCHED_LAUNCH(false, 1);
