@@ -18,7 +18,7 @@ SAMPLE_REC_BYTES = 64
 CHECK_MAX_NODES = 131072
 SCORE_STEP_BYTES, SCORE_TILE_BYTES, SCORE_UNIT_BYTES = 64, 128, 16
 SCORE_IMAGE_BYTES = 43008
-PAIR_STEP_BYTES, PAIR_TILE_BYTES, PAIR_IMAGE_BYTES = 24, 80, 55296
+PAIR_STEP_BYTES, PAIR_TILE_BYTES, PAIR_IMAGE_BYTES, PAIR_TILE_UNITS = 24, 80, 55296, 3328
 FOLD_EDGE_BYTES, FOLD_NODE_BYTES = 48, 16
 SAMPLE_TILE_BYTES, SAMPLE_IMAGE_BYTES = 160, 19456
 SCORE_PIECE, SCORE_SIDE_BYTES = 8192, 8192

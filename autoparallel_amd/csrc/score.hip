@@ -357,6 +357,9 @@ score_compact_kernel(apc_problem p, const double* __restrict__ per_arg,
 // loads of the next edge's matrix are issued before the draws of the current
 // one.  Matrices larger than a buffer are taken in several tiles; very large
 // ones and the default rows of edges without a producer are read in place.
+// Random assignments are faster as a stream of pieces (score_stream.hip, 7.3 -> 5.9 ms for
+// 524 288 of a window of the planner DAG); this walk is for explicit ones, and for graphs or memory that
+// do not allow the stream.
 // The sums of an assignment run in node order, then argument order, as in
 // score_kernel: same results, bit for bit, as scoring the entry arrays that a
 // build with the same clamp_inf wrote.
@@ -665,7 +668,8 @@ constexpr int kFoldLds = 2 * kTermTile * 3 * 8;      // two tiles of three terms
 // read from the three arrays.  The arrays of a graph with large blocks are read at random from
 // memory, two 64-byte lines and a third for a flag byte per pair; the matrices, an eighth of their
 // size, stay in L2 while the workgroups walk the graph side by side: 16 384 given assignments of
-// that window 1 580 -> 820 us, 32 000 random ones of the Llama-3-8B graph 1 970 -> 1 190.
+// that window 1 580 -> 820 us, 32 000 random ones of the Llama-3-8B graph 1 970 -> 1 190.  With scratch memory for
+// records of the edges score_fold.hip does this in 570 and 650.
 // kShift: log2 of the assignments of a workgroup, 6 at most; at 6 a wavefront's lanes share
 // their edge and read its record through the scalar cache.
 template <bool kRandom, int kShift, bool kTable>

@@ -290,7 +290,6 @@ score_images_walk_kernel(const char* __restrict__ images, int n_tile, const uint
 #pragma unroll
       for (int g = 0; g < kN; g += kUnroll) {
         // what the build makes of a matrix element, added up
-        double comm[kUnroll];
         bool adds[kUnroll];
 #pragma unroll
         for (int u = g; u < g + kUnroll; ++u) {

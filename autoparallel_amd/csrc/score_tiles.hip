@@ -15,8 +15,9 @@
 // the edges find their producer's; explicit choices are read a tile ahead into the same place.
 // Below, it is the chain of LDS reads of a step and the few wavefronts a CU has to hide it.
 // Measured, from records and by tiles: 2^20 random assignments of that graph 15.4 -> 10.4 ms, of the 16-layer
-// mixture-of-experts graph 8.4 -> 5.7 (explicit ones, and few random ones, are faster from tile images,
-// score_images.hip; explicit ones are walked here where there is no room for the images).  Not better: step records in LDS instead of scalar loads
+// mixture-of-experts graph 8.4 -> 5.7 (random ones that carry no sums are faster from images of
+// finished entries, score_pairs.hip, 7.3 ms for the first figure; explicit ones, and few random ones, from tile images,
+// score_images.hip; they are walked here where there is no room for the images).  Not better: step records in LDS instead of scalar loads
 // (11.8 for the first figure; eight readfirstlane a step).
 // Sums run in node order, then argument order, as in score_kernel: the same bits.
 #include <algorithm>

@@ -31,11 +31,11 @@ _SCORE_TERMS_BELOW = 114688
 # 2.49, 2.90 and 2.80, 2.91, explicit, at 81 920 and 90 112 2.48, 2.70 and 3.16, 2.70; 12-layer GPT-2 graph 0.77, 0.81 and
 # 0.86, 0.81, and 0.64, 0.72 and 0.81, 0.72.
 _SCORE_TERMS_UP_TO_IMAGES = {"random": 114688, "explicit": 81920}
-# Random assignments that carry no sums: from images of finished entries beyond these many, the second where a tile of
-# theirs has few argument rows, for which its beginning counts.  In ms, finished entries, tile images (from 262 144 on lanes of
-# several), terms: 12-layer GPT-2 graph (10 rows a tile), 90 112 0.62, 0.81, 0.66, 131 072 0.64, 0.81, 0.87, 262 144 0.98,
-# 1.22, 2^20 2.24, 3.42; Llama-3-8B graph (4.2), 131 072 2.98, 2.91, 2.80, 163 840 3.31, 3.65, 3.45, 262 144 3.68, 4.68,
-# 2^20 7.24, 10.41; MoE graph (4.9), 131 072 1.59, 1.57, 1.53.
+# Random assignments that carry no sums: from images of finished entries beyond these many, the second where a tile has
+# room for few argument rows of the graph's mean size, so that its beginning counts.  In ms, finished entries, tile images (from 262 144 on lanes of
+# several), terms: 12-layer GPT-2 graph (173 rows), 90 112 0.62, 0.81, 0.66, 131 072 0.64, 0.81, 0.87, 262 144 0.98,
+# 1.22, 2^20 2.24, 3.42; Llama-3-8B graph (5.1), 131 072 2.98, 2.91, 2.80, 163 840 3.31, 3.65, 3.45, 262 144 3.68, 4.68,
+# 2^20 7.24, 10.41; MoE graph (6.0), 131 072 1.59, 1.57, 1.53.
 _SCORE_PAIRS = True
 _SCORE_PAIRS_FROM, _SCORE_PAIRS_ROWS = (81920, 131072), 8
 # Else, random assignments up to which tile images are walked with a lane each; beyond, lanes take two or four, which
@@ -732,6 +732,7 @@ class CostEngine:
         cost is (comm + per_arg) + transition or its clamp (checked on the device
         when the records are made); else the 32-byte records that carry the cost
         (apc_score_packed)."""
+        g = self.g
         stream = self._stream()
         capturing = self._capturing(stream)
         clamp = self._standing_clamp() if _SCORE_FROM_TABLE else None
@@ -772,9 +773,10 @@ class CostEngine:
             return out
         from_table &= self._versioned  # else an edit would go unnoticed
         if from_table and _SCORE_FROM_TILES and not self.large_blocks and _SCORE_PAIRS and (
-                assign is None and init is None and count > _SCORE_PAIRS_FROM[0]):
+                assign is None and init is None and count > _SCORE_PAIRS_FROM[
+                    0 if g.num_entries * _SCORE_PAIRS_ROWS <= g.num_edges * _lib.PAIR_TILE_UNITS else 1]):
             pairs = self._pair_tiles(first_node)
-            if pairs is not None and (count > _SCORE_PAIRS_FROM[1] or pairs[1] >= _SCORE_PAIRS_ROWS * pairs[3]):
+            if pairs is not None:
                 steps, n_step, d_tiles, n_tile = pairs
                 scratch = self._scratch((n_tile + 1) * _lib.PAIR_IMAGE_BYTES)
                 if scratch is not None:
@@ -1183,7 +1185,8 @@ class CostEngine:
                         row_filter: Optional[dict] = None):
         """``count`` assignments drawn node by node among the strategies that select
         no forbidden (non-finite) entry against the choices made for the node's
-        producers (apc_pack_allowed_columns, then apc_sample_feasible).  Returns
+        producers (apc_pack_allowed_columns, then apc_sample_feasible_tiles, apc_sample_steps or
+        apc_sample_feasible, by strategies, batch and layout).  Returns
         (assign uint16[n_node, count] on the device, n_fallback int32[count]: nodes
         that had no such strategy and took the plain draw).  ``assign``/``first_node``:
         rows below first_node are given (a window of a larger graph); ``node_gid``:
