@@ -27,9 +27,10 @@ struct FoldEdge {
   uint32_t row;             // length of a matrix row
   uint32_t terms;           // the node's per-argument terms
   uint32_t node, src;       // what the draws start from, or the rows of explicit choices
-  uint32_t sizes;           // strategies of the node (bits 0-15) and the producer
+  uint32_t sdst;            // strategies of the node
   int32_t mult;
-  uint32_t dst_list, src_list, flags, reserved;
+  uint32_t dst_list, src_list, flags;
+  uint32_t ssrc;            // and of the producer, 32 bits each: a node's number of them has no other bound
 };
 struct FoldNode { uint32_t terms, node, nstrat; int32_t nargs; };
 constexpr uint32_t kSource = 1, kTransition = 2, kSqueezed = 4;
@@ -54,13 +55,13 @@ fold_records_kernel(apc_problem p, const double* __restrict__ table, const int32
     r.terms = (uint32_t)ed.comp_base;
     r.node = key(ed.node);
     r.src = has_src ? key(ed.src_node) : 0u;
-    r.sizes = (uint32_t)ed.sdst | (uint32_t)ed.ssrc << 16;
+    r.sdst = (uint32_t)ed.sdst;
     r.mult = p.node_multiplier[ed.node];
     r.dst_list = squeezed ? ed.dst_list : 0u;
     r.src_list = squeezed ? ed.src_list : 0u;
     r.flags = (has_src ? kSource : 0u) | (has_src && (ed.flags & APC_EDGE_SCORE_TRANSITION) ? kTransition : 0u) |
               (squeezed ? kSqueezed : 0u);
-    r.reserved = 0;
+    r.ssrc = (uint32_t)ed.ssrc;
     edges[i] = r;
   }
   if (first_node + i < p.n_node) {
@@ -128,8 +129,8 @@ score_terms_kernel(const FoldEdge* __restrict__ edges, int n_edges, const FoldNo
     auto choose = [&](const Rec& r) -> Choices {
       Choices c;
       if (kRandom) {
-        c.o = draw(r.e[1][0], r.e[1][2] & 0xFFFFu);
-        c.j = draw(r.e[1][1], r.e[1][2] >> 16);
+        c.o = draw(r.e[1][0], r.e[1][2]);
+        c.j = draw(r.e[1][1], r.e[2][3]);
         c.v = draw(r.n[1], r.n[2]);
       } else {
         c.o = my_assign[(size_t)r.e[1][0] * stride];

@@ -7,6 +7,8 @@ import torch
 from autoparallel_amd import engine as engine_mod
 from autoparallel_amd import graphgen
 from autoparallel_amd.engine import CostEngine
+from autoparallel_amd.packed import DT_F32, GraphBuilder, NodeDesc
+from oracle import cost_oracle as O
 
 pytestmark = pytest.mark.gpu
 
@@ -64,3 +66,48 @@ def test_the_table_stands_for_the_arrays_only_while_it_does(engines):
         array.mul_(2.0)
         assert not (got == _bits(eng.score_random(3, 0, 70))).all()
     eng.build()
+
+
+def _graph_of_wide_nodes():
+    """A chain of nodes with more strategies than 16 bits count, between ones with few: as consumers and as producers."""
+    b = GraphBuilder((2, 2), 8)
+    rng = np.random.default_rng(7)
+    codes = [0x00, 0x40, 0x41, 0x80]
+    metas = [b.meta((64 << v, 96), (96, 1), 4, DT_F32) for v in range(7)]
+
+    def specs(m, n):
+        return [b.spec(m, (codes[x], codes[y])) for x, y in rng.integers(0, 4, (n, 2))]
+
+    for v, n in enumerate((3, 70000, 2, 65536, 3, 65535, 65537 * 2)):
+        out = [[s] for s in specs(metas[v], n)]
+        if v in (0, 5):
+            b.add_node(NodeDesc(f"in{v}", in_specs=out, out_specs=out, inputs=[], default_rows=[[[0.0]] for _ in out]))
+        else:
+            u = 4 if v == 6 else v - 1
+            b.add_node(NodeDesc(f"v{v}", in_specs=[[s] for s in specs(metas[u], n)], out_specs=out, inputs=[u]))
+    return b.pack()
+
+
+@pytest.mark.parametrize("table_mode", ["full", "compressed"])
+def test_draws_among_more_strategies_than_16_bits_count(table_mode, monkeypatch):
+    """Both counts of an edge are drawn with in full: a walk that keeps them in 16 bits draws among 4 464 of 70 000
+    and among one of 65 536."""
+    g = _graph_of_wide_nodes()
+    eng = CostEngine(g, table_mode=table_mode).build()
+    ids = np.arange(g.num_nodes, dtype=np.int32)
+    ref = O.GraphOracle(g).build()
+    for count in (70, 600, 5000, 40000):
+        init = torch.arange(count * 6, dtype=torch.float64, device="cuda").reshape(count, 6)
+        got = []
+        for from_table in (True, False):
+            monkeypatch.setattr(engine_mod, "_SCORE_FROM_TABLE", from_table)
+            monkeypatch.setattr(engine_mod, "_SCORE_SMALL_FROM_TABLE", from_table)
+            got.append([_bits(eng.score_random(11, 5, count)), _bits(eng.score_random_window(11, 5, count, ids, 1, init=init))])
+            assert (eng.last_score_backend == "block_table_terms") == from_table
+        assert all((a == b).all() for a, b in zip(*got))
+        scores = got[0][0].view(np.float64)
+        for a in (0, 1, count - 1):
+            chosen = eng.random_assignment(11, 5 + a)
+            want = O.score_assignment(g, ref["comm"], ref["transition"], ref["compute"], chosen)
+            assert tuple(scores[a, :4]) == tuple(float(x) for x in want)
+    assert max(int(eng.random_assignment(11, a).max()) for a in (5, 6)) > 65535
