@@ -21,6 +21,7 @@ SCORE_IMAGE_BYTES = 43008
 PAIR_STEP_BYTES, PAIR_TILE_BYTES, PAIR_IMAGE_BYTES, PAIR_TILE_UNITS = 24, 80, 55296, 3328
 FOLD_EDGE_BYTES, FOLD_NODE_BYTES = 48, 16
 SAMPLE_TILE_BYTES, SAMPLE_IMAGE_BYTES = 160, 19456
+SAMPLE_TILE_DEPTH = 30  # the word that holds it in the first tile
 SCORE_PIECE, SCORE_SIDE_BYTES = 8192, 8192
 SCORE_PIECE_BYTES, SCORE_PIECE_SCRATCH = 32, 96  # a record, and what a call needs beside it
 

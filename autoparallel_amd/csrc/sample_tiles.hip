@@ -325,7 +325,8 @@ int apc_sample_tiles(int32_t n_node, int32_t n_edge, const int32_t* node_edge_of
   try {
     int t = -1;
     std::unordered_map<int32_t, int> far;
-    std::vector<int32_t> fresh;
+    std::vector<int32_t> fresh, level((size_t)(n_node - first_node));  // nodes of the longest chain that ends in it
+    int32_t depth = 0;
     for (int v = first_node; v < n_node; ++v) {
       const int e0 = node_edge_off[v], e1 = node_edge_off[v + 1];
       if (e0 < 0 || e0 > e1 || e1 > n_edge) return fail(APC_ERR_INVALID, "apc_sample_tiles: node_edge_off is no list of offsets%s");
@@ -335,6 +336,7 @@ int apc_sample_tiles(int32_t n_node, int32_t n_edge, const int32_t* node_edge_of
       for (int e = e0; e < e1; ++e) {
         const int u = edge_src[e];
         if (u >= v || (u >= 0 && (edge_ssrc[e] < 1 || edge_ssrc[e] > kMaxStrategies))) return 0;
+        if (u >= first_node) level[seq] = std::max(level[seq], level[u - first_node]);
         if (u >= 0 && (u < first_node || seq - (u - first_node) >= kRing) && !far.count(u) &&
             std::find(fresh.begin(), fresh.end(), u) == fresh.end())
           fresh.push_back(u);
@@ -367,7 +369,9 @@ int apc_sample_tiles(int32_t n_node, int32_t n_edge, const int32_t* node_edge_of
       }
       ++tile.n_node;
       tile.n_edge += e1 - e0;
+      depth = std::max(depth, ++level[seq]);
     }
+    if (t >= 0) tiles[0].depth = depth;
     *n_tile = t + 1;
   } catch (const std::exception&) {
     return fail(APC_ERR_INVALID, "apc_sample_tiles: out of host memory%s");

@@ -67,10 +67,18 @@ _SCORE_PER_LANE = 0  # assignments per lane of the compact scorer; 0: the librar
 # window of the planner DAG of 1 600 nodes 5.49, 6.33 and 6.34, 6.30, of 60 nodes 0.242, 0.260 and 0.270, 0.262.
 _SAMPLE_LANES_FROM = {2: 458752, 16: 229376}
 _SAMPLE_WAVES = 0  # 2 or 16: tests
-# Graphs of at most 64 strategies a node: by tiles of nodes through LDS, whatever the batch.  In ms, tiles, and wavefronts
+# Graphs of at most 64 strategies a node: by tiles of nodes through LDS.  In ms, tiles, and wavefronts
 # or lanes: Llama-3-8B graph, 100, 131 072 and 524 288 assignments 2.0, 2.4, 7.2 and 3.0, 5.1, 21.2; 12-layer GPT-2 graph,
 # 100 and 131 072 0.66, 0.86 and 0.91, 1.56.
 _SAMPLE_TILES = True
+# But not small batches on graphs with work for sixteen wavefronts: tiles go node by node, wavefronts by the depth of
+# the graph.  What each takes, us: tiles, in all, per node and per tile; a step, in all and per argument row of the mean
+# node, for every 16 384 assignments (a workgroup of 64 on each CU).  In us, tiles and wavefronts at 16 384, 32 768, 49 152
+# and 65 536: random DAG of 800 nodes (1.4 rows a node, 52 steps) 298, 312, 302, 306 and 102, 177, 254, 328, of 60 nodes
+# 55, 56, 56, 56 and 35, 45, 55, 65, of 4 000 1 394, 1 456, 1 402, 1 408 and 409, 779, 1 152, 1 527; 800 nodes of six rows
+# 802, 792, 780, 782 and 247, 466, 685, 906, and of one, producers up to 20 back (81 steps), 264, 277, 268, 270 and 126, 222,
+# 325, 407.  The rule takes the shorter one at each of these.
+_SAMPLE_TILES_US, _SAMPLE_STEP_US = (24.0, 0.16, 3.0), (1.0, 0.3)
 # Layouts of a kind (by first_node) an engine makes.  They stay until the engine goes, since a launch on
 # another stream or in a graph may still read one; calls beyond take the route that needs none.
 _LAYOUTS_KEPT = 16
@@ -416,6 +424,7 @@ class CostEngine:
         self._built_marks = self._array_marks()
         self._recs_marks: tuple = ()
         self.last_score_backend = "entry_arrays"  # what the last batch was scored from
+        self.last_sample_backend = ""  # how the last feasible draws were made: by "tiles", "steps" or "lanes"
 
     def synchronize(self) -> None:
         torch.cuda.synchronize(self.device)
@@ -1125,7 +1134,7 @@ class CostEngine:
         return colbits, d_off, max_words
 
     def _sample_tiles(self, first_node: int):
-        """(apc_sample_tile records, argument rows' places, both on the device, tiles, wide) of
+        """(apc_sample_tile records, argument rows' places, both on the device, tiles, wide, depth of the graph) of
         apc_sample_feasible_tiles for the walk from ``first_node`` on, or None: a graph such a walk does not take, or no
         layout at hand (_layout)."""
         return self._layout("sample_tiles", first_node, lambda: self._make_sample_tiles(first_node))
@@ -1146,7 +1155,18 @@ class CostEngine:
         if n_tile.value == 0:
             return None
         return (torch.from_numpy(tiles[:n_tile.value]).to(self.device), torch.from_numpy(rows).to(self.device),
-                n_tile.value, int(nstrat[first_node:].max() > 32))
+                n_tile.value, int(nstrat[first_node:].max() > 32), int(tiles[0].view(np.int32)[_lib.SAMPLE_TILE_DEPTH]))
+
+    def _steps_before_tiles(self, first_node: int, count: int, tiles):
+        """_sample_steps where sixteen wavefronts in steps are faster than ``tiles``, else None."""
+        n, n_edge = self.g.num_nodes - first_node, self.g.num_edges - int(self.g.node_edge_off[first_node])
+        n_tile, depth = tiles[2], tiles[4]
+        by_tiles = _SAMPLE_TILES_US[0] + _SAMPLE_TILES_US[1] * n + _SAMPLE_TILES_US[2] * n_tile
+        step = -(-count // 16384) * (_SAMPLE_STEP_US[0] + _SAMPLE_STEP_US[1] * n_edge / n)
+        if n < 6 * depth or max(depth, n / 16) * step >= by_tiles:  # two wavefronts, or too many steps in any layout
+            return None
+        steps = self._sample_steps(first_node)
+        return steps if steps is not None and steps[2] == 16 and steps[1] * step < by_tiles else None
 
     def _sample_steps(self, first_node: int):
         """(records on the device, steps, wavefronts) of apc_sample_feasible_steps for the walk
@@ -1229,17 +1249,23 @@ class CostEngine:
             d_keep = torch.from_numpy(np.concatenate(words).view(np.int64)).to(self.device)
             d_keep_off = torch.from_numpy(keep_off).to(self.device)
         tiles = self._sample_tiles(first_node) if _SAMPLE_TILES and not _SAMPLE_WAVES and count > 0 else None
-        scratch = None if tiles is None else self._scratch((tiles[2] + 1) * _lib.SAMPLE_IMAGE_BYTES)
+        steps = scratch = None
+        if tiles is not None:
+            steps = self._steps_before_tiles(first_node, count, tiles)
+            if steps is None:
+                scratch = self._scratch((tiles[2] + 1) * _lib.SAMPLE_IMAGE_BYTES)
         if scratch is not None:
-            d_tiles, d_rows, n_tile, wide = tiles
+            d_tiles, d_rows, n_tile, wide, _ = tiles
             _lib.check(
                 self.lib.apc_sample_feasible_tiles(
                     C.byref(self.problem), self._ptr(d_tiles), n_tile, self._ptr(d_rows), self._ptr(colbits),
                     self._ptr(d_off), self._ptr(scratch), int(seed), int(first), int(count), self._ptr(d_gid),
                     self._ptr(d_keep), self._ptr(d_keep_off), wide, self._ptr(assign), self._ptr(fallback), self._stream()),
                 "apc_sample_feasible_tiles")
+            self.last_sample_backend = "tiles"
             return assign, fallback
-        steps = self._sample_steps(first_node) if count < max(_SAMPLE_LANES_FROM.values()) else None
+        if steps is None and count < max(_SAMPLE_LANES_FROM.values()):
+            steps = self._sample_steps(first_node)
         if steps is not None and count < _SAMPLE_LANES_FROM[steps[2]]:
             recs, n_step, n_waves = steps
             _lib.check(
@@ -1248,6 +1274,7 @@ class CostEngine:
                     int(seed), int(first), int(count), self._ptr(d_gid), self._ptr(d_keep), self._ptr(d_keep_off),
                     self._ptr(assign), self._ptr(fallback), self._stream()),
                 "apc_sample_feasible_steps")
+            self.last_sample_backend = "steps"
             return assign, fallback
         _lib.check(
             self.lib.apc_sample_feasible(
@@ -1255,6 +1282,7 @@ class CostEngine:
                 self._ptr(d_gid), int(first_node), self._ptr(d_keep), self._ptr(d_keep_off), self._ptr(assign),
                 self._ptr(fallback), self._stream()),
             "apc_sample_feasible")
+        self.last_sample_backend = "lanes"
         return assign, fallback
 
     def random_assignment(self, seed: int, a: int) -> np.ndarray:

@@ -736,7 +736,8 @@ typedef struct apc_sample_tile {
   int32_t seq0; /* node0 - first_node */
   int32_t n_far;
   int32_t far[APC_SAMPLE_TILE_FAR];
-  int32_t reserved[10];
+  int32_t depth; /* in tile 0: nodes of the longest chain from first_node on */
+  int32_t reserved[9];
 } apc_sample_tile; /* 160 bytes */
 int apc_sample_tiles(int32_t n_node, int32_t n_edge, const int32_t* node_edge_off, const int32_t* edge_src,
                      const int32_t* edge_ssrc, const int32_t* node_nstrat, int32_t first_node, apc_sample_tile* tiles,

@@ -77,6 +77,11 @@ def test_layout(name, first_node):
                 assert t["far"][at - RING] == u and at - RING < t["n_far"] and u < asked
         v += int(t["n_node"])
     assert v == g.num_nodes
+    level = np.zeros(v, int)  # nodes of the longest chain that ends in a node
+    for u in range(first_node, v):
+        src = g.edge_src_node[g.node_edge_off[u]:g.node_edge_off[u + 1]]
+        level[u] = 1 + max((level[x] for x in src if x >= first_node), default=0)
+    assert tiles[0]["reserved"][0] == level.max() and (tiles[1:]["reserved"] == 0).all()
 
 
 def test_layout_leaves_other_graphs_alone():
@@ -109,11 +114,42 @@ def test_draws_equal_the_lane_walks(name, count, monkeypatch):
                 out += [a.view(torch.int16).cpu(), f.cpu()]
         return out
 
+    monkeypatch.setattr(engine_mod, "_SAMPLE_TILES_US", (0.0, 0.0, 0.0))  # also where steps would be faster
     assert eng._sample_tiles(first_node) is not None
     got = draws()
+    assert eng.last_sample_backend == "tiles"
     monkeypatch.setattr(engine_mod, "_SAMPLE_TILES", False)
     monkeypatch.setattr(engine_mod, "_SAMPLE_LANES_FROM", {2: 0, 16: 0})
     want = draws()
+    assert eng.last_sample_backend == "lanes"
     assert all(torch.equal(a, b) for a, b in zip(got, want))
     if name == "many_args":
         assert max(int(f.max()) for f in want[1::2]) > 0  # nodes that fall back do occur
+
+
+# small batches of a graph with work for sixteen wavefronts go in steps, larger ones and decoders by tiles; the same draws
+@pytest.mark.gpu
+@pytest.mark.parametrize("name,first_node,count,route", [
+    ("dag", 0, 100, "steps"), ("dag", 0, 16385, "steps"), ("dag", 0, 49152, "steps"), ("dag", 0, 49153, "tiles"),
+    ("dag", 90, 33, "steps"), ("small_dag", 0, 32768, "steps"), ("small_dag", 0, 65537, "tiles"), ("gpt2", 0, 1, "tiles"),
+    ("llama_8x8", 0, 65, "tiles")])
+def test_which_graphs_are_drawn_in_steps(name, first_node, count, route, monkeypatch):
+    g = {"dag": lambda: graphgen.stress_graph(400, (2, 2, 4), seed=1, s_min=2, s_max=20),
+         "small_dag": lambda: graphgen.stress_graph(60, (2, 2, 4), seed=1, s_min=2, s_max=20),
+         **{k: lambda k=k: GRAPHS[k]()[0] for k in GRAPHS}}[name]()
+    eng = engine_mod.CostEngine(g).build()
+    gen = torch.Generator(device="cuda").manual_seed(count)
+    nstrat = torch.from_numpy(g.node_nstrat.astype(np.int32)).cuda()[:, None]
+    given = (torch.randint(0, 1 << 30, (g.num_nodes, count), device="cuda", generator=gen, dtype=torch.int32)
+             % nstrat).to(torch.int16).view(torch.uint16)
+
+    def draw():
+        a, f = eng.sample_feasible(3, 17, count, first_node=first_node, assign=given.clone())
+        return a.view(torch.int16), f, eng.last_sample_backend
+
+    got = draw()
+    assert got[2] == route
+    monkeypatch.setattr(engine_mod, "_SAMPLE_TILES", False)
+    monkeypatch.setattr(engine_mod, "_SAMPLE_LANES_FROM", {2: 0, 16: 0})
+    want = draw()
+    assert want[2] == "lanes" and torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
