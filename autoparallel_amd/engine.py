@@ -424,6 +424,7 @@ class CostEngine:
         self._built_marks = self._array_marks()
         self._recs_marks: tuple = ()
         self.last_score_backend = "entry_arrays"  # what the last batch was scored from
+        self.last_score_entry = ""  # and by which entry point of the library
         self.last_sample_backend = ""  # how the last feasible draws were made: by "tiles", "steps" or "lanes"
 
     def synchronize(self) -> None:
@@ -678,25 +679,26 @@ class CostEngine:
                 return self._score_terms(clamp, assign, seed, first, count, d_gid, first_node, init, out, stream)
         return self._score_arrays(assign, seed, first, count, d_gid, first_node, init, out, stream)
 
+    def _launch_score(self, name: str, *args) -> None:
+        _lib.check(getattr(self.lib, name)(*args), name)
+        self.last_score_entry = name
+
     def _score_arrays(self, assign, seed, first, count, d_gid, first_node, init, out, stream) -> torch.Tensor:
         args = (C.byref(self.problem), self._ptr(self.per_arg), self._ptr(self.comm), self._ptr(self.cost),
                 self._ptr(self.flags))
         if assign is not None:
-            _lib.check(
-                self.lib.apc_score_assignments_window(
-                    *args, self._ptr(assign), int(count), int(first_node), self._ptr(init), self._ptr(out), stream),
-                "apc_score_assignments_window")
+            self._launch_score(
+                "apc_score_assignments_window",
+                *args, self._ptr(assign), int(count), int(first_node), self._ptr(init), self._ptr(out), stream)
         elif d_gid is None:
-            _lib.check(
-                self.lib.apc_score_random_assignments(
-                    *args, int(seed), int(first), int(count), self._ptr(out), stream),
-                "apc_score_random_assignments")
+            self._launch_score(
+                "apc_score_random_assignments",
+                *args, int(seed), int(first), int(count), self._ptr(out), stream)
         else:
-            _lib.check(
-                self.lib.apc_score_random_window(
-                    *args, int(seed), int(first), int(count), self._ptr(d_gid), int(first_node), self._ptr(init),
-                    self._ptr(out), stream),
-                "apc_score_random_window")
+            self._launch_score(
+                "apc_score_random_window",
+                *args, int(seed), int(first), int(count), self._ptr(d_gid), int(first_node), self._ptr(init),
+                self._ptr(out), stream)
         self.last_score_backend = "entry_arrays"
         return out
 
@@ -708,19 +710,17 @@ class CostEngine:
             scratch = self._scratch((g.num_edges - first_edge) * _lib.FOLD_EDGE_BYTES
                                     + (g.num_nodes - first_node) * _lib.FOLD_NODE_BYTES)
         if scratch is not None:
-            _lib.check(
-                self.lib.apc_score_terms(
-                    C.byref(self.problem), self._ptr(self.per_arg), self._ptr(self.table), self._ptr(scratch),
-                    self._ptr(assign), int(seed), int(first), int(count), self._ptr(d_gid), int(first_node), first_edge,
-                    clamp, self._ptr(init), self._ptr(out), stream),
-                "apc_score_terms")
+            self._launch_score(
+                "apc_score_terms",
+                C.byref(self.problem), self._ptr(self.per_arg), self._ptr(self.table), self._ptr(scratch),
+                self._ptr(assign), int(seed), int(first), int(count), self._ptr(d_gid), int(first_node), first_edge,
+                clamp, self._ptr(init), self._ptr(out), stream)
         else:
-            _lib.check(
-                self.lib.apc_score_fold_table(
-                    C.byref(self.problem), self._ptr(self.per_arg), self._ptr(self.table), self._ptr(assign), int(seed),
-                    int(first), int(count), self._ptr(d_gid), int(first_node), clamp, self._ptr(init),
-                    self._ptr(out), stream),
-                "apc_score_fold_table")
+            self._launch_score(
+                "apc_score_fold_table",
+                C.byref(self.problem), self._ptr(self.per_arg), self._ptr(self.table), self._ptr(assign), int(seed),
+                int(first), int(count), self._ptr(d_gid), int(first_node), clamp, self._ptr(init),
+                self._ptr(out), stream)
         self.last_score_backend = "block_table_terms"
         return out
 
@@ -761,23 +761,21 @@ class CostEngine:
                 d_pieces, n_piece, n_item = pieces
                 scratch = self._scratch(n_item * _lib.SCORE_SIDE_BYTES + n_piece * _lib.SCORE_PIECE_SCRATCH)
                 if scratch is not None:
-                    _lib.check(
-                        self.lib.apc_score_stream(
-                            C.byref(self.problem), self._ptr(self.per_arg), self._ptr(self.table), self._ptr(d_pieces),
-                            n_piece, n_item, self._ptr(scratch), int(seed), int(first), int(count), self._ptr(d_gid),
-                            clamp, self._ptr(init), self._ptr(out), stream),
-                        "apc_score_stream")
+                    self._launch_score(
+                        "apc_score_stream",
+                        C.byref(self.problem), self._ptr(self.per_arg), self._ptr(self.table), self._ptr(d_pieces),
+                        n_piece, n_item, self._ptr(scratch), int(seed), int(first), int(count), self._ptr(d_gid),
+                        clamp, self._ptr(init), self._ptr(out), stream)
                     self.last_score_backend = "block_table"
                     return out
             aux = self._score_edge_aux(d_gid)
-            _lib.check(
-                self.lib.apc_score_table(
-                    C.byref(self.problem), self._ptr(self.per_arg), self._ptr(self.table),
-                    C.c_void_p(aux.data_ptr()), self._ptr(assign),
-                    int(seed), int(first), int(count), self._ptr(d_gid), int(first_node), self.g.num_nodes,
-                    clamp, min(_SCORE_PER_LANE, 4),
-                    self._ptr(init), self._ptr(out), stream),
-                "apc_score_table")
+            self._launch_score(
+                "apc_score_table",
+                C.byref(self.problem), self._ptr(self.per_arg), self._ptr(self.table),
+                C.c_void_p(aux.data_ptr()), self._ptr(assign),
+                int(seed), int(first), int(count), self._ptr(d_gid), int(first_node), self.g.num_nodes,
+                clamp, min(_SCORE_PER_LANE, 4),
+                self._ptr(init), self._ptr(out), stream)
             self.last_score_backend = "block_table"
             return out
         from_table &= self._versioned  # else an edit would go unnoticed
@@ -789,12 +787,11 @@ class CostEngine:
                 steps, n_step, d_tiles, n_tile = pairs
                 scratch = self._scratch((n_tile + 1) * _lib.PAIR_IMAGE_BYTES)
                 if scratch is not None:
-                    _lib.check(
-                        self.lib.apc_score_pairs(
-                            C.byref(self.problem), self._ptr(self.per_arg), self._ptr(self.table), self._ptr(steps),
-                            n_step, self._ptr(d_tiles), n_tile, self._ptr(scratch), int(seed), int(first), int(count),
-                            self._ptr(d_gid), clamp, self._ptr(out), stream),
-                        "apc_score_pairs")
+                    self._launch_score(
+                        "apc_score_pairs",
+                        C.byref(self.problem), self._ptr(self.per_arg), self._ptr(self.table), self._ptr(steps),
+                        n_step, self._ptr(d_tiles), n_tile, self._ptr(scratch), int(seed), int(first), int(count),
+                        self._ptr(d_gid), clamp, self._ptr(out), stream)
                     self.last_score_backend = "block_table_tiles"
                     return out
         if from_table and _SCORE_FROM_TILES and not self.large_blocks and (
@@ -811,13 +808,12 @@ class CostEngine:
                     scratch = self._scratch(tiles[1] * _lib.SCORE_STEP_BYTES)
             if scratch is not None:
                 steps, n_step, d_tiles, n_tile, units = tiles
-                _lib.check(
-                    getattr(self.lib, name)(
-                        C.byref(self.problem), self._ptr(self.per_arg), self._ptr(self.table), self._ptr(steps), n_step,
-                        self._ptr(d_tiles), n_tile, self._ptr(units), self._ptr(scratch), self._ptr(assign),
-                        int(seed), int(first), int(count), self._ptr(d_gid), clamp, self._ptr(init),
-                        self._ptr(out), stream),
-                    name)
+                self._launch_score(
+                    name,
+                    C.byref(self.problem), self._ptr(self.per_arg), self._ptr(self.table), self._ptr(steps), n_step,
+                    self._ptr(d_tiles), n_tile, self._ptr(units), self._ptr(scratch), self._ptr(assign),
+                    int(seed), int(first), int(count), self._ptr(d_gid), clamp, self._ptr(init),
+                    self._ptr(out), stream)
                 self.last_score_backend = "block_table_tiles"
                 return out
         terms_below = table_from if large and _SCORE_TERMS_BELOW else _SCORE_TERMS_BELOW
@@ -852,20 +848,18 @@ class CostEngine:
             self._recs_valid = True
             self._recs_marks = self._array_marks()
         if self._recs_compact:
-            _lib.check(
-                self.lib.apc_score_compact(
-                    C.byref(self.problem), self._ptr(self.per_arg), self._ptr(self._recs), self._ptr(assign),
-                    int(seed), int(first), int(count), self._ptr(d_gid), int(first_node), self.g.num_nodes,
-                    _SCORE_PER_LANE, self._ptr(init), self._ptr(out), self._stream()),
-                "apc_score_compact")
+            self._launch_score(
+                "apc_score_compact",
+                C.byref(self.problem), self._ptr(self.per_arg), self._ptr(self._recs), self._ptr(assign),
+                int(seed), int(first), int(count), self._ptr(d_gid), int(first_node), self.g.num_nodes,
+                _SCORE_PER_LANE, self._ptr(init), self._ptr(out), self._stream())
             self.last_score_backend = "compact_records"
             return out
-        _lib.check(
-            self.lib.apc_score_packed(
-                C.byref(self.problem), self._ptr(self.per_arg), self._ptr(self._recs), self._ptr(assign),
-                int(seed), int(first), int(count), self._ptr(d_gid), int(first_node), self._ptr(init),
-                self._ptr(out), self._stream()),
-            "apc_score_packed")
+        self._launch_score(
+            "apc_score_packed",
+            C.byref(self.problem), self._ptr(self.per_arg), self._ptr(self._recs), self._ptr(assign),
+            int(seed), int(first), int(count), self._ptr(d_gid), int(first_node), self._ptr(init),
+            self._ptr(out), self._stream())
         self.last_score_backend = "records"
         return out
 

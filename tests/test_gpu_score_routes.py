@@ -1,0 +1,65 @@
+"""Which entry point scores a batch by default, on both sides of every line between two of them, and that the sums are
+the same bits there as from the entry arrays."""
+import numpy as np
+import pytest
+import torch
+
+from autoparallel_amd import engine as engine_mod
+from autoparallel_amd import graphgen
+from autoparallel_amd.engine import CostEngine
+
+pytestmark = pytest.mark.gpu
+
+# blocks that images of finished entries take many of at a time and few (2.6), and large ones
+GRAPHS = {
+    "small": lambda: graphgen.gpt2_graph((4,), 4, vocab=4096, seq=512, batch=64),
+    "middling": lambda: graphgen.stress_graph(130, (2, 2, 4), seed=1, s_min=34, s_max=38),
+    "large": lambda: graphgen.stress_graph(60, (2, 2, 4), seed=1, s_min=95, s_max=110),  # two pieces a matrix
+}
+
+
+@pytest.fixture(scope="module")
+def engines():
+    return {name: CostEngine(make(), table_mode="full").build() for name, make in GRAPHS.items()}
+
+
+# kind: random, the same with carried sums, explicit
+ROUTES = [
+    ("small", "random", 3000, "apc_score_terms"), ("small", "explicit", 3000, "apc_score_terms"),
+    ("small", "random", 81920, "apc_score_terms"), ("small", "random", 81921, "apc_score_pairs"),
+    ("middling", "random", 114687, "apc_score_terms"), ("middling", "random", 114689, "apc_score_images"),
+    ("middling", "random", 131072, "apc_score_images"), ("middling", "random", 131073, "apc_score_pairs"),
+    ("small", "carried", 114687, "apc_score_terms"), ("small", "carried", 114689, "apc_score_images"),
+    ("small", "carried", 196608, "apc_score_images"), ("small", "carried", 196609, "apc_score_from_tiles"),
+    ("small", "explicit", 81920, "apc_score_terms"), ("small", "explicit", 81921, "apc_score_images"),
+    ("small", "explicit", 262145, "apc_score_images"),
+    ("large", "random", 131072, "apc_score_terms"), ("large", "carried", 131072, "apc_score_terms"),
+    ("large", "random", 262144, "apc_score_stream"), ("large", "carried", 262144, "apc_score_stream"),
+    ("large", "explicit", 196607, "apc_score_terms"), ("large", "explicit", 196608, "apc_score_table"),
+]
+
+
+@pytest.mark.parametrize("name,kind,count,entry", ROUTES)
+def test_routes(engines, name, kind, count, entry, monkeypatch):
+    eng = engines[name]
+    g = eng.g
+    gen = torch.Generator(device="cuda").manual_seed(count)
+    ids = np.arange(g.num_nodes, dtype=np.int32)
+    if kind == "explicit":
+        nstrat = torch.from_numpy(g.node_nstrat.astype(np.int32)).cuda()[:, None]
+        assign = (torch.randint(0, 1 << 30, (g.num_nodes, count), device="cuda", generator=gen, dtype=torch.int32)
+                  % nstrat).to(torch.int16)
+    elif kind == "carried":
+        init = torch.rand((count, 6), dtype=torch.float64, device="cuda", generator=gen)
+
+    def score():
+        out = (eng.score(assign) if kind == "explicit" else eng.score_random(11, 5, count) if kind == "random"
+               else eng.score_random_window(11, 5, count, ids, 3, init=init))
+        return out.view(torch.int64), eng.last_score_entry, eng.last_score_backend
+
+    got = score()
+    assert got[1] == entry and got[2].startswith("block_table")
+    monkeypatch.setattr(engine_mod, "_SCORE_FROM_TABLE", False)
+    monkeypatch.setattr(engine_mod, "_SCORE_SMALL_FROM_TABLE", False)
+    want = score()
+    assert want[2] == ("compact_records" if count >= 32768 else "entry_arrays") and torch.equal(got[0], want[0])
