@@ -22,10 +22,10 @@ _SCORE_FROM_TABLE = True  # the three ways of scoring a graph with large blocks 
 _SCORE_COMPACT = True
 _SCORE_SMALL_FROM_TABLE = True
 _SCORE_FROM_TILES = True  # small blocks: matrices through LDS by tiles, while the table stands for the arrays
-# Below, the terms of a few assignments gathered side by side are faster than a walk over records with a lane per
-# assignment: random ones of a window of the planner DAG, 98 304 and 114 688 assignments, 2.49 and 2.98 ms against 3.83 and
+# Below (seven rounds of 16 384, and one more; 0 switches them off above _SCORE_LANES_FROM: tests), the terms of a few
+# assignments gathered side by side are faster than a walk over records with a lane per assignment: random ones of a window of the planner DAG, 98 304 and 114 688 assignments, 2.49 and 2.98 ms against 3.83 and
 # 3.87, explicit ones 3.10 and 3.79 against 4.40 and 4.45.
-_SCORE_TERMS_BELOW = 114688
+_SCORE_TERMS_BELOW = 114689
 # The same where the walk is one over tile images, which is as long for one assignment as for the 65 536 that are a
 # wavefront a SIMD; terms go in rounds of 16 384.  In ms, terms and images: Llama-3-8B graph, random, at 114 688 and 131 072
 # 2.49, 2.90 and 2.80, 2.91, explicit, at 81 920 and 90 112 2.48, 2.70 and 3.16, 2.70; 12-layer GPT-2 graph 0.77, 0.81 and
@@ -794,9 +794,10 @@ class CostEngine:
                         self._ptr(d_gid), clamp, self._ptr(out), stream)
                     self.last_score_backend = "block_table_tiles"
                     return out
-        if from_table and _SCORE_FROM_TILES and not self.large_blocks and (
-                count > _SCORE_TERMS_UP_TO_IMAGES["random" if assign is None else "explicit"]
-                or not _SCORE_SMALL_FROM_TABLE or _SCORE_TERMS_BELOW <= count):
+        terms_up_to = -1
+        if _SCORE_SMALL_FROM_TABLE:
+            terms_up_to = min(_SCORE_TERMS_UP_TO_IMAGES["random" if assign is None else "explicit"], _SCORE_TERMS_BELOW - 1)
+        if from_table and _SCORE_FROM_TILES and not self.large_blocks and count > terms_up_to:
             name, scratch = "apc_score_images", None
             if assign is not None or count <= _SCORE_IMAGES_UP_TO:
                 tiles = self._score_tiles(first_node, True)
@@ -816,8 +817,10 @@ class CostEngine:
                     self._ptr(out), stream)
                 self.last_score_backend = "block_table_tiles"
                 return out
-        terms_below = table_from if large and _SCORE_TERMS_BELOW else _SCORE_TERMS_BELOW
-        if from_table and count < max(terms_below, _SCORE_TERMS_BELOW) and _SCORE_SMALL_FROM_TABLE:
+        terms_below = _SCORE_TERMS_BELOW
+        if large and terms_below:
+            terms_below = max(terms_below, table_from)
+        if from_table and count < terms_below and _SCORE_SMALL_FROM_TABLE:
             return self._score_terms(clamp, assign, seed, first, count, d_gid, first_node, init, out, stream)
         recs_stand = (self._recs_valid and self._unchanged(self._recs_marks)
                       and (capturing or not self._recorded_writes))  # else replayed since, or not

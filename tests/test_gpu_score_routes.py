@@ -27,9 +27,9 @@ def engines():
 ROUTES = [
     ("small", "random", 3000, "apc_score_terms"), ("small", "explicit", 3000, "apc_score_terms"),
     ("small", "random", 81920, "apc_score_terms"), ("small", "random", 81921, "apc_score_pairs"),
-    ("middling", "random", 114687, "apc_score_terms"), ("middling", "random", 114689, "apc_score_images"),
+    ("middling", "random", 114688, "apc_score_terms"), ("middling", "random", 114689, "apc_score_images"),
     ("middling", "random", 131072, "apc_score_images"), ("middling", "random", 131073, "apc_score_pairs"),
-    ("small", "carried", 114687, "apc_score_terms"), ("small", "carried", 114689, "apc_score_images"),
+    ("small", "carried", 114688, "apc_score_terms"), ("small", "carried", 114689, "apc_score_images"),
     ("small", "carried", 196608, "apc_score_images"), ("small", "carried", 196609, "apc_score_from_tiles"),
     ("small", "explicit", 81920, "apc_score_terms"), ("small", "explicit", 81921, "apc_score_images"),
     ("small", "explicit", 262145, "apc_score_images"),
