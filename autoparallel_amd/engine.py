@@ -45,6 +45,14 @@ _SCORE_PAIRS_FROM, _SCORE_PAIRS_ROWS = (81920, 131072), 8
 _SCORE_IMAGES_UP_TO = 196608
 _SCORE_STREAM = True  # random assignments on graphs with large blocks: matrices as a stream of pieces through LDS
 _SCORE_TERM_RECORDS = True  # terms side by side from records of the edges and nodes, made in front of them
+# But not where a graph is a few of the smallest batches' tiles: there the records' own launch costs more than it saves.
+# Up to so many (assignments; edges or nodes on graphs with small blocks; with large ones, whose entries a workgroup waits
+# for longer in the form without records) it is one launch.  In us, a call alone and among others, with records and
+# without: 1-layer GPT-2 graph (318 edges), random, 100 30.6, 15.7 and 25.9, 11.1, 1 000 28.9, 15.8 and 27.0, 11.2, 2 000 29.5,
+# 15.8 and 28.4, 12.6; 3 layers (786), 100 33.8, 16.3 and 31.1, 15.5, 1 000 33.3, 16.3 and 32.4, 16.7; 6 layers (1 488), explicit,
+# 100 40.5, 21.4 and 38.4, 22.1; 1-layer 70B decoder (318, 341 strategies), 100 31.1, 16.0 and 26.0, 10.8, 2 000 34.5, 17.5 and
+# 39.3, 20.8; 2 layers (583), 1 000 34.9, 17.9 and 36.6, 20.9.
+_SCORE_TERM_FIELDS_UP_TO = ((256, 1536, 1536), (1024, 800, 384), (2048, 384, 192))
 # Matrices of up to this many LDS tiles (64 KB each) go through LDS in the table scorer, larger
 # ones are read in place.  Measured on a 3 000-node window of the stress DAG, 2^20 assignments:
 # 17.9 ms with 1, 17.4 with 2, 18.0 with 4, 18.35 with 8 or 16.  (A lower bound, small matrices
@@ -705,8 +713,10 @@ class CostEngine:
     def _score_terms(self, clamp, assign, seed, first, count, d_gid, first_node, init, out, stream) -> torch.Tensor:
         g = self.g
         first_edge = int(g.node_edge_off[first_node])
+        rows = max(g.num_edges - first_edge, g.num_nodes - first_node)
+        few = next((most[2 if self.large_blocks else 1] for most in _SCORE_TERM_FIELDS_UP_TO if count <= most[0]), 0)
         scratch = None
-        if _SCORE_TERM_RECORDS and first_node < g.num_nodes and first_edge < g.num_edges:
+        if _SCORE_TERM_RECORDS and rows > few and first_node < g.num_nodes and first_edge < g.num_edges:
             scratch = self._scratch((g.num_edges - first_edge) * _lib.FOLD_EDGE_BYTES
                                     + (g.num_nodes - first_node) * _lib.FOLD_NODE_BYTES)
         if scratch is not None:

@@ -1,4 +1,4 @@
-"""Small batches are scored in groups of 4 to 64 assignments whose terms are gathered side by
+"""Small batches are scored in groups of 1 to 64 assignments whose terms are gathered side by
 side; every row has to have the bits of the walk that takes one lane per assignment."""
 import numpy as np
 import pytest
@@ -24,37 +24,52 @@ def _bits(t):
     return t.cpu().numpy().view(np.uint64)
 
 
-# 1 << shift assignments a workgroup: up to 1024, 4096, 8192, 16383, and beyond
-@pytest.mark.parametrize("count", [1, 3, 5, 1024, 1025, 4096, 4097, 8193, 16383, 16385])
+# 1 << shift assignments a workgroup: from records 1 up to 256, 2 up to 512, and so on to 64 up to 16 384 and beyond, there
+# with two workgroups a CU; without them 4 up to 1 024, 8 up to 4 096, 16 up to 8 192, 32 up to 16 383, 64 beyond
+@pytest.mark.parametrize("count", [1, 3, 5, 256, 257, 512, 513, 1024, 1025, 2048, 2049, 4096, 4097, 8192, 8193, 16383, 16384,
+                                   16385])
 @pytest.mark.parametrize("which", [0, 1])
 def test_groups_have_the_bits_of_the_lane_walk(engines, which, count, monkeypatch):
     eng, gid, first_node = engines[which]
     g = eng.g
+    eng.set_node_multiplier(np.arange(g.num_nodes) % 4 - 1 if count % 2 else np.ones(g.num_nodes))
+    eng.build(clamp_inf=count % 3 != 0)
     rng = np.random.default_rng(count)
     assign = torch.from_numpy((rng.integers(0, 1 << 20, (g.num_nodes, count)) % g.node_nstrat[:, None]).astype(np.int16)).cuda()
-    init = torch.from_numpy(rng.integers(0, 1000, (count, 6)).astype(np.float64)).cuda()
+    init = torch.from_numpy(rng.random((count, 6)) * 1000).cuda()
+    init[:, [3, 5]] = init[:, [3, 5]].floor()  # counts, but for the rows below
+    init[::3] = -0.0
+    init[1::5] = 0.5
+    init[2::7] = torch.inf
     ids = np.arange(g.num_nodes, dtype=np.int32) if gid is None else gid
 
     def all_scores():
         return [_bits(x) for x in (
             eng.score_random(11, 5, count), eng.score(assign),
             eng.score_random_window(11, 5, count, ids, first_node, init=init),
-            eng.score_random_window(11, 5, count, ids, g.num_nodes, init=init),  # nothing to add
+            eng.score_random_window(11, 5, count, ids, g.num_nodes, init=init.abs()),  # nothing to add
             eng.score_window(assign, first_node, init=init))]
 
+    monkeypatch.setattr(engine_mod, "_SCORE_TERM_FIELDS_UP_TO", ())
     from_table = all_scores()
+    assert eng.last_score_entry == "apc_score_terms"
+    monkeypatch.setattr(engine_mod, "_SCORE_TERM_RECORDS", False)
+    from_fields = all_scores()
+    assert eng.last_score_entry == "apc_score_fold_table"
     monkeypatch.setattr(engine_mod, "_SCORE_SMALL_FROM_TABLE", False)
     from_arrays = all_scores()
-    monkeypatch.setattr(engine_mod, "_SCORE_LANES_FROM", 1)  # one lane per assignment, from records
+    assert eng.last_score_backend == "entry_arrays"
+    monkeypatch.setattr(engine_mod, "_SCORE_LANES_FROM", 1)  # one lane per assignment, from records of the entries
     monkeypatch.setattr(engine_mod, "_SCORE_FROM_TABLE", False)
     want = all_scores()
-    for a, b, c in zip(from_table, from_arrays, want):
-        assert (a == c).all() and (b == c).all()
+    for a, b, c, d in zip(from_table, from_fields, from_arrays, want):
+        assert (a == d).all() and (b == d).all() and (c == d).all()
 
 
 def test_the_table_stands_for_the_arrays_only_while_it_does(engines):
     """Clamped and unclamped builds; and where the arrays were edited, the arrays decide."""
     eng = engines[0][0]
+    eng.set_node_multiplier(np.ones(eng.g.num_nodes))
     for clamp in (False, True):
         eng.build(clamp_inf=clamp)
         got = _bits(eng.score_random(3, 0, 70))
@@ -96,6 +111,7 @@ def test_draws_among_more_strategies_than_16_bits_count(table_mode, monkeypatch)
     eng = CostEngine(g, table_mode=table_mode).build()
     ids = np.arange(g.num_nodes, dtype=np.int32)
     ref = O.GraphOracle(g).build()
+    monkeypatch.setattr(engine_mod, "_SCORE_TERM_FIELDS_UP_TO", ())
     for count in (70, 600, 5000, 40000):
         init = torch.arange(count * 6, dtype=torch.float64, device="cuda").reshape(count, 6)
         got = []

@@ -14,7 +14,9 @@ pytestmark = pytest.mark.gpu
 GRAPHS = {
     "small": lambda: graphgen.gpt2_graph((4,), 4, vocab=4096, seq=512, batch=64),
     "middling": lambda: graphgen.stress_graph(130, (2, 2, 4), seed=1, s_min=34, s_max=38),
+    "smallest": lambda: graphgen.gpt2_graph((4,), 1, vocab=4096, seq=512, batch=64),
     "large": lambda: graphgen.stress_graph(60, (2, 2, 4), seed=1, s_min=95, s_max=110),  # two pieces a matrix
+    "larger": lambda: graphgen.stress_graph(240, (2, 2, 4), seed=1, s_min=95, s_max=100),
 }
 
 
@@ -25,6 +27,11 @@ def engines():
 
 # kind: random, the same with carried sums, explicit
 ROUTES = [
+    ("small", "random", 256, "apc_score_fold_table"), ("small", "explicit", 257, "apc_score_terms"),
+    ("smallest", "random", 257, "apc_score_fold_table"), ("smallest", "explicit", 1024, "apc_score_fold_table"),
+    ("smallest", "carried", 2048, "apc_score_fold_table"), ("smallest", "random", 2049, "apc_score_terms"),
+    ("large", "carried", 2048, "apc_score_fold_table"), ("large", "explicit", 2049, "apc_score_terms"),
+    ("larger", "random", 1024, "apc_score_fold_table"), ("larger", "random", 1025, "apc_score_terms"),
     ("small", "random", 3000, "apc_score_terms"), ("small", "explicit", 3000, "apc_score_terms"),
     ("small", "random", 81920, "apc_score_terms"), ("small", "random", 81921, "apc_score_pairs"),
     ("middling", "random", 114688, "apc_score_terms"), ("middling", "random", 114689, "apc_score_images"),
