@@ -105,6 +105,36 @@ def xgmi_config_struct(cfg) -> _lib.ApcXgmiConfig:
     return c
 
 
+def matrix_sizes(g: PackedGraph, compressed: bool) -> np.ndarray:
+    """int64[num_edges]: elements of an edge's matrix in the block table, of distinct words where it is compressed; 0
+    where it has none."""
+    _, block_off, _, table_off, usrc, udst = g.block_table(compressed)
+    size = g.edge_ssrc.astype(np.int64) * g.edge_sdst
+    squeezed = (table_off >= 0) & (usrc > 0)
+    if squeezed.any():
+        block = np.searchsorted(block_off, table_off[squeezed], side="right") - 1
+        size[squeezed] = usrc[squeezed].astype(np.int64) * udst[block]
+    size[table_off < 0] = 0
+    return size
+
+
+def piece_counts(g: PackedGraph, size: np.ndarray, first_node: int):
+    """(pieces, items) of the list apc_score_pieces makes for the walk from ``first_node`` on over matrices of
+    ``size`` elements (matrix_sizes), or None where it makes none: what the choice of a scorer needs to know of it."""
+    if first_node >= g.num_nodes or size.max(initial=0) > 0x7FFFFFFF - _lib.SCORE_PIECE:
+        return None
+    first_edge = int(g.node_edge_off[first_node])
+    nstrat, ssrc = g.node_nstrat[first_node:], g.edge_ssrc[first_edge:]
+    most = 10 * int(nstrat.max()), 2 * int(ssrc.max(initial=0))
+    if max(most) > _lib.SCORE_SIDE_BYTES or (sum(most) > _lib.SCORE_SIDE_BYTES and int(
+            (10 * nstrat[g.edge_node[first_edge:] - first_node] + 2 * ssrc).max(initial=0)) > _lib.SCORE_SIDE_BYTES):
+        return None
+    # an edge without a matrix is one piece, too, as is a node without an argument row
+    pieces = np.maximum(size[first_edge:] + (_lib.SCORE_PIECE - 1), _lib.SCORE_PIECE) // _lib.SCORE_PIECE
+    bare = int((np.diff(g.node_edge_off[first_node:]) == 0).sum())
+    return int(pieces.sum()) + bare, len(pieces) + bare
+
+
 def make_model(mesh_shape, devices_per_host: int, device_name: str, order_mode: int = 0,
                topo_config=None) -> _lib.ApcModel:
     """Cost-model constants for a mesh on a named device (raises ApcError for a
@@ -255,7 +285,7 @@ class CostEngine:
 
         self._keep: Dict[str, torch.Tensor] = {}
         self._layouts: Dict[str, dict] = {"score_tiles": {}, "score_tiles_explicit": {}, "sample_steps": {},
-                                          "score_pieces": {}, "sample_tiles": {}, "pair_tiles": {}}
+                                          "score_pieces": {}, "piece_counts": {}, "sample_tiles": {}, "pair_tiles": {}}
 
         # The problem is some thirty arrays, most of them a few kilobytes: they go up in
         # one copy.  An array is laid into a pinned staging buffer and gets its address
@@ -763,9 +793,11 @@ class CostEngine:
             if assign is not None:
                 table_from *= _SCORE_TABLE_EXPLICIT
             elif _SCORE_STREAM:
-                pieces = self._score_pieces(first_node)
-                if pieces is not None:
-                    table_from *= max(1.0, pieces[1] / pieces[2] / _SCORE_TABLE_PIECES)
+                counts = self._layout("piece_counts", first_node, lambda: piece_counts(g, self._matrix_sizes(), first_node))
+                if counts is not None:
+                    table_from *= max(1.0, counts[0] / counts[1] / _SCORE_TABLE_PIECES)
+                    if count >= table_from:  # else the list need not be made
+                        pieces = self._score_pieces(first_node)
         if from_table and large and count >= table_from:
             if pieces is not None:
                 d_pieces, n_piece, n_item = pieces
@@ -960,17 +992,16 @@ class CostEngine:
         ``first_node`` on, or None: a node with too many strategies, nothing to score, or no layout at hand."""
         return self._layout("score_pieces", first_node, lambda: self._make_score_pieces(first_node))
 
+    def _matrix_sizes(self) -> np.ndarray:
+        if "matrix_sizes" not in self._keep:
+            self._keep["matrix_sizes"] = matrix_sizes(self.g, self.table_mode == "compressed")
+        return self._keep["matrix_sizes"]
+
     def _make_score_pieces(self, first_node: int):
         g = self.g
         compressed = self.table_mode == "compressed"
-        _, block_off, _, table_off, usrc, udst = g.block_table(compressed)
-        # rows and columns of a matrix: of distinct words where it is compressed
-        size = g.edge_ssrc.astype(np.int64) * g.edge_sdst
-        squeezed = (table_off >= 0) & (usrc > 0)
-        if squeezed.any():
-            block = np.searchsorted(block_off, table_off[squeezed], side="right") - 1
-            size[squeezed] = usrc[squeezed].astype(np.int64) * udst[block]
-        if g.num_edges and size.max() > 0x7FFFFFFF - _lib.SCORE_PIECE:
+        size = self._matrix_sizes()
+        if size.max(initial=0) > 0x7FFFFFFF - _lib.SCORE_PIECE:
             return None
         size = size.astype(np.int32)
         edges = np.ascontiguousarray(g.edge_records(compressed))

@@ -70,3 +70,11 @@ def test_routes(engines, name, kind, count, entry, monkeypatch):
     monkeypatch.setattr(engine_mod, "_SCORE_SMALL_FROM_TABLE", False)
     want = score()
     assert want[2] == ("compact_records" if count >= 32768 else "entry_arrays") and torch.equal(got[0], want[0])
+
+
+def test_no_list_of_pieces_is_made_to_choose_the_terms():
+    eng = CostEngine(GRAPHS["large"](), table_mode="full").build()
+    eng.score_random(11, 5, 131072)
+    assert eng.last_score_entry == "apc_score_terms" and not eng._layouts["score_pieces"]
+    eng.score_random(11, 5, 262144)
+    assert eng.last_score_entry == "apc_score_stream" and eng._layouts["score_pieces"][0] is not None

@@ -59,6 +59,27 @@ def test_pieces(name, first_node, scale):
 def test_pieces_leave_other_graphs_alone():
     g = graphgen.stress_graph(6, (4, 8, 8), seed=4, s_min=1030, s_max=1100)
     assert len(_pieces(g, 0, np.full(g.num_edges, 100, np.int32))[1]) == 0
+    sizes = engine_mod.matrix_sizes(g, False)
+    assert engine_mod.piece_counts(g, sizes, 0) is None and engine_mod.piece_counts(g, sizes, g.num_nodes) is None
+
+
+@pytest.mark.parametrize("compressed", [False, True])
+@pytest.mark.parametrize("first_node", [0, 9])
+@pytest.mark.parametrize("name", [*GRAPHS, "widest", "wider"])
+def test_counts_are_those_of_the_list(name, first_node, compressed):
+    """What the choice of a scorer asks, without a list: at the largest counts of strategies that a list takes, too."""
+    wide = {"widest": 682, "wider": 683}  # 12 bytes of a side image a strategy, of 8 192
+    g = GRAPHS[name]() if name in GRAPHS else graphgen.stress_graph(12, (4, 8, 8), seed=4, s_min=wide[name], s_max=wide[name])
+    edges = np.ascontiguousarray(g.edge_records(compressed))
+    off, nstrat = [np.ascontiguousarray(x, np.int32) for x in (g.node_edge_off, g.node_nstrat)]
+    sizes = engine_mod.matrix_sizes(g, compressed)
+    msize = sizes.astype(np.int32)
+    out, n, items = np.zeros(g.num_nodes + int((msize // 8192 + 1).sum()), PIECE), C.c_int32(), C.c_int32()
+    _lib.check(_lib.load().apc_score_pieces(
+        edges.ctypes.data, g.num_edges, g.num_nodes, off.ctypes.data, nstrat.ctypes.data, msize.ctypes.data, first_node,
+        out.ctypes.data, len(out), C.byref(n), C.byref(items)), "apc_score_pieces")
+    assert engine_mod.piece_counts(g, sizes, first_node) == ((n.value, items.value) if n.value else None)
+    assert (n.value == 0) == (name == "wider")
 
 
 # one assignment a lane up to 2^18, then two, then four, then a second launch; a workgroup of five wavefronts
