@@ -105,6 +105,15 @@ def xgmi_config_struct(cfg) -> _lib.ApcXgmiConfig:
     return c
 
 
+def score_tile_room(g: PackedGraph):
+    """(steps and tiles, units) that apc_score_tiles may need room for: a step per argument row, and per node without
+    one; a unit per 32 elements of a step's matrix, and of its node's terms, which every tile that the node goes on in
+    places again."""
+    rows = np.maximum(np.diff(g.node_edge_off), 1).astype(np.int64)
+    units = ((g.edge_sdst.astype(np.int64) * g.edge_ssrc + 31) // 32).sum() + (rows * ((g.node_nstrat + 31) // 32)).sum()
+    return g.num_nodes + g.num_edges, max(int(units), 1)
+
+
 def matrix_sizes(g: PackedGraph, compressed: bool) -> np.ndarray:
     """int64[num_edges]: elements of an edge's matrix in the block table, of distinct words where it is compressed; 0
     where it has none."""
@@ -942,9 +951,7 @@ class CostEngine:
             a = [np.ascontiguousarray(x, t) for x, t in (
                 (g.node_edge_off, np.int32), (g.node_nstrat, np.int32), (g.node_nargs, np.int32),
                 (g.node_comp_off, np.int64))]
-            max_step = g.num_nodes + g.num_edges
-            chunks = (g.edge_sdst.astype(np.int64) * g.edge_ssrc + 31) // 32
-            max_unit = int(chunks.sum() + ((g.node_nstrat.astype(np.int64) + 31) // 32).sum()) + max_step
+            max_step, max_unit = score_tile_room(g)
             steps = np.empty((max_step, _lib.SCORE_STEP_BYTES), np.uint8)
             tiles = np.empty((max_step, _lib.SCORE_TILE_BYTES), np.uint8)
             units = np.empty((max_unit, _lib.SCORE_UNIT_BYTES), np.uint8)

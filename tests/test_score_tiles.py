@@ -6,7 +6,7 @@ import numpy as np
 import pytest
 import torch
 
-from autoparallel_amd import _lib, graphgen
+from autoparallel_amd import _lib, graphgen, packed
 from autoparallel_amd import engine as engine_mod
 
 STEP = np.dtype([(k, "<i4") for k in ("node", "src", "nstrat", "ssrc", "nargs", "flags", "mat", "pa", "row_node",
@@ -16,7 +16,22 @@ TILE = np.dtype([(k, "<i4") for k in ("step0", "step1", "unit0", "unit1", "n_row
                 + [("row", "<i4", 16), ("reserved", "<i4", 10)])
 DOUBLES = 5120
 
+def _default_rows(n=6, strategies=250, columns=11, rows=3):
+    """Nodes with argument rows without a producer, whose default values fill a tile each: the terms of a node are placed
+    in every tile that it goes on in."""
+    b = packed.GraphBuilder((2, 2), 4)
+    m = b.meta((64, 96), (96, 1), 4, packed.DT_F32)
+    tuples = [(x, y) for x in (0x00, 0x40, 0x41, 0x80) for y in (0x00, 0x40, 0x41, 0x80)]
+    specs = [b.spec(m, tuples[o % 16]) for o in range(strategies)]
+    for v in range(n):
+        b.add_node(packed.NodeDesc(
+            f"n{v}", in_specs=[[x] * rows for x in specs], out_specs=[[x] for x in specs], inputs=[],
+            default_rows=[[[0.5 * j + a + o * v for j in range(columns)] for a in range(rows)] for o in range(strategies)]))
+    return b.pack()
+
+
 GRAPHS = {
+    "default_rows": _default_rows,
     "gpt2_2x3": lambda: graphgen.gpt2_graph((2, 3), 1, vocab=4096, seq=512, batch=64),
     "moe_8x8": lambda: graphgen.moe_graph((8, 8), 1, vocab=4096, seq=512, batch=64),
     "stress_60": lambda: graphgen.stress_graph(150, (2, 2, 4), seed=4, s_min=2, s_max=60),
@@ -44,6 +59,8 @@ def _layout(g, first_node, explicit):
 def test_layout(name, first_node, explicit):
     g = GRAPHS[name]()
     edges, steps, tiles, units = _layout(g, first_node, explicit)
+    room = engine_mod.score_tile_room(g)
+    assert max(len(steps), len(tiles)) <= room[0] and len(units) <= room[1]
     assert (STEP.itemsize, TILE.itemsize, UNIT.itemsize) == (64, 128, 16)
     table_size = int(g.block_table(False)[1][-1])
     e, v, ring, at = int(g.node_edge_off[first_node]), first_node - 1, {}, 0
