@@ -400,6 +400,7 @@ int apc_sample_feasible_tiles(const apc_problem* p, const apc_sample_tile* tiles
   const int lds = 2 * kImageBytes + kSlots * n_lane;
   void (*const kernel)(const char*, int, uint64_t, int64_t, int64_t, int64_t, uint16_t*, int32_t*) =
       wide ? sample_tiles_kernel<true> : sample_tiles_kernel<false>;
+  if (int rc = check_lds_from_0(reinterpret_cast<const void*>(kernel), "sample_tiles_kernel")) return rc;
   hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
   if (e != hipSuccess) return fail(APC_ERR_LAUNCH, "hipFuncSetAttribute(sample_tiles_kernel): %s", hipGetErrorString(e));
   for (int64_t a0 = 0; a0 < n_assign; a0 += part) {

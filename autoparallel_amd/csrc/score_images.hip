@@ -376,8 +376,9 @@ int launch_walk(const char* images, int n_tile, const uint16_t* assign, int64_t 
                 int64_t first, int64_t n_assign, int clamp_inf, const double* init, double* out, int n_lane,
                 hipStream_t stream) {
   const int lds = 2 * kImageBytes + (kAhead + 1) * kRowSlots * n_lane * 2;
-  hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(score_images_walk_kernel<kFrom, kAhead>),
-                                     hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+  const void* const kernel = reinterpret_cast<const void*>(score_images_walk_kernel<kFrom, kAhead>);
+  if (int rc = check_lds_from_0(kernel, "score_images_walk_kernel")) return rc;
+  hipError_t e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
   if (e != hipSuccess) return fail(APC_ERR_LAUNCH, "hipFuncSetAttribute(score_images_walk_kernel): %s", hipGetErrorString(e));
   hipLaunchKernelGGL((score_images_walk_kernel<kFrom, kAhead>), dim3((unsigned)((n_assign + n_lane - 1) / n_lane)),
                      dim3(n_lane), lds, stream, images, n_tile, assign, stride, row_len, seed, first, n_assign, clamp_inf,

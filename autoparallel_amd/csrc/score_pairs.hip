@@ -449,6 +449,7 @@ int apc_score_pairs(const apc_problem* p, const double* per_arg, const double* t
   void (*const kernel)(const char*, int, uint64_t, int64_t, int64_t, double*) =
       per == 1 ? score_pairs_kernel<1> : per == 2 ? score_pairs_kernel<2> : score_pairs_kernel<4>;
   const int lds = 2 * kImageBytes + kSlots * n_lane * per;
+  if (int rc = check_lds_from_0(reinterpret_cast<const void*>(kernel), "score_pairs_kernel")) return rc;
   hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
   if (e != hipSuccess) return fail(APC_ERR_LAUNCH, "hipFuncSetAttribute(score_pairs_kernel): %s", hipGetErrorString(e));
   for (int64_t a0 = 0; a0 < n_assign; a0 += part) {

@@ -38,5 +38,16 @@ __device__ __forceinline__ void load4_lds(const void* g, uint32_t lds) {
                : "=&s"(saved) : "s"(lds), "v"(g) : "memory");
 }
 
+// The words of an image name places in LDS counted from 0, so that a read needs no addition: right while a kernel that
+// reads them has nothing in front of its dynamic part, neither a __shared__ variable nor an array that the compiler
+// moved there.  Asked of the built kernel before every launch.
+inline int check_lds_from_0(const void* kernel, const char* name) {
+  hipFuncAttributes a;
+  hipError_t e = hipFuncGetAttributes(&a, kernel);
+  if (e != hipSuccess) return fail(APC_ERR_LAUNCH, "hipFuncGetAttributes: %s", hipGetErrorString(e));
+  if (a.sharedSizeBytes != 0) return fail(APC_ERR_UNSUPPORTED, "%s: the dynamic part of its LDS does not begin at 0", name);
+  return 0;
+}
+
 }  // namespace apc_tiles
 #endif  // APC_SCORE_TILES_H_
