@@ -47,6 +47,8 @@ constexpr int kKindMask = 0xC0, kShard = 0x40, kPartial = 0x80, kArgMask = 0x3F;
 constexpr int kPartialSum = 0x80;
 constexpr int kBlock = 256;
 
+constexpr int kFinite = 0x1F8;  // v_cmp_class: normal, denormal, zero
+
 typedef double double2_t __attribute__((ext_vector_type(2)));
 typedef long long ll2_t __attribute__((ext_vector_type(2)));
 
@@ -56,13 +58,17 @@ typedef long long ll2_t __attribute__((ext_vector_type(2)));
 // scorer and sampler takes it from here.  The walks are bound by instructions, and a 64-bit mix
 // with a modulo that was here before took a quarter of them.
 // ---------------------------------------------------------------------------
-__host__ __device__ __forceinline__ uint32_t finalise32(uint32_t h) {  // murmur3's finaliser
-  h ^= h >> 16;
+__host__ __device__ __forceinline__ uint32_t fold16(uint32_t h) { return h ^ (h >> 16); }
+
+__host__ __device__ __forceinline__ uint32_t finalise32_folded(uint32_t h) {  // what follows fold16 in finalise32
   h *= 0x85EBCA6Bu;
   h ^= h >> 13;
   h *= 0xC2B2AE35u;
-  h ^= h >> 16;
-  return h;
+  return fold16(h);
+}
+
+__host__ __device__ __forceinline__ uint32_t finalise32(uint32_t h) {  // murmur3's finaliser
+  return finalise32_folded(fold16(h));
 }
 
 // the part of every draw of assignment a that does not depend on the node
@@ -80,6 +86,13 @@ __host__ __device__ __forceinline__ uint32_t node_key(int32_t gid) { return (uin
 __host__ __device__ __forceinline__ uint32_t plain_draw(uint32_t h0, int32_t gid, int32_t nstrat) {
   const uint32_t h = finalise32(h0 ^ node_key(gid));
   return (uint32_t)(((uint64_t)h * (uint64_t)(uint32_t)nstrat) >> 32);
+}
+
+// A draw from a hash and a key that are folded by themselves in front of a walk, since
+// fold16(x ^ y) == fold16(x) ^ fold16(y): two instructions less.  Keys: node_key(gid), for the
+// rank draw node_key(gid) ^ kRankSalt.
+__device__ __forceinline__ uint32_t folded_draw(uint32_t folded_hash, uint32_t folded_key, uint32_t count) {
+  return __umulhi(finalise32_folded(folded_hash ^ folded_key), count);
 }
 
 // the sampler's rank draw hashes the node's key with this, so that it is not the plain draw's

@@ -61,8 +61,6 @@ typedef const __attribute__((address_space(3))) uint8_t* lds_u8_ptr_t;
 typedef __attribute__((address_space(3))) uint8_t* lds_u8_out_t;
 typedef const __attribute__((address_space(3))) uint64_t* lds_u64_ptr_t;
 
-__device__ __forceinline__ uint32_t fold16(uint32_t h) { return h ^ (h >> 16); }  // finalise32's first half step
-
 __device__ __forceinline__ int columns_of(const apc_problem& p, int e) {
   return p.edges[e].src_node >= 0 ? p.edges[e].ssrc : 1;
 }
@@ -276,10 +274,7 @@ sample_tiles_kernel(const char* __restrict__ images, int n_tile, uint64_t seed, 
       const int i1 = i + 1 < n_node ? i + 1 : i;
       const uint32_t j0 = choice(word(node.w.arg[0].choices, i1)), j1 = choice(word(node.w.arg[1].choices, i1));
       const uint64_t c_before = column(word(node.w.before, i), pick);
-      uint32_t h = (h0 ^ word(node.w.key_rank, i)) * 0x85EBCA6Bu;  // rank_draw by the node's key
-      h ^= h >> 13;
-      h *= 0xC2B2AE35u;
-      h ^= h >> 16;
+      const uint32_t h = finalise32_folded(h0 ^ word(node.w.key_rank, i));  // rank_draw by the node's key
       uint64_t m = rest & c_before;
       if (m_more >> i & 1) {
         const uint32_t n_more = word(node.w.n_more, i);
@@ -293,10 +288,7 @@ sample_tiles_kernel(const char* __restrict__ images, int n_tile, uint64_t seed, 
       const uint32_t r = __umulhi(h, count);
       pick = kWide && (m_wide >> i & 1) ? nth_bit<true>(m, r) : nth_bit<false>(m, r);
       if (__ballot(count == 0)) {
-        uint32_t g = (h0 ^ word(node.w.key_plain, i)) * 0x85EBCA6Bu;  // plain_draw
-        g ^= g >> 13;
-        g *= 0xC2B2AE35u;
-        g ^= g >> 16;
+        const uint32_t g = finalise32_folded(h0 ^ word(node.w.key_plain, i));  // plain_draw
         pick = count == 0 ? __umulhi(g, word(node.w.nstrat, i)) : pick;
         fallbacks += count == 0;
       }

@@ -17,7 +17,6 @@
 namespace {
 
 constexpr int kTermLanes = 768;
-constexpr int kFinite = 0x1F8;  // v_cmp_class: normal, denormal, zero
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 // a pointer made of a number is one to anywhere: its loads are flat ones, which a wait for LDS waits for, too
 typedef const __attribute__((address_space(1))) double* global_f64_ptr_t;
@@ -35,8 +34,6 @@ struct FoldEdge {
 struct FoldNode { uint32_t terms, node, nstrat; int32_t nargs; };
 constexpr uint32_t kSource = 1, kTransition = 2, kSqueezed = 4;
 static_assert(sizeof(FoldEdge) == 48 && sizeof(FoldNode) == 16, "layout");
-
-__device__ __forceinline__ uint32_t fold16(uint32_t h) { return h ^ (h >> 16); }  // finalise32's first half step
 
 __global__ void __launch_bounds__(kBlock)
 fold_records_kernel(apc_problem p, const double* __restrict__ table, const int32_t* __restrict__ node_gid, int first_node,
@@ -120,11 +117,7 @@ score_terms_kernel(const FoldEdge* __restrict__ edges, int n_edges, const FoldNo
       return r;
     };
     auto draw = [&](uint32_t key, uint32_t nstrat) -> uint32_t {  // plain_draw by the node's key
-      uint32_t h = (h0 ^ key) * 0x85EBCA6Bu;
-      h ^= h >> 13;
-      h *= 0xC2B2AE35u;
-      h ^= h >> 16;
-      return __umulhi(h, nstrat);
+      return folded_draw(h0, key, nstrat);
     };
     auto choose = [&](const Rec& r) -> Choices {
       Choices c;

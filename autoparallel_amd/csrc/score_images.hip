@@ -29,7 +29,6 @@ constexpr int kHeadBytes = 2048;  // of an image: edges, nodes, rows, Head
 constexpr int kNodesAt = 1024, kRowsAt = 1536, kHeadAt = 1792;
 constexpr int kImageBytes = APC_SCORE_IMAGE_BYTES;
 constexpr int kUnroll = 4;
-constexpr int kFinite = 0x1F8;  // v_cmp_class: normal, denormal, zero
 typedef const __attribute__((address_space(3))) uint16_t* lds_u16_ptr_t;
 typedef const __attribute__((address_space(3))) double* lds_f64_ptr_t;
 constexpr int kRowSlots = kRows + 1;  // the last one: zeros, the choice of a missing producer
@@ -63,8 +62,6 @@ struct Head {
 };
 static_assert(sizeof(EdgeWords) * kTileSteps <= kNodesAt && sizeof(NodeWords) * kTileSteps <= kRowsAt - kNodesAt &&
               sizeof(RowWords) * kRows <= kHeadAt - kRowsAt && sizeof(Head) + kHeadAt <= kHeadBytes, "an image's head");
-
-__device__ __forceinline__ uint32_t fold16(uint32_t h) { return h ^ (h >> 16); }  // finalise32's first half step
 
 __device__ __forceinline__ int image_doubles(const apc_score_tile& t, const apc_score_unit* __restrict__ units) {
   const apc_score_unit last = units[t.unit1 - 1];  // the units of a tile fill its buffer in order
@@ -251,13 +248,8 @@ score_images_walk_kernel(const char* __restrict__ images, int n_tile, const uint
       const u32x2_t row = reinterpret_cast<const u32x2_t*>(img + kRowsAt)[lane & (kRows - 1)];
       for (int r0 = 0; r0 < n_row; r0 += kUnroll) {  // past n_row: nodes drawn again, never read
 #pragma unroll
-        for (int u = 0; u < kUnroll; ++u) {
-          uint32_t h = (h0 ^ word(row[0], r0 + u)) * 0x85EBCA6Bu;  // plain_draw by the node's key
-          h ^= h >> 13;
-          h *= 0xC2B2AE35u;
-          h ^= h >> 16;
-          rows[(r0 + u) * n_lane] = (uint16_t)__umulhi(h, word(row[1], r0 + u));
-        }
+        for (int u = 0; u < kUnroll; ++u)  // plain_draw by the node's key
+          rows[(r0 + u) * n_lane] = (uint16_t)folded_draw(h0, word(row[0], r0 + u), word(row[1], r0 + u));
       }
     }
     const uint32_t at_rows = (uint32_t)(uintptr_t)(lds_ptr_t)rows;

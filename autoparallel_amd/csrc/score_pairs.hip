@@ -49,8 +49,6 @@ typedef const __attribute__((address_space(3))) double* lds_f64_ptr_t;
 typedef const __attribute__((address_space(3))) double2_t* lds_f64x2_ptr_t;
 typedef uint16_t u16x2_t __attribute__((ext_vector_type(2)));
 
-__device__ __forceinline__ uint32_t fold16(uint32_t h) { return h ^ (h >> 16); }  // finalise32's first half step
-
 __global__ void __launch_bounds__(kBlock)
 pair_images_kernel(apc_problem p, const double* __restrict__ per_arg, const double* __restrict__ table,
                    const apc_pair_step* __restrict__ steps, const apc_pair_tile* __restrict__ tiles, int n_tile,
@@ -200,13 +198,7 @@ score_pairs_kernel(const char* __restrict__ images, int n_tile, uint64_t seed, i
       const uint32_t key = word(row.key, r), w = word(row.nstrat, r), nstrat = w & 0xFFFFu;
       uint32_t packed = 0;
 #pragma unroll
-      for (int k = 0; k < kPer; ++k) {
-        uint32_t h = (h0[k] ^ key) * 0x85EBCA6Bu;  // plain_draw by the node's key
-        h ^= h >> 13;
-        h *= 0xC2B2AE35u;
-        h ^= h >> 16;
-        packed |= __umulhi(h, nstrat) << (8 * k);
-      }
+      for (int k = 0; k < kPer; ++k) packed |= folded_draw(h0[k], key, nstrat) << (8 * k);  // plain_draw by the node's key
       *(row_out_t)(uintptr_t)(my_rows + (w >> 16)) = (packed_t)packed;
     }
     auto choices = [&](uint32_t at) -> uint32_t { return *(row_ptr_t)(uintptr_t)(my_rows + at); };

@@ -30,7 +30,6 @@ constexpr int kPieceDoubles = APC_SCORE_PIECE;  // 64 KB
 constexpr int kSideBytes = APC_SCORE_SIDE_BYTES;
 constexpr int kRingBytes = 160 * 1024;
 constexpr int kAheadMost = 16;  // pieces under way
-constexpr int kFinite = 0x1F8;  // v_cmp_class: normal, denormal, zero
 static_assert(2 * (kPieceDoubles * 8 + kSideBytes) <= kRingBytes, "a piece and the next one");
 
 typedef const __attribute__((address_space(1))) double* global_f64_ptr_t;
@@ -61,8 +60,6 @@ struct AskRec {
 static_assert(sizeof(WalkRec) == 64 && sizeof(AskRec) == 32 && sizeof(apc_score_piece) == 32, "layout");
 // A side image: per-argument terms by choice, then the matrix row of every choice and the column of every choice of the
 // producer, 16 bits each.
-
-__device__ __forceinline__ uint32_t fold16(uint32_t h) { return h ^ (h >> 16); }  // finalise32's first half step
 
 __global__ void __launch_bounds__(kBlock)
 score_pieces_kernel(apc_problem p, const double* __restrict__ per_arg, const double* __restrict__ table,
@@ -155,11 +152,7 @@ score_stream_kernel(const WalkRec* __restrict__ walk, const AskRec* __restrict__
     asm volatile("" : "+v"(t_compute[k]), "+v"(t_comm[k]), "+v"(obj[k]));
   }
   auto draw = [&](int k, uint32_t key, uint32_t nstrat) -> uint32_t {  // plain_draw by the node's key
-    uint32_t h = (h0[k] ^ key) * 0x85EBCA6Bu;
-    h ^= h >> 13;
-    h *= 0xC2B2AE35u;
-    h ^= h >> 16;
-    return __umulhi(h, nstrat);
+    return folded_draw(h0[k], key, nstrat);
   };
   // by 32-bit addresses: a pointer that may go elsewhere makes flat loads, and those wait for the copies, too
   auto lds_f64 = [](uint32_t at) -> double { return *(lds_f64_ptr_t)(uintptr_t)at; };
