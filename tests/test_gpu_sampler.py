@@ -28,6 +28,17 @@ def CostEngine():
     return CostEngine
 
 
+def _routes(eng, monkeypatch):
+    """The three walks there are, each with the switches that lead to it; the draws behind have to have taken it."""
+    monkeypatch.setattr(engine_mod, "_SAMPLE_TILES_US", (0.0, 0.0, 0.0))  # no steps before tiles
+    for route in ("tiles", "steps", "lanes"):
+        monkeypatch.setattr(engine_mod, "_SAMPLE_TILES", route == "tiles")
+        if route == "lanes":
+            monkeypatch.setattr(engine_mod, "_SAMPLE_LANES_FROM", {2: 0, 16: 0})
+        yield route
+        assert eng.last_sample_backend == route
+
+
 @pytest.mark.parametrize("name", list(GRAPHS))
 def test_sampled_assignments_equal_the_oracles(CostEngine, name, monkeypatch):
     g = GRAPHS[name]()
@@ -59,17 +70,29 @@ def test_sampled_assignments_equal_the_oracles(CostEngine, name, monkeypatch):
     # and the plain draws of the same counters do select forbidden variables on these graphs
     plain = eng.score_random(9, 1000, n).cpu().numpy()
     assert (plain[:, 5] > 0).mean() > (scores[:, 5] > 0).mean()
-    # a large batch: the same choices for the same counters, in steps and by lanes
+    # a large batch: the same choices for the same counters, by tiles, in steps and by lanes
     a = 65535
     want, want_fb = O.sample_feasible(g, forbidden, 9, 1000 + a)
-    for lanes in (False, True):
-        if lanes:
-            monkeypatch.setattr(engine_mod, "_SAMPLE_LANES_FROM", {2: 0, 16: 0})
+    for _ in _routes(eng, monkeypatch):
         for count in (n, 65536):  # a lane walk of few wavefronts is another instance of the kernel
             big, big_fb = eng.sample_feasible(seed=9, first=1000, count=count)
             assert np.array_equal(big[:, :n].cpu().numpy(), assign)
             assert np.array_equal(big_fb[:n].cpu().numpy(), fallback)
         assert big[:, a].cpu().numpy().tolist() == want and int(big_fb[a]) == want_fb
+
+
+def test_draws_where_there_is_no_room_for_images(CostEngine, monkeypatch):
+    """Without scratch memory for its images a batch goes in steps, or by lanes: the same draws."""
+    g = GRAPHS["llama_1layer_2x4"]()
+    eng = CostEngine(g).build(clamp_inf=True)
+    for count, other in ((65, "steps"), (70001, "steps"), (458752, "lanes")):
+        want = eng.sample_feasible(seed=3, first=0, count=count)
+        assert eng.last_sample_backend == "tiles"
+        with monkeypatch.context() as m:
+            m.setattr(eng, "_scratch", lambda nbytes: None)
+            got = eng.sample_feasible(seed=3, first=0, count=count)
+        assert eng.last_sample_backend == other
+        assert torch.equal(got[0].view(torch.int16), want[0].view(torch.int16)) and torch.equal(got[1], want[1])
 
 
 def test_sampler_continues_from_given_rows(CostEngine):
@@ -180,11 +203,9 @@ def test_filtered_draws_equal_the_oracle_and_never_fall_back(CostEngine, monkeyp
     for a in range(0, n, 7):
         want, want_fb = O.sample_feasible(g, forbidden, 4, a, row_filter=filters)
         assert assign[:, a].tolist() == want and want_fb == 0, a
-    # the launches that fill the chip, in steps and by lanes (another instance of the kernel for
+    # the launches that fill the chip, by tiles, in steps and by lanes (another instance of the kernel for
     # few wavefronts): the same draws
-    for lanes in (False, True):
-        if lanes:
-            monkeypatch.setattr(engine_mod, "_SAMPLE_LANES_FROM", {2: 0, 16: 0})
+    for _ in _routes(eng, monkeypatch):
         for count in (n, 65536):
             big, big_fb = eng.sample_feasible(seed=4, first=0, count=count, row_filter=filters)
             assert int(big_fb.sum().item()) == 0 and (big[:, :n].cpu().numpy() == assign).all()

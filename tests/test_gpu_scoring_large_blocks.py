@@ -1,5 +1,5 @@
 """Scoring of graphs with large edge blocks: from the block table through LDS
-(apc_score_table), from compact records (apc_score_compact) and from the
+(apc_score_table, apc_score_stream), from compact records (apc_score_compact) and from the
 32-byte records (apc_score_packed), each against the scorer that reads the
 three entry arrays, bit for bit; and that one against the oracle."""
 import numpy as np
@@ -26,12 +26,12 @@ def E():
 @pytest.fixture()
 def knobs(E):
     saved = (E._SCORE_FROM_TABLE, E._SCORE_COMPACT, E._SCORE_STAGE_TILES, E._SCORE_PER_LANE, E._SCORE_TABLE_FROM,
-             E._SCORE_LANES_FROM)
+             E._SCORE_LANES_FROM, E._SCORE_STREAM)
     # the table scorer and the record walks whatever the batch size, where a test asks for them
     E._SCORE_TABLE_FROM = 0
     yield E
     (E._SCORE_FROM_TABLE, E._SCORE_COMPACT, E._SCORE_STAGE_TILES, E._SCORE_PER_LANE, E._SCORE_TABLE_FROM,
-     E._SCORE_LANES_FROM) = saved
+     E._SCORE_LANES_FROM, E._SCORE_STREAM) = saved
 
 
 def _same(a, b):
@@ -71,8 +71,8 @@ def test_every_backend_gives_the_sums_of_the_entry_arrays(knobs, name, table_mod
         eng.packed_scoring = True
         eng.large_blocks = True  # the table scorer also for the graph with small blocks
         assert eng._table_clamp == int(clamp)
-        # the table, its matrices through LDS (one tile, several tiles) or read in place
-        E._SCORE_FROM_TABLE = True
+        # the table edge by edge, its matrices through LDS (one tile, several tiles) or read in place
+        E._SCORE_FROM_TABLE, E._SCORE_STREAM = True, False
         for tiles, per in ((8, 0), (0, 4), (1, 2), (64, 4), (8, 1)):
             E._SCORE_STAGE_TILES, E._SCORE_PER_LANE = tiles, per
             eng._keep.pop("score_edge_aux", None)
@@ -82,6 +82,17 @@ def test_every_backend_gives_the_sums_of_the_entry_arrays(knobs, name, table_mod
                 assert (msize > tile).any() and (msize > 0).any()  # several tiles do occur
             for got, ref in zip(_calls(eng, g, assign, half), want):
                 assert _same(got, ref), (name, table_mode, clamp, "table", tiles, per)
+            assert eng.last_score_entry == "apc_score_table"
+        # and as a stream of pieces, where the nodes are not too wide; without room for its scratch edge by edge
+        E._SCORE_STREAM = True
+        for room in (True, False):
+            with pytest.MonkeyPatch.context() as m:
+                if not room:
+                    m.setattr(eng, "_scratch", lambda nbytes: None)
+                for got, ref in zip(_calls(eng, g, assign, half), want):
+                    assert _same(got, ref), (name, table_mode, clamp, "stream", room)
+            stream = room and name != "stress_long_lists"
+            assert eng.last_score_entry == ("apc_score_stream" if stream else "apc_score_table")
         # compact records, then the 32-byte ones
         E._SCORE_FROM_TABLE = False
         for per in (0, 1, 2, 4, 8):

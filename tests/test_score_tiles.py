@@ -106,11 +106,13 @@ def test_layout_leaves_other_graphs_alone():
 
 
 # one assignment a lane up to 2^18, then two, then four (two, and a second launch, if explicit); past 2^20
-# random ones take a second launch too
+# random ones take a second launch too.  As batches are walked where there is room for the images, where there is none,
+# and where there is none for a record per step either.
 @pytest.mark.gpu
-@pytest.mark.parametrize("name,count", [(name, count) for name in GRAPHS for count in (1, 129, 33000, 262145, 524289)]
+@pytest.mark.parametrize("room", ["images", "steps", "none"])
+@pytest.mark.parametrize("name,count", [(name, count) for name in GRAPHS for count in (1, 129, 33000, 200000, 262145, 524289)]
                          + [("gpt2_2x3", 2**20 + 65)])
-def test_scores_have_the_bits_of_the_walk_over_records(name, count, monkeypatch):
+def test_scores_have_the_bits_of_the_walk_over_records(name, count, room, monkeypatch):
     g = GRAPHS[name]()
     eng = engine_mod.CostEngine(g, table_mode="full").build()
     eng.large_blocks = False
@@ -122,22 +124,34 @@ def test_scores_have_the_bits_of_the_walk_over_records(name, count, monkeypatch)
               % nstrat).to(torch.int16)
     init = torch.rand((count, 6), dtype=torch.float64, device="cuda", generator=gen) * 1e6
 
-    def scores(backend):
+    def scores(*backends):
         out = []
-        for score in (lambda: eng.score_random(11, 5, count), lambda: eng.score(assign),
-                      lambda: eng.score_random_window(11, 5, count, gid, 5, init=init),
-                      lambda: eng.score_window(assign, 5, init=init)):
+        for score, backend in zip((
+                lambda: eng.score_random(11, 5, count), lambda: eng.score(assign),
+                lambda: eng.score_random_window(11, 5, count, gid, 5, init=init),
+                lambda: eng.score_window(assign, 5, init=init)), backends):
             out.append(score().view(torch.int64))
-            assert eng.last_score_backend == backend
+            assert backend in (eng.last_score_backend, eng.last_score_entry)
         return out
 
     monkeypatch.setattr(engine_mod, "_SCORE_LANES_FROM", 1)
     monkeypatch.setattr(engine_mod, "_SCORE_TERMS_BELOW", 0)
+    by_entry = {  # random, explicit, and both with carried sums
+        "images": ("apc_score_images" if count <= 131072 else "apc_score_pairs", "apc_score_images",
+                   "apc_score_images" if count <= 196608 else "apc_score_from_tiles", "apc_score_images"),
+        "steps": ("apc_score_from_tiles",) * 4, "none": ("compact_records",) * 4}[room]
+    if name == "stress_60" or name == "default_rows":  # a matrix may be too large for an image of finished entries
+        by_entry = (("block_table_tiles",) if room == "images" else by_entry[:1]) + by_entry[1:]
+    if room != "images":
+        steps = (g.num_nodes + g.num_edges) * _lib.SCORE_STEP_BYTES
+        scratch = eng._scratch
+        monkeypatch.setattr(eng, "_scratch", lambda nbytes: scratch(nbytes) if room == "steps" and nbytes <= steps else None)
+        monkeypatch.setattr(engine_mod, "_SCORE_IMAGES_UP_TO", 1 << 62)
     for clamp in (True, False):
         eng.build(clamp_inf=clamp)
-        got = scores("block_table_tiles")
+        got = scores(*by_entry)
         monkeypatch.setattr(engine_mod, "_SCORE_FROM_TILES", False)
-        want = scores("compact_records")
+        want = scores(*["compact_records"] * 4)
         monkeypatch.setattr(engine_mod, "_SCORE_FROM_TILES", True)
         assert all(torch.equal(a, b) for a, b in zip(got, want))
         eng.set_node_multiplier(mult)  # the layout is kept, the multipliers are the call's
