@@ -22,10 +22,14 @@ _SCORE_FROM_TABLE = True  # the three ways of scoring a graph with large blocks 
 _SCORE_COMPACT = True
 _SCORE_SMALL_FROM_TABLE = True
 _SCORE_FROM_TILES = True  # small blocks: matrices through LDS by tiles, while the table stands for the arrays
-# Below (seven rounds of 16 384, and one more; 0 switches them off above _SCORE_LANES_FROM: tests), the terms of a few
-# assignments gathered side by side are faster than a walk over records with a lane per assignment: random ones of a window of the planner DAG, 98 304 and 114 688 assignments, 2.49 and 2.98 ms against 3.83 and
-# 3.87, explicit ones 3.10 and 3.79 against 4.40 and 4.45.
-_SCORE_TERMS_BELOW = 114689
+_SCORE_TERMS_ABOVE = True  # from _SCORE_LANES_FROM on, too, up to the lines below (tests switch them off)
+# Where a graph with small blocks has no tiles, the terms of so many assignments gathered side by side are faster than a
+# walk over records with a lane per assignment, which takes as long for one as for 2^18 of them.  In ms, terms and records,
+# random at 114 688, 131 072 and 139 264, explicit at 131 072, 163 840 and 172 032: random DAG of 1 200 nodes with up to 150
+# strategies 1.16, 1.43 and 1.42, 1.43 and 1.51, 1.42, and 1.58, 2.26 and 2.22, 2.29 and 2.34, 2.30; of 300 nodes on 4x8x8
+# 0.30, 0.38 and 0.32, 0.38 and 0.34, 0.37, and 0.36, 0.44 and 0.43, 0.45 and 0.45, 0.45.  Graphs whose terms hit the caches
+# more often would gain above, too (Llama-3-8B graph, compressed table, 196 608 5.3, 7.2), but those have tiles.
+_SCORE_TERMS_UP_TO_RECORDS = {"random": 131072, "explicit": 163840}
 # The same where the walk is one over tile images, which is as long for one assignment as for the 65 536 that are a
 # wavefront a SIMD; terms go in rounds of 16 384.  In ms, terms and images: Llama-3-8B graph, random, at 114 688 and 131 072
 # 2.49, 2.90 and 2.80, 2.91, explicit, at 81 920 and 90 112 2.48, 2.70 and 3.16, 2.70; 12-layer GPT-2 graph 0.77, 0.81 and
@@ -845,9 +849,9 @@ class CostEngine:
                         self._ptr(d_gid), clamp, self._ptr(out), stream)
                     self.last_score_backend = "block_table_tiles"
                     return out
-        terms_up_to = -1
-        if _SCORE_SMALL_FROM_TABLE:
-            terms_up_to = min(_SCORE_TERMS_UP_TO_IMAGES["random" if assign is None else "explicit"], _SCORE_TERMS_BELOW - 1)
+        terms_up_to, kind = -1, "random" if assign is None else "explicit"
+        if _SCORE_SMALL_FROM_TABLE and _SCORE_TERMS_ABOVE:
+            terms_up_to = _SCORE_TERMS_UP_TO_IMAGES[kind]
         if from_table and _SCORE_FROM_TILES and not self.large_blocks and count > terms_up_to:
             name, scratch = "apc_score_images", None
             if assign is not None or count <= _SCORE_IMAGES_UP_TO:
@@ -868,10 +872,8 @@ class CostEngine:
                     self._ptr(out), stream)
                 self.last_score_backend = "block_table_tiles"
                 return out
-        terms_below = _SCORE_TERMS_BELOW
-        if large and terms_below:
-            terms_below = max(terms_below, table_from)
-        if from_table and count < terms_below and _SCORE_SMALL_FROM_TABLE:
+        # on a graph with large blocks, what is not scored by the table above
+        if from_table and terms_up_to >= 0 and (large or count <= _SCORE_TERMS_UP_TO_RECORDS[kind]):
             return self._score_terms(clamp, assign, seed, first, count, d_gid, first_node, init, out, stream)
         recs_stand = (self._recs_valid and self._unchanged(self._recs_marks)
                       and (capturing or not self._recorded_writes))  # else replayed since, or not

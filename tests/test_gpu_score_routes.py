@@ -17,6 +17,7 @@ GRAPHS = {
     "smallest": lambda: graphgen.gpt2_graph((4,), 1, vocab=4096, seq=512, batch=64),
     "large": lambda: graphgen.stress_graph(60, (2, 2, 4), seed=1, s_min=95, s_max=110),  # two pieces a matrix
     "larger": lambda: graphgen.stress_graph(240, (2, 2, 4), seed=1, s_min=95, s_max=100),
+    "untiled": lambda: graphgen.stress_graph(30, (2, 2, 4), seed=1, s_min=2, s_max=150),  # small on average only
 }
 
 
@@ -43,6 +44,9 @@ ROUTES = [
     ("large", "random", 131072, "apc_score_terms"), ("large", "carried", 131072, "apc_score_terms"),
     ("large", "random", 262144, "apc_score_stream"), ("large", "carried", 262144, "apc_score_stream"),
     ("large", "explicit", 196607, "apc_score_terms"), ("large", "explicit", 196608, "apc_score_table"),
+    ("untiled", "random", 131072, "apc_score_terms"), ("untiled", "random", 131073, "apc_score_compact"),
+    ("untiled", "carried", 131072, "apc_score_terms"), ("untiled", "carried", 131073, "apc_score_compact"),
+    ("untiled", "explicit", 163840, "apc_score_terms"), ("untiled", "explicit", 163841, "apc_score_compact"),
 ]
 
 
@@ -65,7 +69,7 @@ def test_routes(engines, name, kind, count, entry, monkeypatch):
         return out.view(torch.int64), eng.last_score_entry, eng.last_score_backend
 
     got = score()
-    assert got[1] == entry and got[2].startswith("block_table")
+    assert got[1] == entry and got[2].startswith("block_table") == (entry != "apc_score_compact")
     monkeypatch.setattr(engine_mod, "_SCORE_FROM_TABLE", False)
     monkeypatch.setattr(engine_mod, "_SCORE_SMALL_FROM_TABLE", False)
     want = score()
