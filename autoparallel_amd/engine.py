@@ -66,9 +66,13 @@ _SCORE_STAGE_TILES = 2
 # edge (explicit ones), terms side by side about 9 ns (random) and 12 per edge and 1 000 assignments.  In ms, random ones,
 # terms and table: window of the planner DAG (1.6 pieces an edge), 131 072 and 147 456 assignments 3.64, 4.08 and 4.43, 4.15;
 # 8-layer 70B decoder on 2x2x4 (2.6 pieces), 131 072 2.09, 4.52.  Explicit ones, that window, 163 840 and 196 608 6.03,
-# 7.89 and 7.76, 7.89.  The table it is from this many assignments on, times pieces per edge over 1.5 (random) or 1.5.
+# 7.89 and 7.76, 7.89.  Random ones without a list of pieces (more than 819 strategies; not made before a graph is
+# recorded) go through the table edge by edge, 1.75 us each: that window, 155 648, 163 840 and 172 032 4.28, 5.05 and 4.59, 5.03
+# and 4.98, 5.04, 120 nodes of 830 to 900 strategies, 147 456 and 163 840 0.33, 0.36 and 0.37, 0.36, 60 of 1 030 to 1 100, 163 840
+# and 180 224 0.21, 0.22 and 0.23, 0.22.  The table it is from this many assignments on, times pieces per edge over 1.5
+# (random), or 1.25 (without pieces), or 1.5 (explicit).
 _SCORE_TABLE_FROM = 131072
-_SCORE_TABLE_PIECES, _SCORE_TABLE_EXPLICIT = 1.5, 1.5
+_SCORE_TABLE_PIECES, _SCORE_TABLE_EDGES, _SCORE_TABLE_EXPLICIT = 1.5, 1.25, 1.5
 _SCORE_PER_LANE = 0  # assignments per lane of the compact scorer; 0: the library chooses
 # Assignments from which one lane each beats several wavefronts per 64 assignments, by the number
 # of wavefronts.  Lanes go in rounds of 2^18 that cost the same however full, wavefronts by the
@@ -805,12 +809,16 @@ class CostEngine:
         if from_table and large and count >= table_from and self._versioned:
             if assign is not None:
                 table_from *= _SCORE_TABLE_EXPLICIT
-            elif _SCORE_STREAM:
-                counts = self._layout("piece_counts", first_node, lambda: piece_counts(g, self._matrix_sizes(), first_node))
+            else:
+                counts = None
+                if _SCORE_STREAM:
+                    counts = self._layout("piece_counts", first_node, lambda: piece_counts(g, self._matrix_sizes(), first_node))
                 if counts is not None:
                     table_from *= max(1.0, counts[0] / counts[1] / _SCORE_TABLE_PIECES)
                     if count >= table_from:  # else the list need not be made
                         pieces = self._score_pieces(first_node)
+                if pieces is None:
+                    table_from = max(table_from, _SCORE_TABLE_FROM * _SCORE_TABLE_EDGES)
         if from_table and large and count >= table_from:
             if pieces is not None:
                 d_pieces, n_piece, n_item = pieces
