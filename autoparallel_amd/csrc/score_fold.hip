@@ -7,9 +7,9 @@
 // one record per edge and per node with all a pair needs, and nothing is waited for where it is asked for: records a tile
 // (with explicit choices two) ahead, choices a tile ahead, and a tile's terms are formed while the next tile's
 // entries are on their way.
-// Measured, MI355X, fields and records, us: 2 000 random assignments of the 12-layer GPT-2 graph 50 -> 36, of the
-// Llama-3-8B graph 143 -> 115, 100 93 -> 66, 32 768 1 188 -> 650; 16 384 explicit ones of a 1 600-node window of the
-// planner DAG 811 -> 567, 2 000 165 -> 131.  What bounds it: few assignments, the chain of additions (4.6 ns a term, of
+// Measured, MI355X, fields and records, us: 2 000 random assignments of the 12-layer GPT-2 graph 50 -> 33, of the
+// Llama-3-8B graph 143 -> 94, 100 93 -> 64, 32 768 1 188 -> 629; 16 384 explicit ones of a 1 600-node window of the
+// planner DAG 811 -> 567, 2 000 165 -> 126.  What bounds it: few assignments, the chain of additions (4.6 ns a term, of
 // which 3.6 are the addition's latency); 2 000 and more, the gathering lanes' instructions (0.43 busy at 2 000, three
 // hashes per edge and node); explicit ones on large blocks, the misses of a draw's entry.
 #include "apc_device.h"
@@ -110,10 +110,14 @@ score_terms_kernel(const FoldEdge* __restrict__ edges, int n_edges, const FoldNo
       const int row = row_of(t, u);
       const u32x4_t* const e = reinterpret_cast<const u32x4_t*>(edges + max(min(row, n_edges - 1), 0));
       Rec r;
+      // The node's record in front of the edge's where 4 to 32 lanes read the same ones: 2 000, 4 000 and 8 000 random
+      // assignments of the Llama-3-8B graph 113, 195 and 353 -> 93, 162 and 301 us, but 16 000 489 -> 504.
+      constexpr bool kNodeFirst = kShift >= 2 && kShift < 6;
+      if (kNodeFirst) r.n = *reinterpret_cast<const u32x4_t*>(nodes + min(row, n_nodes - 1));
       r.e[0] = e[0];
       r.e[1] = e[1];
       r.e[2] = e[2];
-      r.n = *reinterpret_cast<const u32x4_t*>(nodes + min(row, n_nodes - 1));
+      if (!kNodeFirst) r.n = *reinterpret_cast<const u32x4_t*>(nodes + min(row, n_nodes - 1));
       return r;
     };
     auto draw = [&](uint32_t key, uint32_t nstrat) -> uint32_t {  // plain_draw by the node's key
