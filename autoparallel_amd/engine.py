@@ -742,42 +742,45 @@ class CostEngine:
         args = (C.byref(self.problem), self._ptr(self.per_arg), self._ptr(self.comm), self._ptr(self.cost),
                 self._ptr(self.flags))
         if assign is not None:
-            self._launch_score(
-                "apc_score_assignments_window",
+            self.last_score_entry = "apc_score_assignments_window"
+            rc = self.lib.apc_score_assignments_window(
                 *args, self._ptr(assign), int(count), int(first_node), self._ptr(init), self._ptr(out), stream)
         elif d_gid is None:
-            self._launch_score(
-                "apc_score_random_assignments",
-                *args, int(seed), int(first), int(count), self._ptr(out), stream)
+            self.last_score_entry = "apc_score_random_assignments"
+            rc = self.lib.apc_score_random_assignments(*args, int(seed), int(first), int(count), self._ptr(out), stream)
         else:
-            self._launch_score(
-                "apc_score_random_window",
+            self.last_score_entry = "apc_score_random_window"
+            rc = self.lib.apc_score_random_window(
                 *args, int(seed), int(first), int(count), self._ptr(d_gid), int(first_node), self._ptr(init),
                 self._ptr(out), stream)
+        _lib.check(rc, self.last_score_entry)
         self.last_score_backend = "entry_arrays"
         return out
 
     def _score_terms(self, clamp, assign, seed, first, count, d_gid, first_node, init, out, stream) -> torch.Tensor:
         g = self.g
         first_edge = int(g.node_edge_off[first_node])
-        rows = max(g.num_edges - first_edge, g.num_nodes - first_node)
-        few = next((most[2 if self.large_blocks else 1] for most in _SCORE_TERM_FIELDS_UP_TO if count <= most[0]), 0)
-        scratch = None
-        if _SCORE_TERM_RECORDS and rows > few and first_node < g.num_nodes and first_edge < g.num_edges:
-            scratch = self._scratch((g.num_edges - first_edge) * _lib.FOLD_EDGE_BYTES
-                                    + (g.num_nodes - first_node) * _lib.FOLD_NODE_BYTES)
+        n_edge, n_node = g.num_edges - first_edge, g.num_nodes - first_node
+        few, scratch = 0, None
+        for most, small, large in _SCORE_TERM_FIELDS_UP_TO:
+            if count <= most:
+                few = large if self.large_blocks else small
+                break
+        if _SCORE_TERM_RECORDS and n_edge > 0 and n_node > 0 and (n_edge > few or n_node > few):
+            scratch = self._scratch(n_edge * _lib.FOLD_EDGE_BYTES + n_node * _lib.FOLD_NODE_BYTES)
         if scratch is not None:
-            self._launch_score(
-                "apc_score_terms",
+            self.last_score_entry = "apc_score_terms"
+            rc = self.lib.apc_score_terms(
                 C.byref(self.problem), self._ptr(self.per_arg), self._ptr(self.table), self._ptr(scratch),
                 self._ptr(assign), int(seed), int(first), int(count), self._ptr(d_gid), int(first_node), first_edge,
                 clamp, self._ptr(init), self._ptr(out), stream)
         else:
-            self._launch_score(
-                "apc_score_fold_table",
+            self.last_score_entry = "apc_score_fold_table"
+            rc = self.lib.apc_score_fold_table(
                 C.byref(self.problem), self._ptr(self.per_arg), self._ptr(self.table), self._ptr(assign), int(seed),
                 int(first), int(count), self._ptr(d_gid), int(first_node), clamp, self._ptr(init),
                 self._ptr(out), stream)
+        _lib.check(rc, self.last_score_entry)
         self.last_score_backend = "block_table_terms"
         return out
 
