@@ -51,12 +51,13 @@ _SCORE_STREAM = True  # random assignments on graphs with large blocks: matrices
 _SCORE_TERM_RECORDS = True  # terms side by side from records of the edges and nodes, made in front of them
 # But not where a graph is a few of the smallest batches' tiles: there the records' own launch costs more than it saves.
 # Up to so many (assignments; edges or nodes on graphs with small blocks; with large ones, whose entries a workgroup waits
-# for longer in the form without records) it is one launch.  In us, a call alone and among others, with records and
-# without: 1-layer GPT-2 graph (318 edges), random, 100 30.6, 15.7 and 25.9, 11.1, 1 000 28.9, 15.8 and 27.0, 11.2, 2 000 29.5,
-# 15.8 and 28.4, 12.6; 3 layers (786), 100 33.8, 16.3 and 31.1, 15.5, 1 000 33.3, 16.3 and 32.4, 16.7; 6 layers (1 488), explicit,
-# 100 40.5, 21.4 and 38.4, 22.1; 1-layer 70B decoder (318, 341 strategies), 100 31.1, 16.0 and 26.0, 10.8, 2 000 34.5, 17.5 and
-# 39.3, 20.8; 2 layers (583), 1 000 34.9, 17.9 and 36.6, 20.9.
-_SCORE_TERM_FIELDS_UP_TO = ((256, 1536, 1536), (1024, 800, 384), (2048, 384, 192))
+# for longer in the form without records) it is one launch.  In us, a call among others, from records and without: small
+# blocks, 1-layer GPT-2 graph (318 edges), random, 100 and 2 048 assignments 15.6, 10.6 and 15.6, 12.9; 2 layers (552), 1 024 and
+# 1 500 15.5, 14.2 and 15.4, 16.3; 3 layers (786), 600 and 1 024 15.7, 16.0 and 15.8, 16.8; 4 layers (1 020), 256 17.8, 17.4;
+# 5-layer Llama-3-8B graph (1 378), 100 19.9, 20.8.  Large blocks, 1-layer 70B decoder (318), 100, 1 024 and 1 500 15.6, 10.5
+# and 15.5, 14.8 and 16.0, 18.2; windows of the planner DAG of 60 nodes (102), 100 and 2 048 34.2, 30.4 and 34.5, 33.3, of 140
+# (255), 600 and 1 024 35.3, 34.9 and 36.2, 37.2, of 300 (559), 256 38.2, 40.0.
+_SCORE_TERM_FIELDS_UP_TO = ((256, 1152, 512), (640, 640, 320), (1024, 640, 192), (2048, 384, 192))
 # Matrices of up to this many LDS tiles (64 KB each) go through LDS in the table scorer, larger
 # ones are read in place.  Measured on a 3 000-node window of the stress DAG, 2^20 assignments:
 # 17.9 ms with 1, 17.4 with 2, 18.0 with 4, 18.35 with 8 or 16.  (A lower bound, small matrices

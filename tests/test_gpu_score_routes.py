@@ -16,7 +16,7 @@ GRAPHS = {
     "middling": lambda: graphgen.stress_graph(130, (2, 2, 4), seed=1, s_min=34, s_max=38),
     "smallest": lambda: graphgen.gpt2_graph((4,), 1, vocab=4096, seq=512, batch=64),
     "large": lambda: graphgen.stress_graph(60, (2, 2, 4), seed=1, s_min=95, s_max=110),  # two pieces a matrix
-    "larger": lambda: graphgen.stress_graph(240, (2, 2, 4), seed=1, s_min=95, s_max=100),
+    "larger": lambda: graphgen.stress_graph(200, (2, 2, 4), seed=1, s_min=95, s_max=100),
     "untiled": lambda: graphgen.stress_graph(30, (2, 2, 4), seed=1, s_min=2, s_max=150),  # small on average only
     "widest": lambda: graphgen.stress_graph(8, (2, 2, 4), seed=1, s_min=820, s_max=900),  # no list of pieces
 }
@@ -33,7 +33,7 @@ ROUTES = [
     ("smallest", "random", 257, "apc_score_fold_table"), ("smallest", "explicit", 1024, "apc_score_fold_table"),
     ("smallest", "carried", 2048, "apc_score_fold_table"), ("smallest", "random", 2049, "apc_score_terms"),
     ("large", "carried", 2048, "apc_score_fold_table"), ("large", "explicit", 2049, "apc_score_terms"),
-    ("larger", "random", 1024, "apc_score_fold_table"), ("larger", "random", 1025, "apc_score_terms"),
+    ("larger", "random", 640, "apc_score_fold_table"), ("larger", "random", 641, "apc_score_terms"),
     ("small", "random", 3000, "apc_score_terms"), ("small", "explicit", 3000, "apc_score_terms"),
     ("small", "random", 81920, "apc_score_terms"), ("small", "random", 81921, "apc_score_pairs"),
     ("middling", "random", 114688, "apc_score_terms"), ("middling", "random", 114689, "apc_score_images"),
