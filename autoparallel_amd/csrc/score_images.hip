@@ -8,7 +8,8 @@
 // know to ask for the next tile.  A copy is then consecutive memory, 4 KB per instruction group; explicit choices come
 // the same way, rows of 16 bits straight into LDS, a tile further ahead where three buffers fit (they come from memory,
 // and a tile lasts about as long as that takes); the words of an edge are in the lanes' registers (lane i: edge i) and
-// come from there with v_readlane; and eight edges are walked side by side without a branch.
+// come from there with v_readlane; and eight edges are walked side by side, with one branch per four, taken where one of them
+// is not of the common kind.
 // Measured, MI355X, Llama-3-8B graph (8 533 edges): 131 072 explicit assignments 5.7 -> 2.6 ms, 262 144 6.7 -> 3.8,
 // 131 072 random ones 4.8 -> 2.9; the images (43 MB) take 20 us of that.  What bounds it: at 262 144 about as much
 // the LDS (20 cycles of reads per edge and wavefront and the copies, half of the time) as instructions (0.5 busy; 41

@@ -12,10 +12,12 @@
 // (apc_score_pieces works out where and when): with one piece under way at a time a copy is its latency, 0.8 us a piece
 // whatever its size.
 // Measured, MI355X, window of the planner DAG of 1 600 nodes (2 967 edges, 194 MB of matrices), edge by edge and as a
-// stream: 131 072 random assignments 5.28 -> 4.09 ms, 524 288 6.41 -> 5.22, 2^20 8.93 -> 7.12.  What bounds it: at 131 072
-// the copies (3.2 ms by themselves: 0.9 us latency over the 75 KB that are under way beside a piece in use; four
-// consecutive buffers of 32 KB reach 1.8 ms), at 2^20 instructions, two hashes per edge and assignment first of all.
-// Not better: pieces of 44 KB (5.70 ms for 524 288), a piece asked for by one wavefront (6.06) or by all of them (6.40).
+// stream: calls with carried sums, repeated on one set of inputs, 196 608 random assignments 5.27 -> 4.21 ms, 524 288
+// 6.54 -> 5.48, 2^20 9.48 -> 7.40; on inputs that change from call to call, so that the matrices come from memory,
+// 524 288 7.3 -> 5.9.  What bounds it: with the fewest lanes the copies (3.2 ms by themselves: 0.9 us latency over the
+// 75 KB that are under way beside a piece in use; four consecutive buffers of 32 KB reach 1.8 ms), at 2^20 instructions,
+// two hashes per edge and assignment first of all.  Not better, at 524 288: pieces of 44 KB (9% longer), a piece asked for
+// by one wavefront (16%) or by all of them (23%).
 // Sums run in node order, then argument order, as in score_kernel: the same bits.
 #include <algorithm>
 

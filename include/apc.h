@@ -754,9 +754,9 @@ int apc_score_fold_table(const apc_problem* p, const double* per_arg, const doub
                          uint64_t seed, int64_t first, int64_t n_assign, const int32_t* node_gid, int32_t first_node,
                          int32_t clamp_inf, const double* init, double* out, void* stream);
 
-/* The same from records of edges and nodes, which a launch in front makes: first_edge is node_edge_off[first_node],
- * below n_edge, and first_node below n_node.  scratch: 16-byte aligned, 48 bytes per edge from first_edge on and 16 per node
- * from first_node on. */
+/* The same from records of edges and nodes, which a launch in front makes (1 to 64 assignments a workgroup): first_edge is
+ * node_edge_off[first_node], below n_edge, and first_node below n_node.  scratch: 16-byte aligned, 48 bytes per edge from
+ * first_edge on and 16 per node from first_node on. */
 int apc_score_terms(const apc_problem* p, const double* per_arg, const double* table, void* scratch,
                     const uint16_t* assign, uint64_t seed, int64_t first, int64_t n_assign, const int32_t* node_gid,
                     int32_t first_node, int32_t first_edge, int32_t clamp_inf, const double* init, double* out,
