@@ -74,6 +74,21 @@ _SCORE_STAGE_TILES = 2
 # (random), or 1.25 (without pieces), or 1.5 (explicit).
 _SCORE_TABLE_FROM = 131072
 _SCORE_TABLE_PIECES, _SCORE_TABLE_EDGES, _SCORE_TABLE_EXPLICIT = 1.5, 1.25, 1.5
+# But random ones edge by edge where many matrices are more than two tiles: the stream copies every piece of them to each CU,
+# edge by edge they are read in place, an entry a draw, which is little while few assignments share them.  What an edge
+# takes, us: as a stream, a piece and, at 2^20 assignments, the draws on top; edge by edge, at least, a tile, a matrix in
+# place, and on top at 2^20, in all, for a matrix in place, and, by the square, where nearly all are (no copies then keep
+# the CUs at the same matrix).  Terms, ns for an edge and 1 000 assignments: at least, with a
+# matrix, and for each MB of the block table, at most so much.  In ms, terms, stream and edge by edge, at 131 072, 262 144, 524 288
+# and 2^20: 2-layer 70B decoder on 2x2x4 (2.9 pieces an edge, 0.41 in place, 21 MB) 0.56, 1.51, 0.97 and 1.13, 1.58, 0.97 and
+# 2.34, 1.76, 1.26 and 4.76, 2.16, 1.88; 8 layers of it, compressed (2.3, 0.25, 16 MB) 2.06, 4.53, 3.99 and 4.03, 4.77, 3.99 and
+# 8.01, 5.38, 4.98 and 16.0, 6.74, 7.18; 300-node DAG, not compressed, 140 to 170 strategies (3.4, 1.0, 79 MB) 0.63, 1.33, 0.65 and
+# 1.43, 1.40, 0.64 and 3.06, 1.53, 1.26 and 6.35, 1.84, 3.59 (786 432: 4.71, 1.70, 2.66); 95 to 110 (2.0, 0, 35 MB) 0.48, 0.70, 0.98 and 1.17, 0.75, 1.00 and
+# 2.65, 0.88, 1.12 and 5.63, 1.16, 1.38; compressed, 250 to 300 (1.8, 0.24, 23 MB) 0.35, 0.47, 0.54 and 0.70, 0.50, 0.55 and
+# 1.44, 0.58, 0.68 and 2.94, 0.75, 0.98; 400-node window of the planner DAG, not compressed (5.1, 0.41, 429 MB) 1.68, 9.83, 2.52
+# and 3.65, 9.90, 2.51 and 7.87, 10.2, 3.42 and 16.3, 11.1, 5.42.
+_SCORE_STREAM_US, _SCORE_TABLE_US = (0.92, 1.15), (1.05, 0.7, 0.85, 1.1, 1.7, 3.5)
+_SCORE_TERMS_NS = (2.2, 4.5, 0.05, 8.0)
 _SCORE_PER_LANE = 0  # assignments per lane of the compact scorer; 0: the library chooses
 # Assignments from which one lane each beats several wavefronts per 64 assignments, by the number
 # of wavefronts.  Lanes go in rounds of 2^18 that cost the same however full, wavefronts by the
@@ -151,6 +166,22 @@ def piece_counts(g: PackedGraph, size: np.ndarray, first_node: int):
     pieces = np.maximum(size[first_edge:] + (_lib.SCORE_PIECE - 1), _lib.SCORE_PIECE) // _lib.SCORE_PIECE
     bare = int((np.diff(g.node_edge_off[first_node:]) == 0).sum())
     return int(pieces.sum()) + bare, len(pieces) + bare
+
+
+def large_block_costs(counts, size: np.ndarray, tile: int, table_mb: float):
+    """What an edge of the walk takes by the three ways of scoring random assignments on large blocks, up to 2^18 and
+    what a batch of 2^20 adds (lanes take several): ((stream, on top), (edge by edge, on top, and by the square)), us, and the
+    terms, ns for 1 000 of them.  ``counts``: piece_counts; ``size``: matrix_sizes of the walk's edges; ``tile``: elements of an LDS tile."""
+    n_piece, n_item = counts
+    staged = size <= _SCORE_STAGE_TILES * tile
+    tiles = int((-(-size[staged] // tile)).sum()) / n_item
+    matrices, in_place = int((size > 0).sum()) / n_item, int((~staged).sum()) / n_item
+    least, per_tile, per_in_place, top, top_in_place, top_all_in_place = _SCORE_TABLE_US
+    terms, per_matrix, per_mb, most_mb = _SCORE_TERMS_NS
+    return ((_SCORE_STREAM_US[0] * n_piece / n_item, _SCORE_STREAM_US[1]),
+            (least + per_tile * tiles + per_in_place * in_place, top + top_in_place * in_place,
+             top_all_in_place if in_place > 0.9 * matrices else 0.0),
+            terms + matrices * (per_matrix + min(most_mb, per_mb * table_mb)))
 
 
 def make_model(mesh_shape, devices_per_host: int, device_name: str, order_mode: int = 0,
@@ -303,7 +334,7 @@ class CostEngine:
 
         self._keep: Dict[str, torch.Tensor] = {}
         self._layouts: Dict[str, dict] = {"score_tiles": {}, "score_tiles_explicit": {}, "sample_steps": {},
-                                          "score_pieces": {}, "piece_counts": {}, "sample_tiles": {}, "pair_tiles": {}}
+                                          "score_pieces": {}, "piece_counts": {}, "large_block_costs": {}, "sample_tiles": {}, "pair_tiles": {}}
 
         # The problem is some thirty arrays, most of them a few kilobytes: they go up in
         # one copy.  An array is laid into a pinned staging buffer and gets its address
@@ -788,8 +819,8 @@ class CostEngine:
     def _score_packed(self, assign, seed, first, count, d_gid, first_node, init, out) -> torch.Tensor:
         """Scoring of a large batch.  A graph with large blocks: from the block
         table while the entry arrays are what the last build made of it
-        (apc_score_stream, or apc_score_table for explicit assignments and more strategies than that takes; 5x the
-        rate of any walk over records there).  Else,
+        (apc_score_stream, or apc_score_table for explicit assignments, more strategies than that takes, and where
+        large_block_costs says so; 5x the rate of any walk over records there).  Else,
         and for graphs with small blocks: up to _SCORE_TERMS_UP_TO_IMAGES assignments with
         the terms gathered side by side from the table (apc_score_terms), from
         there on by tiles of edges (random ones apc_score_pairs: 7.2 ms for 2^20 assignments of the Llama-3-8B graph,
@@ -817,11 +848,14 @@ class CostEngine:
                 counts = None
                 if _SCORE_STREAM:
                     counts = self._layout("piece_counts", first_node, lambda: piece_counts(g, self._matrix_sizes(), first_node))
-                if counts is not None:
+                edge_by_edge_us = self._edge_by_edge_us(counts, first_node, count, capturing)
+                if edge_by_edge_us is not None:
+                    table_from = max(table_from, 1e6 * edge_by_edge_us[0] / edge_by_edge_us[1])
+                elif counts is not None:
                     table_from *= max(1.0, counts[0] / counts[1] / _SCORE_TABLE_PIECES)
                     if count >= table_from:  # else the list need not be made
                         pieces = self._score_pieces(first_node)
-                if pieces is None:
+                if pieces is None and edge_by_edge_us is None:
                     table_from = max(table_from, _SCORE_TABLE_FROM * _SCORE_TABLE_EDGES)
         if from_table and large and count >= table_from:
             if pieces is not None:
@@ -1012,6 +1046,21 @@ class CostEngine:
         """(apc_score_piece records on the device, pieces, items) of apc_score_stream for the walk from
         ``first_node`` on, or None: a node with too many strategies, nothing to score, or no layout at hand."""
         return self._layout("score_pieces", first_node, lambda: self._make_score_pieces(first_node))
+
+    def _edge_by_edge_us(self, counts, first_node: int, count: int, capturing: bool):
+        """(us an edge, ns the terms of one take for 1 000 assignments) where ``count`` random assignments are faster from the
+        table edge by edge than as a stream of the pieces of ``counts``, else None."""
+        if counts is None or (capturing and "score_edge_aux" not in self._keep):  # its records cannot be made meanwhile
+            return None
+        costs = self._layout("large_block_costs", first_node, lambda: large_block_costs(
+            counts, self._matrix_sizes()[self.g.node_edge_off[first_node]:], int(self.lib.apc_score_table_tile()),
+            self.table.numel() * 8e-6))
+        if costs is None:
+            return None
+        (stream, stream_top), (table, table_top, table_top2), terms = costs
+        filled = max(min(count, 1 << 20) - (1 << 18), 0) / ((1 << 20) - (1 << 18))
+        table += (table_top + table_top2 * filled) * filled
+        return (table, terms) if table < stream + stream_top * filled else None
 
     def _matrix_sizes(self) -> np.ndarray:
         if "matrix_sizes" not in self._keep:

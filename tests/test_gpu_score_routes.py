@@ -18,6 +18,7 @@ GRAPHS = {
     "large": lambda: graphgen.stress_graph(60, (2, 2, 4), seed=1, s_min=95, s_max=110),  # two pieces a matrix
     "larger": lambda: graphgen.stress_graph(200, (2, 2, 4), seed=1, s_min=95, s_max=100),
     "untiled": lambda: graphgen.stress_graph(30, (2, 2, 4), seed=1, s_min=2, s_max=150),  # small on average only
+    "in_place": lambda: graphgen.stress_graph(40, (2, 2, 4), seed=1, s_min=140, s_max=170),  # three or four pieces a matrix
     "widest": lambda: graphgen.stress_graph(8, (2, 2, 4), seed=1, s_min=820, s_max=900),  # no list of pieces
 }
 
@@ -45,6 +46,8 @@ ROUTES = [
     ("large", "random", 131072, "apc_score_terms"), ("large", "carried", 131072, "apc_score_terms"),
     ("large", "random", 262144, "apc_score_stream"), ("large", "carried", 262144, "apc_score_stream"),
     ("large", "explicit", 196607, "apc_score_terms"), ("large", "explicit", 196608, "apc_score_table"),
+    ("in_place", "random", 240000, "apc_score_terms"), ("in_place", "random", 300000, "apc_score_table"),
+    ("in_place", "carried", 300000, "apc_score_table"), ("in_place", "random", 1 << 20, "apc_score_stream"),
     ("widest", "random", 163839, "apc_score_terms"), ("widest", "random", 163840, "apc_score_table"),
     ("widest", "carried", 163839, "apc_score_terms"), ("widest", "carried", 163840, "apc_score_table"),
     ("untiled", "random", 131072, "apc_score_terms"), ("untiled", "random", 131073, "apc_score_compact"),

@@ -26,12 +26,13 @@ def E():
 @pytest.fixture()
 def knobs(E):
     saved = (E._SCORE_FROM_TABLE, E._SCORE_COMPACT, E._SCORE_STAGE_TILES, E._SCORE_PER_LANE, E._SCORE_TABLE_FROM,
-             E._SCORE_LANES_FROM, E._SCORE_STREAM)
+             E._SCORE_LANES_FROM, E._SCORE_STREAM, E._SCORE_TABLE_US)
     # the table scorer and the record walks whatever the batch size, where a test asks for them
     E._SCORE_TABLE_FROM = 0
+    E._SCORE_TABLE_US = (1e9, 0, 0, 0, 0, 0)  # the stream, unless it is switched off
     yield E
     (E._SCORE_FROM_TABLE, E._SCORE_COMPACT, E._SCORE_STAGE_TILES, E._SCORE_PER_LANE, E._SCORE_TABLE_FROM,
-     E._SCORE_LANES_FROM, E._SCORE_STREAM) = saved
+     E._SCORE_LANES_FROM, E._SCORE_STREAM, E._SCORE_TABLE_US) = saved
 
 
 def _same(a, b):
