@@ -122,6 +122,11 @@ def xgmi_config_struct(cfg) -> _lib.ApcXgmiConfig:
     """apc_xgmi_config from any object with XGMITopoConfig's fields."""
     if isinstance(cfg, _lib.ApcXgmiConfig):
         return cfg
+# Nor on the smallest graphs, where two wavefronts have few steps.  In all and a step, and the assignments up to which that
+# holds (beyond, it grows with them).  In us, among others, tiles and two wavefronts, 16 384, 65 536, 131 072 and 196 608: random
+# DAG of 30 nodes (16 steps) 25.6, 17.6 and 26.5, 18.6 and 30.2, 25.0 and 32.5, 37.3, of 60 33.7, 29.7 and 35.4, 31.2 and 40.7,
+# 44.0 and 47.0, 67.5, of 100 46.8, 45.8 and 49.6, 48.2; 1-layer GPT-2 graph (243 nodes, 122 steps) 88.5, 101.4.
+_SAMPLE_TWO_US, _SAMPLE_TWO_UP_TO = (13.0, 0.85), 100000
     c = _lib.ApcXgmiConfig()
     c.gpus_per_node, c.links_per_gpu = int(cfg.gpus_per_node), int(cfg.links_per_gpu)
     c.link_gbps, c.nic_gbps = float(cfg.link_gbps), float(cfg.nic_gbps)
@@ -1266,12 +1271,19 @@ class CostEngine:
                 n_tile.value, int(nstrat[first_node:].max() > 32), int(tiles[0].view(np.int32)[_lib.SAMPLE_TILE_DEPTH]))
 
     def _steps_before_tiles(self, first_node: int, count: int, tiles):
-        """_sample_steps where sixteen wavefronts in steps are faster than ``tiles``, else None."""
+        """_sample_steps where sixteen wavefronts in steps, or two on the smallest graphs, are faster than ``tiles``, else
+        None."""
         n, n_edge = self.g.num_nodes - first_node, self.g.num_edges - int(self.g.node_edge_off[first_node])
         n_tile, depth = tiles[2], tiles[4]
         by_tiles = _SAMPLE_TILES_US[0] + _SAMPLE_TILES_US[1] * n + _SAMPLE_TILES_US[2] * n_tile
         step = -(-count // 16384) * (_SAMPLE_STEP_US[0] + _SAMPLE_STEP_US[1] * n_edge / n)
-        if n < 6 * depth or max(depth, n / 16) * step >= by_tiles:  # two wavefronts, or too many steps in any layout
+        if n < 6 * depth:  # two wavefronts
+            two = _SAMPLE_TWO_US[1] * max(1.0, count / _SAMPLE_TWO_UP_TO)
+            if _SAMPLE_TWO_US[0] + two * max(depth, n / 2) >= by_tiles:
+                return None
+            steps = self._sample_steps(first_node)
+            return steps if steps is not None and _SAMPLE_TWO_US[0] + two * steps[1] < by_tiles else None
+        if max(depth, n / 16) * step >= by_tiles:  # too many steps in any layout
             return None
         steps = self._sample_steps(first_node)
         return steps if steps is not None and steps[2] == 16 and steps[1] * step < by_tiles else None

@@ -127,15 +127,18 @@ def test_draws_equal_the_lane_walks(name, count, monkeypatch):
         assert max(int(f.max()) for f in want[1::2]) > 0  # nodes that fall back do occur
 
 
-# small batches of a graph with work for sixteen wavefronts go in steps, larger ones and decoders by tiles; the same draws
+# small batches of a graph with work for sixteen wavefronts go in steps, larger ones and decoders by tiles, the smallest
+# graphs in steps of two; the same draws
 @pytest.mark.gpu
 @pytest.mark.parametrize("name,first_node,count,route", [
     ("dag", 0, 100, "steps"), ("dag", 0, 16385, "steps"), ("dag", 0, 49152, "steps"), ("dag", 0, 49153, "tiles"),
-    ("dag", 90, 33, "steps"), ("small_dag", 0, 32768, "steps"), ("small_dag", 0, 65537, "tiles"), ("gpt2", 0, 1, "tiles"),
+    ("dag", 90, 33, "steps"), ("small_dag", 0, 32768, "steps"), ("small_dag", 0, 65537, "tiles"), ("smallest_dag", 0, 65536, "steps"),
+    ("smallest_dag", 0, 131072, "steps"), ("smallest_dag", 0, 196608, "tiles"), ("gpt2", 0, 1, "tiles"),
     ("llama_8x8", 0, 65, "tiles")])
 def test_which_graphs_are_drawn_in_steps(name, first_node, count, route, monkeypatch):
     g = {"dag": lambda: graphgen.stress_graph(400, (2, 2, 4), seed=1, s_min=2, s_max=20),
          "small_dag": lambda: graphgen.stress_graph(60, (2, 2, 4), seed=1, s_min=2, s_max=20),
+         "smallest_dag": lambda: graphgen.stress_graph(30, (2, 2, 4), seed=1, s_min=2, s_max=20),
          **{k: lambda k=k: GRAPHS[k]()[0] for k in GRAPHS}}[name]()
     eng = engine_mod.CostEngine(g).build()
     gen = torch.Generator(device="cuda").manual_seed(count)
