@@ -42,6 +42,13 @@ _SCORE_TERMS_UP_TO_IMAGES = {"random": 114688, "explicit": 81920}
 # 2^20 7.24, 10.41; MoE graph (6.0), 131 072 1.59, 1.57, 1.53.
 _SCORE_PAIRS = True
 _SCORE_PAIRS_FROM, _SCORE_PAIRS_ROWS = (81920, 131072), 8
+# Not where a graph is a few tiles, which the walks without images in front go through meanwhile.  In us, finished entries,
+# tile images and lanes of several, at 131 072, 262 144 and 2^20: random DAG of 39 edges (5 tiles of finished entries, 3 of
+# images) 28.6, 23.2, 28.1 and 35.0, 30.5, 29.5 and 64.1, 94.9, 56.4, of 61, 524 288 55.2 and, lanes of several, 51.5, of 84
+# (11, 8) 40.2, 39.1, 51.0 and 51.9, 56.8, 51.6 and 103, 200, 116.  Explicit ones beyond 2^18, tile images and lanes of several,
+# 524 288 and 2^20: 39 edges 52.2, 43.6 and 92.4, 83.7, 84 (8 tiles) 94.7, 85.0 and 177, 168, 138 (13) 138, 138.  And explicit
+# ones up to 114 688 go by their terms where a tile has few edges: 100-node DAG of 10 to 60 strategies (3.4), 98 304 98 and 67.
+_SCORE_PAIRS_TILES, _SCORE_IMAGES_TILES, _SCORE_IMAGES_EDGES = 10, 12, 4
 # Else, random assignments up to which tile images are walked with a lane each; beyond, lanes take two or four, which
 # share a tile's draws of far producers and unpacking.  In ms, images and lanes of several, at 196 608 and 262 144:
 # Llama-3-8B graph 3.65, 4.59 and 4.48, 4.68; 12-layer GPT-2 graph 1.06, 1.31 and 1.31, 1.21.  Explicit ones at any number: at
@@ -889,7 +896,7 @@ class CostEngine:
                 assign is None and init is None and count > _SCORE_PAIRS_FROM[
                     0 if g.num_entries * _SCORE_PAIRS_ROWS <= g.num_edges * _lib.PAIR_TILE_UNITS else 1]):
             pairs = self._pair_tiles(first_node)
-            if pairs is not None:
+            if pairs is not None and pairs[3] >= _SCORE_PAIRS_TILES:
                 steps, n_step, d_tiles, n_tile = pairs
                 scratch = self._scratch((n_tile + 1) * _lib.PAIR_IMAGE_BYTES)
                 if scratch is not None:
@@ -903,7 +910,11 @@ class CostEngine:
         terms_up_to, kind = -1, "random" if assign is None else "explicit"
         if _SCORE_SMALL_FROM_TABLE and _SCORE_TERMS_ABOVE:
             terms_up_to = _SCORE_TERMS_UP_TO_IMAGES[kind]
-        if from_table and _SCORE_FROM_TILES and not self.large_blocks and count > terms_up_to:
+        by_tiles = from_table and _SCORE_FROM_TILES and not self.large_blocks and count > terms_up_to
+        if by_tiles and assign is not None and terms_up_to >= 0 and count <= _SCORE_TERMS_UP_TO_IMAGES["random"]:
+            tiles = self._score_tiles(first_node, True)
+            by_tiles = tiles is None or self._walk_from(first_node)[1] >= tiles[3] * _SCORE_IMAGES_EDGES
+        if by_tiles:
             name, scratch = "apc_score_images", None
             if assign is not None or count <= _SCORE_IMAGES_UP_TO:
                 tiles = self._score_tiles(first_node, True)
@@ -911,7 +922,7 @@ class CostEngine:
                     scratch = self._scratch((tiles[3] + 1) * _lib.SCORE_IMAGE_BYTES)
             if scratch is None:
                 name, tiles = "apc_score_from_tiles", self._score_tiles(first_node, assign is not None)
-                if tiles is not None:
+                if tiles is not None and (tiles[3] >= _SCORE_IMAGES_TILES or count <= 1 << 18):
                     scratch = self._scratch(tiles[1] * _lib.SCORE_STEP_BYTES)
             if scratch is not None:
                 steps, n_step, d_tiles, n_tile, units = tiles

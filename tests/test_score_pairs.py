@@ -100,6 +100,7 @@ def test_scores_have_the_bits_of_the_walk_over_records(name, count, monkeypatch)
 
     monkeypatch.setattr(engine_mod, "_SCORE_LANES_FROM", 1)
     monkeypatch.setattr(engine_mod, "_SCORE_TERMS_ABOVE", False)
+    monkeypatch.setattr(engine_mod, "_SCORE_PAIRS_TILES", 1)
     monkeypatch.setattr(engine_mod, "_SCORE_PAIRS_FROM", (0, 0))
     for mult in (np.ones(g.num_nodes, np.int32), np.arange(g.num_nodes, dtype=np.int32) % 3 - 1):
         eng.set_node_multiplier(mult)  # the layout is kept, the multipliers are the call's

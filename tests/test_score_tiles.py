@@ -136,6 +136,8 @@ def test_scores_have_the_bits_of_the_walk_over_records(name, count, room, monkey
 
     monkeypatch.setattr(engine_mod, "_SCORE_LANES_FROM", 1)
     monkeypatch.setattr(engine_mod, "_SCORE_TERMS_ABOVE", False)
+    monkeypatch.setattr(engine_mod, "_SCORE_PAIRS_TILES", 1)
+    monkeypatch.setattr(engine_mod, "_SCORE_IMAGES_TILES", 1)
     by_entry = {  # random, explicit, and both with carried sums
         "images": ("apc_score_images" if count <= 131072 else "apc_score_pairs", "apc_score_images",
                    "apc_score_images" if count <= 196608 else "apc_score_from_tiles", "apc_score_images"),
@@ -190,6 +192,8 @@ def test_images_have_the_bits_of_the_walk_over_records(name, count, skip, monkey
 
     monkeypatch.setattr(engine_mod, "_SCORE_LANES_FROM", 1)
     monkeypatch.setattr(engine_mod, "_SCORE_TERMS_ABOVE", False)
+    monkeypatch.setattr(engine_mod, "_SCORE_PAIRS_TILES", 1)
+    monkeypatch.setattr(engine_mod, "_SCORE_IMAGES_TILES", 1)
     monkeypatch.setattr(engine_mod, "_SCORE_IMAGES_UP_TO", 1 << 20)
     monkeypatch.setattr(engine_mod, "_SCORE_PAIRS", False)
     got = scores("block_table_tiles")
