@@ -64,7 +64,11 @@ _SCORE_TERM_RECORDS = True  # terms side by side from records of the edges and n
 # 5-layer Llama-3-8B graph (1 378), 100 19.9, 20.8.  Large blocks, 1-layer 70B decoder (318), 100, 1 024 and 1 500 15.6, 10.5
 # and 15.5, 14.8 and 16.0, 18.2; windows of the planner DAG of 60 nodes (102), 100 and 2 048 34.2, 30.4 and 34.5, 33.3, of 140
 # (255), 600 and 1 024 35.3, 34.9 and 36.2, 37.2, of 300 (559), 256 38.2, 40.0.
-_SCORE_TERM_FIELDS_UP_TO = ((256, 1152, 512), (640, 640, 320), (1024, 640, 192), (2048, 384, 192))
+# Of the smallest graphs larger batches, too: random DAG of 11 edges, 32 768 and 65 536 13.7, 9.6 and 15.6, 12.3, of 39, 5 000,
+# 16 384 and 32 768 14.0, 11.5 and 14.0, 9.7 and 14.0, 11.2, of 61, 32 768 16.2, 13.6, of 84, 16 384 and 32 768 14.1, 12.1 and
+# 13.9, 17.6, of 138, 5 000 15.2, 16.7; large blocks, 39, 5 000 and 16 384 13.7, 11.9 and 13.6, 10.0.
+_SCORE_TERM_FIELDS_UP_TO = ((256, 1152, 512), (640, 640, 320), (1024, 640, 192), (2048, 384, 192), (16384, 96, 96), (32768, 64, 48),
+                               (65536, 16, 16))
 # Matrices of up to this many LDS tiles (64 KB each) go through LDS in the table scorer, larger
 # ones are read in place.  Measured on a 3 000-node window of the stress DAG, 2^20 assignments:
 # 17.9 ms with 1, 17.4 with 2, 18.0 with 4, 18.35 with 8 or 16.  (A lower bound, small matrices
@@ -90,8 +94,8 @@ _SCORE_TABLE_PIECES, _SCORE_TABLE_EDGES, _SCORE_TABLE_EXPLICIT = 1.5, 1.25, 1.5
 # and 2^20: 2-layer 70B decoder on 2x2x4 (2.9 pieces an edge, 0.41 in place, 21 MB) 0.56, 1.51, 0.97 and 1.13, 1.58, 0.97 and
 # 2.34, 1.76, 1.26 and 4.76, 2.16, 1.88; 8 layers of it, compressed (2.3, 0.25, 16 MB) 2.06, 4.53, 3.99 and 4.03, 4.77, 3.99 and
 # 8.01, 5.38, 4.98 and 16.0, 6.74, 7.18; 300-node DAG, not compressed, 140 to 170 strategies (3.4, 1.0, 79 MB) 0.63, 1.33, 0.65 and
-# 1.43, 1.40, 0.64 and 3.06, 1.53, 1.26 and 6.35, 1.84, 3.59 (786 432: 4.71, 1.70, 2.66); 95 to 110 (2.0, 0, 35 MB) 0.48, 0.70, 0.98 and 1.17, 0.75, 1.00 and
-# 2.65, 0.88, 1.12 and 5.63, 1.16, 1.38; compressed, 250 to 300 (1.8, 0.24, 23 MB) 0.35, 0.47, 0.54 and 0.70, 0.50, 0.55 and
+# 1.43, 1.40, 0.64 and 3.06, 1.53, 1.26 and 6.35, 1.84, 3.59 (786 432: 4.71, 1.70, 2.66); 95 to 110 (2.0, 0, 35 MB) 0.48, 0.70,
+# 0.98 and 1.17, 0.75, 1.00 and 2.65, 0.88, 1.12 and 5.63, 1.16, 1.38; compressed, 250 to 300 (1.8, 0.24, 23 MB) 0.35, 0.47, 0.54 and 0.70, 0.50, 0.55 and
 # 1.44, 0.58, 0.68 and 2.94, 0.75, 0.98; 400-node window of the planner DAG, not compressed (5.1, 0.41, 429 MB) 1.68, 9.83, 2.52
 # and 3.65, 9.90, 2.51 and 7.87, 10.2, 3.42 and 16.3, 11.1, 5.42.
 _SCORE_STREAM_US, _SCORE_TABLE_US = (0.92, 1.15), (1.05, 0.7, 0.85, 1.1, 1.7, 3.5)
@@ -118,6 +122,11 @@ _SAMPLE_TILES = True
 # 802, 792, 780, 782 and 247, 466, 685, 906, and of one, producers up to 20 back (81 steps), 264, 277, 268, 270 and 126, 222,
 # 325, 407.  The rule takes the shorter one at each of these.
 _SAMPLE_TILES_US, _SAMPLE_STEP_US = (24.0, 0.16, 3.0), (1.0, 0.3)
+# Nor on the smallest graphs, where two wavefronts have few steps.  In all and a step, and the assignments up to which that
+# holds (beyond, it grows with them).  In us, among others, tiles and two wavefronts, 16 384, 65 536, 131 072 and 196 608: random
+# DAG of 30 nodes (16 steps) 25.6, 17.6 and 26.5, 18.6 and 30.2, 25.0 and 32.5, 37.3, of 60 33.7, 29.7 and 35.4, 31.2 and 40.7,
+# 44.0 and 47.0, 67.5, of 100 46.8, 45.8 and 49.6, 48.2; 1-layer GPT-2 graph (243 nodes, 122 steps) 88.5, 101.4.
+_SAMPLE_TWO_US, _SAMPLE_TWO_UP_TO = (13.0, 0.85), 100000
 # Layouts of a kind (by first_node) an engine makes.  They stay until the engine goes, since a launch on
 # another stream or in a graph may still read one; calls beyond take the route that needs none.
 _LAYOUTS_KEPT = 16
@@ -129,11 +138,6 @@ def xgmi_config_struct(cfg) -> _lib.ApcXgmiConfig:
     """apc_xgmi_config from any object with XGMITopoConfig's fields."""
     if isinstance(cfg, _lib.ApcXgmiConfig):
         return cfg
-# Nor on the smallest graphs, where two wavefronts have few steps.  In all and a step, and the assignments up to which that
-# holds (beyond, it grows with them).  In us, among others, tiles and two wavefronts, 16 384, 65 536, 131 072 and 196 608: random
-# DAG of 30 nodes (16 steps) 25.6, 17.6 and 26.5, 18.6 and 30.2, 25.0 and 32.5, 37.3, of 60 33.7, 29.7 and 35.4, 31.2 and 40.7,
-# 44.0 and 47.0, 67.5, of 100 46.8, 45.8 and 49.6, 48.2; 1-layer GPT-2 graph (243 nodes, 122 steps) 88.5, 101.4.
-_SAMPLE_TWO_US, _SAMPLE_TWO_UP_TO = (13.0, 0.85), 100000
     c = _lib.ApcXgmiConfig()
     c.gpus_per_node, c.links_per_gpu = int(cfg.gpus_per_node), int(cfg.links_per_gpu)
     c.link_gbps, c.nic_gbps = float(cfg.link_gbps), float(cfg.nic_gbps)
@@ -183,7 +187,8 @@ def piece_counts(g: PackedGraph, size: np.ndarray, first_node: int):
 def large_block_costs(counts, size: np.ndarray, tile: int, table_mb: float):
     """What an edge of the walk takes by the three ways of scoring random assignments on large blocks, up to 2^18 and
     what a batch of 2^20 adds (lanes take several): ((stream, on top), (edge by edge, on top, and by the square)), us, and the
-    terms, ns for 1 000 of them.  ``counts``: piece_counts; ``size``: matrix_sizes of the walk's edges; ``tile``: elements of an LDS tile."""
+    terms, ns for 1 000 of them.  ``counts``: piece_counts; ``size``: matrix_sizes of the walk's edges; ``tile``: elements of
+    an LDS tile."""
     n_piece, n_item = counts
     staged = size <= _SCORE_STAGE_TILES * tile
     tiles = int((-(-size[staged] // tile)).sum()) / n_item
@@ -346,7 +351,8 @@ class CostEngine:
 
         self._keep: Dict[str, torch.Tensor] = {}
         self._layouts: Dict[str, dict] = {"score_tiles": {}, "score_tiles_explicit": {}, "sample_steps": {},
-                                          "score_pieces": {}, "piece_counts": {}, "large_block_costs": {}, "sample_tiles": {}, "pair_tiles": {}}
+                                          "score_pieces": {}, "piece_counts": {}, "large_block_costs": {},
+                                          "sample_tiles": {}, "pair_tiles": {}}
 
         # The problem is some thirty arrays, most of them a few kilobytes: they go up in
         # one copy.  An array is laid into a pinned staging buffer and gets its address
@@ -502,6 +508,7 @@ class CostEngine:
         # are large (_score_packed), else records made from the arrays on first use,
         # stale after anything rewrites the arrays.
         self.packed_scoring = g.num_edges > 0 and g.num_entries > 0
+        self._whole_walk = self._walk_from(0)
         self.large_blocks = g.num_edges > 0 and g.num_entries / g.num_edges >= _LARGE_BLOCKS_FROM
         self._recs: Optional[torch.Tensor] = None
         self._recs_valid = False
@@ -801,10 +808,14 @@ class CostEngine:
         self.last_score_backend = "entry_arrays"
         return out
 
+    def _walk_from(self, first_node: int):
+        """(first edge, edges, nodes) of the walk from ``first_node`` on."""
+        first_edge = int(self.g.node_edge_off[first_node])
+        return first_edge, self.g.num_edges - first_edge, self.g.num_nodes - first_node
+
     def _score_terms(self, clamp, assign, seed, first, count, d_gid, first_node, init, out, stream) -> torch.Tensor:
         g = self.g
-        first_edge = int(g.node_edge_off[first_node])
-        n_edge, n_node = g.num_edges - first_edge, g.num_nodes - first_node
+        first_edge, n_edge, n_node = self._whole_walk if first_node == 0 else self._walk_from(first_node)
         few, scratch = 0, None
         for most, small, large in _SCORE_TERM_FIELDS_UP_TO:
             if count <= most:
@@ -918,11 +929,11 @@ class CostEngine:
             name, scratch = "apc_score_images", None
             if assign is not None or count <= _SCORE_IMAGES_UP_TO:
                 tiles = self._score_tiles(first_node, True)
-                if tiles is not None:
+                if tiles is not None and (tiles[3] >= _SCORE_IMAGES_TILES or count <= 1 << 18):
                     scratch = self._scratch((tiles[3] + 1) * _lib.SCORE_IMAGE_BYTES)
             if scratch is None:
                 name, tiles = "apc_score_from_tiles", self._score_tiles(first_node, assign is not None)
-                if tiles is not None and (tiles[3] >= _SCORE_IMAGES_TILES or count <= 1 << 18):
+                if tiles is not None:
                     scratch = self._scratch(tiles[1] * _lib.SCORE_STEP_BYTES)
             if scratch is not None:
                 steps, n_step, d_tiles, n_tile, units = tiles

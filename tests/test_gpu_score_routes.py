@@ -14,6 +14,8 @@ pytestmark = pytest.mark.gpu
 GRAPHS = {
     "small": lambda: graphgen.gpt2_graph((4,), 4, vocab=4096, seq=512, batch=64),
     "middling": lambda: graphgen.stress_graph(130, (2, 2, 4), seed=1, s_min=34, s_max=38),
+    "tiny": lambda: graphgen.stress_graph(30, (2, 2, 4), seed=1, s_min=2, s_max=20),  # 39 edges, three tiles
+    "tiled": lambda: graphgen.stress_graph(100, (2, 2, 4), seed=1, s_min=10, s_max=60),  # 3.4 edges a tile
     "smallest": lambda: graphgen.gpt2_graph((4,), 1, vocab=4096, seq=512, batch=64),
     "large": lambda: graphgen.stress_graph(60, (2, 2, 4), seed=1, s_min=95, s_max=110),  # two pieces a matrix
     "larger": lambda: graphgen.stress_graph(200, (2, 2, 4), seed=1, s_min=95, s_max=100),
@@ -33,16 +35,20 @@ ROUTES = [
     ("small", "random", 256, "apc_score_fold_table"), ("small", "explicit", 257, "apc_score_terms"),
     ("smallest", "random", 257, "apc_score_fold_table"), ("smallest", "explicit", 1024, "apc_score_fold_table"),
     ("smallest", "carried", 2048, "apc_score_fold_table"), ("smallest", "random", 2049, "apc_score_terms"),
-    ("large", "carried", 2048, "apc_score_fold_table"), ("large", "explicit", 2049, "apc_score_terms"),
+    ("large", "carried", 16384, "apc_score_fold_table"), ("large", "explicit", 16385, "apc_score_terms"),
     ("larger", "random", 640, "apc_score_fold_table"), ("larger", "random", 641, "apc_score_terms"),
-    ("small", "random", 3000, "apc_score_terms"), ("small", "explicit", 3000, "apc_score_terms"),
+    ("tiny", "random", 16384, "apc_score_fold_table"), ("tiny", "explicit", 32768, "apc_score_fold_table"),
+    ("tiny", "carried", 32769, "apc_score_terms"), ("tiny", "random", 131072, "apc_score_images"),
+    ("tiny", "random", 196609, "apc_score_from_tiles"), ("tiny", "explicit", 262144, "apc_score_images"),
+    ("tiny", "explicit", 262145, "apc_score_from_tiles"), ("small", "random", 3000, "apc_score_terms"), ("small", "explicit", 3000, "apc_score_terms"),
     ("small", "random", 81920, "apc_score_terms"), ("small", "random", 81921, "apc_score_pairs"),
     ("middling", "random", 114688, "apc_score_terms"), ("middling", "random", 114689, "apc_score_images"),
     ("middling", "random", 131072, "apc_score_images"), ("middling", "random", 131073, "apc_score_pairs"),
     ("small", "carried", 114688, "apc_score_terms"), ("small", "carried", 114689, "apc_score_images"),
     ("small", "carried", 196608, "apc_score_images"), ("small", "carried", 196609, "apc_score_from_tiles"),
     ("small", "explicit", 81920, "apc_score_terms"), ("small", "explicit", 81921, "apc_score_images"),
-    ("small", "explicit", 262145, "apc_score_images"),
+    ("small", "explicit", 262145, "apc_score_images"), ("tiled", "explicit", 114688, "apc_score_terms"),
+    ("tiled", "explicit", 114689, "apc_score_images"),
     ("large", "random", 131072, "apc_score_terms"), ("large", "carried", 131072, "apc_score_terms"),
     ("large", "random", 262144, "apc_score_stream"), ("large", "carried", 262144, "apc_score_stream"),
     ("large", "explicit", 196607, "apc_score_terms"), ("large", "explicit", 196608, "apc_score_table"),
