@@ -94,3 +94,26 @@ def test_no_list_of_pieces_is_made_to_choose_the_terms():
     assert eng.last_score_entry == "apc_score_terms" and not eng._layouts["score_pieces"]
     eng.score_random(11, 5, 262144)
     assert eng.last_score_entry == "apc_score_stream" and eng._layouts["score_pieces"][0] is not None
+
+
+@pytest.mark.parametrize("eager,entry", [(300000, "apc_score_table"), (1 << 20, "apc_score_stream")])
+def test_a_recorded_batch_takes_the_walk_whose_layout_is_there(eager, entry):
+    """Nothing can be copied to the device meanwhile: edge by edge, where that is faster and its records were made, else the
+    stream, where its list was."""
+    count = 300000
+    eng = CostEngine(GRAPHS["in_place"](), table_mode="full").build()
+    eng.score_random(11, 5, eager)
+    assert eng.last_score_entry == entry
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        got = eng.score_random(11, 5, count)
+    assert eng.last_score_entry == entry
+    want = eng.score_random(11, 5, count)
+    assert eng.last_score_entry == "apc_score_table"
+    for _ in range(3):
+        got.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(got.view(torch.int64), want.view(torch.int64))
+        want = eng.score_random(11, 5, count)
